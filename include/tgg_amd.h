@@ -159,7 +159,9 @@ int tgg_m_grouped_gemm_fp8_out(const void* A, const void* B, void* codes, float*
  *   (what cub::DeviceRadixSort::SortPairs + moe_permute_topK_row_map produce, permute.cu:40-101, :541-548), or -1 when
  *   dropped or when the destination is >= num_out_tokens (0 = keep all).  tokens_per_expert (optional, int32 or int64
  *   [num_experts]) receives the per-expert row counts, i.e. the size_per_group argument of the grouped GEMMs.
- *   workspace: device memory of at least tgg_moe_sort_workspace_bytes(...) bytes, contents irrelevant before and after.
+ *   workspace: device memory of at least tgg_moe_sort_workspace_bytes(...) bytes, contents irrelevant before and after
+ *   (small problems need none: the function then reports 0 and the pointer may be null).
+ * tgg_moe_permute: tgg_moe_permute_map and tgg_moe_permute_rows in one call (one or two launches in all).
  * tgg_moe_permute_rows: permuted[row_id_map[k, t], :] = input[t, :] for every kept assignment.
  * tgg_moe_unpermute: output[t, :] = sum_k probs[t, k] * input[row_id_map[k, t], :] over kept assignments, fp32
  *   arithmetic, one rounding to the activation type (probs may be null: plain sum; also the backward of permute_rows).
@@ -169,6 +171,9 @@ int tgg_moe_sort_workspace_bytes(int64_t num_tokens, int topk, int num_experts, 
 int tgg_moe_permute_map(const int32_t* indices, int64_t num_tokens, int topk, int num_experts, int64_t num_out_tokens,
                         int32_t* row_id_map, void* tokens_per_expert, int counts_i64, void* workspace,
                         int64_t workspace_bytes, void* stream);
+int tgg_moe_permute(const void* input, void* permuted, const int32_t* indices, int64_t num_tokens, int topk,
+                    int num_experts, int64_t num_out_tokens, int hidden, int dtype, int32_t* row_id_map,
+                    void* tokens_per_expert, int counts_i64, void* workspace, int64_t workspace_bytes, void* stream);
 /* tgg_moe_permute_map without the workspace argument, for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The
  * sort's temporaries live in a fixed 8 MiB + 8 KiB array inside the library's device code (one copy per GPU, held

@@ -122,3 +122,29 @@ def test_feeds_the_grouped_gemm(dev):
             ref[t] += probs[t, k] * yk
     err = (out.float().cpu() - ref).abs().max() / ref.abs().max()
     assert err <= 2.0 ** -7, float(err)
+
+
+@pytest.mark.parametrize("num_token,num_expert,topk,hidden", [
+    (1024, 128, 8, 40), (1025, 128, 8, 40),        # the last one-launch size and the first one behind it
+    (3001, 1024, 7, 8), (9001, 5, 3, 24),          # table columns shared by no / many threads, ragged last chunk
+    (33000, 1000, 8, 8), (70001, 1, 2, 8),         # a table that needs the scan launch; a single expert
+    (8, 1024, 1100, 16), (20, 600, 500, 2056)])    # more assignments per token than one batch holds; several batches
+def test_sort_paths(dev, num_token, num_expert, topk, hidden):
+    """Every path of the sort at its edges: map, counts and moved rows are bit-exact, with ids drawn with repetition,
+    dropped assignments and a capacity that cuts the last experts off."""
+    g = torch.Generator().manual_seed(num_token)
+    indices = torch.randint(-1, num_expert, (num_token, topk), generator=g, dtype=torch.int32)
+    x = torch.randn(num_token, hidden, generator=g).to(torch.bfloat16)
+    kept = int((indices >= 0).sum())
+    for cap in (0, kept - kept // 5):
+        ref_map = permute_ref.row_id_map(indices, cap)
+        rmap, counts = ops.permute_map(indices.to(dev), cap, num_experts=num_expert)
+        assert torch.equal(rmap.cpu(), ref_map)
+        assert torch.equal(counts.cpu().long(), permute_ref.tokens_per_expert(indices, num_expert))
+        perm, rmap2 = ops.permute(x.to(dev), indices.to(dev), num_out_tokens=cap, num_experts=num_expert)
+        assert torch.equal(rmap2.cpu(), ref_map)
+        rows = cap if cap else kept
+        token_of = torch.empty(rows, dtype=torch.int64)
+        live = ref_map >= 0
+        token_of[ref_map[live].long()] = torch.arange(topk * num_token)[live] % num_token
+        assert torch.equal(perm[:rows].cpu(), x[token_of])

@@ -490,23 +490,43 @@ int tgg_moe_sort_workspace_bytes(int64_t num_tokens, int topk, int num_experts, 
   if (!bytes) return set_error("null pointer");
   if (num_tokens < 0 || topk < 1) return set_error("bad num_tokens / topk");
   if (num_experts < 1 || num_experts > 1024) return set_error("num_experts=%d outside [1, 1024]", num_experts);
-  *bytes = moe_sort_workspace_bytes(num_tokens * topk, num_experts);
+  *bytes = moe_sort_workspace_bytes(num_tokens, topk, num_experts);
+  return 0;
+}
+
+// What the sorting entry points with a workspace check alike.
+static int check_moe_sort(const int32_t* indices, int64_t num_tokens, int topk, int num_experts, const int32_t* row_id_map,
+                          const void* workspace, int64_t workspace_bytes) {
+  if (num_tokens < 0 || topk < 1) return set_error("bad num_tokens / topk");
+  if (num_tokens * topk >= (1ll << 31)) return set_error("num_tokens * topk must stay below 2^31");
+  if (num_experts < 1 || num_experts > 1024) return set_error("num_experts=%d outside [1, 1024]", num_experts);
+  const int64_t need = moe_sort_workspace_bytes(num_tokens, topk, num_experts);
+  if ((need > 0 && !workspace) || (num_tokens > 0 && (!indices || !row_id_map))) return set_error("null pointer");
+  if (workspace_bytes < need)
+    return set_error("workspace of %lld bytes is too small (need %lld)", (long long)workspace_bytes, (long long)need);
   return 0;
 }
 
 int tgg_moe_permute_map(const int32_t* indices, int64_t num_tokens, int topk, int num_experts, int64_t num_out_tokens,
                         int32_t* row_id_map, void* tokens_per_expert, int counts_i64, void* workspace,
                         int64_t workspace_bytes, void* stream) {
-  if (num_tokens < 0 || topk < 1) return set_error("bad num_tokens / topk");
-  if (num_tokens * topk >= (1ll << 31)) return set_error("num_tokens * topk must stay below 2^31");
-  if (num_experts < 1 || num_experts > 1024) return set_error("num_experts=%d outside [1, 1024]", num_experts);
-  if (!workspace || (num_tokens > 0 && (!indices || !row_id_map))) return set_error("null pointer");
-  if (workspace_bytes < moe_sort_workspace_bytes(num_tokens * topk, num_experts))
-    return set_error("workspace of %lld bytes is too small (need %lld)", (long long)workspace_bytes,
-                     (long long)moe_sort_workspace_bytes(num_tokens * topk, num_experts));
+  if (int e = check_moe_sort(indices, num_tokens, topk, num_experts, row_id_map, workspace, workspace_bytes)) return e;
   const int64_t capacity = num_out_tokens > 0 ? num_out_tokens : num_tokens * topk;
   return launch_moe_permute_map(indices, num_tokens, topk, num_experts, capacity, row_id_map, tokens_per_expert,
                                 counts_i64, workspace, (hipStream_t)stream);
+}
+
+int tgg_moe_permute(const void* input, void* permuted, const int32_t* indices, int64_t num_tokens, int topk,
+                    int num_experts, int64_t num_out_tokens, int hidden, int dtype, int32_t* row_id_map,
+                    void* tokens_per_expert, int counts_i64, void* workspace, int64_t workspace_bytes, void* stream) {
+  int64_t rb;
+  if (moe_row_bytes(hidden, dtype, &rb)) return 1;
+  if (int e = check_moe_sort(indices, num_tokens, topk, num_experts, row_id_map, workspace, workspace_bytes)) return e;
+  if (num_tokens > 0 && (!input || !permuted)) return set_error("null pointer");
+  if (!aligned16(input) || !aligned16(permuted)) return set_error("activation pointers must be 16-byte aligned");
+  const int64_t capacity = num_out_tokens > 0 ? num_out_tokens : num_tokens * topk;
+  return launch_moe_permute(input, permuted, rb, indices, num_tokens, topk, num_experts, capacity, row_id_map,
+                            tokens_per_expert, counts_i64, workspace, (hipStream_t)stream);
 }
 
 int tgg_moe_permute_map_static(const int32_t* indices, int64_t num_tokens, int topk, int num_experts,
