@@ -244,41 +244,22 @@ TGG_DEV void gemm_fast_body(const GemmParams& p) {
   // The workgroup's pos-th tile (-1 past its last one).  Static: the walk above.  Queued (K-grouped, whose tiles
   // cost what their groups have tokens, with the groups in order of decreasing size): tile ids are drawn from a
   // counter in global memory, so a workgroup that drew expensive tiles simply draws fewer -- the greedy schedule
-  // that evens out what no fixed assignment can.  Thread 0 draws and passes the ids to the other waves through a
-  // ring of eight words in the group table's scan scratch; readers use plain LDS reads, so an id must be drawn a
-  // workgroup barrier before anyone can ask for it.  Who asks first is the copy stream: it runs two slabs ahead of
-  // the multiplies and looks the next tile up as soon as it has requested a tile's last slab.  Thread 0 draws once
-  // per tile, right before the barrier of the tile's first slab (what it writes there is seen by all from the
-  // next slab on at the latest), and draws on through short tiles until it has drawn one of at least
-  // kLongTile slabs -- that one gives the next draw time enough -- or is kQueueAhead tiles ahead (enough for any
-  // run of one-slab tiles).  So a workgroup commits itself to one expensive tile beyond the one in work, not more:
-  // committing to several is what spoils the balance when a workgroup has only a dozen tiles in all.  Ids at or
-  // beyond the tile count end the workgroup's sequence; the counter only grows, so all later ones are too.
-  constexpr int kQueueAhead = 5, kLongTile = 5;
-  int32_t* const qring = reinterpret_cast<int32_t*>(sched_rw.scan_);
+  // that evens out what no fixed assignment can.  Wave 0 draws (QueueDraw in sched.hpp) and passes the ids to the
+  // other waves through a ring of words in the group table's scan scratch; readers use plain LDS reads, so an id must
+  // be in the ring a workgroup barrier before anyone can ask for it.  Who asks first is the copy stream, which looks
+  // the next tile up as soon as it has requested a tile's last slab.
+  QueueDraw<C::BM, C::BN, SchedTableT<kFastMaxGroups>> draw(p, sched_rw, (int)num_tiles, BK, queued && wave == 0);
   const int total_tiles = (int)num_tiles;
   auto tile_at = [&](int pos) -> int {
     if (queued) {
-      const int id = __builtin_amdgcn_readfirstlane(qring[pos & 7]);
+      const int id = __builtin_amdgcn_readfirstlane(draw.ring(pos));
       return id < total_tiles ? id : -1;
     }
     const int64_t id = walk.first + (int64_t)pos * walk.stride;
     return id < walk.end ? (int)id : -1;
   };
-  int q_drawn = 0, q_victim = 0;  // thread 0: ids drawn so far, counters found exhausted (see sched_draw_tile)
-  // thread 0: makes sure the ids of tiles from..from+kQueueAhead-1 are drawn, up to the first long tile
-  auto draw_from = [&](int from) {
-    for (int j = from; j < from + kQueueAhead; ++j) {
-      if (j >= q_drawn) {
-        qring[j & 7] = sched_draw_tile(p.queue, total_tiles, q_victim);
-        ++q_drawn;
-      }
-      const int id = qring[j & 7];
-      if (id >= total_tiles || slabs_of(sched_tile<C::BM, C::BN>(p, sched, id)) >= kLongTile) break;
-    }
-  };
   if (queued) {
-    if (threadIdx.x == 0) draw_from(0);
+    draw.first();
     __syncthreads();
   }
   TileIo feed;
@@ -376,6 +357,7 @@ TGG_DEV void gemm_fast_body(const GemmParams& p) {
     feed.a_rem -= A_KMAJOR ? BK * 2 : BK;
     feed.b_base += b_step;
     feed.b_rem -= B_KMAJOR ? BK * 2 : BK;
+    if (LAYOUT == LAYOUT_TN) draw.count(feed.issued, feed.kt_n);
     feed.issued += 1;
     if (counted && feed.issued >= feed.kt_n) feed_seek(feed_pos + 1);
     if (DEEP) begin_b(sc, buf_b);
@@ -549,14 +531,16 @@ TGG_DEV void gemm_fast_body(const GemmParams& p) {
       const char* sn = smem + C::a_off((ring + 1) & 1);
       const char* sba = smem + C::b_off(DEEP ? ring3 : (ring & 1));
       const char* sbn = smem + C::b_off(DEEP ? ring3n : ((ring + 1) & 1));
+      int want = 0;
+      if constexpr (LAYOUT == LAYOUT_TN) {
+        want = draw.wanted();
+        if (__builtin_expect(want, 0)) draw.request();
+      }
       half(0, 0, sa, sba, 1, READ_EARLY, NC / 2);
       half(0, 1, sa, sba, 1, READ_ROLL, -1, true);
       half(1, 0, sn, sbn, 0, READ_NONE, -1);
       wait_vmcnt<WAIT_N>();
-      // queued: this tile's draw, where this wave has no copies in flight (the wait for the counter's answer then
-      // waits for nothing else) and in front of the barrier: wave 0 is the first-served wave of its SIMD and tends
-      // to reach the barrier early, so part of the answer's latency falls into time it would spend waiting there
-      if (LAYOUT == LAYOUT_TN && queued && kt == 0 && threadIdx.x == 0) draw_from(tile_pos + 1);
+      if (LAYOUT == LAYOUT_TN && draw.live) draw.take(want);
       __syncthreads();
       sc = sc_next;
       half(1, 1, sn, sbn, 0, READ_CATCH_UP, 0);
@@ -814,7 +798,7 @@ bool fast_supported(const GemmParams& p, int dt, int layout) {
   if (p.G > kFastMaxGroups) return false;
   if ((p.N & 7) != 0) return false;
   if (layout == LAYOUT_TN) {
-    if (p.mode != MODE_KG) return false;
+    if (p.mode != MODE_KG && p.mode != MODE_KG_COUNT) return false;
     if ((p.m_total & 7) != 0) return false;
     return p.m_total * 2 * 64 < (1ll << 30) && (int64_t)p.N * 2 * 64 < (1ll << 30);
   }

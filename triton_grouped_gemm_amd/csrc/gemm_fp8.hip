@@ -176,34 +176,20 @@ TGG_DEV void gemm_fp8_body(const GemmParams& p) {
   // interleaved sweeps); K-grouped: interleaved, since a tile's cost follows its group's token count.
   const TileWalk walk64 = sched_walk(num_tiles, !KGROUP && p.tile_split);
   struct { int first, end, stride; } walk = {(int)walk64.first, (int)walk64.end, (int)walk64.stride};
-  // The workgroup's pos-th tile (-1 past its last one): the static walk, or, queued, ids drawn from the counter in
-  // global memory by thread 0 and passed on through a ring of eight words in the group table's scan scratch: one
-  // draw per tile, on through short tiles up to the first one of kLongTile slabs or kQueueAhead tiles ahead (the
-  // protocol and why it is safe are described in gemm_fast.hip).
-  constexpr int kQueueAhead = 5, kLongTile = 5;
-  int32_t* const qring = reinterpret_cast<int32_t*>(sched_rw.scan_);
+  // The workgroup's pos-th tile (-1 past its last one): the static walk, or, queued, ids drawn from the counters in
+  // global memory by wave 0 and passed on through a ring in the group table's scan scratch (QueueDraw in sched.hpp).
+  QueueDraw<C::BM, C::BN, SchedTableT<kFastMaxGroups>> draw(p, sched_rw, (int)num_tiles, BKB, queued && wave == 0);
   const int total_tiles = (int)num_tiles;
   auto tile_at = [&](int pos) -> int {
     if (queued) {
-      const int id = __builtin_amdgcn_readfirstlane(qring[pos & 7]);
+      const int id = __builtin_amdgcn_readfirstlane(draw.ring(pos));
       return id < total_tiles ? id : -1;
     }
     const int64_t id = walk.first + (int64_t)pos * walk.stride;
     return id < walk.end ? (int)id : -1;
   };
-  int q_drawn = 0, q_victim = 0;  // thread 0: ids drawn so far, counters found exhausted (see sched_draw_tile)
-  auto draw_from = [&](int from) {
-    for (int j = from; j < from + kQueueAhead; ++j) {
-      if (j >= q_drawn) {
-        qring[j & 7] = sched_draw_tile(p.queue, total_tiles, q_victim);
-        ++q_drawn;
-      }
-      const int id = qring[j & 7];
-      if (id >= total_tiles || slabs_of(sched_tile<C::BM, C::BN>(p, sched, id)) >= kLongTile) break;
-    }
-  };
   if (queued) {
-    if (threadIdx.x == 0) draw_from(0);
+    draw.first();
     __syncthreads();
   }
   TileIo feed;
@@ -290,6 +276,7 @@ TGG_DEV void gemm_fp8_body(const GemmParams& p) {
     feed.b_base += BKB;
     feed.b_left -= BKB;
     feed.s_base += (uint64_t)p.m_total * 4;
+    if (KGROUP) draw.count(feed.issued, feed.kt_n);
     feed.issued += 1;
     if (live && feed.issued >= feed.kt_n) feed_seek(feed_pos + 1);
     if (DEEP) begin_b(sc, buf_b);
@@ -444,6 +431,11 @@ TGG_DEV void gemm_fp8_body(const GemmParams& p) {
         for (int i = 0; i < C::TM; ++i) srow[i] = ss[16 * i];
       }
       SlabCopy scn;
+      int want = 0;
+      if constexpr (KGROUP) {
+        want = draw.wanted();
+        if (__builtin_expect(want, 0)) draw.request();
+      }
 #pragma unroll
       for (int i = 0; i < C::TM; ++i) {
         __builtin_amdgcn_sched_barrier(0);
@@ -454,8 +446,7 @@ TGG_DEV void gemm_fp8_body(const GemmParams& p) {
           // fragment was requested a row block ago) are complete: after the barrier the buffer is overwritten
           wait_vmcnt_lgkmcnt0<WAIT_N>();
           if (BLOCK) asm volatile("" : "+v"(sbv_next));  // everything older than the newest B copies has landed: touching it costs no wait
-          // queued: this tile's draw, where this wave has nothing in flight, in front of the barrier (gemm_fast.hip)
-          if (KGROUP && queued && kt == 0 && threadIdx.x == 0) draw_from(tile_pos + 1);
+          if (KGROUP && draw.live) draw.take(want);
           __syncthreads();
           sc = scn;
           fa[0] = load_frag(sn + wm0 * 128);

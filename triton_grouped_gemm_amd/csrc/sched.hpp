@@ -389,20 +389,78 @@ TGG_HD int sched_queue_id(int n, int xq, int R) {
 // workgroup that drew expensive tiles draws fewer.  A workgroup whose own XCD has nothing left takes from the
 // next XCD's counter, and so on round the ring: what the deal leaves uneven is evened out at the end.  For every
 // counter the ids grow with the number of draws, so one id at or beyond `total` means that counter is exhausted.
-// `victim` (0 at first; kept by the drawing thread) counts the counters found exhausted so far; returns an id at
-// or beyond `total` when all eight are.
-TGG_DEV int sched_draw_tile(int32_t* queue, int total, int& victim) {
-  const int P = (int)gridDim.x;
-  if ((P & 7) != 0) return atomicAdd(queue, 1);
-  const int x = (int)blockIdx.x & 7, R = P >> 3;
-  while (victim < 8) {
-    const int xq = (x + victim) & 7;
-    const int id = sched_queue_id(atomicAdd(queue + xq, 1), xq, R);
-    if (id < total) return id;
-    ++victim;
+//
+// One wave of each workgroup draws for it.  A draw costs a round trip to the counter (about a microsecond), which on
+// tiles of a slab or two is as long as the tile, so it is requested at the start of a slab and taken at the slab's
+// own wait for its copies, in front of the barrier; only when the copy stream is about to run out of drawn tiles does
+// the wave draw on the spot.  It draws when fewer than kAhead slabs are drawn and not yet requested by the copy
+// stream, so a workgroup commits itself to its next expensive tile a few slabs before it needs it and not earlier:
+// committing to several is what spoils the balance when a workgroup has only a dozen tiles in all.  Measured against a
+// draw on the spot per tile, 128 groups of 2048 x 1536 outputs: bf16, 64 / 256 / 1024 tokens per group 203 / 303 / 853 ->
+// 167 / 285 / 819 us (4096: the same), FP8, 128 / 256 / 1024 tokens 241 / 258 / 586 -> 199 / 224 / 582 us.  kAhead 2, 4, 8:
+// FP8 at 128 tokens 222, 206, 199 us, no difference at 4096.  The branches are marked unlikely: laid out inside the
+// slab loop they cost 1-1.5 % of a long FP8 launch.
+template <int BM, int BN, class Table>
+struct QueueDraw {
+  static constexpr int kRing = 16;  // > tiles between the one in work and the last drawn: 3 + kAhead one-slab tiles
+  static constexpr int kAhead = 8;
+  const GemmParams& p;
+  Table& t;
+  const int total, slab_k;
+  int ahead = 0;             // slabs drawn and not yet requested by the copy stream (kept by every wave's begin_slab, read by the drawing wave)
+  int drawn = 0, victim = 0;  // tiles drawn; counters found exhausted
+  int live;                   // 1 in the wave that draws, until it has put the end marker in the ring (integers, not
+                              // truth values, so that they stay in scalar registers)
+  int answer;                 // lane 0: the counter's value once the wave's memory operations have been waited for
+
+  TGG_DEV QueueDraw(const GemmParams& p_, Table& t_, int total_, int slab_k_, bool drawing)
+      : p(p_), t(t_), total(total_), slab_k(slab_k_), live(drawing ? 1 : 0) {}
+
+  TGG_DEV int32_t& ring(int pos) { return reinterpret_cast<int32_t*>(t.scan_)[pos & (kRing - 1)]; }
+  TGG_DEV bool spread() const { return (gridDim.x & 7) == 0; }  // eight counters; else one
+  TGG_DEV int counter() const { return spread() ? ((int)(blockIdx.x & 7) + victim) & 7 : 0; }
+  TGG_DEV int wanted() { live = __builtin_amdgcn_readfirstlane(live); return ahead < kAhead ? live : 0; }
+  // begin_slab has requested a slab of the tile (issued < slabs: there was one left)
+  TGG_DEV void count(int issued, int slabs) { ahead -= (int)((uint32_t)(issued - slabs) >> 31); }
+
+  // n: the value drawn from the current counter
+  TGG_DEV void accept(int n) {
+    const int id = spread() ? sched_queue_id(n, counter(), (int)gridDim.x >> 3) : n;
+    if (id < total) {
+      const int per_group = (int)((p.m_total + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+      const int rows = __builtin_amdgcn_readfirstlane(t.rows[t.tile0[id / per_group]]);
+      ring(drawn++) = id;
+      ahead += rows > 0 ? (rows + slab_k - 1) / slab_k : 1;  // an empty group's tile has one slab of nothing
+    } else if (++victim >= (spread() ? 8 : 1)) {
+      ring(drawn++) = total;
+      live = 0;
+    }
   }
-  return total;
-}
+
+  TGG_DEV void draw_now() {
+    int n = 0;
+    if (lane_id() == 0) n = atomicAdd(p.queue + counter(), 1);
+    accept(__builtin_amdgcn_readfirstlane(n));
+  }
+
+  TGG_DEV void first() { while (wanted()) draw_now(); }
+
+  // Requests a draw; `answer` is in flight until take().  Only lane 0 adds, by the execution mask and not by a branch:
+  // a branch of lanes would join in front of take(), and the compiler must have no reason to move `answer`.
+  TGG_DEV void request() {
+    const int32_t* const at = p.queue + counter();
+    uint64_t saved;
+    asm volatile("s_mov_b64 %1, exec\n\ts_mov_b64 exec, 1\n\tglobal_atomic_add %0, %2, %3, off sc0\n\ts_mov_b64 exec, %1"
+                 : "=v"(answer), "=&s"(saved) : "v"(at), "v"(1) : "memory");
+  }
+
+  // The drawing wave, after it has waited for all of its memory operations and in front of a workgroup barrier.
+  TGG_DEV void take(int requested) {
+    asm volatile("" : "+v"(answer));  // arrived: not to be read any earlier than here
+    if (__builtin_expect(requested, 0)) accept(__builtin_amdgcn_readfirstlane(answer));
+    while (__builtin_expect(ahead <= 1 && live, 0)) draw_now();  // the next slab's request may ask for the next tile
+  }
+};
 
 // End of a queued launch: every workgroup reports here once it has drawn its last id (the draw that found all eight
 // counters exhausted has returned by then), and the workgroup that reports last puts the nine words back to zero, so
