@@ -77,6 +77,12 @@ int tgg_k_grouped_gemm(const void* A, const void* B, void* C, const int32_t* sta
 int tgg_k_grouped_gemm_queued(const void* A, const void* B, void* C, const int32_t* start, const int32_t* end, int G,
                               int Mdim, int N, int64_t Ktot, int dtype, int num_cu, int32_t* queue, void* stream);
 
+/* tgg_k_grouped_gemm_queued with segments that follow one another in group order and `sizes` (int32 or int64 [G]) tokens
+ * each: the kernel makes their starts itself, as k_grouped_gemm does from size_per_group when it gets no bounds
+ * (gemm/BF16/k_grouped_gemm_TMA.py:217-294).  queue may be NULL. */
+int tgg_k_grouped_gemm_sizes(const void* A, const void* B, void* C, const void* sizes, int sizes_i64, int G, int Mdim,
+                             int N, int64_t Ktot, int dtype, int num_cu, int32_t* queue, void* stream);
+
 /* C = (Aq . Bq[g]^T) * a_scale[r] * b_scale[g*N+n].  Replaces gmm_fp8_act_per_channel_w_per_expert
  * (gemm/FP8/m_grouped_gemm_channel_expert.py:139-198). */
 int tgg_m_grouped_gemm_fp8_channel(const void* Aq, const float* a_scale, const void* Bq, const float* b_scale,

@@ -514,3 +514,23 @@ def test_k_grouped_work_queue_equals_fixed_assignment(dev, sizes, num_cu):
     assert int(queue.abs().sum()) == 0
     check_16bit_gemm(drawn, gemm_ref.gmm_dw(a.cpu(), b.cpu(), sizes), gemm_ref.gmm_dw(a.cpu(), b.cpu(), sizes, fp32=True),
                      "queued K-grouped")
+
+
+@pytest.mark.parametrize("sizes", [
+    [1], [0, 0, 5], [64, 0, 1, 128, 63, 65, 0, 200],
+    [(i * 37) % 70 for i in range(130)],           # one-slab tiles: the copy stream runs several tiles ahead
+    [700, 3, 0, 700, 64, 64, 1, 1, 1, 1500, 320],  # short and long tiles in turn
+    [i % 5 for i in range(600)]])                  # beyond the tuned kernels' table
+@pytest.mark.parametrize("size_dtype,extra", [(torch.int32, 0), (torch.int64, 9), (torch.int64, -3)])
+def test_k_grouped_from_sizes_equals_explicit_bounds(dev, sizes, size_dtype, extra):
+    """Segments from the sizes alone, bit for bit what explicit starts and ends give: tokens beyond the last segment
+    (extra > 0) belong to nobody, sizes that add up to more than there are tokens (extra < 0) are clipped."""
+    total, Mdim, N = max(sum(sizes) + extra, 1), 264, 520
+    gen = torch.Generator().manual_seed(len(sizes))
+    a = torch.randn(total, Mdim, generator=gen).to(torch.bfloat16).to(dev)
+    b = torch.randn(total, N, generator=gen).to(torch.bfloat16).to(dev)
+    s = torch.tensor(sizes, dtype=size_dtype, device=dev)
+    end = s.cumsum(0)
+    want = k_grouped_gemm(a, b, s, (end - s).to(torch.int32), end.to(torch.int32))
+    for _ in range(3):
+        assert torch.equal(k_grouped_gemm(a, b, s), want)

@@ -29,6 +29,7 @@ SIGNATURES = {
     "tgg_m_grouped_gemm_masked": [_P, _P, _P, _P, _I, _I, _L, _L, _I, _I, _I, _I, _I, _P],
     "tgg_k_grouped_gemm": [_P, _P, _P, _P, _P, _I, _I, _I, _L, _I, _I, _P],
     "tgg_k_grouped_gemm_queued": [_P, _P, _P, _P, _P, _I, _I, _I, _L, _I, _I, _P, _P],
+    "tgg_k_grouped_gemm_sizes": [_P, _P, _P, _P, _I, _I, _I, _I, _L, _I, _I, _P, _P],
     "tgg_m_grouped_gemm_fp8_channel": [_P, _P, _P, _P, _P, _P, _I, _I, _L, _I, _I, _I, _I, _I, _I, _P],
     "tgg_k_grouped_gemm_fp8_channel": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _L, _I, _I, _I, _P],
     "tgg_k_grouped_gemm_fp8_channel_queued": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _L, _I, _I, _I, _P, _P],

@@ -136,6 +136,14 @@ static GemmParams params_k_grouped(const void* A, const void* B, void* C, const 
   return p;
 }
 
+// the segments of the shared reduction axis follow one another in group order, `sizes` says how long they are
+static GemmParams params_k_grouped_sizes(const void* A, const void* B, void* C, const void* sizes, int sizes_i64, int G,
+                                         int Mdim, int N, int64_t Ktot, int num_cu, int32_t* queue) {
+  GemmParams p = params_k_grouped(A, B, C, nullptr, nullptr, G, Mdim, N, Ktot, num_cu, queue);
+  p.mode = MODE_KG_COUNT; p.sizes = sizes; p.sizes_i64 = sizes_i64;
+  return p;
+}
+
 static GemmParams params_fp8_channel(const void* Aq, const float* a_scale, const void* Bq, const float* b_scale,
                                      void* C, const void* sizes, int sizes_i64, int G, int64_t M, int N, int K,
                                      int num_cu) {
@@ -362,6 +370,16 @@ int tgg_k_grouped_gemm_queued(const void* A, const void* B, void* C, const int32
   if (dtype != TGG_BF16 && dtype != TGG_F16) return set_error("data type code %d not supported", dtype);
   if ((Mdim & 7) || (N & 7)) return set_error("Mdim and N must be multiples of 8 (16-byte rows), got %d, %d", Mdim, N);
   const GemmParams p = params_k_grouped(A, B, C, start, end, G, Mdim, N, Ktot, num_cu, queue);
+  return dispatch_16bit(p, dtype, 2, (hipStream_t)stream);
+}
+
+int tgg_k_grouped_gemm_sizes(const void* A, const void* B, void* C, const void* sizes, int sizes_i64, int G, int Mdim,
+                             int N, int64_t Ktot, int dtype, int num_cu, int32_t* queue, void* stream) {
+  if (int e = check_common(A, B, C, sizes, G, N, TGG_MAX_GROUPS)) return e;
+  if (Mdim < 1 || Ktot < 0) return set_error("bad Mdim=%d or Ktot=%lld", Mdim, (long long)Ktot);
+  if (dtype != TGG_BF16 && dtype != TGG_F16) return set_error("data type code %d not supported", dtype);
+  if ((Mdim & 7) || (N & 7)) return set_error("Mdim and N must be multiples of 8 (16-byte rows), got %d, %d", Mdim, N);
+  const GemmParams p = params_k_grouped_sizes(A, B, C, sizes, sizes_i64, G, Mdim, N, Ktot, num_cu, queue);
   return dispatch_16bit(p, dtype, 2, (hipStream_t)stream);
 }
 

@@ -57,13 +57,17 @@ def k_grouped_gemm(A: Tensor, B: Tensor, size_per_group: Tensor, group_start: Op
     K_TOTAL, M_DIM, N_DIM, num_groups = _check_k_grouped_gemm_inputs(A, B, size_per_group, trans_b)
     assert 1 <= num_groups <= _native.MAX_GROUPS, f"between 1 and {_native.MAX_GROUPS} groups are supported"
     C = A.new_empty(num_groups, M_DIM, N_DIM)
+    # tile-id counters of the kernel's work queue (a tile costs what its group has tokens; see include/tgg_amd.h)
+    queue = _native.work_queue(A.device, queue)
     if group_start is None or group_end is None:
-        group_end = size_per_group.cumsum(0)
-        group_start = group_end - size_per_group
+        # the kernel makes the segments' starts itself (five launches of 5 us when torch makes them)
+        sizes = size_per_group.contiguous()
+        _native.call("tgg_k_grouped_gemm_sizes", A.data_ptr(), B.data_ptr(), C.data_ptr(), sizes.data_ptr(),
+                     int(sizes.dtype == torch.int64), num_groups, M_DIM, N_DIM, K_TOTAL, _dtype_code(A.dtype),
+                     int(numSM), queue.data_ptr(), _native.stream_of(A))
+        return C
     group_start = group_start.to(device=A.device, dtype=torch.int32).contiguous()
     group_end = group_end.to(device=A.device, dtype=torch.int32).contiguous()
-    # tile-id counter of the kernel's work queue (a tile costs what its group has tokens; see include/tgg_amd.h)
-    queue = _native.work_queue(A.device, queue)
     _native.call("tgg_k_grouped_gemm_queued", A.data_ptr(), B.data_ptr(), C.data_ptr(), group_start.data_ptr(),
                  group_end.data_ptr(), num_groups, M_DIM, N_DIM, K_TOTAL, _dtype_code(A.dtype), int(numSM),
                  queue.data_ptr(), _native.stream_of(A))
