@@ -126,6 +126,10 @@ int tgg_m_grouped_gemm_fp8_block_placed(const void* Aq, const float* sa, const v
 int tgg_trans_per_block_quant_expand_128x(const void* x, void* codes, float* scales, const void* sizes,
                                           int sizes_i64, int G, int64_t M, int N, int64_t M_expand, int fmt,
                                           void* stream);
+/* The same; padded_sizes (optional, [G] in the integer type of sizes) receives the sizes rounded up to 128. */
+int tgg_trans_per_block_quant_expand_128x_padded(const void* x, void* codes, float* scales, const void* sizes,
+                                                 int sizes_i64, int G, int64_t M, int N, int64_t M_expand,
+                                                 void* padded_sizes, int fmt, void* stream);
 
 /* bf16 x [M,K] -> codes [M,K], scales [M,K/128] (scales_mn_major=0) or stored transposed [K/128,M]
  * (scales_mn_major=1); 1x128 recipe.  Replaces per_token_cast_to_fp8

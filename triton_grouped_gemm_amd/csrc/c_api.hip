@@ -51,7 +51,7 @@ int num_cus() {
   return cached[dev];
 }
 
-int launch_trans_quant128(const void*, void*, float*, const GemmParams&, int64_t, int, hipStream_t);
+int launch_trans_quant128(const void*, void*, float*, const GemmParams&, int64_t, void*, int, hipStream_t);
 int launch_token_cast128(const void*, void*, float*, int64_t, int, int, int, hipStream_t);
 int launch_block_cast128(const void*, void*, float*, int, int, int, int, hipStream_t);
 int launch_cvt_fp8(const float*, void*, int64_t, int, hipStream_t);
@@ -458,16 +458,22 @@ int tgg_m_grouped_gemm_fp8_block_placed(const void* Aq, const float* sa, const v
 int tgg_trans_per_block_quant_expand_128x(const void* x, void* codes, float* scales, const void* sizes,
                                           int sizes_i64, int G, int64_t M, int N, int64_t M_expand, int fmt,
                                           void* stream) {
+  return tgg_trans_per_block_quant_expand_128x_padded(x, codes, scales, sizes, sizes_i64, G, M, N, M_expand, nullptr, fmt, stream);
+}
+
+int tgg_trans_per_block_quant_expand_128x_padded(const void* x, void* codes, float* scales, const void* sizes,
+                                                 int sizes_i64, int G, int64_t M, int N, int64_t M_expand,
+                                                 void* padded_sizes, int fmt, void* stream) {
   if ((!x && M > 0) || !codes || !scales || !sizes) return set_error("null pointer");
   if (G < 1 || G > TGG_MAX_GROUPS) return set_error("G=%d outside [1, %d]", G, TGG_MAX_GROUPS);
   if (N < 128 || (N & 127)) return set_error("N must be a positive multiple of 128, got %d", N);
   if (M < 0 || M_expand < 0 || (M_expand & 127)) return set_error("M_expand must be a multiple of 128");
   if (M_expand < ((M + 127) / 128) * 128) return set_error("M_expand=%lld too small for M=%lld", (long long)M_expand, (long long)M);
   if (!aligned16(x) || !aligned16(codes)) return set_error("operand pointers must be 16-byte aligned");
-  if (M_expand == 0) return 0;
+  if (M_expand == 0 && !padded_sizes) return 0;
   GemmParams p = zero_params();
   p.sizes = sizes; p.sizes_i64 = sizes_i64; p.G = G; p.mode = MODE_MG; p.m_total = M; p.N = N;
-  return launch_trans_quant128(x, codes, scales, p, M_expand, fmt, (hipStream_t)stream);
+  return launch_trans_quant128(x, codes, scales, p, M_expand, padded_sizes, fmt, (hipStream_t)stream);
 }
 
 int tgg_per_token_cast_to_fp8(const void* x, void* codes, float* scales, int64_t M, int K, int fmt,

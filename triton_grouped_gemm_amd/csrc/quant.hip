@@ -62,10 +62,18 @@ template <int MAXG> struct TransSmem {
 // Read: thread (rr = tid/16, cv = tid%16) owns rows rr*8 .. rr*8+7, columns cv*8 .. cv*8+7.
 // LDS holds the transposed codes: byte (c, r) at c*128 + ((r/16) ^ ((c/8)%8))*16 + r%16.
 // MAXG sizes the group table in LDS: the small one lets twice as many workgroups share a CU.
+// padded (optional): the sizes rounded up to 128, in their own integer type.
 template <int FMT, int MAXG>
 __global__ __launch_bounds__(256) void trans_quant128_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ codes,
-                                                            float* __restrict__ scales, GemmParams p, int64_t m_expand) {
+                                                            float* __restrict__ scales, GemmParams p, int64_t m_expand,
+                                                            void* __restrict__ padded) {
   __shared__ TransSmem<MAXG> sm;
+  if (padded && blockIdx.x == 0) {
+    for (int g = threadIdx.x; g < p.G; g += 256) {
+      if (p.sizes_i64) ((int64_t*)padded)[g] = (((const int64_t*)p.sizes)[g] + 127) & ~(int64_t)127;
+      else ((int32_t*)padded)[g] = (((const int32_t*)p.sizes)[g] + 127) & ~127;
+    }
+  }
   sched_init<128>(p, sm.sched);
   const int N = p.N;
   const int tiles_n = N >> 7;
@@ -274,8 +282,8 @@ __global__ void cvt_fp8_kernel(const float* __restrict__ in, uint8_t* __restrict
 
 }  // namespace
 
-int launch_trans_quant128(const void* x, void* codes, float* scales, const GemmParams& p, int64_t m_expand, int fmt,
-                          hipStream_t s) {
+int launch_trans_quant128(const void* x, void* codes, float* scales, const GemmParams& p, int64_t m_expand, void* padded,
+                          int fmt, hipStream_t s) {
   const int64_t tiles = (m_expand >> 7) * (int64_t)(p.N >> 7);
   int64_t grid = (int64_t)num_cus() * 8;
   if (grid > tiles) grid = tiles;
@@ -285,11 +293,11 @@ int launch_trans_quant128(const void* x, void* codes, float* scales, const GemmP
   uint8_t* co = (uint8_t*)codes;
   const bool small = p.G <= 256;
   if (fmt == DT_E4M3) {
-    if (small) hipLaunchKernelGGL((trans_quant128_kernel<DT_E4M3, 256>), g, b, 0, s, xi, co, scales, p, m_expand);
-    else hipLaunchKernelGGL((trans_quant128_kernel<DT_E4M3, kMaxGroups>), g, b, 0, s, xi, co, scales, p, m_expand);
+    if (small) hipLaunchKernelGGL((trans_quant128_kernel<DT_E4M3, 256>), g, b, 0, s, xi, co, scales, p, m_expand, padded);
+    else hipLaunchKernelGGL((trans_quant128_kernel<DT_E4M3, kMaxGroups>), g, b, 0, s, xi, co, scales, p, m_expand, padded);
   } else if (fmt == DT_E5M2) {
-    if (small) hipLaunchKernelGGL((trans_quant128_kernel<DT_E5M2, 256>), g, b, 0, s, xi, co, scales, p, m_expand);
-    else hipLaunchKernelGGL((trans_quant128_kernel<DT_E5M2, kMaxGroups>), g, b, 0, s, xi, co, scales, p, m_expand);
+    if (small) hipLaunchKernelGGL((trans_quant128_kernel<DT_E5M2, 256>), g, b, 0, s, xi, co, scales, p, m_expand, padded);
+    else hipLaunchKernelGGL((trans_quant128_kernel<DT_E5M2, kMaxGroups>), g, b, 0, s, xi, co, scales, p, m_expand, padded);
   } else {
     return set_error("unsupported fp8 format code %d", fmt);
   }

@@ -32,13 +32,13 @@ def trans_per_block_quant_expand_128x(input_tensor: torch.Tensor, size_per_group
     _native.require_gpu(input_tensor)
     assert input_tensor.is_contiguous(), "input_tensor must be contiguous"
     sizes, is64 = _sizes_on_device(size_per_group, input_tensor.device)
-    size_per_group_padding = torch.div(sizes + (group_size - 1), group_size, rounding_mode="floor") * group_size
+    size_per_group_padding = torch.empty_like(sizes)  # written by the kernel
     M_EXPAND = M + group_size * num_experts - M % group_size
     output_tensor = input_tensor.new_empty((N, M_EXPAND), dtype=dtype)
     output_scales = input_tensor.new_empty((N // group_size, M_EXPAND // group_size), dtype=torch.float32)
-    _native.call("tgg_trans_per_block_quant_expand_128x", input_tensor.data_ptr(), output_tensor.data_ptr(),
+    _native.call("tgg_trans_per_block_quant_expand_128x_padded", input_tensor.data_ptr(), output_tensor.data_ptr(),
                  output_scales.data_ptr(), sizes.data_ptr(), is64, num_experts, M, N, M_EXPAND,
-                 _native.FP8_CODE[dtype], _native.stream_of(input_tensor))
+                 size_per_group_padding.data_ptr(), _native.FP8_CODE[dtype], _native.stream_of(input_tensor))
     return output_tensor, output_scales, size_per_group_padding
 
 
