@@ -164,3 +164,47 @@ def test_per_block_cast_bit_exact(dev, shape):
         sb = scales.cpu().numpy().reshape((xs.shape[0],) + rs.shape)[b]
         assert np.array_equal(sb.view(np.uint32), rs.view(np.uint32))
         assert np.array_equal(cb, rc)
+
+
+@pytest.mark.parametrize("dtype", [torch.float8_e4m3fn, torch.float8_e5m2])
+@pytest.mark.parametrize("kind", ["tiny", "denormal", "huge", "mixed", "inf", "zeros"])
+def test_trans_quant_at_the_ends_of_the_range(dev, dtype, kind):
+    """Bit-exact where the scale is clamped, where quotients underflow (zeros keep their sign), and in blocks whose values
+    leave the range of the exact reciprocal method (beyond 1e30, infinities)."""
+    g = torch.Generator().manual_seed(7)
+    sizes, N = [130, 0, 5, 300, 128], 256
+    x = torch.randn(sum(sizes), N, generator=g)
+    if kind == "tiny":
+        x *= 1e-10
+    elif kind == "denormal":
+        x *= 1e-38
+    elif kind == "huge":
+        x *= 3e37
+    elif kind == "mixed":  # bf16 bit patterns, finite
+        x = torch.randint(-(1 << 15), 1 << 15, x.shape, generator=g, dtype=torch.int16).view(torch.bfloat16).float()
+        x[~x.isfinite()] = 1.0
+    elif kind == "inf":
+        x[::50, ::60] = float("inf")
+        x[7::50, ::60] = float("-inf")
+    else:
+        x = torch.zeros_like(x).copysign(x)
+    _check_trans_quant(dev, x.to(torch.bfloat16), sizes, dtype, torch.int64)
+
+
+def test_trans_quant_ignores_nan_in_the_scale(dev):
+    """A NaN does not count towards its block's maximum: the other values of the block get the codes they get without it."""
+    sizes = [100, 156]
+    x = _randn((256, 128), 5, 2.0)
+    y = x.clone()
+    y[::9, ::7] = float("nan")
+    x[::9, ::7] = 0.0
+    s = torch.tensor(sizes, dtype=torch.int32, device=dev)
+    cx, sx, _ = trans_per_block_quant_expand_128x(x.to(dev), s)
+    cy, sy, _ = trans_per_block_quant_expand_128x(y.to(dev), s)
+    assert torch.equal(sx, sy)
+    rows = torch.arange(256) % 9 == 0
+    cols = torch.arange(128) % 7 == 0
+    place = torch.cat([torch.arange(100), 128 + torch.arange(156)])  # output column of every input row
+    same = ~(rows[:, None] & cols[None, :])
+    a, b = (c.view(torch.uint8).cpu()[:, place].t() for c in (cx, cy))
+    assert torch.equal(a[same], b[same])
