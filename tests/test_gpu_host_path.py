@@ -1,0 +1,108 @@
+"""The native call path (csrc/host.cpp): it takes the ordinary eager call and gives what the operator and the wrapper give;
+it leaves everything else -- gradients, tracing modes, operands that need conversion, invalid arguments -- to them."""
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from triton_grouped_gemm_amd import _native, ops
+from triton_grouped_gemm_amd.gemm.BF16.k_grouped_gemm import k_grouped_gemm
+from triton_grouped_gemm_amd.gemm.BF16.m_grouped_gemm import m_grouped_gemm
+from triton_grouped_gemm_amd.gemm.BF16.m_grouped_gemm_masked_TMA import m_grouped_gemm_masked
+from triton_grouped_gemm_amd.gemm.FP8.m_grouped_gemm_channel_expert import gmm_fp8_act_per_channel_w_per_expert
+
+
+def test_cpu_operands_are_left_to_the_wrapper():
+    a, b, s = torch.zeros(8, 8, dtype=torch.bfloat16), torch.zeros(1, 8, 8, dtype=torch.bfloat16), torch.tensor([8])
+    assert _native.host().m_grouped_gemm(a, b, s, True, -1) is None
+    with pytest.raises(AssertionError, match="GPU"):
+        m_grouped_gemm(a, b, s, True)
+
+
+def _operands(dev, dtype=torch.bfloat16, trans_b=True):
+    g = torch.Generator().manual_seed(3)
+    sizes = torch.tensor([70, 0, 33, 97], dtype=torch.int32, device=dev)
+    a = torch.randn(200, 72, generator=g).to(dtype).to(dev)
+    b = torch.randn(*((4, 40, 72) if trans_b else (4, 72, 40)), generator=g).to(dtype).to(dev)
+    return a, b, sizes
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("trans_b", [True, False])
+@pytest.mark.parametrize("wide", [False, True])
+def test_direct_call_equals_the_operator(dev, dtype, trans_b, wide):
+    a, b, sizes = _operands(dev, dtype, trans_b)
+    sizes = sizes.to(torch.int64) if wide else sizes
+    want = torch.ops.moe.m_grouped_gemm(a, b, sizes, trans_b)
+    got = _native.host().m_grouped_gemm(a, b, sizes, trans_b, -1)
+    assert got is not None and got.dtype == dtype and torch.equal(got, want)
+    assert torch.equal(m_grouped_gemm(A=a, B=b, size_per_group=sizes, trans_b=trans_b, numSM=8), want)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):  # the caller's current stream is the one that is used
+        other = m_grouped_gemm(a * 2, b, sizes, trans_b)
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(other, torch.ops.moe.m_grouped_gemm(a * 2, b, sizes, trans_b))
+
+
+@pytest.mark.gpu
+def test_what_is_left_to_the_operator(dev):
+    a, b, sizes = _operands(dev)
+    host = _native.host()
+    call = lambda x=a, w=b, s=sizes, t=True: host.m_grouped_gemm(x, w, s, t, -1)
+    assert call() is not None
+    assert call(x=a.clone().requires_grad_(True)) is None
+    with torch.no_grad():
+        assert call(x=a.clone().requires_grad_(True)) is not None
+    assert call(x=a[:, :64]) is None and call(x=a.t().contiguous().t()) is None and call(x=a.float()) is None
+    assert call(s=sizes.cpu()) is None and call(s=sizes[:3]) is None and call(s=sizes.float()) is None and call(t=1) is None
+    class Tensor2(torch.Tensor):
+        pass
+    assert call(x=a.as_subclass(Tensor2)) is None
+    seen = []
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+    with Watch():
+        out = m_grouped_gemm(a, b, sizes, True)
+    assert any("m_grouped_gemm" in f for f in seen) and torch.equal(out, call())
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode(allow_non_fake_inputs=False) as mode:
+        fake = m_grouped_gemm(mode.from_tensor(a), mode.from_tensor(b), mode.from_tensor(sizes), True)
+        assert type(fake).__name__ == "FakeTensor" and tuple(fake.shape) == (200, 40)
+    with pytest.raises(AssertionError, match="K of A should be equal"):
+        m_grouped_gemm(a[:, :64].contiguous(), b, sizes, True)
+    with pytest.raises(TypeError):
+        host.m_grouped_gemm(a, b)
+
+
+@pytest.mark.gpu
+def test_other_entry_points_agree_with_their_wrappers(dev):
+    """Strided copies of the operands, which the native path refuses, against the same operands as they are."""
+    a, b, sizes = _operands(dev)
+    grad = torch.randn(200, 56, device=dev).to(torch.bfloat16)
+    end = sizes.cumsum(0).int()
+    assert torch.equal(k_grouped_gemm(a, grad, sizes), k_grouped_gemm(a, grad, sizes, end - sizes, end))
+    lhs = torch.randn(4 * 128, 72, device=dev).to(torch.bfloat16)
+    outs = [torch.zeros(4 * 128, 40, device=dev, dtype=torch.bfloat16) for _ in range(2)]
+    assert m_grouped_gemm_masked(lhs, b, outs[0], sizes, 128) is None
+    assert m_grouped_gemm_masked(lhs, b, outs[1], sizes, 128, 1) is None
+    assert torch.equal(*outs) and outs[0].any()
+    a8, b8 = torch.randn(200, 80, device=dev).to(torch.float8_e4m3fn), torch.randn(4, 48, 80, device=dev).to(torch.float8_e4m3fn)
+    sa, sb = torch.rand(200, 1, device=dev), torch.rand(4, 48, device=dev)
+    for out_type in (torch.float16, torch.bfloat16):
+        got = gmm_fp8_act_per_channel_w_per_expert(a8, sa, b8, sb, sizes, out_type)
+        assert got.dtype == out_type
+        assert torch.equal(got, gmm_fp8_act_per_channel_w_per_expert(a8, sa.double(), b8, sb, sizes, out_type))
+    idx = torch.randint(0, 4, (200, 2), device=dev, dtype=torch.int32)
+    x = a.clone().requires_grad_(True)
+    rows, where = ops.permute(x, idx, num_experts=4)
+    with torch.no_grad():
+        direct = ops.permute(x, idx, num_experts=4)
+    assert rows.requires_grad and not direct[0].requires_grad
+    assert torch.equal(rows, direct[0]) and torch.equal(where, direct[1])
+    probs = torch.rand(200, 2, device=dev)
+    assert torch.equal(ops.unpermute(direct[0], where, probs), ops.unpermute(rows, where, probs))
+    assert torch.equal(ops.permute_map(idx, num_experts=4)[0], ops.permute_map(idx.long(), num_experts=4)[0])

@@ -1,4 +1,4 @@
-"""ctypes binding of libtgg_amd.so (the C ABI declared in include/tgg_amd.h).
+"""ctypes binding of libtgg_amd.so (the C ABI declared in include/tgg_amd.h), and the native call path over it.
 
 There is no fallback: if the shared library is missing or a call fails, the
 caller gets an exception.
@@ -57,6 +57,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_host = None
 
 
 def load() -> ctypes.CDLL:
@@ -77,6 +78,18 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+def host():
+    """The extension module of csrc/host.cpp: each of its functions does one entry point's ordinary eager call (plain
+    contiguous tensors on the current GPU, nothing recorded, no mode active) and returns None for any other, which then
+    takes the wrapper's own way through checks, conversions and the operator."""
+    global _host
+    if _host is None:
+        load()
+        from . import _host as module
+        _host = module
+    return _host
+
+
 def last_error() -> str:
     return load().tgg_last_error().decode()
 
@@ -92,7 +105,7 @@ def set_option(key: str, value: int) -> None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 _work_queues = {}
@@ -111,7 +124,7 @@ def work_queue(device: torch.device, queue: Optional[torch.Tensor] = None) -> to
         return queue
     if torch.cuda.is_current_stream_capturing():
         return torch.zeros(QUEUE_WORDS, dtype=torch.int32, device=device)
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, torch._C._cuda_getCurrentRawStream(device.index))
     q = _work_queues.get(key)
     if q is None:
         q = _work_queues[key] = torch.zeros(QUEUE_WORDS, dtype=torch.int32, device=device)

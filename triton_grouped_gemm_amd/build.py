@@ -1,4 +1,5 @@
-"""Compile csrc/*.hip for gfx950 into libtgg_amd.so next to this file.
+"""Compile csrc/*.hip for gfx950 into libtgg_amd.so next to this file, and csrc/host.cpp (the native call path of the
+Python entry points, an extension module over torch's C++ API) into _host.so beside it.
 
 ``python -m triton_grouped_gemm_amd.build`` (or ``build_library()``) runs hipcc once per
 translation unit in parallel and links the objects.  hipcc cross-compiles, so no
@@ -10,12 +11,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libtgg_amd.so"
+HOST_PATH = PKG_DIR / "_host.so"
 ARCH = "gfx950"
 # packed fp32 VALU forms are switched off for every HIP translation unit
 HIPCC_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-Xclang", "-target-feature", "-Xclang",
@@ -36,6 +39,23 @@ def _run(cmd):
     if proc.returncode != 0:
         raise RuntimeError("command failed: " + " ".join(map(str, cmd)) + "\n" + err)
     return err
+
+
+def _compile_host(obj: Path):
+    """csrc/host.cpp against torch's headers, by the host compiler."""
+    from torch.utils.cpp_extension import include_paths
+    includes = [*include_paths("cuda"), sysconfig.get_paths()["include"]]
+    _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          *(f"-I{d}" for d in includes), "-c", str(CSRC / "host.cpp"), "-o", str(obj)])
+
+
+def _link_host(obj: Path):
+    """_host.so: finds libtgg_amd.so beside itself and torch's libraries where the running process has loaded them."""
+    from torch.utils.cpp_extension import library_paths
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    _run([shutil.which("g++") or "g++", "-shared", "-o", str(tmp), str(obj), *(f"-L{d}" for d in library_paths("cuda")),
+          "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", f"-L{PKG_DIR}", f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN"])
+    os.replace(tmp, HOST_PATH)
 
 
 def build_library(verbose: bool = False, jobs: int | None = None) -> Path:
@@ -62,11 +82,15 @@ def build_library(verbose: bool = False, jobs: int | None = None) -> Path:
         if verbose and msg.strip():
             print(msg, file=sys.stderr)
 
+    host_obj = obj_dir / "host.o"
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(_compile_host, host_obj)
         list(pool.map(compile_one, zip(sources, objs)))
+        host.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     _run([hipcc, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)])
     os.replace(tmp, LIB_PATH)
+    _link_host(host_obj)
     return LIB_PATH
 
 

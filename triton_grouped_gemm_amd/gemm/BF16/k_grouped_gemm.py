@@ -54,6 +54,10 @@ def k_grouped_gemm(A: Tensor, B: Tensor, size_per_group: Tensor, group_start: Op
     ``queue`` (not in the reference): the kernel's tile counters, ``_native.QUEUE_WORDS`` zeroed int32 on A's device
     that the caller owns -- for callers that must not allocate inside the call (graph capture); the kernel hands them
     back zeroed.  By default the library keeps one such tensor per device and stream."""
+    if group_start is None and group_end is None and not trans_b and A.is_cuda:
+        C = _native.host().k_grouped_gemm(A, B, size_per_group, numSM, _native.work_queue(A.device, queue))
+        if C is not None:
+            return C
     K_TOTAL, M_DIM, N_DIM, num_groups = _check_k_grouped_gemm_inputs(A, B, size_per_group, trans_b)
     assert 1 <= num_groups <= _native.MAX_GROUPS, f"between 1 and {_native.MAX_GROUPS} groups are supported"
     C = A.new_empty(num_groups, M_DIM, N_DIM)

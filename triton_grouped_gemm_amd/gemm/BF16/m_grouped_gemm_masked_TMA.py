@@ -18,6 +18,8 @@ def m_grouped_gemm_masked(lhs: Tensor, rhs: Tensor, out: Tensor, masked_m: Tenso
                           trans_b: bool = True) -> None:
     """lhs ``[G*m_max, K]``, rhs ``[G, N, K]``, out ``[G*m_max, N]``; ``expected_m`` is the row
     stride ``m_max`` between groups (the reference kernel uses it that way, :107-111)."""
+    if _native.host().m_grouped_gemm_masked(lhs, rhs, out, masked_m, expected_m, trans_b) is not None:
+        return None
     assert lhs.dim() == 2
     assert rhs.dim() == 3
     M, K = lhs.shape
