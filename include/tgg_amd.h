@@ -142,6 +142,11 @@ int tgg_per_token_cast_to_fp8(const void* x, void* codes, float* scales, int64_t
 int tgg_per_block_cast_to_fp8(const void* x, void* codes, float* scales, int batch, int R, int C, int fmt,
                               void* stream);
 
+/* Activation scales stored [M, kblocks] (row-major, as per_token_cast_to_fp8 of
+ * gemm/FP8/m_grouped_gemm_channel_expert.py:217-222 returns them) into the [kblocks, M] storage that the block-scaled GEMM
+ * streams (sa_mn_major = 1). */
+int tgg_scales_to_mn_major(const float* in, float* out, int64_t M, int kblocks, void* stream);
+
 /* Element-wise fp32 -> fp8 code with the conversion the quantizers use (test hook for the
  * `.to(torch.float8_*)` casts of the recipes above). */
 int tgg_cvt_f32_to_fp8(const float* in, void* out, int64_t n, int fmt, void* stream);

@@ -106,3 +106,37 @@ def test_other_entry_points_agree_with_their_wrappers(dev):
     probs = torch.rand(200, 2, device=dev)
     assert torch.equal(ops.unpermute(direct[0], where, probs), ops.unpermute(rows, where, probs))
     assert torch.equal(ops.permute_map(idx, num_experts=4)[0], ops.permute_map(idx.long(), num_experts=4)[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [128, 640, 8192])  # 1, 5 and 64 scale blocks per row
+@pytest.mark.parametrize("sizes", [[64], [1, 0, 200, 128], [130] * 5])
+def test_contiguous_entry_points_check_the_total_and_take_both_scale_layouts(dev, k, sizes):
+    """Row-major activation scales (turned by a kernel) give the bits of K-block-major ones; sizes that do not add up to A's
+    rows raise the reference's ValueError, before anything is written where the caller brings the output."""
+    from triton_grouped_gemm_amd.gemm.deep_gemm_ops import m_grouped_bf16_nt_contiguous, m_grouped_fp8_nt_contiguous
+    from triton_grouped_gemm_amd.quant.fp8_cast import per_block_cast_to_fp8, per_token_cast_to_fp8
+    s = torch.tensor(sizes, dtype=torch.int32, device=dev)
+    m, g, n = sum((v + 127) // 128 * 128 for v in sizes), len(sizes), 136
+    x = torch.randn(m, k, device=dev).to(torch.bfloat16)
+    w = torch.randn(g, n, k, device=dev).to(torch.bfloat16)
+    rows = torch.cat([torch.arange(v, device=dev) + i for v, i in
+                      zip(sizes, torch.tensor([0, *[(v + 127) // 128 * 128 for v in sizes]]).cumsum(0).tolist())])
+    wq = per_block_cast_to_fp8(w)
+    outs = [m_grouped_fp8_nt_contiguous(per_token_cast_to_fp8(x, scales_mn_major=mn), wq, sz)
+            for mn in (True, False) for sz in (s, s.long())]
+    assert all(torch.equal(o[rows], outs[0][rows]) for o in outs)
+    xq = per_token_cast_to_fp8(x)
+    kept = torch.zeros(m, n, dtype=torch.bfloat16, device=dev)
+    assert m_grouped_fp8_nt_contiguous(xq, wq, s, out=kept) is kept and torch.equal(kept[rows], outs[0][rows])
+    plain = m_grouped_bf16_nt_contiguous(x, w, s)
+    assert torch.equal(m_grouped_bf16_nt_contiguous(x, w, s, out=kept)[rows], plain[rows])
+    bad = s.clone()
+    bad[0] += 128
+    kept.fill_(7.0)
+    for call in (lambda **kw: m_grouped_fp8_nt_contiguous(xq, wq, bad, **kw), lambda **kw: m_grouped_bf16_nt_contiguous(x, w, bad, **kw)):
+        with pytest.raises(ValueError, match=f"expected M={m + 128}, got M={m}"):
+            call()
+        with pytest.raises(ValueError, match="padded expert rows"):
+            call(out=kept)
+    assert bool((kept == 7.0).all())

@@ -54,6 +54,7 @@ int num_cus() {
 int launch_trans_quant128(const void*, void*, float*, const GemmParams&, int64_t, void*, int, hipStream_t);
 int launch_token_cast128(const void*, void*, float*, int64_t, int, int, int, hipStream_t);
 int launch_block_cast128(const void*, void*, float*, int, int, int, int, hipStream_t);
+int launch_scales_transpose(const float*, float*, int64_t, int, hipStream_t);
 int launch_cvt_fp8(const float*, void*, int64_t, int, hipStream_t);
 bool fast_supported(const GemmParams& p, int dt, int layout);
 int launch_fast_16bit(const GemmParams& p, int dt, int layout, hipStream_t s);
@@ -490,6 +491,12 @@ int tgg_per_block_cast_to_fp8(const void* x, void* codes, float* scales, int bat
   if (batch < 0 || R < 0 || C < 0) return set_error("negative shape");
   if (!aligned16(x) || !aligned16(codes)) return set_error("operand pointers must be 16-byte aligned");
   return launch_block_cast128(x, codes, scales, batch, R, C, fmt, (hipStream_t)stream);
+}
+
+int tgg_scales_to_mn_major(const float* in, float* out, int64_t M, int kblocks, void* stream) {
+  if (!in || !out) return set_error("null pointer");
+  if (M < 0 || kblocks < 0 || (M + 63) / 64 >= (1ll << 24)) return set_error("bad M=%lld or kblocks=%d", (long long)M, kblocks);
+  return launch_scales_transpose(in, out, M, kblocks, (hipStream_t)stream);
 }
 
 int tgg_cvt_f32_to_fp8(const float* in, void* out, int64_t n, int fmt, void* stream) {

@@ -8,10 +8,12 @@
 // decided here that the wrappers do not decide too, and no state is kept.
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <c10/core/Event.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -252,7 +254,124 @@ PyObject* unpermute(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// The padded total of a contiguous layout against the rows of A (the reference reads it back too,
+// gemm/deep_gemm_ops.py:49-51).  The read-back is enqueued in front of the GEMM and waited for behind it, so the GPU has the
+// GEMM to work on meanwhile; the GEMM never touches rows at or beyond M, whatever the sizes say.
+class TotalCheck {
+ public:
+  TotalCheck(const at::Tensor& sizes, int64_t block_m, int64_t m)
+      : sizes_(sizes.to(at::TensorOptions(sizes.options()).device(at::kCPU), /*non_blocking=*/true)), event_(c10::DeviceType::CUDA),
+        block_m_(block_m), m_(m) {
+    // torch's streams and events carry the device type CUDA
+    const auto current = c10::hip::getCurrentHIPStream();
+    event_.record(c10::Stream(c10::Stream::UNSAFE, sizes.device(), current.id()));
+  }
+  // Whether the rows are as many as the sizes say; raises otherwise.
+  bool passes() {
+    Py_BEGIN_ALLOW_THREADS
+    event_.synchronize();
+    Py_END_ALLOW_THREADS
+    int64_t total = 0;
+    for (int64_t g = 0; g < sizes_.size(0); ++g) {
+      const int64_t v = sizes_.scalar_type() == at::kLong ? (int32_t)sizes_.const_data_ptr<int64_t>()[g] : sizes_.const_data_ptr<int32_t>()[g];
+      const int64_t up = v + block_m_ - 1;
+      total += (up >= 0 ? up / block_m_ : -((block_m_ - 1 - up) / block_m_)) * block_m_;
+    }
+    if (total == m_) return true;
+    PyErr_Format(PyExc_ValueError, "A must include padded expert rows: expected M=%lld, got M=%lld", (long long)total, (long long)m_);
+    return false;
+  }
+
+ private:
+  at::Tensor sizes_;
+  c10::Event event_;
+  const int64_t block_m_, m_;
+};
+
+bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
+
+// (a, b, sizes, out or None, block_m) -> out
+PyObject* m_grouped_bf16_contiguous(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  TGG_ARGS(5);
+  TGG_TENSOR(a, 0);
+  TGG_TENSOR(b, 1);
+  TGG_TENSOR(sizes, 2);
+  TGG_INT(block_m, 4);
+  if (a.dim() != 2 || b.dim() != 3 || capturing()) Py_RETURN_NONE;
+  const int64_t m = a.size(0), k = a.size(1), g = b.size(0), n = b.size(1);
+  if (a.scalar_type() != at::kBFloat16 || b.scalar_type() != at::kBFloat16 || b.size(2) != k || (n & 7) || (k & 7) || block_m < 1 ||
+      g > kMaxGroupsOther || !sizes_ok(sizes, g) || !a.is_contiguous() || !b.is_contiguous())
+    Py_RETURN_NONE;
+  at::Tensor c;
+  TotalCheck check(sizes, block_m, m);
+  if (args[3] != Py_None) {
+    TGG_TENSOR(out, 3);
+    if (out.scalar_type() != at::kBFloat16 || !out.is_contiguous() || out.numel() != m * n || out.requires_grad()) Py_RETURN_NONE;
+    if (!check.passes()) return nullptr;  // the caller's tensor stays as it is
+    c = out;
+  } else {
+    c = at::empty({m, n}, a.options());
+  }
+  PyObject* const result = done("tgg_m_grouped_gemm_padded", tgg_m_grouped_gemm_padded(a.data_ptr(), b.data_ptr(), c.data_ptr(),
+                                sizes.data_ptr(), is64(sizes), (int)g, m, (int)n, (int)k, (int)block_m, TGG_BF16, -1, stream()), c);
+  if (result && args[3] == Py_None && !check.passes()) {
+    Py_DECREF(result);
+    return nullptr;
+  }
+  return result;
+  END_HANDLE_TH_ERRORS
+}
+
+// (a codes, a scales, b codes, b scales, sizes, out or None, block_m) -> out
+PyObject* m_grouped_fp8_contiguous(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  TGG_ARGS(7);
+  TGG_TENSOR(a, 0);
+  TGG_TENSOR(sa_in, 1);
+  TGG_TENSOR(b, 2);
+  TGG_TENSOR(sb, 3);
+  TGG_TENSOR(sizes, 4);
+  TGG_INT(block_m, 6);
+  if (a.dim() != 2 || b.dim() != 3 || sa_in.dim() != 2 || sb.dim() != 3 || capturing()) Py_RETURN_NONE;
+  const int64_t m = a.size(0), k = a.size(1), g = b.size(0), n = b.size(1), kb = (k + 127) / 128, nb = (n + 127) / 128;
+  if (a.scalar_type() != at::kFloat8_e4m3fn || b.scalar_type() != at::kFloat8_e4m3fn || b.size(2) != k || (k & 15) || block_m < 128 ||
+      block_m % 128 || sa_in.size(0) != m || sa_in.size(1) != kb || sb.size(0) != g || sb.size(1) != nb || sb.size(2) != kb ||
+      sa_in.scalar_type() != at::kFloat || sb.scalar_type() != at::kFloat || !sb.is_contiguous() || g > kMaxGroupsOther ||
+      !sizes_ok(sizes, g) || !a.is_contiguous() || !b.is_contiguous() || m == 0)
+    Py_RETURN_NONE;
+  const bool mn_major = kb == 1 || (sa_in.stride(0) == 1 && sa_in.stride(1) == m);
+  if (!mn_major && !sa_in.is_contiguous()) Py_RETURN_NONE;
+  at::Tensor c;
+  TotalCheck check(sizes, block_m, m);
+  if (args[5] != Py_None) {
+    TGG_TENSOR(out, 5);
+    if (out.scalar_type() != at::kBFloat16 || !out.is_contiguous() || out.numel() != m * n || out.requires_grad()) Py_RETURN_NONE;
+    if (!check.passes()) return nullptr;  // the caller's tensor stays as it is
+    c = out;
+  } else {
+    c = at::empty({m, n}, a.options().dtype(at::kBFloat16));
+  }
+  at::Tensor sa = sa_in;
+  if (!mn_major) {  // the kernel streams one K block of all rows at a time
+    sa = at::empty({kb, m}, sa_in.options());
+    if (int rc = tgg_scales_to_mn_major((const float*)sa_in.data_ptr(), (float*)sa.data_ptr(), m, (int)kb, stream()))
+      return done("tgg_scales_to_mn_major", rc, c);
+  }
+  PyObject* const result = done("tgg_m_grouped_gemm_fp8_block", tgg_m_grouped_gemm_fp8_block(a.data_ptr(), (const float*)sa.data_ptr(),
+                                b.data_ptr(), (const float*)sb.data_ptr(), c.data_ptr(), sizes.data_ptr(), is64(sizes), (int)g, m, (int)n,
+                                (int)k, (int)block_m, 1, -1, stream()), c);
+  if (result && args[5] == Py_None && !check.passes()) {
+    Py_DECREF(result);
+    return nullptr;
+  }
+  return result;
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"m_grouped_bf16_contiguous", (PyCFunction)(void*)m_grouped_bf16_contiguous, METH_FASTCALL, nullptr},
+    {"m_grouped_fp8_contiguous", (PyCFunction)(void*)m_grouped_fp8_contiguous, METH_FASTCALL, nullptr},
     {"m_grouped_gemm", (PyCFunction)(void*)m_grouped_gemm, METH_FASTCALL, nullptr},
     {"m_grouped_gemm_masked", (PyCFunction)(void*)m_grouped_gemm_masked, METH_FASTCALL, nullptr},
     {"k_grouped_gemm", (PyCFunction)(void*)k_grouped_gemm, METH_FASTCALL, nullptr},

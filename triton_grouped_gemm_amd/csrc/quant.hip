@@ -384,6 +384,27 @@ __global__ __launch_bounds__(256) void block_cast128_kernel(const uint16_t* __re
   }
 }
 
+// [rows, cols] -> [cols, rows] for activation scales (cols = K / 128, a few dozen).  A workgroup takes 64 rows: one run
+// of memory in, 64-float runs out, 64 columns at a time through LDS.
+__global__ __launch_bounds__(256) void scales_transpose_kernel(const float* __restrict__ in, float* __restrict__ out,
+                                                              int64_t rows, int cols) {
+  __shared__ float t[64][65];
+  const int64_t r0 = (int64_t)blockIdx.x * 64;
+  const int n = (int)min((int64_t)64, rows - r0);
+  for (int c0 = 0; c0 < cols; c0 += 64) {
+    const int w = min(64, cols - c0);
+    for (int i = threadIdx.x; i < n * w; i += 256) {
+      const int r = i / w, c = i - r * w;
+      t[c][r] = in[(r0 + r) * cols + c0 + c];
+    }
+    __syncthreads();
+    const int r = threadIdx.x & 63;
+    if (r < n)
+      for (int c = threadIdx.x >> 6; c < w; c += 4) out[(int64_t)(c0 + c) * rows + r0 + r] = t[c][r];
+    __syncthreads();
+  }
+}
+
 template <int FMT>
 __global__ void cvt_fp8_kernel(const float* __restrict__ in, uint8_t* __restrict__ out, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -438,6 +459,12 @@ int launch_block_cast128(const void* x, void* codes, float* scales, int batch, i
   else
     return set_error("unsupported fp8 format code %d", fmt);
   return check_launch("block_cast128");
+}
+
+int launch_scales_transpose(const float* in, float* out, int64_t rows, int cols, hipStream_t s) {
+  if (rows == 0 || cols == 0) return 0;
+  hipLaunchKernelGGL(scales_transpose_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(256), 0, s, in, out, rows, cols);
+  return check_launch("scales_transpose");
 }
 
 int launch_cvt_fp8(const float* in, void* out, int64_t n, int fmt, hipStream_t s) {

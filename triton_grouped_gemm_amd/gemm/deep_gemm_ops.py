@@ -45,7 +45,7 @@ def _check_contiguous_layout(a: torch.Tensor, b: torch.Tensor, size_per_group: t
     # device.  While the stream is being captured into a graph no such read is possible, so the check is left out
     # there: the kernels never touch rows at or beyond M, whatever the sizes say.
     if not (size_per_group.is_cuda and torch.cuda.is_current_stream_capturing()):
-        expected_m = int(round_up_to_alignment(size_per_group.to(dtype=torch.int32), block_m).sum().item())
+        expected_m = int(round_up_to_alignment(size_per_group.cpu().to(dtype=torch.int32), block_m).sum())
         if m != expected_m:
             raise ValueError(f"A must include padded expert rows: expected M={expected_m}, got M={m}")
     if grouped_layout is not None:
@@ -126,6 +126,10 @@ def m_grouped_bf16_nt_contiguous(a: torch.Tensor, b: torch.Tensor, size_per_grou
                                  block_m: int = 128, use_psum_layout: bool = False) -> torch.Tensor:
     """a ``[M_padded, K]`` bf16, b ``[G, N, K]`` bf16 -> ``[M_padded, N]`` bf16
     (reference gemm/deep_gemm_ops.py:24-57)."""
+    if grouped_layout is None:
+        result = _native.host().m_grouped_bf16_contiguous(a, b, size_per_group, out, block_m)
+        if result is not None:
+            return result
     m, n, k, g = _check_contiguous_layout(a, b, size_per_group, block_m, grouped_layout, use_psum_layout, "a")
     if a.dtype != torch.bfloat16 or b.dtype != torch.bfloat16:
         raise ValueError("a and b must be bfloat16")
@@ -164,6 +168,10 @@ def m_grouped_fp8_nt_contiguous(a: Tuple[torch.Tensor, torch.Tensor], b: Tuple[t
     """
     a_codes, a_scale = a
     b_codes, b_scale = b
+    if grouped_layout is None and recipe_a in (None, (1, 128)) and recipe_b in (None, (128, 128)):
+        result = _native.host().m_grouped_fp8_contiguous(a_codes, a_scale, b_codes, b_scale, size_per_group, out, block_m)
+        if result is not None:
+            return result
     m, n, k, g = _check_contiguous_layout(a_codes, b_codes, size_per_group, block_m, grouped_layout,
                                           use_psum_layout, "a[0]")
     if recipe_a not in (None, (1, 128)) or recipe_b not in (None, (128, 128)):
