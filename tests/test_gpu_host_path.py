@@ -79,6 +79,40 @@ def test_what_is_left_to_the_operator(dev):
 
 
 @pytest.mark.gpu
+def test_forward_mode_and_tracing_are_left_to_the_autograd_functions(dev):
+    """A tangent or a trace must not be dropped: the autograd functions refuse the one and are recorded in the other."""
+    import torch.autograd.forward_ad as fwd
+    a, b, sizes = _operands(dev)
+    idx = torch.randint(0, 4, (200, 2), device=dev, dtype=torch.int32)
+    rows, where = ops.permute(a, idx, num_experts=4)
+    probs = torch.rand(200, 2, device=dev)
+    with fwd.dual_level():
+        for call in (lambda: ops.gmm(fwd.make_dual(a, a), b, sizes, True), lambda: ops.gmm(a, fwd.make_dual(b, b), sizes, True),
+                     lambda: ops.permute(fwd.make_dual(a, a), idx, num_experts=4),
+                     lambda: ops.unpermute(rows, where, fwd.make_dual(probs, probs))):
+            with pytest.raises(RuntimeError, match="jvp|forward"):
+                call()
+    traced = torch.jit.trace(lambda x: m_grouped_gemm(x, b, sizes, True), (a,), check_trace=False)
+    assert torch.equal(traced(a * 2), m_grouped_gemm(a * 2, b, sizes, True))
+
+
+@pytest.mark.gpu
+def test_permute_gives_zeros_where_no_gradient_arrives(dev):
+    class Stop(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.sum()
+
+        @staticmethod
+        def backward(ctx, _):
+            return None
+    x = torch.randn(16, 8, device=dev, requires_grad=True)
+    idx = torch.randint(0, 4, (16, 2), device=dev, dtype=torch.int32)
+    grad, = torch.autograd.grad(Stop.apply(ops.permute(x, idx, num_experts=4)[0]), x)
+    assert torch.equal(grad, torch.zeros_like(x))
+
+
+@pytest.mark.gpu
 def test_other_entry_points_agree_with_their_wrappers(dev):
     """Strided copies of the operands, which the native path refuses, against the same operands as they are."""
     a, b, sizes = _operands(dev)

@@ -24,7 +24,8 @@ namespace {
 
 constexpr int64_t kMaxGroups = 1024, kMaxGroupsOther = 512, kMaxExperts = 1024;
 
-// A plain torch.Tensor (or Parameter) on the current GPU, without functorch or Python layers around it; null otherwise.
+// A plain torch.Tensor (or Parameter) on the current GPU, without functorch or Python layers around it and without a
+// forward-mode tangent (the wrappers' autograd functions have no jvp and say so); null otherwise.
 // device: the current GPU, looked up (-1 before) once a tensor on some GPU has been seen.
 const at::Tensor* plain(PyObject* o, c10::DeviceIndex& device) {
   if (!THPVariable_CheckExact(o)) return nullptr;
@@ -34,13 +35,14 @@ const at::Tensor* plain(PyObject* o, c10::DeviceIndex& device) {
   if (t.device().index() != device) return nullptr;
   static const c10::DispatchKeySet layered({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
                                             c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize,
-                                            c10::DispatchKey::Conjugate, c10::DispatchKey::Negative});
-  return t.key_set().has_any(layered) ? nullptr : &t;
+                                            c10::DispatchKey::Conjugate, c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor,
+                                            c10::DispatchKey::Batched});
+  return t.key_set().has_any(layered) || t._fw_grad(/*level=*/0).defined() ? nullptr : &t;
 }
 
 bool modes_active() {
   static const c10::DispatchKeySet watched({c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::Functionalize,
-                                            c10::DispatchKey::Python});
+                                            c10::DispatchKey::Python, c10::DispatchKey::Tracer});
   return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() ||
          c10::impl::tls_local_dispatch_key_set().included_.has_any(watched);
 }
