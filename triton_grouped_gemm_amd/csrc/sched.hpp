@@ -445,13 +445,13 @@ struct QueueDraw {
 
   TGG_DEV void first() { while (wanted()) draw_now(); }
 
-  // Requests a draw; `answer` is in flight until take().  Only lane 0 adds, by the execution mask and not by a branch:
-  // a branch of lanes would join in front of take(), and the compiler must have no reason to move `answer`.
+  // Requests a draw; `answer` is in flight until take().  A builtin, so that the compiler knows of the register in flight
+  // and waits wherever it might touch it.  The address is made a lane's own: for one that the wave shares the compiler
+  // merges the lanes' additions and reads the result back on the spot, which is the wait that this is to avoid.
   TGG_DEV void request() {
-    const int32_t* const at = p.queue + counter();
-    uint64_t saved;
-    asm volatile("s_mov_b64 %1, exec\n\ts_mov_b64 exec, 1\n\tglobal_atomic_add %0, %2, %3, off sc0\n\ts_mov_b64 exec, %1"
-                 : "=v"(answer), "=&s"(saved) : "v"(at), "v"(1) : "memory");
+    int at = counter();
+    asm("" : "+v"(at));
+    if (lane_id() == 0) answer = __hip_atomic_fetch_add(p.queue + at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
   // The drawing wave, after it has waited for all of its memory operations and in front of a workgroup barrier.
