@@ -128,6 +128,7 @@ def test_feeds_the_grouped_gemm(dev):
     (1024, 128, 8, 40), (1025, 128, 8, 40),        # the last one-launch size and the first one behind it
     (3001, 1024, 7, 8), (9001, 5, 3, 24),          # table columns shared by no / many threads, ragged last chunk
     (33000, 1000, 8, 8), (70001, 1, 2, 8),         # a table that needs the scan launch; a single expert
+    (8533, 64, 8, 2048), (8534, 64, 8, 2048),      # the last rows moved by the placing launch and the first by their own
     (8, 1024, 1100, 16), (20, 600, 500, 2056)])    # more assignments per token than one batch holds; several batches
 def test_sort_paths(dev, num_token, num_expert, topk, hidden):
     """Every path of the sort at its edges: map, counts and moved rows are bit-exact, with ids drawn with repetition,

@@ -17,8 +17,13 @@
 // destination = expert start + assignments of the expert in front; row_id_map[k * tokens + t] gets it (or -1 for
 // dropped assignments: expert -1, or destination beyond the capacity).
 //
-// Measured against four launches for the sort and one for the rows: 8192 tokens x top-8, 128 experts, 4 KB rows 72 ->
-// 61 us (of which the rows alone take 49); 24 tokens 26 -> 4.4 us.
+//   * rows of more than kPlaceMoveBytes: the placing launch makes the map and a launch with a workgroup per token moves
+//     the rows.  A thousand placing workgroups stream at 4.9 TB/s and the short ones at 5.6, which outweighs the launch
+//     from 300 to 600 MB read and written on (moved by the placing launch / by their own: top-8 of 4096 4 KB rows 29 /
+//     34 us, 12288 101 / 103, 24576 197 / 182, 81920 645 / 577; top-1 of 81920 2 KB rows 77 / 68; 8192 rows, with the
+//     unpermute and both gradients behind it, 304 / 316).
+// Measured against four launches for the sort and one for the rows: 8192 tokens x top-8, 128 experts, 4 KB rows 70 ->
+// 67 us, 81920 tokens 589 -> 577, 4096 tokens 43 -> 29, 24 tokens 26 -> 4.4.
 //
 // The row movers are streaming kernels (16-byte accesses, fp32 arithmetic), bound by memory:
 //   place           reads each token row once and writes it to its up to topK destinations
@@ -37,6 +42,7 @@ constexpr int kCountThreads = 1024;
 constexpr int kMaxExperts = 1024;
 constexpr int64_t kSmallAssignments = 8192;  // one-launch sort up to here
 constexpr int64_t kTableEntries = 16384;     // the placing workgroups sum the count table themselves up to here
+constexpr int64_t kPlaceMoveBytes = 300ll << 20;  // the placing workgroups move the rows too up to here (bytes read and written)
 constexpr int kPlaceThreads = 512;
 constexpr int kBatch = 1024;                 // assignments whose destinations a placing workgroup holds at a time
 
@@ -513,7 +519,8 @@ int launch_moe_permute(const void* in, void* out, int64_t row_bytes, const int32
   const int64_t n = tokens * topk, cus = num_cus();
   MoveArgs a;
   a.chunks16 = (int)(row_bytes / 16);
-  const bool move = in && tokens > 0 && a.chunks16 <= (1 << 20);  // a batch's chunks are counted in 32 bits
+  const bool move = in && tokens > 0 && a.chunks16 <= (1 << 20) &&  // a batch's chunks are counted in 32 bits
+                    (small_sort(n, topk) || (n + tokens) * row_bytes <= kPlaceMoveBytes);
   a.in = move ? (const i32x4_t*)in : nullptr;
   a.out = (i32x4_t*)out;
   a.indices = indices;
