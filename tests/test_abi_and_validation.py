@@ -2,6 +2,8 @@
 validation raises the reference's errors before anything touches a GPU."""
 import ctypes
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import pytest
@@ -75,6 +77,25 @@ def test_group_count_limits_per_entry_point():
     assert "G=1025 outside [1, 1024]" in _native.last_error()
     assert lib.tgg_k_grouped_gemm(p, p, p, p, p, _native.MAX_GROUPS + 1, 128, 128, 1024, 0, -1, None) == 1
     assert "G=1025 outside [1, 1024]" in _native.last_error()
+
+
+def test_empty_expert_assignment_returns_from_the_sort():
+    """No tokens, for every number of experts per token: the sort returns (with an error where there is no GPU to launch
+    on) and needs no workspace.  In a process of its own: a division by zero ends the whole process."""
+    code = """
+import ctypes
+from triton_grouped_gemm_amd import _native
+lib = _native.load()
+need = ctypes.c_int64(-1)
+for topk in (1, 8, 1024, 1025, 1100):
+    assert lib.tgg_moe_sort_workspace_bytes(0, topk, 8, ctypes.byref(need)) == 0 and need.value == 0, need.value
+    lib.tgg_moe_permute_map(None, 0, topk, 8, 0, None, None, 0, None, 0, None)
+    lib.tgg_moe_permute_map_static(None, 0, topk, 8, 0, None, None, 0, None)
+    lib.tgg_moe_permute(None, None, None, 0, topk, 8, 0, 64, 0, None, None, 0, None, 0, None)
+print("returned")
+"""
+    run = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0 and "returned" in run.stdout, (run.returncode, run.stderr[-500:])
 
 
 def test_reference_import_paths_resolve():

@@ -106,6 +106,12 @@ def test_empty_input_passes_through(dev):
     assert out.numel() == 0 and rmap is None
 
 
+@pytest.mark.parametrize("topk", [1, 8, 1024, 1100])
+def test_empty_assignment_counts_are_zero(dev, topk):
+    rmap, counts = ops.permute_map(torch.empty((0, topk), dtype=torch.int32, device=dev), num_experts=40)
+    assert rmap.numel() == 0 and torch.equal(counts.cpu(), torch.zeros(40, dtype=torch.int32))
+
+
 def test_feeds_the_grouped_gemm(dev):
     """permute -> grouped GEMM with the counts as size_per_group -> unpermute equals the dense per-token formula."""
     T, E, H, N, topk = 512, 8, 128, 64, 2

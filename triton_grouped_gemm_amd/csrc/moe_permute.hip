@@ -503,8 +503,9 @@ SortWorkspace carve(void* base, int64_t n, int num_experts) {
   return w;
 }
 
-// Whether the one-launch sort takes the problem.
-bool small_sort(int64_t n, int topk) { return n <= kSmallAssignments && topk <= kBatch; }
+// Whether the one-launch sort takes the problem.  No assignments at all are always its own: the counting and placing
+// launches would have empty grids.
+bool small_sort(int64_t n, int topk) { return n == 0 || (n <= kSmallAssignments && topk <= kBatch); }
 
 }  // namespace
 
