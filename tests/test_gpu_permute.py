@@ -112,6 +112,17 @@ def test_empty_assignment_counts_are_zero(dev, topk):
     assert rmap.numel() == 0 and torch.equal(counts.cpu(), torch.zeros(40, dtype=torch.int32))
 
 
+def test_unpermute_without_probs_asks_for_an_entry_per_row(dev):
+    """More rows than map entries (a capacity above the token count) are refused, not read beyond the map."""
+    x, indices, _ = _case(100, 8, 64, 1, torch.bfloat16)
+    rows, rmap = ops.permute(x.to(dev), indices.to(dev), num_out_tokens=160, num_experts=8)
+    assert rows.shape == (160, 64) and rmap.numel() == 100
+    for r in (rows, rows.clone().requires_grad_(True)):
+        with pytest.raises(RuntimeError, match="`row_id_map` shape mismatch! Expect 160, but got 100"):
+            ops.unpermute(r, rmap)
+    assert torch.equal(ops.unpermute(rows[:100].contiguous(), rmap).cpu(), x)
+
+
 def test_feeds_the_grouped_gemm(dev):
     """permute -> grouped GEMM with the counts as size_per_group -> unpermute equals the dense per-token formula."""
     T, E, H, N, topk = 512, 8, 128, 64, 2

@@ -249,6 +249,8 @@ PyObject* unpermute(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     tokens = probs.size(0);
     topk = probs.size(1);
     weights = (const float*)probs.data_ptr();
+  } else if (map.numel() < tokens) {  // fewer entries than rows of x: the wrapper raises
+    Py_RETURN_NONE;
   }
   at::Tensor out = at::empty({tokens, x.size(1)}, x.options());
   return done("tgg_moe_unpermute", tgg_moe_unpermute(x.data_ptr(), out.data_ptr(), (const int32_t*)map.data_ptr(), weights, tokens,
