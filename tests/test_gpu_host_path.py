@@ -174,3 +174,23 @@ def test_contiguous_entry_points_check_the_total_and_take_both_scale_layouts(dev
         with pytest.raises(ValueError, match="padded expert rows"):
             call(out=kept)
     assert bool((kept == 7.0).all())
+
+
+@pytest.mark.gpu
+def test_one_block_of_activation_scales_with_any_stride(dev):
+    """K = 128: a column of a wider scale tensor and one scale expanded over the rows give what contiguous copies give, on
+    the native path (sizes on the GPU) and through the wrapper (sizes on the host)."""
+    from triton_grouped_gemm_amd.gemm.deep_gemm_ops import m_grouped_fp8_nt_contiguous
+    from triton_grouped_gemm_amd.quant.fp8_cast import per_block_cast_to_fp8
+    g = torch.Generator().manual_seed(11)
+    s = torch.tensor([128, 100, 0], dtype=torch.int32, device=dev)
+    codes = torch.randn(256, 128, generator=g).to(dev).to(torch.float8_e4m3fn)
+    wq = per_block_cast_to_fp8(torch.randn(3, 72, 128, generator=g).to(torch.bfloat16).to(dev))
+    wide = torch.rand(256, 5, generator=g).to(dev) + 0.5
+    for scale in (wide[:, 3:4], wide[7:8, :1].expand(256, 1), wide[:, 2:3].contiguous()):
+        want = m_grouped_fp8_nt_contiguous((codes, scale.clone(memory_format=torch.contiguous_format)), wq, s)
+        for sizes in (s, s.cpu()):
+            got = m_grouped_fp8_nt_contiguous((codes, scale), wq, sizes)
+            assert torch.equal(got[:228], want[:228])
+    exact = codes.float()[:128] @ (wq[0][0].float() * wq[1][0, 0, 0]).t() * wide[:128, 2:3]
+    assert float((want[:128].float() - exact).abs().max() / exact.abs().max()) < 2.0 ** -7

@@ -344,7 +344,7 @@ PyObject* m_grouped_fp8_contiguous(PyObject*, PyObject* const* args, Py_ssize_t 
       sa_in.scalar_type() != at::kFloat || sb.scalar_type() != at::kFloat || !sb.is_contiguous() || g > kMaxGroupsOther ||
       !sizes_ok(sizes, g) || !a.is_contiguous() || !b.is_contiguous() || m == 0)
     Py_RETURN_NONE;
-  const bool mn_major = kb == 1 || (sa_in.stride(0) == 1 && sa_in.stride(1) == m);
+  const bool mn_major = kb == 1 ? sa_in.is_contiguous() : sa_in.stride(0) == 1 && sa_in.stride(1) == m;
   if (!mn_major && !sa_in.is_contiguous()) Py_RETURN_NONE;
   at::Tensor c;
   TotalCheck check(sizes, block_m, m);

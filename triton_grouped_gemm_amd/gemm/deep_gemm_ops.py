@@ -193,7 +193,9 @@ def m_grouped_fp8_nt_contiguous(a: Tuple[torch.Tensor, torch.Tensor], b: Tuple[t
     # the tuned kernel streams the activation scales one K block (= one row of a [K/128, M] array) per
     # slab: a scale tensor that is already stored that way (strides (1, M)) is used as is
     sa = a_scale.to(torch.float32)
-    if sa.stride() != (1, m) and kb > 1:
+    if kb <= 1:
+        sa = sa.contiguous()  # one block: the rows' scales behind one another (a column of a wider tensor is copied)
+    elif sa.stride() != (1, m):
         sa = sa.t().contiguous().t()
     sb = b_scale.to(torch.float32).contiguous()
     if grouped_layout is not None and not use_psum_layout:  # per-row form: experts' regions in any order
