@@ -186,6 +186,18 @@ def test_contiguous_entry_validation():
         m_grouped_fp8_nt_contiguous((aq, torch.zeros(256, 1)), (bq, torch.zeros(2, 1, 1)), s, recipe_a=(1, 64))
 
 
+@pytest.mark.parametrize("rows,groups", [(6, 1), (6, 3), (1, 1), (1, 4)])
+def test_expert_major_scales_are_stored_as_the_kernel_reads_them(rows, groups):
+    """Element (row, g) at g * rows + row of the storage, whatever the strides of the scales that came in."""
+    from triton_grouped_gemm_amd.gemm.FP8.k_grouped_gemm_channel_expert import _expert_major
+    wide = torch.arange(rows * groups * 4, dtype=torch.float32).view(rows * 2, groups * 2)
+    for scale in (wide[:rows, :groups], wide[::2, 1::2], wide[:1, :1].expand(rows, groups), wide.t()[:groups, :rows].t(),
+                  torch.rand(groups, rows).t()):
+        got = _expert_major(scale, rows, groups)
+        assert torch.equal(got, scale)
+        assert torch.equal(torch.as_strided(got, (rows * groups,), (1,)), scale.t().reshape(-1))
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_native, "_lib", None)
     monkeypatch.setattr(_native, "LIB_PATH", tmp_path / "libtgg_amd.so")

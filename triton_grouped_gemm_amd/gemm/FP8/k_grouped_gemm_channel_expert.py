@@ -23,9 +23,7 @@ def _expert_major(scale: Tensor, rows: int, groups: int) -> Tensor:
     ``[rows, G]`` tensor already has strides ``(1, rows)``."""
     assert tuple(scale.shape) == (rows, groups), f"scale must have shape ({rows}, {groups})"
     s = scale.to(torch.float32)
-    if s.stride() == (1, rows) or groups == 1:
-        return s
-    return s.t().contiguous().t()
+    return s if s.stride() == (1, rows) else s.t().contiguous().t()
 
 
 def matmul(x_fp8: Tensor, x_scale: Tensor, y_fp8: Tensor, y_scale: Tensor, tokens_per_expert: Tensor,
