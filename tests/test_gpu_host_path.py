@@ -194,3 +194,22 @@ def test_one_block_of_activation_scales_with_any_stride(dev):
             assert torch.equal(got[:228], want[:228])
     exact = codes.float()[:128] @ (wq[0][0].float() * wq[1][0, 0, 0]).t() * wide[:128, 2:3]
     assert float((want[:128].float() - exact).abs().max() / exact.abs().max()) < 2.0 ** -7
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", range(4))
+def test_fp8_gemm_refuses_the_gradient_of_every_operand(dev, which):
+    """The operator has no derivative: backward through it says so, whichever operand asks for a gradient, and a call
+    that records nothing is answered as before."""
+    sizes = torch.tensor([5, 0, 11], dtype=torch.int32, device=dev)
+    operands = [torch.randn(16, 32, device=dev).to(torch.float8_e4m3fn), torch.rand(16, 1, device=dev),
+                torch.randn(3, 24, 32, device=dev).to(torch.float8_e4m3fn), torch.rand(3, 24, device=dev)]
+    want = gmm_fp8_act_per_channel_w_per_expert(*operands, sizes)
+    operands[which] = torch.nn.Parameter(operands[which])
+    out = gmm_fp8_act_per_channel_w_per_expert(*operands, sizes)
+    assert out.requires_grad and torch.equal(out, want)
+    with pytest.raises(RuntimeError, match="autograd"):
+        out.sum().backward()
+    with torch.no_grad():
+        out = gmm_fp8_act_per_channel_w_per_expert(*operands, sizes)
+    assert not out.requires_grad and torch.equal(out, want)

@@ -162,7 +162,7 @@ PyObject* m_grouped_gemm_fp8_channel(PyObject*, PyObject* const* args, Py_ssize_
   TGG_TENSOR(sb, 3);
   TGG_TENSOR(sizes, 4);
   TGG_TRUTH(fp16, 5);
-  if (a.dim() != 2 || b.dim() != 3 || records(sa) || records(sb)) Py_RETURN_NONE;
+  if (a.dim() != 2 || b.dim() != 3 || records(a) || records(sa) || records(b) || records(sb)) Py_RETURN_NONE;
   const int64_t m = a.size(0), k = a.size(1), g = b.size(0), n = b.size(1);
   const int fa = code8(a), fb = code8(b);
   if (fa < 0 || fb < 0 || b.size(2) != k || sa.numel() != m || sb.numel() != g * n || sa.scalar_type() != at::kFloat ||
