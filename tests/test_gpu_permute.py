@@ -123,6 +123,36 @@ def test_unpermute_without_probs_asks_for_an_entry_per_row(dev):
     assert torch.equal(ops.unpermute(rows[:100].contiguous(), rmap).cpu(), x)
 
 
+@pytest.mark.parametrize("num_token,hidden,topk", [
+    (102400, 512, 3), (102401, 512, 3), (110000, 504, 3),  # the row width and the size from which rows are taken singly
+    (50001, 1544, 4), (16001, 2640, 5), (70001, 2048, 2)])  # 4 waves a token, the last one ragged; 6; pairs
+def test_unpermute_of_many_rows_equals_its_parts(dev, num_token, hidden, topk):
+    """The sum of a token's rows has the same bits however many of them are in flight: a large call against calls on
+    runs of its tokens, and those against fp32 torch."""
+    g = torch.Generator(device=dev).manual_seed(num_token)
+    rows = torch.randn(num_token * topk, hidden, device=dev, dtype=torch.bfloat16, generator=g)
+    rmap = torch.randperm(num_token * topk, device=dev, generator=g).int()
+    rmap[::11] = -1
+    probs = torch.rand(num_token, topk, device=dev, generator=g)
+    for p in (probs, torch.ones_like(probs)):
+        whole = ops.unpermute(rows, rmap, p)
+        for t0 in range(0, num_token, num_token // 5):
+            part = slice(t0, min(num_token, t0 + num_token // 5))
+            src = rmap.view(topk, num_token)[:, part].contiguous()
+            assert torch.equal(whole[part], ops.unpermute(rows, src.reshape(-1), p[part].contiguous()))
+        picked = torch.where((src >= 0)[..., None], rows[src.clamp_min(0).long()].float(), 0.0)
+        _close(whole[part], (picked * p[part].t()[..., None]).sum(0).cpu(), torch.bfloat16, topk + 1)
+
+
+@pytest.mark.parametrize("num_token,hidden", [(2 ** 24 + 5, 8), (2 ** 23 + 3, 1032)])
+def test_unpermute_beyond_the_waves_of_one_launch(dev, num_token, hidden):
+    """More pieces (64 chunks of a token) than the launch has waves: one a token, and three."""
+    rows = torch.empty(num_token, hidden, device=dev, dtype=torch.bfloat16)
+    rows.view(torch.int16).copy_((torch.arange(num_token * hidden, device=dev) % 16001).view(num_token, hidden))
+    rmap = torch.arange(num_token - 1, -1, -1, device=dev, dtype=torch.int32)
+    assert torch.equal(ops.unpermute(rows, rmap), rows.flip(0))
+
+
 def test_feeds_the_grouped_gemm(dev):
     """permute -> grouped GEMM with the counts as size_per_group -> unpermute equals the dense per-token formula."""
     T, E, H, N, topk = 512, 8, 128, 64, 2

@@ -377,18 +377,29 @@ template <> struct Elem<DT_F32> {
 };
 
 // out[t, :] = sum_k prob[t, k] * in[row_id_map[k * tokens + t], :]   (prob == nullptr: plain sum)
-// A wave takes 64 neighbouring 16-byte chunks of one token (so the map and the weights are scalar loads) and requests
-// KU rows before it adds the first: 8192 x top-8 rows of 4 KB in 48-50 us, 6.1 TB/s (the card copies at 4.9 and reads at
-// 6.2), a little faster than one row at a time by a workgroup per token, and without idle waves on narrow rows.
+// Bound by memory.  A wave takes 64 neighbouring 16-byte chunks of one token (so the map and the weights are scalar loads,
+// and narrow rows leave no wave idle) and requests KU rows before it adds the first (one_row_at_a_time below says how
+// many).  A workgroup per token, one row at a time, against this: 8192 x top-6 rows of 528 B 12.6 -> 6.3 us, 8192 x top-8 of
+// 4 KB 47.0 -> 46.2 (6.3 TB/s; the card copies at 4.9 and reads at 6.2), of 14 KB 218 -> 206, 81920 x top-8 of 4 KB 574 ->
+// 572, 65536 x top-1 of 4 KB 100.6 -> 101.4.  A wave of a top-1 launch has two short loads to wait for, so what it does
+// before it requests its row shows: a 64-bit division for its token and a wait for the weight cost 2.5 % there.
 template <int DT, int KU>
 __global__ __launch_bounds__(256) void moe_unpermute_kernel(const char* __restrict__ in, char* __restrict__ out,
                                                             const int32_t* __restrict__ row_id_map,
                                                             const float* __restrict__ prob, int64_t tokens, int topk,
-                                                            int chunks16, int waves_per_token, int64_t waves) {
+                                                            int chunks16, uint32_t waves_per_token, int shift,
+                                                            uint32_t step_tokens, uint32_t step_pieces) {
   constexpr int N = Elem<DT>::N;
-  for (int64_t w = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); w < waves; w += (int64_t)gridDim.x * 4) {
-    const int64_t t = w / waves_per_token;
-    const int c = (int)(w - t * waves_per_token) * 64 + lane_id();
+  // the launch's waves, four a workgroup and at most 2^24, walk the pieces of all tokens in order
+  const uint32_t w = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t first = shift >= 0 ? w >> shift : w / waves_per_token;
+  uint32_t piece = w - first * waves_per_token;
+  for (int64_t t = first; t < tokens; t += step_tokens, piece += step_pieces) {
+    if (piece >= waves_per_token) {
+      piece -= waves_per_token;
+      if (++t >= tokens) break;
+    }
+    const int c = (int)piece * 64 + lane_id();
     if (c >= chunks16) continue;
     float acc[N];
 #pragma unroll
@@ -402,8 +413,10 @@ __global__ __launch_bounds__(256) void moe_unpermute_kernel(const char* __restri
         const int k = k0 + u;
         const int src = k < topk ? row_id_map[(int64_t)k * tokens + t] : -1;
         kept[u] = src >= 0;
-        weight[u] = prob && k < topk ? prob[t * topk + k] : 1.f;
-        if (kept[u]) row[u] = *(const i32x4_t*)(in + ((int64_t)src * chunks16 + c) * 16);
+        if (kept[u]) {  // the weight behind the row's request, which would otherwise wait for it too
+          row[u] = *(const i32x4_t*)(in + ((int64_t)src * chunks16 + c) * 16);
+          weight[u] = prob ? prob[t * topk + k] : 1.f;
+        }
       }
 #pragma unroll
       for (int u = 0; u < KU; ++u)
@@ -631,16 +644,29 @@ int launch_moe_permute_rows(const void* in, void* out, const int32_t* row_id_map
     else LAUNCH(4); \
   } while (0)
 
+// The forward kernel one row at a time: from 400 MiB read and written on, where the rows come from memory rather than from
+// the memory-side cache and are the faster the fewer are in flight at once (top-8 rows of 4 KB, four / one: 144 MiB 23.0 /
+// 22.6 us, 288 MiB 46.5 / 46.9, 432 MiB 89.3 / 88.7, 1700 MiB 347.5 / 338.2; top-4 and top-6 alike).  Top-2 rows are 0.6 %
+// faster in pairs at every size; rows below 1 KB (several tokens a workgroup) want all requests they can have (512 B, top-8,
+// 864 MiB: 199.7 / 224.9).
+static bool one_row_at_a_time(int64_t tokens, int topk, int c16) {
+  return topk > 2 && c16 >= 64 && tokens * (topk + 1) * c16 * 16 > (400ll << 20);
+}
+
 template <int DT>
 static void launch_unpermute_dt(const void* in, void* out, const int32_t* row_id_map, const float* prob, int64_t tokens,
                                 int topk, int c16, hipStream_t s) {
   const int per_token = (c16 + 63) / 64;
-  const int64_t waves = tokens * per_token, wgs = (waves + 3) / 4;
+  const int64_t wgs = (tokens * per_token + 3) / 4;
   const dim3 grid((unsigned)(wgs < (1 << 22) ? wgs : 1 << 22));  // a launch's threads stay below 2^32
+  const uint32_t step_tokens = grid.x * 4 / per_token, step_pieces = grid.x * 4 % per_token;
+  const int shift = (per_token & (per_token - 1)) == 0 ? __builtin_ctz(per_token) : -1;
 #define TGG_LAUNCH(KU) \
   hipLaunchKernelGGL((moe_unpermute_kernel<DT, KU>), grid, dim3(256), 0, s, (const char*)in, (char*)out, \
-                     row_id_map, prob, tokens, topk, c16, per_token, waves)
-  TGG_BY_TOPK(TGG_LAUNCH);
+                     row_id_map, prob, tokens, topk, c16, (uint32_t)per_token, shift, step_tokens, step_pieces)
+  if (topk <= 1 || one_row_at_a_time(tokens, topk, c16)) TGG_LAUNCH(1);
+  else if (topk <= 2) TGG_LAUNCH(2);
+  else TGG_LAUNCH(4);
 #undef TGG_LAUNCH
 }
 
