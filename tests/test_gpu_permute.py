@@ -153,6 +153,34 @@ def test_unpermute_beyond_the_waves_of_one_launch(dev, num_token, hidden):
     assert torch.equal(ops.unpermute(rows, rmap), rows.flip(0))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("num_token,chunks,topk", [
+    (16384, 256, 3), (16385, 256, 3), (16385, 256, 8), (20001, 256, 1), (18000, 240, 2), (18000, 241, 2), (17001, 257, 5)])
+def test_unpermute_backward_of_many_rows_equals_its_parts(dev, dtype, num_token, chunks, topk):
+    """The gradients have the same bits on either side of the sizes that take rows singly: a large call against calls on
+    runs of its tokens, and those against fp32 torch."""
+    g = torch.Generator(device=dev).manual_seed(num_token + chunks)
+    hidden = chunks * 16 // torch.empty(0, dtype=dtype).element_size()
+    rows = torch.randn(num_token * topk, hidden, device=dev, generator=g).to(dtype).requires_grad_(True)
+    grad = torch.randn(num_token, hidden, device=dev, generator=g).to(dtype)
+    rmap = torch.randperm(num_token * topk, device=dev, generator=g).int()
+    rmap[::7] = -1
+    probs = torch.rand(num_token, topk, device=dev, generator=g).requires_grad_(True)
+    whole = torch.autograd.grad(ops.unpermute(rows, rmap, probs), (rows, probs), grad)
+    for t0 in range(0, num_token, num_token // 4):
+        part = slice(t0, min(num_token, t0 + num_token // 4))
+        src = rmap.view(topk, num_token)[:, part].contiguous()
+        p = probs.detach()[part].contiguous().requires_grad_(True)
+        got = torch.autograd.grad(ops.unpermute(rows, src.reshape(-1), p), (rows, p), grad[part])
+        kept = src[src >= 0].long()
+        assert torch.equal(got[0][kept], whole[0][kept]) and torch.equal(got[1], whole[1][part])
+    scaled = (p.detach().t()[..., None] * grad[part].float())[src >= 0]
+    _close(got[0][kept], scaled.cpu(), dtype)
+    dots = torch.where(src >= 0, (rows.detach()[src.clamp_min(0).long()].double() * grad[part].double()).sum(-1), 0.0).t()
+    # a sum of `hidden` products of normal numbers in fp32: the error grows like the square root of their number
+    assert float((got[1].double() - dots).abs().max()) < 8 * 2.0 ** -24 * hidden
+
+
 def test_feeds_the_grouped_gemm(dev):
     """permute -> grouped GEMM with the counts as size_per_group -> unpermute equals the dense per-token formula."""
     T, E, H, N, topk = 512, 8, 128, 64, 2

@@ -434,7 +434,7 @@ __global__ __launch_bounds__(256) void moe_unpermute_kernel(const char* __restri
 // act_grad[dest, :] = prob[t, k] * grad[t, :];  prob_grad[t, k] = sum_h grad[t, h] * fwd_in[dest, h]
 // One workgroup per token; KU forward rows are requested together and their dot products reduced together, with one
 // barrier for all (two per row before): 8192 x top-8 rows of 4 KB 118 -> 113 us, 5.05 TB/s, half of it written.
-template <int DT, int KU>
+template <int DT, int KU, bool SINGLE>
 __global__ __launch_bounds__(256) void moe_unpermute_bwd_kernel(const char* __restrict__ grad, const char* __restrict__ fwd_in,
                                                                 const int32_t* __restrict__ row_id_map,
                                                                 const float* __restrict__ prob, char* __restrict__ act_grad,
@@ -451,14 +451,14 @@ __global__ __launch_bounds__(256) void moe_unpermute_bwd_kernel(const char* __re
     for (int u = 0; u < KU; ++u) {
       const int k = k0 + u;
       dest[u] = k < topk ? row_id_map[(int64_t)k * tokens + t] : -1;
-      weight[u] = prob && k < topk ? prob[t * topk + k] : 1.f;
+      weight[u] = prob && k < topk && (!SINGLE || dest[u] >= 0) ? prob[t * topk + k] : 1.f;
       dot[u] = 0.f;
     }
     for (int c = threadIdx.x; c < chunks16; c += 256) {
       i32x4_t row[KU];
       float g[N];
       Elem<DT>::unpack(*(const i32x4_t*)(grad + (t * chunks16 + c) * 16), g);
-      if (prob_grad) {
+      if (prob_grad && !SINGLE) {
 #pragma unroll
         for (int u = 0; u < KU; ++u)
           if (dest[u] >= 0) row[u] = *(const i32x4_t*)(fwd_in + ((int64_t)dest[u] * chunks16 + c) * 16);
@@ -471,6 +471,10 @@ __global__ __launch_bounds__(256) void moe_unpermute_bwd_kernel(const char* __re
           for (int j = 0; j < N; ++j) s[j] = weight[u] * g[j];
           Elem<DT>::store(act_grad + ((int64_t)dest[u] * chunks16 + c) * 16, s);
           if (prob_grad) {
+            if (SINGLE) {
+              asm volatile("" ::: "memory");  // the store stays in front of the read
+              row[u] = *(const i32x4_t*)(fwd_in + ((int64_t)dest[u] * chunks16 + c) * 16);
+            }
             float x[N];
             Elem<DT>::unpack(row[u], x);
 #pragma unroll
@@ -637,13 +641,6 @@ int launch_moe_permute_rows(const void* in, void* out, const int32_t* row_id_map
 
 // KU, the rows of a token that a wave requests before it uses the first (the topK loop runs in groups of KU): 2 and 4
 // measure the same on top-8 rows, 8 is 3-5 % slower in the forward kernel and 11 % in the backward one (registers).
-#define TGG_BY_TOPK(LAUNCH) \
-  do { \
-    if (topk <= 1) LAUNCH(1); \
-    else if (topk <= 2) LAUNCH(2); \
-    else LAUNCH(4); \
-  } while (0)
-
 // The forward kernel one row at a time: from 400 MiB read and written on, where the rows come from memory rather than from
 // the memory-side cache and are the faster the fewer are in flight at once (top-8 rows of 4 KB, four / one: 144 MiB 23.0 /
 // 22.6 us, 288 MiB 46.5 / 46.9, 432 MiB 89.3 / 88.7, 1700 MiB 347.5 / 338.2; top-4 and top-6 alike).  Top-2 rows are 0.6 %
@@ -670,13 +667,23 @@ static void launch_unpermute_dt(const void* in, void* out, const int32_t* row_id
 #undef TGG_LAUNCH
 }
 
+// The backward kernel one row at a time, stored before the forward row is read: where a row is one chunk for (nearly) every
+// thread of the workgroup and the gradient has more than 64 MiB.  Rows of 4 KB, batches / one: top-8 of 8192 tokens 112.2 /
+// 115.8 us, of 12288 172.2 / 172.5, of 24576 340.0 / 339.4, of 81920 1136 / 1115; top-4 of 29491 223.6 / 219.3; top-2 of 65536
+// 258 / 247; top-1 of 28672 66.0 / 65.1.  Shorter rows leave threads idle, longer ones are several chunks a thread: batches
+// are better there with top-8 (rows of 3.5 KB by 2 %, of 5.6 KB by 5 %, of 8 KB by 2.5 %).
+static bool single_backward(int64_t tokens, int c16) { return c16 > 240 && c16 <= 256 && tokens * c16 * 16 > (64ll << 20); }
+
 template <int DT>
 static void launch_unpermute_bwd_dt(const void* grad, const void* fwd_in, const int32_t* row_id_map, const float* prob,
                                     void* act_grad, float* prob_grad, int64_t tokens, int topk, int c16, hipStream_t s) {
-#define TGG_LAUNCH(KU) \
-  hipLaunchKernelGGL((moe_unpermute_bwd_kernel<DT, KU>), dim3((unsigned)tokens), dim3(256), 0, s, (const char*)grad, \
+#define TGG_LAUNCH(KU, SINGLE) \
+  hipLaunchKernelGGL((moe_unpermute_bwd_kernel<DT, KU, SINGLE>), dim3((unsigned)tokens), dim3(256), 0, s, (const char*)grad, \
                      (const char*)fwd_in, row_id_map, prob, (char*)act_grad, prob_grad, tokens, topk, c16)
-  TGG_BY_TOPK(TGG_LAUNCH);
+  if (single_backward(tokens, c16)) TGG_LAUNCH(1, true);
+  else if (topk <= 1) TGG_LAUNCH(1, false);
+  else if (topk <= 2) TGG_LAUNCH(2, false);
+  else TGG_LAUNCH(4, false);
 #undef TGG_LAUNCH
 }
 
