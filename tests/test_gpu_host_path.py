@@ -1,5 +1,11 @@
 """The native call path (csrc/host.cpp): it takes the ordinary eager call and gives what the operator and the wrapper give;
 it leaves everything else -- gradients, tracing modes, operands that need conversion, invalid arguments -- to them."""
+import ctypes
+import re
+import subprocess
+import sysconfig
+from pathlib import Path
+
 import pytest
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
@@ -16,6 +22,25 @@ def test_cpu_operands_are_left_to_the_wrapper():
     assert _native.host().m_grouped_gemm(a, b, s, True, -1) is None
     with pytest.raises(AssertionError, match="GPU"):
         m_grouped_gemm(a, b, s, True)
+
+
+def test_the_interpreter_lock_is_taken_again_when_an_exception_passes(tmp_path):
+    """The scope in which the native call path gives up the lock, as it stands in its source, left by an exception: the
+    handler that makes a Python error of it needs the lock.  Nothing else in that source gives the lock up."""
+    source = (Path(_native.__file__).parent / "csrc" / "host.cpp").read_text()
+    assert "_ALLOW_THREADS" not in source and "PyEval_SaveThread" in source
+    scope = re.search(r"class Unlocked \{.*?\n\};", source, re.S).group(0)
+    (tmp_path / "probe.cpp").write_text("#include <Python.h>\n#include <stdexcept>\n" + scope + """
+extern "C" int locked_after_throw() {
+  try { const Unlocked unlocked; if (PyGILState_Check()) return -1; throw std::runtime_error("x"); } catch (...) {}
+  const int held = PyGILState_Check();
+  if (!held) PyGILState_Ensure();
+  return held;
+}""")
+    so = tmp_path / "probe.so"
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", f"-I{sysconfig.get_paths()['include']}", str(tmp_path / "probe.cpp"),
+                    "-o", str(so)], check=True)
+    assert ctypes.PyDLL(str(so)).locked_after_throw() == 1
 
 
 def _operands(dev, dtype=torch.bfloat16, trans_b=True):

@@ -73,6 +73,18 @@ PyObject* done(const char* name, int rc, const at::Tensor& result) {
   return THPVariable_Wrap(result);
 }
 
+// The interpreter lock is given up in the scope of one of these, and taken again also where an exception leaves it.
+class Unlocked {
+ public:
+  Unlocked() : state_(PyEval_SaveThread()) {}
+  ~Unlocked() { PyEval_RestoreThread(state_); }
+  Unlocked(const Unlocked&) = delete;
+  Unlocked& operator=(const Unlocked&) = delete;
+
+ private:
+  PyThreadState* const state_;
+};
+
 #define TGG_ARGS(n) \
   if (nargs != (n)) { PyErr_SetString(PyExc_TypeError, "wrong number of arguments"); return nullptr; } \
   if (modes_active()) Py_RETURN_NONE; \
@@ -272,9 +284,10 @@ class TotalCheck {
   }
   // Whether the rows are as many as the sizes say; raises otherwise.
   bool passes() {
-    Py_BEGIN_ALLOW_THREADS
-    event_.synchronize();
-    Py_END_ALLOW_THREADS
+    {
+      const Unlocked unlocked;
+      event_.synchronize();
+    }
     int64_t total = 0;
     for (int64_t g = 0; g < sizes_.size(0); ++g) {
       const int64_t v = sizes_.scalar_type() == at::kLong ? (int32_t)sizes_.const_data_ptr<int64_t>()[g] : sizes_.const_data_ptr<int32_t>()[g];
