@@ -3,7 +3,9 @@ it leaves everything else -- gradients, tracing modes, operands that need conver
 import ctypes
 import re
 import subprocess
+import sys
 import sysconfig
+import threading
 from pathlib import Path
 
 import pytest
@@ -238,3 +240,46 @@ def test_fp8_gemm_refuses_the_gradient_of_every_operand(dev, which):
     with torch.no_grad():
         out = gmm_fp8_act_per_channel_w_per_expert(*operands, sizes)
     assert not out.requires_grad and torch.equal(out, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("entry", ["gemm", "masked", "k_grouped", "fp8", "permute_map", "permute", "unpermute", "bf16_padded", "fp8_padded"])
+def test_other_threads_run_while_a_call_allocates_and_launches(dev, entry):
+    """A thread that waits for the interpreter lock gets it during the calls, without asking the interpreter to switch
+    (the switch interval is set beyond the test's length)."""
+    a, b, sizes = _operands(dev)
+    a8, b8 = torch.randn(200, 80, device=dev).to(torch.float8_e4m3fn), torch.randn(4, 48, 80, device=dev).to(torch.float8_e4m3fn)
+    sa, sb = torch.rand(200, 1, device=dev), torch.rand(4, 48, device=dev)
+    lhs, out = torch.randn(512, 72, device=dev).to(torch.bfloat16), torch.empty(512, 40, device=dev, dtype=torch.bfloat16)
+    idx = torch.randint(0, 4, (200, 2), device=dev, dtype=torch.int32)
+    rows, where = ops.permute(a, idx, num_experts=4)
+    probs, queue = torch.rand(200, 2, device=dev), _native.work_queue(a.device)
+    x16, x8 = (torch.randn(384, 80, device=dev).to(t) for t in (torch.bfloat16, torch.float8_e4m3fn))
+    w16, row_scale, block_scale = b8.to(torch.bfloat16), torch.rand(384, 1, device=dev), torch.rand(4, 1, 1, device=dev)
+    host = _native.host()
+    call = {"gemm": lambda: host.m_grouped_gemm(a, b, sizes, True, -1),
+            "masked": lambda: host.m_grouped_gemm_masked(lhs, b, out, sizes, 128, True),
+            "k_grouped": lambda: host.k_grouped_gemm(a, a, sizes, -1, queue),
+            "fp8": lambda: host.m_grouped_gemm_fp8_channel(a8, sa, b8, sb, sizes, True),
+            "permute_map": lambda: host.permute_map(idx, 0, 4, False), "permute": lambda: host.permute(a, idx, 0, 4),
+            "unpermute": lambda: host.unpermute(rows, where, probs),
+            "bf16_padded": lambda: host.m_grouped_bf16_contiguous(x16, w16, sizes, None, 128),
+            "fp8_padded": lambda: host.m_grouped_fp8_contiguous(x8, row_scale, b8, block_scale, sizes, None, 128)}[entry]
+    assert call() is not None
+    gate, seen = threading.Lock(), []
+    gate.acquire()
+    waiting = threading.Thread(target=lambda: (gate.acquire(), seen.append(1)), daemon=True)
+    interval = sys.getswitchinterval()
+    try:
+        waiting.start()
+        sys.setswitchinterval(1000.0)
+        gate.release()
+        for _ in range(500):
+            call()
+            if seen:
+                break
+        assert seen
+    finally:
+        sys.setswitchinterval(interval)
+        waiting.join()
+    torch.cuda.synchronize()

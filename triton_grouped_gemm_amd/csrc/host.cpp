@@ -73,7 +73,9 @@ PyObject* done(const char* name, int rc, const at::Tensor& result) {
   return THPVariable_Wrap(result);
 }
 
-// The interpreter lock is given up in the scope of one of these, and taken again also where an exception leaves it.
+// The interpreter lock is given up in the scope of one of these, and taken again also where an exception leaves it: the
+// allocation and the launch can both block (a device allocation; a stream with a full queue) and must not stop the other
+// host threads.  Giving it up and taking it back does not show in the time of a call (5.2 us of host time either way).
 class Unlocked {
  public:
   Unlocked() : state_(PyEval_SaveThread()) {}
@@ -115,9 +117,15 @@ PyObject* m_grouped_gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (dt < 0 || b.scalar_type() != a.scalar_type() || b.size(trans_b ? 2 : 1) != k || (n & 7) || (k & 7) || g > kMaxGroups ||
       !sizes_ok(sizes, g) || !a.is_contiguous() || !b.is_contiguous())
     Py_RETURN_NONE;
-  at::Tensor c = at::empty({m, n}, a.options());
-  return done("tgg_m_grouped_gemm", tgg_m_grouped_gemm(a.data_ptr(), b.data_ptr(), c.data_ptr(), sizes.data_ptr(), is64(sizes),
-              (int)g, m, (int)n, (int)k, trans_b, dt, (int)num_cu, stream()), c);
+  at::Tensor c;
+  int rc;
+  {
+    const Unlocked unlocked;
+    c = at::empty({m, n}, a.options());
+    rc = tgg_m_grouped_gemm(a.data_ptr(), b.data_ptr(), c.data_ptr(), sizes.data_ptr(), is64(sizes), (int)g, m, (int)n, (int)k,
+                            trans_b, dt, (int)num_cu, stream());
+  }
+  return done("tgg_m_grouped_gemm", rc, c);
   END_HANDLE_TH_ERRORS
 }
 
@@ -138,8 +146,13 @@ PyObject* m_grouped_gemm_masked(PyObject*, PyObject* const* args, Py_ssize_t nar
       (n & 7) || (k & 7) || m % 128 || out.size(0) != m || out.size(1) != n || stride < 0 || g * stride > m ||
       g > kMaxGroupsOther || !sizes_ok(sizes, g) || !a.is_contiguous() || !b.is_contiguous() || !out.is_contiguous())
     Py_RETURN_NONE;
-  return done("tgg_m_grouped_gemm_masked", tgg_m_grouped_gemm_masked(a.data_ptr(), b.data_ptr(), out.data_ptr(), sizes.data_ptr(),
-              is64(sizes), (int)g, stride, m, (int)n, (int)k, trans_b, dt, -1, stream()), out);
+  int rc;
+  {
+    const Unlocked unlocked;
+    rc = tgg_m_grouped_gemm_masked(a.data_ptr(), b.data_ptr(), out.data_ptr(), sizes.data_ptr(), is64(sizes), (int)g, stride, m,
+                                   (int)n, (int)k, trans_b, dt, -1, stream());
+  }
+  return done("tgg_m_grouped_gemm_masked", rc, out);
   END_HANDLE_TH_ERRORS
 }
 
@@ -158,9 +171,15 @@ PyObject* k_grouped_gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (dt < 0 || b.scalar_type() != a.scalar_type() || b.size(0) != kt || (m & 7) || (n & 7) || g < 1 || g > kMaxGroups ||
       !sizes_ok(sizes, g) || !a.is_contiguous() || !b.is_contiguous() || ((uintptr_t)a.data_ptr() & 15) || ((uintptr_t)b.data_ptr() & 15))
     Py_RETURN_NONE;
-  at::Tensor c = at::empty({g, m, n}, a.options());
-  return done("tgg_k_grouped_gemm_sizes", tgg_k_grouped_gemm_sizes(a.data_ptr(), b.data_ptr(), c.data_ptr(), sizes.data_ptr(),
-              is64(sizes), (int)g, (int)m, (int)n, kt, dt, (int)num_cu, (int32_t*)queue.data_ptr(), stream()), c);
+  at::Tensor c;
+  int rc;
+  {
+    const Unlocked unlocked;
+    c = at::empty({g, m, n}, a.options());
+    rc = tgg_k_grouped_gemm_sizes(a.data_ptr(), b.data_ptr(), c.data_ptr(), sizes.data_ptr(), is64(sizes), (int)g, (int)m, (int)n, kt,
+                                  dt, (int)num_cu, (int32_t*)queue.data_ptr(), stream());
+  }
+  return done("tgg_k_grouped_gemm_sizes", rc, c);
   END_HANDLE_TH_ERRORS
 }
 
@@ -181,10 +200,16 @@ PyObject* m_grouped_gemm_fp8_channel(PyObject*, PyObject* const* args, Py_ssize_
       sb.scalar_type() != at::kFloat || !sa.is_contiguous() || !sb.is_contiguous() || g > kMaxGroupsOther ||
       !sizes_ok(sizes, g) || !a.is_contiguous() || !b.is_contiguous())
     Py_RETURN_NONE;
-  at::Tensor c = at::empty({m, n}, a.options().dtype(fp16 ? at::kHalf : at::kBFloat16));
-  return done("tgg_m_grouped_gemm_fp8_channel", tgg_m_grouped_gemm_fp8_channel(a.data_ptr(), (const float*)sa.data_ptr(), b.data_ptr(),
-              (const float*)sb.data_ptr(), c.data_ptr(), sizes.data_ptr(), is64(sizes), (int)g, m, (int)n, (int)k, fa, fb,
-              fp16 ? TGG_F16 : TGG_BF16, -1, stream()), c);
+  at::Tensor c;
+  int rc;
+  {
+    const Unlocked unlocked;
+    c = at::empty({m, n}, a.options().dtype(fp16 ? at::kHalf : at::kBFloat16));
+    rc = tgg_m_grouped_gemm_fp8_channel(a.data_ptr(), (const float*)sa.data_ptr(), b.data_ptr(), (const float*)sb.data_ptr(), c.data_ptr(),
+                                        sizes.data_ptr(), is64(sizes), (int)g, m, (int)n, (int)k, fa, fb, fp16 ? TGG_F16 : TGG_BF16,
+                                        -1, stream());
+  }
+  return done("tgg_m_grouped_gemm_fp8_channel", rc, c);
   END_HANDLE_TH_ERRORS
 }
 
@@ -214,12 +239,17 @@ PyObject* permute_map(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   TGG_TRUTH(wide, 3);
   if (idx.dim() != 2 || idx.scalar_type() != at::kInt || !idx.is_contiguous() || experts < 1 || experts > kMaxExperts) Py_RETURN_NONE;
   const int64_t tokens = idx.size(0), topk = idx.size(1);
-  at::Tensor map = at::empty({tokens * topk}, idx.options());
-  at::Tensor counts = at::empty({experts}, idx.options().dtype(wide ? at::kLong : at::kInt));
-  int64_t bytes;
-  const at::Tensor ws = sort_workspace(tokens, topk, experts, idx, bytes);
-  const int rc = tgg_moe_permute_map((const int32_t*)idx.data_ptr(), tokens, (int)topk, (int)experts, keep, (int32_t*)map.data_ptr(),
-                                     counts.data_ptr(), wide, ws.defined() ? ws.data_ptr() : nullptr, bytes, stream());
+  at::Tensor map, counts;
+  int rc;
+  {
+    const Unlocked unlocked;
+    map = at::empty({tokens * topk}, idx.options());
+    counts = at::empty({experts}, idx.options().dtype(wide ? at::kLong : at::kInt));
+    int64_t bytes;
+    const at::Tensor ws = sort_workspace(tokens, topk, experts, idx, bytes);
+    rc = tgg_moe_permute_map((const int32_t*)idx.data_ptr(), tokens, (int)topk, (int)experts, keep, (int32_t*)map.data_ptr(),
+                             counts.data_ptr(), wide, ws.defined() ? ws.data_ptr() : nullptr, bytes, stream());
+  }
   return rc != 0 ? done("tgg_moe_permute_map", rc, map) : pair(map, counts);
   END_HANDLE_TH_ERRORS
 }
@@ -236,12 +266,17 @@ PyObject* permute(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       x.size(0) != idx.size(0) || code_act(x) < 0 || experts < 1 || experts > kMaxExperts)
     Py_RETURN_NONE;
   const int64_t tokens = idx.size(0), topk = idx.size(1), hidden = x.size(1), rows = keep > 0 ? keep : tokens * topk;
-  at::Tensor map = at::empty({tokens * topk}, idx.options()), out = at::empty({rows, hidden}, x.options());
-  int64_t bytes;
-  const at::Tensor ws = sort_workspace(tokens, topk, experts, idx, bytes);
-  const int rc = tgg_moe_permute(x.data_ptr(), out.data_ptr(), (const int32_t*)idx.data_ptr(), tokens, (int)topk, (int)experts, keep,
-                                 (int)hidden, code_act(x), (int32_t*)map.data_ptr(), nullptr, 0, ws.defined() ? ws.data_ptr() : nullptr,
-                                 bytes, stream());
+  at::Tensor map, out;
+  int rc;
+  {
+    const Unlocked unlocked;
+    map = at::empty({tokens * topk}, idx.options());
+    out = at::empty({rows, hidden}, x.options());
+    int64_t bytes;
+    const at::Tensor ws = sort_workspace(tokens, topk, experts, idx, bytes);
+    rc = tgg_moe_permute(x.data_ptr(), out.data_ptr(), (const int32_t*)idx.data_ptr(), tokens, (int)topk, (int)experts, keep, (int)hidden,
+                         code_act(x), (int32_t*)map.data_ptr(), nullptr, 0, ws.defined() ? ws.data_ptr() : nullptr, bytes, stream());
+  }
   return rc != 0 ? done("tgg_moe_permute", rc, map) : pair(out, map);
   END_HANDLE_TH_ERRORS
 }
@@ -264,46 +299,66 @@ PyObject* unpermute(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   } else if (map.numel() < tokens) {  // fewer entries than rows of x: the wrapper raises
     Py_RETURN_NONE;
   }
-  at::Tensor out = at::empty({tokens, x.size(1)}, x.options());
-  return done("tgg_moe_unpermute", tgg_moe_unpermute(x.data_ptr(), out.data_ptr(), (const int32_t*)map.data_ptr(), weights, tokens,
-              (int)topk, (int)x.size(1), code_act(x), stream()), out);
+  at::Tensor out;
+  int rc;
+  {
+    const Unlocked unlocked;
+    out = at::empty({tokens, x.size(1)}, x.options());
+    rc = tgg_moe_unpermute(x.data_ptr(), out.data_ptr(), (const int32_t*)map.data_ptr(), weights, tokens, (int)topk, (int)x.size(1),
+                           code_act(x), stream());
+  }
+  return done("tgg_moe_unpermute", rc, out);
   END_HANDLE_TH_ERRORS
 }
 
 // The padded total of a contiguous layout against the rows of A (the reference reads it back too,
 // gemm/deep_gemm_ops.py:49-51).  The read-back is enqueued in front of the GEMM and waited for behind it, so the GPU has the
 // GEMM to work on meanwhile; the GEMM never touches rows at or beyond M, whatever the sizes say.
-class TotalCheck {
+class PaddedTotal {
  public:
-  TotalCheck(const at::Tensor& sizes, int64_t block_m, int64_t m)
+  PaddedTotal(const at::Tensor& sizes, int64_t block_m)
       : sizes_(sizes.to(at::TensorOptions(sizes.options()).device(at::kCPU), /*non_blocking=*/true)), event_(c10::DeviceType::CUDA),
-        block_m_(block_m), m_(m) {
+        block_m_(block_m) {
     // torch's streams and events carry the device type CUDA
     const auto current = c10::hip::getCurrentHIPStream();
     event_.record(c10::Stream(c10::Stream::UNSAFE, sizes.device(), current.id()));
   }
-  // Whether the rows are as many as the sizes say; raises otherwise.
-  bool passes() {
-    {
-      const Unlocked unlocked;
-      event_.synchronize();
-    }
+  int64_t wait() {
+    event_.synchronize();
     int64_t total = 0;
     for (int64_t g = 0; g < sizes_.size(0); ++g) {
       const int64_t v = sizes_.scalar_type() == at::kLong ? (int32_t)sizes_.const_data_ptr<int64_t>()[g] : sizes_.const_data_ptr<int32_t>()[g];
       const int64_t up = v + block_m_ - 1;
       total += (up >= 0 ? up / block_m_ : -((block_m_ - 1 - up) / block_m_)) * block_m_;
     }
-    if (total == m_) return true;
-    PyErr_Format(PyExc_ValueError, "A must include padded expert rows: expected M=%lld, got M=%lld", (long long)total, (long long)m_);
-    return false;
+    return total;
   }
 
  private:
   at::Tensor sizes_;
   c10::Event event_;
-  const int64_t block_m_, m_;
+  const int64_t block_m_;
 };
+
+// Runs `gemm`, which returns the C ABI's code, with the total looked at behind it, or in front of it where the result is the
+// caller's tensor, which then stays as it is if the total is wrong.
+template <class Gemm>
+PyObject* padded_gemm(const char* name, const at::Tensor& sizes, int64_t block_m, int64_t m, const at::Tensor& c, bool callers, Gemm gemm) {
+  int rc = 0;
+  int64_t total = m;
+  {
+    const Unlocked unlocked;
+    PaddedTotal padded(sizes, block_m);
+    if (callers) total = padded.wait();
+    if (total == m) rc = gemm();
+    if (rc == 0 && !callers) total = padded.wait();
+  }
+  if (total != m) {
+    PyErr_Format(PyExc_ValueError, "A must include padded expert rows: expected M=%lld, got M=%lld", (long long)total, (long long)m);
+    return nullptr;
+  }
+  return done(name, rc, c);
+}
 
 bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
 
@@ -321,22 +376,17 @@ PyObject* m_grouped_bf16_contiguous(PyObject*, PyObject* const* args, Py_ssize_t
       g > kMaxGroupsOther || !sizes_ok(sizes, g) || !a.is_contiguous() || !b.is_contiguous())
     Py_RETURN_NONE;
   at::Tensor c;
-  TotalCheck check(sizes, block_m, m);
-  if (args[3] != Py_None) {
+  const bool callers = args[3] != Py_None;
+  if (callers) {
     TGG_TENSOR(out, 3);
     if (out.scalar_type() != at::kBFloat16 || !out.is_contiguous() || out.numel() != m * n || out.requires_grad()) Py_RETURN_NONE;
-    if (!check.passes()) return nullptr;  // the caller's tensor stays as it is
     c = out;
-  } else {
-    c = at::empty({m, n}, a.options());
   }
-  PyObject* const result = done("tgg_m_grouped_gemm_padded", tgg_m_grouped_gemm_padded(a.data_ptr(), b.data_ptr(), c.data_ptr(),
-                                sizes.data_ptr(), is64(sizes), (int)g, m, (int)n, (int)k, (int)block_m, TGG_BF16, -1, stream()), c);
-  if (result && args[3] == Py_None && !check.passes()) {
-    Py_DECREF(result);
-    return nullptr;
-  }
-  return result;
+  return padded_gemm("tgg_m_grouped_gemm_padded", sizes, block_m, m, c, callers, [&] {
+    if (!callers) c = at::empty({m, n}, a.options());
+    return tgg_m_grouped_gemm_padded(a.data_ptr(), b.data_ptr(), c.data_ptr(), sizes.data_ptr(), is64(sizes), (int)g, m, (int)n, (int)k,
+                                     (int)block_m, TGG_BF16, -1, stream());
+  });
   END_HANDLE_TH_ERRORS
 }
 
@@ -360,29 +410,22 @@ PyObject* m_grouped_fp8_contiguous(PyObject*, PyObject* const* args, Py_ssize_t 
   const bool mn_major = kb == 1 ? sa_in.is_contiguous() : sa_in.stride(0) == 1 && sa_in.stride(1) == m;
   if (!mn_major && !sa_in.is_contiguous()) Py_RETURN_NONE;
   at::Tensor c;
-  TotalCheck check(sizes, block_m, m);
-  if (args[5] != Py_None) {
+  const bool callers = args[5] != Py_None;
+  if (callers) {
     TGG_TENSOR(out, 5);
     if (out.scalar_type() != at::kBFloat16 || !out.is_contiguous() || out.numel() != m * n || out.requires_grad()) Py_RETURN_NONE;
-    if (!check.passes()) return nullptr;  // the caller's tensor stays as it is
     c = out;
-  } else {
-    c = at::empty({m, n}, a.options().dtype(at::kBFloat16));
   }
-  at::Tensor sa = sa_in;
-  if (!mn_major) {  // the kernel streams one K block of all rows at a time
-    sa = at::empty({kb, m}, sa_in.options());
-    if (int rc = tgg_scales_to_mn_major((const float*)sa_in.data_ptr(), (float*)sa.data_ptr(), m, (int)kb, stream()))
-      return done("tgg_scales_to_mn_major", rc, c);
-  }
-  PyObject* const result = done("tgg_m_grouped_gemm_fp8_block", tgg_m_grouped_gemm_fp8_block(a.data_ptr(), (const float*)sa.data_ptr(),
-                                b.data_ptr(), (const float*)sb.data_ptr(), c.data_ptr(), sizes.data_ptr(), is64(sizes), (int)g, m, (int)n,
-                                (int)k, (int)block_m, 1, -1, stream()), c);
-  if (result && args[5] == Py_None && !check.passes()) {
-    Py_DECREF(result);
-    return nullptr;
-  }
-  return result;
+  return padded_gemm("tgg_m_grouped_gemm_fp8_block", sizes, block_m, m, c, callers, [&] {
+    if (!callers) c = at::empty({m, n}, a.options().dtype(at::kBFloat16));
+    at::Tensor sa = sa_in;
+    if (!mn_major) {  // the kernel streams one K block of all rows at a time
+      sa = at::empty({kb, m}, sa_in.options());
+      if (int rc = tgg_scales_to_mn_major((const float*)sa_in.data_ptr(), (float*)sa.data_ptr(), m, (int)kb, stream())) return rc;
+    }
+    return tgg_m_grouped_gemm_fp8_block(a.data_ptr(), (const float*)sa.data_ptr(), b.data_ptr(), (const float*)sb.data_ptr(), c.data_ptr(),
+                                        sizes.data_ptr(), is64(sizes), (int)g, m, (int)n, (int)k, (int)block_m, 1, -1, stream());
+  });
   END_HANDLE_TH_ERRORS
 }
 
