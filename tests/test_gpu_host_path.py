@@ -26,6 +26,34 @@ def test_cpu_operands_are_left_to_the_wrapper():
         m_grouped_gemm(a, b, s, True)
 
 
+def test_the_operators_are_their_definitions():
+    """The entry points that are operators are the operators' definitions, with what belongs to one; an implementation for
+    all devices takes the native path out.  In a process of its own: registrations last."""
+    code = """
+import inspect, torch
+from triton_grouped_gemm_amd.gemm.BF16.m_grouped_gemm import m_grouped_gemm
+from triton_grouped_gemm_amd.gemm.FP8.m_grouped_gemm_channel_expert import gmm_fp8_act_per_channel_w_per_expert as fp8
+a, b, s = torch.randn(8, 8), torch.randn(1, 8, 8), torch.tensor([8])
+for op, args, name in ((m_grouped_gemm, (a, b, s), 'm_grouped_gemm'),
+                       (fp8, (a, a[:, :1], b, b[:, 0], s), 'gmm_fp8_act_per_channel_w_per_expert')):
+    assert isinstance(op, torch.library.CustomOpDef) and op.__name__ == name and op.__doc__
+    assert list(inspect.signature(op).parameters)[0] == 'A' and not op.replaced
+    op.register_autograd(lambda ctx, g: (g * 3, *[None] * (len(args) - 1)))
+    op.register_kernel('cpu')(lambda x, *rest: x + 1)
+    x = a.clone().requires_grad_(True)
+    out = op(x, *args[1:])
+    out.sum().backward()
+    assert torch.equal(out, a + 1) and torch.equal(x.grad, torch.full_like(a, 3.0)) and not op.replaced
+    assert torch.equal(torch.compile(lambda *t: op(*t) * 2, fullgraph=True, backend='eager')(*args), (a + 1) * 2)
+    torch.library.opcheck(op, args, test_utils='test_schema')
+    op.register_kernel(None)(lambda x, *rest: x + 2)
+    assert op.replaced
+print("checked")
+"""
+    run = subprocess.run([sys.executable, "-c", code], cwd=Path(_native.__file__).parents[1], capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0 and "checked" in run.stdout, run.stderr[-2000:]
+
+
 def test_the_interpreter_lock_is_taken_again_when_an_exception_passes(tmp_path):
     """The scope in which the native call path gives up the lock, as it stands in its source, left by an exception: the
     handler that makes a Python error of it needs the lock.  Nothing else in that source gives the lock up."""
@@ -283,3 +311,32 @@ def test_other_threads_run_while_a_call_allocates_and_launches(dev, entry):
         sys.setswitchinterval(interval)
         waiting.join()
     torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("key", ["CUDA", "AutocastCUDA", "AutogradCUDA"])
+def test_what_others_register_for_the_operators_is_what_runs(dev, key):
+    a, b, sizes = _operands(dev)
+    a8, b8 = torch.randn(200, 80, device=dev).to(torch.float8_e4m3fn), torch.randn(4, 48, 80, device=dev).to(torch.float8_e4m3fn)
+    eight = (a8, torch.rand(200, 1, device=dev), b8, torch.rand(4, 48, device=dev), sizes)
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=key == "AutocastCUDA"):
+        plain = m_grouped_gemm(a, b, sizes, True), gmm_fp8_act_per_channel_w_per_expert(*eight)
+        with torch.library._scoped_library("moe", "IMPL") as moe, torch.library._scoped_library("myfp8", "IMPL") as myfp8:
+            moe.impl("m_grouped_gemm", lambda x, *rest: x.new_full((2,), 7.0), key)
+            myfp8.impl("gmm_fp8_act_per_channel_w_per_expert", lambda x, scale, *rest: scale.new_full((3,), 9.0), key)
+            assert m_grouped_gemm(a, b, sizes, True).tolist() == [7.0] * 2 and ops.gmm(a, b, sizes, True).tolist() == [7.0] * 2
+            assert gmm_fp8_act_per_channel_w_per_expert(*eight).tolist() == [9.0] * 3
+        again = m_grouped_gemm(a, b, sizes, True), gmm_fp8_act_per_channel_w_per_expert(*eight)
+        assert torch.equal(plain[0], again[0]) and torch.equal(plain[1], again[1])
+
+
+@pytest.mark.gpu
+def test_the_profiler_shows_the_operators(dev):
+    a, b, sizes = _operands(dev)
+    a8, b8 = torch.randn(200, 80, device=dev).to(torch.float8_e4m3fn), torch.randn(4, 48, 80, device=dev).to(torch.float8_e4m3fn)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], record_shapes=True) as seen:
+        ops.gmm(a, b, sizes, True)
+        gmm_fp8_act_per_channel_w_per_expert(a8, torch.rand(200, 1, device=dev), b8, torch.rand(4, 48, device=dev), sizes)
+    shapes = {e.name: e.input_shapes for e in seen.events()}
+    assert shapes["moe::m_grouped_gemm"][:2] == [[200, 72], [4, 40, 72]]
+    assert shapes["myfp8::gmm_fp8_act_per_channel_w_per_expert"][:2] == [[200, 80], [200, 1]]

@@ -91,6 +91,18 @@ def host():
     return _host
 
 
+class EagerOp(torch.library.CustomOpDef):
+    """A custom operator whose own eager calls go to the kernel directly where that gives what the operator would: its
+    subclasses' ``__call__`` asks the native call path first.  It stays the operator's definition (``register_autograd``,
+    ``register_kernel``, ``opcheck`` and the rest), and an implementation that is registered for it is the one that runs:
+    the native path looks for those the dispatcher has for GPU tensors, ``replaced`` says that there is one for all devices."""
+    replaced = False
+
+    def register_kernel(self, device_types, *rest):
+        self.replaced = self.replaced or device_types is None
+        return super().register_kernel(device_types, *rest)
+
+
 def last_error() -> str:
     return load().tgg_last_error().decode()
 

@@ -8,6 +8,8 @@
 // decided here that the wrappers do not decide too, and no state is kept.
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/core/dispatch/Dispatcher.h>
+#include <ATen/record_function.h>
 #include <c10/core/Event.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -45,6 +47,14 @@ bool modes_active() {
                                             c10::DispatchKey::Python, c10::DispatchKey::Tracer});
   return c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled() ||
          c10::impl::tls_local_dispatch_key_set().included_.has_any(watched);
+}
+
+// Whether the dispatcher has an implementation or a rule of someone else's for the operator on GPU tensors (the operator's
+// own ones serve all devices): a call then goes through it.
+bool replaced(const c10::OperatorName& op) {
+  const auto handle = c10::Dispatcher::singleton().findOp(op);
+  return handle && (handle->hasKernelForDispatchKey(c10::DispatchKey::CUDA) || handle->hasKernelForDispatchKey(c10::DispatchKey::AutocastCUDA) ||
+                    handle->hasKernelForDispatchKey(c10::DispatchKey::AutogradCUDA));
 }
 
 bool records(const at::Tensor& t) { return t.requires_grad() && c10::GradMode::is_enabled(); }
@@ -117,6 +127,9 @@ PyObject* m_grouped_gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (dt < 0 || b.scalar_type() != a.scalar_type() || b.size(trans_b ? 2 : 1) != k || (n & 7) || (k & 7) || g > kMaxGroups ||
       !sizes_ok(sizes, g) || !a.is_contiguous() || !b.is_contiguous())
     Py_RETURN_NONE;
+  static const c10::OperatorName op("moe::m_grouped_gemm", "");
+  if (replaced(op)) Py_RETURN_NONE;
+  RECORD_FUNCTION(op.name, std::vector<c10::IValue>({a, b, sizes, trans_b, (int64_t)num_cu}));  // under the operator's name
   at::Tensor c;
   int rc;
   {
@@ -200,6 +213,9 @@ PyObject* m_grouped_gemm_fp8_channel(PyObject*, PyObject* const* args, Py_ssize_
       sb.scalar_type() != at::kFloat || !sa.is_contiguous() || !sb.is_contiguous() || g > kMaxGroupsOther ||
       !sizes_ok(sizes, g) || !a.is_contiguous() || !b.is_contiguous())
     Py_RETURN_NONE;
+  static const c10::OperatorName op("myfp8::gmm_fp8_act_per_channel_w_per_expert", "");
+  if (replaced(op)) Py_RETURN_NONE;
+  RECORD_FUNCTION(op.name, std::vector<c10::IValue>({a, sa, b, sb, sizes}));
   at::Tensor c;
   int rc;
   {

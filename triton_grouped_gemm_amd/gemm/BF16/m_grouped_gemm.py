@@ -14,6 +14,7 @@ from typing import Optional, Tuple
 
 import torch
 from torch import Tensor
+from torch.compiler import is_compiling
 
 from ... import _native
 
@@ -90,26 +91,32 @@ def _m_grouped_gemm_launch(A: Tensor, B: Tensor, C: Tensor, size_per_group: Tens
 
 
 @torch.library.custom_op("moe::m_grouped_gemm", mutates_args=())
-def _m_grouped_gemm_op(A: Tensor, B: Tensor, size_per_group: Tensor, trans_b: bool = False, numSM: int = -1) -> Tensor:
+def m_grouped_gemm(A: Tensor, B: Tensor, size_per_group: Tensor, trans_b: bool = False, numSM: int = -1) -> Tensor:
     M, K = A.shape
     N = B.shape[1] if trans_b else B.shape[2]
     C = A.new_empty(M, N)
     return _m_grouped_gemm_launch(A, B, C, size_per_group, trans_b, numSM)
 
 
-@_m_grouped_gemm_op.register_fake
+@m_grouped_gemm.register_fake
 def _(A: Tensor, B: Tensor, size_per_group: Tensor, trans_b: bool = False, numSM: int = -1) -> Tensor:
     M, K = A.shape
     N = B.shape[1] if trans_b else B.shape[2]
     return A.new_empty(M, N)
 
 
-def m_grouped_gemm(A: Tensor, B: Tensor, size_per_group: Tensor, trans_b: bool = False, numSM: int = -1) -> Tensor:
+class _MGroupedGemm(_native.EagerOp):
     """``C[r] = A[r] @ B[g(r)]^T`` (``trans_b``) or ``A[r] @ B[g(r)]``; rows past ``sum(size_per_group)``
     are left uninitialised, as in the reference (:435-447).  The operator ``moe::m_grouped_gemm``; an ordinary eager
     call goes to the kernel directly (16 -> 5 us of host time)."""
-    if not torch.compiler.is_compiling():
-        C = _native.host().m_grouped_gemm(A, B, size_per_group, trans_b, numSM)
-        if C is not None:
-            return C
-    return _m_grouped_gemm_op(A, B, size_per_group, trans_b, numSM)
+    __name__ = "m_grouped_gemm"
+
+    def __call__(self, A: Tensor, B: Tensor, size_per_group: Tensor, trans_b: bool = False, numSM: int = -1) -> Tensor:
+        if not (self.replaced or is_compiling()):
+            C = (_native._host or _native.host()).m_grouped_gemm(A, B, size_per_group, trans_b, numSM)
+            if C is not None:
+                return C
+        return super().__call__(A, B, size_per_group, trans_b, numSM)
+
+
+m_grouped_gemm.__class__ = _MGroupedGemm

@@ -9,14 +9,15 @@ from __future__ import annotations
 
 import torch
 from torch import Tensor
+from torch.compiler import is_compiling
 
 from ... import _native
 from ..BF16.m_grouped_gemm import _sizes_on_device
 
 
 @torch.library.custom_op("myfp8::gmm_fp8_act_per_channel_w_per_expert", mutates_args=())
-def _gmm_fp8_op(A: Tensor, A_scale: Tensor, B: Tensor, B_scale: Tensor, size_per_group: Tensor,
-                dtype_out: torch.dtype = torch.float16) -> Tensor:
+def gmm_fp8_act_per_channel_w_per_expert(A: Tensor, A_scale: Tensor, B: Tensor, B_scale: Tensor,
+                                         size_per_group: Tensor, dtype_out: torch.dtype = torch.float16) -> Tensor:
     assert A.dim() == 2
     assert B.dim() == 3
     M, K = A.shape
@@ -42,18 +43,24 @@ def _gmm_fp8_op(A: Tensor, A_scale: Tensor, B: Tensor, B_scale: Tensor, size_per
     return C
 
 
-@_gmm_fp8_op.register_fake
+@gmm_fp8_act_per_channel_w_per_expert.register_fake
 def _(A, A_scale, B, B_scale, size_per_group, dtype_out=torch.float16):
     return A.new_empty(A.shape[0], B.shape[1], dtype=dtype_out)
 
 
-def gmm_fp8_act_per_channel_w_per_expert(A: Tensor, A_scale: Tensor, B: Tensor, B_scale: Tensor,
-                                         size_per_group: Tensor, dtype_out: torch.dtype = torch.float16) -> Tensor:
+class _ChannelExpertGemm(_native.EagerOp):
     """A ``[M, K]`` fp8, A_scale ``[M, 1]`` fp32, B ``[G, N, K]`` fp8, B_scale fp32 with ``G*N`` entries
     (element ``g*N + n`` scales column n of expert g).  The operator of this name; an ordinary eager call goes to the
     kernel directly."""
-    if dtype_out in _native.DTYPE_CODE and not torch.compiler.is_compiling():
-        C = _native.host().m_grouped_gemm_fp8_channel(A, A_scale, B, B_scale, size_per_group, dtype_out == torch.float16)
-        if C is not None:
-            return C
-    return _gmm_fp8_op(A, A_scale, B, B_scale, size_per_group, dtype_out)
+    __name__ = "gmm_fp8_act_per_channel_w_per_expert"
+
+    def __call__(self, A: Tensor, A_scale: Tensor, B: Tensor, B_scale: Tensor, size_per_group: Tensor,
+                 dtype_out: torch.dtype = torch.float16) -> Tensor:
+        if dtype_out in _native.DTYPE_CODE and not (self.replaced or is_compiling()):
+            C = (_native._host or _native.host()).m_grouped_gemm_fp8_channel(A, A_scale, B, B_scale, size_per_group, dtype_out == torch.float16)
+            if C is not None:
+                return C
+        return super().__call__(A, A_scale, B, B_scale, size_per_group, dtype_out)
+
+
+gmm_fp8_act_per_channel_w_per_expert.__class__ = _ChannelExpertGemm
