@@ -82,6 +82,26 @@ def test_trans_quant_bit_exact_wide_many_groups(dev):
     _check_trans_quant(dev, x, sizes, torch.float8_e5m2, torch.int64)
 
 
+@pytest.mark.parametrize("groups", [1, 63, 64, 65, 200, 255, 256, 257, 600, 1000, 1023, 1024])
+@pytest.mark.parametrize("wide", [False, True])
+def test_trans_quant_finds_the_rows_of_every_group(dev, groups, wide):
+    """Group counts around the ones at which a lane of the row search walks one size more and at which a workgroup takes
+    several blocks, empty and ragged groups; sizes that reach beyond the matrix are cut off at its end."""
+    sizes = [(i * 53 + groups) % 290 * (i % 7 > 1) for i in range(groups)]
+    sizes[-1] = 129
+    x = _randn((sum(sizes), 640 if groups in (257, 1024) else 128), 93)  # one block of columns, and a run of four with one more
+    dtype = torch.int64 if wide else torch.int32
+    _check_trans_quant(dev, x, sizes, size_dtype=dtype)
+    m = max(1, sum(sizes) * 2 // 3)
+    left, cut = m, []
+    for v in sizes:
+        cut.append(min(v, left))
+        left -= cut[-1]
+    got = trans_per_block_quant_expand_128x(x[:m].contiguous().to(dev), torch.tensor(sizes, dtype=dtype, device=dev))
+    want = trans_per_block_quant_expand_128x(x[:m].contiguous().to(dev), torch.tensor(cut, dtype=dtype, device=dev))
+    assert torch.equal(got[0].view(torch.uint8), want[0].view(torch.uint8)) and torch.equal(got[1], want[1])
+
+
 @pytest.mark.parametrize("n_chunk", [1, 2])
 def test_trans_quant_ignores_gemm_tile_order_option(dev, n_chunk):
     """The column-chunk option of the GEMM tile order must not reach the quantizer."""

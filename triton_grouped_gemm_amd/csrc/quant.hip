@@ -158,15 +158,22 @@ TGG_DEV void store_nt(void* dst, i32x4_t v) {
   asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 1" : : "v"(dst), "v"(v) : "memory");
 }
 
+// With more than 256 groups a workgroup takes four neighbouring blocks of its row tile one after another: the search for the
+// rows walks 5 to 16 sizes a lane then, in three passes, and costs more than the block.  One block / four, 131072 x 4096
+// values: 512 groups 503 / 395 us, 1024 groups 1036 / 487 (a table that 2048 persistent workgroups made once each: 623, 929);
+// 524288 x 4096: 1550 / 1327, 2659 / 1448 (1605, 1895).  Eight and sixteen blocks leave the last workgroups more to do:
+// 419 and 456 us with 512 groups, 467 and 509 with 1024.
+constexpr int kManyGroups = 256, kManyCols = 4;
+
 // One 128x128 block per workgroup, 256 threads.  Bound by memory: 3 bytes per element, rows of 256 bytes in, rows of 128
-// bytes out.  A workgroup per block lets the hardware fill the chip evenly and beats 2048 workgroups that walk the blocks
+// bytes out.  A workgroup per block (COLS = 1) lets the hardware fill the chip evenly and beats 2048 workgroups that walk the blocks
 // (a copy with this access pattern: 5.2 against 4.9 TB/s), which is why the block finds its rows without a table; streaming
 // stores are worth another 3-15 %.  655360 x 4096 values 1770 -> 1598 us (4.59 -> 5.08 TB/s), 33001 x 4096 98 -> 82 us
 // (4.5 -> 5.4 TB/s), of which the division's share is small: it overlaps the memory traffic of the other blocks of a CU.
 // Read: thread (rr = tid/16, cv = tid%16) owns rows rr*8 .. rr*8+7, columns cv*8 .. cv*8+7.
 // LDS holds the transposed codes: byte (c, r) at c*128 + ((r/16) ^ ((c/8)%8))*16 + r%16.
 // padded (optional): the sizes rounded up to 128, in their own integer type.
-template <int FMT>
+template <int FMT, int COLS>
 __global__ __launch_bounds__(256) void trans_quant128_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ codes,
                                                             float* __restrict__ scales, GemmParams p, int64_t m_expand,
                                                             void* __restrict__ padded) {
@@ -184,74 +191,77 @@ __global__ __launch_bounds__(256) void trans_quant128_kernel(const uint16_t* __r
       else ((int32_t*)padded)[g] = (((const int32_t*)p.sizes)[g] + 127) & ~127;
     }
   }
-  const int pm = (int)(blockIdx.x / (unsigned)tiles_n), bn = (int)(blockIdx.x % (unsigned)tiles_n);
+  const unsigned runs = COLS > 1 ? ((unsigned)tiles_n + COLS - 1) / COLS : (unsigned)tiles_n;
+  const int pm = (int)(blockIdx.x / runs), bn0 = (int)(blockIdx.x % runs) * COLS;
   if (pm >= m_tiles_all) return;
-  uint8_t* out_base = codes + ((int64_t)bn * 128) * m_expand + (int64_t)pm * 128;
   int64_t row0;
   int rows;
   find_row_tile(p, pm, row0, rows);
-  if (rows < 0) {  // tail beyond the padded groups: zero codes, zero scale
-    const i32x4_t z = {0, 0, 0, 0};
+  for (int bn = bn0; bn < (COLS > 1 ? min(tiles_n, bn0 + COLS) : bn0 + 1); ++bn) {
+    uint8_t* out_base = codes + ((int64_t)bn * 128) * m_expand + (int64_t)pm * 128;
+    if (rows < 0) {  // tail beyond the padded groups: zero codes, zero scale
+      const i32x4_t z = {0, 0, 0, 0};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int c = (tid >> 3) + 32 * i, u = tid & 7;
+        store_nt(out_base + (int64_t)c * m_expand + u * 16, z);
+      }
+      if (tid == 0) scales[(int64_t)bn * m_tiles_all + pm] = 0.f;
+      continue;
+    }
+    i32x4_t v[8];
+    u16x2_t top = {0, 0};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = rr * 8 + i;
+      i32x4_t val = {0, 0, 0, 0};
+      if (r < rows) val = *(const i32x4_t*)(x + (row0 + r) * (int64_t)N + bn * 128 + cv * 8);
+      v[i] = val;
+      top = amax_bits(top, val);
+    }
+    uint32_t bits = top[0] > top[1] ? top[0] : top[1];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const uint32_t o = (uint32_t)__shfl_xor((int)bits, off, 64);
+      bits = o > bits ? o : bits;
+    }
+    if ((tid & 63) == 0) wmax[tid >> 6] = bf16_bits_to_f32(bits);
+    __syncthreads();
+    // the pattern's order survives the conversion to float, except that a NaN makes the sum one
+    const float amax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    const bool numbers = wmax[0] + wmax[1] + wmax[2] + wmax[3] < 4.f * kMaxFastValue;
+    float scale = clampf(amax / fmax_, 1e-12f, 3e38f);
+    if (__builtin_expect(numbers, 1)) {
+      const float inv = 1.0f / scale;
+      // column j of this thread's 8x8 patch -> 8 consecutive r bytes
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float q[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const uint32_t w = (uint32_t)v[i][j >> 1];
+          const float f = __builtin_bit_cast(float, (j & 1) ? (w & 0xffff0000u) : (w << 16));
+          q[i] = clampf(div_by(f, scale, inv), -fmax_, fmax_);
+        }
+        uint2 pk;
+        pk.x = cvt4<FMT>(q[0], q[1], q[2], q[3]);
+        pk.y = cvt4<FMT>(q[4], q[5], q[6], q[7]);
+        const int c = cv * 8 + j;
+        const int slot = (rr >> 1) ^ (cv & 7);
+        *(uint2*)(codes_t + c * 128 + slot * 16 + (rr & 1) * 8) = pk;
+      }
+    } else {
+      scale = trans_block_any<FMT>(x + row0 * (int64_t)N + bn * 128, N, rows, codes_t, wmax);
+    }
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int c = (tid >> 3) + 32 * i, u = tid & 7;
-      store_nt(out_base + (int64_t)c * m_expand + u * 16, z);
+      const i32x4_t o = *(const i32x4_t*)(codes_t + c * 128 + ((u ^ ((c >> 3) & 7)) * 16));
+      store_nt(out_base + (int64_t)c * m_expand + u * 16, o);
     }
-    if (tid == 0) scales[(int64_t)bn * m_tiles_all + pm] = 0.f;
-    return;
+    if (tid == 0) scales[(int64_t)bn * m_tiles_all + pm] = scale;
   }
-  i32x4_t v[8];
-  u16x2_t top = {0, 0};
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int r = rr * 8 + i;
-    i32x4_t val = {0, 0, 0, 0};
-    if (r < rows) val = *(const i32x4_t*)(x + (row0 + r) * (int64_t)N + bn * 128 + cv * 8);
-    v[i] = val;
-    top = amax_bits(top, val);
-  }
-  uint32_t bits = top[0] > top[1] ? top[0] : top[1];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const uint32_t o = (uint32_t)__shfl_xor((int)bits, off, 64);
-    bits = o > bits ? o : bits;
-  }
-  if ((tid & 63) == 0) wmax[tid >> 6] = bf16_bits_to_f32(bits);
-  __syncthreads();
-  // the pattern's order survives the conversion to float, except that a NaN makes the sum one
-  const float amax = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-  const bool numbers = wmax[0] + wmax[1] + wmax[2] + wmax[3] < 4.f * kMaxFastValue;
-  float scale = clampf(amax / fmax_, 1e-12f, 3e38f);
-  if (__builtin_expect(numbers, 1)) {
-    const float inv = 1.0f / scale;
-    // column j of this thread's 8x8 patch -> 8 consecutive r bytes
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float q[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint32_t w = (uint32_t)v[i][j >> 1];
-        const float f = __builtin_bit_cast(float, (j & 1) ? (w & 0xffff0000u) : (w << 16));
-        q[i] = clampf(div_by(f, scale, inv), -fmax_, fmax_);
-      }
-      uint2 pk;
-      pk.x = cvt4<FMT>(q[0], q[1], q[2], q[3]);
-      pk.y = cvt4<FMT>(q[4], q[5], q[6], q[7]);
-      const int c = cv * 8 + j;
-      const int slot = (rr >> 1) ^ (cv & 7);
-      *(uint2*)(codes_t + c * 128 + slot * 16 + (rr & 1) * 8) = pk;
-    }
-  } else {
-    scale = trans_block_any<FMT>(x + row0 * (int64_t)N + bn * 128, N, rows, codes_t, wmax);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int c = (tid >> 3) + 32 * i, u = tid & 7;
-    const i32x4_t o = *(const i32x4_t*)(codes_t + c * 128 + ((u ^ ((c >> 3) & 7)) * 16));
-    store_nt(out_base + (int64_t)c * m_expand + u * 16, o);
-  }
-  if (tid == 0) scales[(int64_t)bn * m_tiles_all + pm] = scale;
 }
 
 // 16 lanes per 1x128 group; each lane 8 elements.  A workgroup's 16 lane groups take 16 neighbouring groups
@@ -417,13 +427,18 @@ int launch_trans_quant128(const void* x, void* codes, float* scales, const GemmP
                           int fmt, hipStream_t s) {
   const int64_t tiles = (m_expand >> 7) * (int64_t)(p.N >> 7);
   if (tiles >= (1ll << 24)) return set_error("a matrix of %lld 128 x 128 blocks is too large for one launch", (long long)tiles);
-  const dim3 g((unsigned)(tiles > 0 ? tiles : 1)), b(256);
-  if (fmt == DT_E4M3)
-    hipLaunchKernelGGL(trans_quant128_kernel<DT_E4M3>, g, b, 0, s, (const uint16_t*)x, (uint8_t*)codes, scales, p, m_expand, padded);
-  else if (fmt == DT_E5M2)
-    hipLaunchKernelGGL(trans_quant128_kernel<DT_E5M2>, g, b, 0, s, (const uint16_t*)x, (uint8_t*)codes, scales, p, m_expand, padded);
-  else
-    return set_error("unsupported fp8 format code %d", fmt);
+#define TGG_LAUNCH(FMT) \
+  do { \
+    if (many) hipLaunchKernelGGL((trans_quant128_kernel<FMT, kManyCols>), g, b, 0, s, (const uint16_t*)x, (uint8_t*)codes, scales, p, m_expand, padded); \
+    else hipLaunchKernelGGL((trans_quant128_kernel<FMT, 1>), g, b, 0, s, (const uint16_t*)x, (uint8_t*)codes, scales, p, m_expand, padded); \
+  } while (0)
+  const bool many = p.G > kManyGroups;
+  const int64_t runs = many ? (m_expand >> 7) * (((p.N >> 7) + kManyCols - 1) / kManyCols) : tiles;
+  const dim3 g((unsigned)(runs > 0 ? runs : 1)), b(256);
+  if (fmt == DT_E4M3) TGG_LAUNCH(DT_E4M3);
+  else if (fmt == DT_E5M2) TGG_LAUNCH(DT_E5M2);
+  else return set_error("unsupported fp8 format code %d", fmt);
+#undef TGG_LAUNCH
   return check_launch("trans_quant128");
 }
 
