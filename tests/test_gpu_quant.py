@@ -42,7 +42,7 @@ def test_hardware_fp8_conversion_equals_software_rne(dev, fmt, code):
     ([5, 0, 130, 128, 1], 256),
     ([0, 0, 0], 128),
     ([300] * 7 + [77], 384),
-    ([3, 0, 17] * 100, 128),  # 300 groups: the large group table
+    ([3, 0, 17] * 100, 128),  # 300 groups: several blocks a workgroup
 ])
 def test_trans_quant_bit_exact(dev, dtype, sizes, N):
     M = sum(sizes)
@@ -76,7 +76,7 @@ def test_trans_quant_bit_exact_wide(dev, N):
 
 
 def test_trans_quant_bit_exact_wide_many_groups(dev):
-    """G > 256 (the large group table) at N = 2048, int64 sizes, e5m2."""
+    """G > 256 (several blocks a workgroup) at N = 2048, int64 sizes, e5m2."""
     sizes = [(i * 53) % 290 for i in range(300)]
     x = _randn((sum(sizes), 2048), 91)
     _check_trans_quant(dev, x, sizes, torch.float8_e5m2, torch.int64)

@@ -19,11 +19,19 @@
 //
 //   * rows of more than kPlaceMoveBytes: the placing launch makes the map and a launch with a workgroup per token moves
 //     the rows.  A thousand placing workgroups stream at 4.9 TB/s and the short ones at 5.6, which outweighs the launch
-//     from 300 to 600 MB read and written on (moved by the placing launch / by their own: top-8 of 4096 4 KB rows 29 /
-//     34 us, 12288 101 / 103, 24576 197 / 182, 81920 645 / 577; top-1 of 81920 2 KB rows 77 / 68; 8192 rows, with the
-//     unpermute and both gradients behind it, 304 / 316).
-// Measured against four launches for the sort and one for the rows: 8192 tokens x top-8, 128 experts, 4 KB rows 70 ->
-// 67 us, 81920 tokens 589 -> 577, 4096 tokens 43 -> 29, 24 tokens 26 -> 4.4.
+//     from 200 to 450 MiB read and written on, by the number of choices: moved by the placing launch / by their own, rows of
+//     4 KB, us
+//                   top-1        top-2        top-4        top-8
+//       150 MiB   32.3 / 35.2  31.9 / 36.2  31.9 / 36.6  32.5 / 36.3
+//       250       55.9 / 52.9  54.3 / 54.0  52.2 / 54.6  59.9 / 55.0
+//       320       74.0 / 66.7  69.5 / 65.6  62.8 / 64.7  72.0 / 66.3
+//       600        147 / 121    138 / 126    132 / 126    140 / 126
+//     Rows of 2 to 14 KB are alike; rows of 1 KB like the placing launch a little longer (top-1, 320 MiB 74.4 / 80.7, 600
+//     151 / 149; top-4, 600 MiB 141 / 148; top-8, 900 MiB 221 / 260).  The line at 300 MiB costs at most a tenth on the wrong
+//     side of it.
+// Against four launches for the sort and one for the rows: 8192 tokens x top-8, 128 experts, 4 KB rows 70 -> 67 us, 81920
+// tokens 589 -> 577, 4096 tokens 43 -> 29, 24 tokens 26 -> 4.4; top-1 to top-8 rows of 1 to 14 KB, 60 to 900 MiB: 0.54 to
+// 0.96 of the time.
 //
 // The row movers are streaming kernels (16-byte accesses, fp32 arithmetic), bound by memory:
 //   place           reads each token row once and writes it to its up to topK destinations
@@ -584,10 +592,10 @@ int launch_moe_permute_map(const int32_t* indices, int64_t tokens, int topk, int
 // ---- the sort without a caller-provided workspace ---------------------------------------------------------------
 // For callers that cannot allocate (HIP graph capture, serving loops): the sort's temporaries live in a fixed
 // array in device memory that is part of the library's code object.  Sized for any problem the entry point
-// accepts: 2^20 assignments, 1024 experts, the smallest chunks (table 4 MiB + rank 4 MiB + two 4 KiB expert rows).  Every GPU the
+// accepts: 2^20 assignments, 1024 experts, the smallest chunks (table 4 MiB + rank 4 MiB + totals 4 KiB, and 4 KiB to spare).  Every GPU the
 // library runs on holds its own copy at its own address until the process ends; all calls on one GPU share it, so
 // calls that overlap on one GPU (different streams) race.  Nothing in it has to start at zero: the counting pass
-// writes every table entry and rank it later reads, the scans write totals and starts.
+// writes every table entry and rank that is read later, the scan of a large table its totals; the one-launch sort uses none of it.
 constexpr int64_t kStaticMaxAssignments = 1ll << 20;
 constexpr size_t kStaticScratchBytes = (size_t)kMaxExperts * (kStaticMaxAssignments / kCountThreads) * 4 + 2 * (size_t)kMaxExperts * 4 +
                                        (size_t)kStaticMaxAssignments * 4;
