@@ -520,7 +520,8 @@ def test_k_grouped_work_queue_equals_fixed_assignment(dev, sizes, num_cu):
     [1], [0, 0, 5], [64, 0, 1, 128, 63, 65, 0, 200],
     [(i * 37) % 70 for i in range(130)],           # one-slab tiles: the copy stream runs several tiles ahead
     [700, 3, 0, 700, 64, 64, 1, 1, 1, 1500, 320],  # short and long tiles in turn
-    [i % 5 for i in range(600)]])                  # beyond the tuned kernels' table
+    [i % 5 for i in range(600)],                   # beyond the tuned kernels' table
+    [(i * 7) % 23 for i in range(513)], [(i * 11) % 19 * (i % 3 > 0) for i in range(1024)]])
 @pytest.mark.parametrize("size_dtype,extra", [(torch.int32, 0), (torch.int64, 9), (torch.int64, -3)])
 def test_k_grouped_from_sizes_equals_explicit_bounds(dev, sizes, size_dtype, extra):
     """Segments from the sizes alone, bit for bit what explicit starts and ends give: tokens beyond the last segment
@@ -534,3 +535,24 @@ def test_k_grouped_from_sizes_equals_explicit_bounds(dev, sizes, size_dtype, ext
     want = k_grouped_gemm(a, b, s, (end - s).to(torch.int32), end.to(torch.int32))
     for _ in range(3):
         assert torch.equal(k_grouped_gemm(a, b, s), want)
+
+
+def test_k_grouped_of_many_groups_takes_no_longer_from_sizes(dev):
+    """1024 groups: the kernel makes the segments' starts in about the time it takes to read them (a single thread that adds
+    them up one by one takes 150 us more, half of this launch again)."""
+    G, Mdim, N = 1024, 264, 520
+    a, b = (torch.randn(4 * G, n, device=dev).to(torch.bfloat16) for n in (Mdim, N))
+    s = torch.full((G,), 4, dtype=torch.int32, device=dev)
+    end = s.cumsum(0).to(torch.int32)
+    start = end - s
+    best = {}
+    for _ in range(20):
+        for name, bounds in (("sizes", ()), ("bounds", (start, end))):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+            for _ in range(3):
+                k_grouped_gemm(a, b, s, *bounds)
+            t1.record()
+            t1.synchronize()
+            best[name] = min(best.get(name, 1e9), t0.elapsed_time(t1))
+    assert best["sizes"] < 1.2 * best["bounds"], best

@@ -5,6 +5,8 @@
 // with a persistent, XCD-aware stride.  No host-side metadata, no workspace, no
 // host/device synchronisation.
 #pragma once
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace tgg {
@@ -127,6 +129,41 @@ TGG_DEV int64_t sched_block_scan(int64_t v, Table& t, int64_t& total) {
   return base + inc - v;
 }
 
+// sched_prefix by the whole workgroup: every thread takes a run of neighbouring groups, the runs meet in two scans.  All
+// threads must call this, with the loaded extents visible to them.
+template <int BM, class Table>
+TGG_DEV void sched_prefix_runs(const GemmParams& p, Table& t) {
+  const int per = (p.G + (int)blockDim.x - 1) / (int)blockDim.x;
+  const int g0 = min(p.G, (int)threadIdx.x * per), g1 = min(p.G, g0 + per);
+  auto step = [&](int64_t sz) { return p.mode == MODE_MG_PAD ? ((sz + p.align - 1) / p.align) * p.align : sz; };
+  int64_t sum = 0, total;
+  for (int g = g0; g < g1; ++g) sum += step(t.rows[g]);
+  int64_t row = sched_block_scan(sum, t, total);
+  const int64_t limit = (p.mode == MODE_KG_COUNT) ? p.k_total : p.m_total;
+  sum = 0;
+  for (int g = g0; g < g1; ++g) {
+    int64_t sz = t.rows[g], start = row;
+    row += step(sz);
+    if (p.mode == MODE_MASKED) {
+      start = (int64_t)g * p.m_stride;
+      if (sz > p.m_stride) sz = p.m_stride;
+    } else if (p.mode == MODE_MG_PAD && p.row_start) {
+      start = (int64_t)p.row_start[g];
+    }
+    if (start < 0 || start >= limit) sz = 0;
+    else if (start + sz > limit) sz = limit - start;
+    t.row0[g] = start;
+    t.rows[g] = (int32_t)sz;
+    sum += (sz + BM - 1) / BM;
+  }
+  int64_t tile = sched_block_scan(sum, t, total);
+  for (int g = g0; g < g1; ++g) {
+    t.tile0[g] = (int32_t)tile;
+    tile += (t.rows[g] + BM - 1) / BM;
+  }
+  if (threadIdx.x == 0) t.tile0[p.G] = (int32_t)total;
+}
+
 // K modes only (a no-op otherwise): fills t.tile0 with the groups in tile-space order once t.rows is final.  All
 // threads of the workgroup must call this; ends with a barrier when it does anything.
 template <class Table>
@@ -150,10 +187,9 @@ TGG_DEV int32_t sched_init(const GemmParams& p, Table& t) {
     for (int g = threadIdx.x; g < p.G; g += blockDim.x) sched_load_group(p, t, g);
     __syncthreads();
     if (p.mode != MODE_KG) {
-      if (threadIdx.x == 0) {
-        sched_prefix<BM>(p, t);
-        t.pad_ = 1 << 30;
-      }
+      if constexpr (std::is_same<Table, SchedTable>::value) sched_prefix_runs<BM>(p, t);
+      else if (threadIdx.x == 0) sched_prefix<BM>(p, t);
+      if (threadIdx.x == 0) t.pad_ = 1 << 30;
       __syncthreads();
     }
     sched_order_groups(p, t);
