@@ -112,6 +112,21 @@ def test_empty_assignment_counts_are_zero(dev, topk):
     assert rmap.numel() == 0 and torch.equal(counts.cpu(), torch.zeros(40, dtype=torch.int32))
 
 
+@pytest.mark.parametrize("num_token,hidden,topk", [
+    (51200, 1024, 1), (51201, 1024, 1), (52000, 1016, 1), (51200, 1024, 2), (51201, 1024, 2)])
+def test_rows_on_either_side_of_a_launch_of_their_own(dev, num_token, hidden, topk):
+    """Sizes at which the placing launch stops to move the rows as well: by the number of choices and the rows' width."""
+    g = torch.Generator(device=dev).manual_seed(num_token + hidden)
+    x = torch.randint(-30000, 30000, (num_token, hidden), device=dev, dtype=torch.int16, generator=g).view(torch.bfloat16)
+    idx = torch.randint(0, 16, (num_token, topk), device=dev, dtype=torch.int32, generator=g)
+    idx[::13, 0] = -1
+    rows, rmap = ops.permute(x, idx, num_experts=16)
+    assert torch.equal(rmap, ops.permute_map(idx, num_experts=16)[0])
+    flat = torch.argsort(torch.where(idx < 0, 99, idx).reshape(-1), stable=True)[:int((idx >= 0).sum())]
+    assert torch.equal(rows[:flat.numel()].view(torch.int16), x.view(torch.int16)[flat // topk])
+    assert torch.equal(rmap.view(topk, num_token)[flat % topk, flat // topk], torch.arange(flat.numel(), device=dev, dtype=torch.int32))
+
+
 def test_unpermute_without_probs_asks_for_an_entry_per_row(dev):
     """More rows than map entries (a capacity above the token count) are refused, not read beyond the map."""
     x, indices, _ = _case(100, 8, 64, 1, torch.bfloat16)

@@ -17,18 +17,19 @@
 // destination = expert start + assignments of the expert in front; row_id_map[k * tokens + t] gets it (or -1 for
 // dropped assignments: expert -1, or destination beyond the capacity).
 //
-//   * rows of more than kPlaceMoveBytes: the placing launch makes the map and a launch with a workgroup per token moves
-//     the rows.  A thousand placing workgroups stream at 4.9 TB/s and the short ones at 5.6, which outweighs the launch
-//     from 200 to 450 MiB read and written on, by the number of choices: moved by the placing launch / by their own, rows of
-//     4 KB, us
+//   * rows of more bytes than place_moves_rows says: the placing launch makes the map and a launch with a workgroup per token
+//     moves the rows.  A thousand placing workgroups stream at 4.9 TB/s and the short ones at 5.6, which outweighs the launch
+//     from 200 to 450 MiB read and written on; but the placing launch leaves more of its rows in the memory-side cache for the
+//     call behind it, so the line is taken from whole passes (permute, unpermute and both gradients; moved by the placing
+//     launch / by their own, rows of 4 KB, 128 experts, us):
 //                   top-1        top-2        top-4        top-8
-//       150 MiB   32.3 / 35.2  31.9 / 36.2  31.9 / 36.6  32.5 / 36.3
-//       250       55.9 / 52.9  54.3 / 54.0  52.2 / 54.6  59.9 / 55.0
-//       320       74.0 / 66.7  69.5 / 65.6  62.8 / 64.7  72.0 / 66.3
-//       600        147 / 121    138 / 126    132 / 126    140 / 126
-//     Rows of 2 to 14 KB are alike; rows of 1 KB like the placing launch a little longer (top-1, 320 MiB 74.4 / 80.7, 600
-//     151 / 149; top-4, 600 MiB 141 / 148; top-8, 900 MiB 221 / 260).  The line at 300 MiB costs at most a tenth on the wrong
-//     side of it.
+//       170 MiB    150 / 148    153 / 152    156 / 153    167 / 166
+//       220        202 / 197    214 / 212    212 / 212    222 / 222
+//       250        231 / 225    237 / 238    241 / 247    255 / 259
+//       299        285 / 275    290 / 295    301 / 316    321 / 331
+//     8 and 1024 experts and rows of 2 to 14 KB are alike.  Rows of 1 KB like the placing launch longer (top-1, 220 MiB 264 /
+//     267, 299 351 / 348).  The permute alone, called over and over: 250 MiB 55.9 / 52.9, 54.3 / 54.0, 52.2 / 54.6, 59.9 / 55.0;
+//     600 MiB 147 / 121, 138 / 126, 132 / 126, 140 / 126.
 // Against four launches for the sort and one for the rows: 8192 tokens x top-8, 128 experts, 4 KB rows 70 -> 67 us, 81920
 // tokens 589 -> 577, 4096 tokens 43 -> 29, 24 tokens 26 -> 4.4; top-1 to top-8 rows of 1 to 14 KB, 60 to 900 MiB: 0.54 to
 // 0.96 of the time.
@@ -50,7 +51,6 @@ constexpr int kCountThreads = 1024;
 constexpr int kMaxExperts = 1024;
 constexpr int64_t kSmallAssignments = 8192;  // one-launch sort up to here
 constexpr int64_t kTableEntries = 16384;     // the placing workgroups sum the count table themselves up to here
-constexpr int64_t kPlaceMoveBytes = 300ll << 20;  // the placing workgroups move the rows too up to here (bytes read and written)
 constexpr int kPlaceThreads = 512;
 constexpr int kBatch = 1024;                 // assignments whose destinations a placing workgroup holds at a time
 
@@ -59,6 +59,12 @@ int64_t count_chunk(int64_t n, int num_experts) {
   int64_t chunk = kCountThreads;
   while (chunk < 8 * kCountThreads && ((n + chunk - 1) / chunk) * num_experts > kTableEntries) chunk *= 2;
   return chunk;
+}
+
+// Whether the placing workgroups move the rows too (see the top of the file): by the bytes read and written.
+bool place_moves_rows(int64_t tokens, int topk, int64_t row_bytes) {
+  const int64_t most = topk == 1 && row_bytes >= 2048 ? 200ll << 20 : 300ll << 20;
+  return tokens * (topk + 1) * row_bytes <= most;
 }
 
 // The lanes of the wave whose (valid) key equals this lane's; keys below 2^bits.
@@ -546,7 +552,7 @@ int launch_moe_permute(const void* in, void* out, int64_t row_bytes, const int32
   MoveArgs a;
   a.chunks16 = (int)(row_bytes / 16);
   const bool move = in && tokens > 0 && a.chunks16 <= (1 << 20) &&  // a batch's chunks are counted in 32 bits
-                    (small_sort(n, topk) || (n + tokens) * row_bytes <= kPlaceMoveBytes);
+                    (small_sort(n, topk) || place_moves_rows(tokens, topk, row_bytes));
   a.in = move ? (const i32x4_t*)in : nullptr;
   a.out = (i32x4_t*)out;
   a.indices = indices;
