@@ -46,16 +46,16 @@ PEAK_HBM_GBS = 8000.0
 # printed only while the hash of that source set still equals the stamp below; after any change to those files it
 # is null until the counters are read again (python bench.py --print-traffic-stamps prints the current hashes).
 MEASURED_TRAFFIC_GB = {
-    "bf16_m_grouped_gateup_nt": (11.63, "gemm16"),
-    "bf16_m_grouped_gateup_nn": (10.29, "gemm16"),
-    "bf16_m_grouped_gateup_fp8_out": (10.94, "gemm16"),
-    "bf16_m_grouped_down_nt": (5.26, "gemm16"),
-    "bf16_m_grouped_down_nn": (5.44, "gemm16"),
+    "bf16_m_grouped_gateup_nt": (11.38, "gemm16"),
+    "bf16_m_grouped_gateup_nn": (9.9, "gemm16"),
+    "bf16_m_grouped_gateup_fp8_out": (10.74, "gemm16"),
+    "bf16_m_grouped_down_nt": (5.24, "gemm16"),
+    "bf16_m_grouped_down_nn": (5.33, "gemm16"),
     "bf16_masked_decode": (2.47, "gemm16"),
-    "bf16_k_grouped_wgrad": (28.5, "gemm16"),
-    "fp8_block_m_grouped": (24.55, "gemm8"),
-    "fp8_channel_m_grouped": (26.27, "gemm8"),
-    "fp8_channel_k_grouped": (16.77, "gemm8"),
+    "bf16_k_grouped_wgrad": (28.75, "gemm16"),
+    "fp8_block_m_grouped": (24.84, "gemm8"),
+    "fp8_channel_m_grouped": (26.96, "gemm8"),
+    "fp8_channel_k_grouped": (16.78, "gemm8"),
     "quant_trans128": (8.12, "quant"),
     "quant_token128": (8.2, "quant"),
     "moe_permute": (3.06, "permute"),      # the row mover (the sort kernels move < 1 % of that)
@@ -68,9 +68,9 @@ TRAFFIC_SOURCES = {
     "permute": ("moe_permute.hip",),
 }
 TRAFFIC_STAMPS = {  # sha256 over the source set's files, first 16 hex digits, at the time of the counter runs
-    "gemm16": "cb51591effa7a809",
-    "gemm8": "a03a1cbc94564fe7",
-    "quant": "a6c28452874ed31c",
+    "gemm16": "f2a0e05e5afc8cad",
+    "gemm8": "54cd90ab5497d50e",
+    "quant": "8debad0aae3b9696",
     "permute": "f5951f56ef17868f",
 }
 

@@ -130,7 +130,10 @@ TGG_DEV int64_t sched_block_scan(int64_t v, Table& t, int64_t& total) {
 }
 
 // sched_prefix by the whole workgroup: every thread takes a run of neighbouring groups, the runs meet in two scans.  All
-// threads must call this, with the loaded extents visible to them.
+// threads must call this, with the loaded extents visible to them.  For the 1024-entry table of the shape-agnostic kernel,
+// whose workgroups have fewer threads than there may be groups: one thread's serial pass is 0.15 us a group, half of a small
+// launch again (K-grouped from sizes, outputs of 264 x 520 and 4 tokens a group: 1024 groups 502 -> 333 us, 600 groups 285 ->
+// 186).  Same values.
 template <int BM, class Table>
 TGG_DEV void sched_prefix_runs(const GemmParams& p, Table& t) {
   const int per = (p.G + (int)blockDim.x - 1) / (int)blockDim.x;
@@ -179,8 +182,8 @@ TGG_DEV void sched_order_groups(const GemmParams& p, Table& t) {
 // takes 0.2 us per group (15 us at 128 groups, a tenth of a decode-sized launch).  Same values as sched_prefix.
 // The tile scan carries the prefix for tiles of half the height along in its upper word: the calling thread's group
 // would start at the returned tile id under that cut, and t.pad_ receives how many tiles more that cut has in all
-// (see sched_use_half_height).  Where the serial pass runs instead, t.pad_ is set so large that no caller prefers
-// the half-height cut.
+// (see sched_use_half_height).  With more groups than threads the serial pass (or sched_prefix_runs) takes the place of the
+// scans, and t.pad_ is set so large that no caller prefers the half-height cut.
 template <int BM, class Table>
 TGG_DEV int32_t sched_init(const GemmParams& p, Table& t) {
   if (p.mode == MODE_KG || p.G > (int)blockDim.x || blockDim.x > 1024) {
