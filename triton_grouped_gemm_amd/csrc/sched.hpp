@@ -420,14 +420,29 @@ TGG_HD int sched_queue_id(int n, int xq, int R) {
   return (pass * 8 + ((pass & 1) ? 7 - xq : xq)) * R + n % R;
 }
 
+// Lane x < 8 holds the value of XCD x's counter.  Bit x of the result: that counter's next draw stands for a tile (a counter
+// only grows: one that has been seen exhausted stays so).  The whole wave calls it.
+TGG_DEV int sched_queue_left(int seen, int total, int R) {
+  const int x = lane_id();
+  return (int)(uint32_t)__ballot(x < 8 && sched_queue_id(seen, x & 7, R) < total);
+}
+
+// The first counter behind `own` (in ring order) among those of the mask `left` (not empty).
+TGG_HD int sched_queue_next(int left, int own) {
+  const int turned = ((left >> own) | (left << (8 - own))) & 0xff;  // bit d: counter own + d
+  return (own + __builtin_ctz(turned)) & 7;
+}
+
 // Work queue of the K-grouped tuned kernels: eight counters in global memory, one per XCD (zero at launch).  The
 // tile space is cut into runs of R neighbouring tiles (R = workgroups per XCD; neighbours are tiles of one group,
 // which share operand panels in an XCD's L2), and the runs are dealt to the XCDs in order of decreasing cost, back
 // and forth (0..7, 7..0, ...) so that no XCD always gets the dearest of eight.  Within an XCD a tile goes to
 // whichever workgroup asks next: like the static interleaved walk the XCD works through runs of neighbours, but a
-// workgroup that drew expensive tiles draws fewer.  A workgroup whose own XCD has nothing left takes from the
-// next XCD's counter, and so on round the ring: what the deal leaves uneven is evened out at the end.  For every
-// counter the ids grow with the number of draws, so one id at or beyond `total` means that counter is exhausted.
+// workgroup that drew expensive tiles draws fewer.  A workgroup whose own XCD has nothing left looks at all
+// counters at once and goes on with the next one in ring order that has tiles, until none has: what the deal leaves uneven is
+// evened out at the end.  (Finding them exhausted by a draw from one counter after the other takes seven more round
+// trips at the end of every launch, half of a small one: bf16, 4 groups of 2048 x 1536, 64 / 256 / 1024 tokens a group 38 / 40 / 56
+// -> 20 / 25 / 56 us; FP8, 4 groups of 768 x 2048, 128 / 1024 tokens 46 / 46 -> 27 / 37 us.)  For every counter the ids grow with the number of draws, so one id at or beyond `total` means that counter is exhausted.
 //
 // One wave of each workgroup draws for it.  A draw costs a round trip to the counter (about a microsecond), which on
 // tiles of a slab or two is as long as the tile, so it is requested at the start of a slab and taken at the slab's
@@ -447,56 +462,75 @@ struct QueueDraw {
   Table& t;
   const int total, slab_k;
   int ahead = 0;             // slabs drawn and not yet requested by the copy stream (kept by every wave's begin_slab, read by the drawing wave)
-  int drawn = 0, victim = 0;  // tiles drawn; counters found exhausted
+  int drawn = 0, xq;          // tiles drawn; the counter to draw from
+  int exhausted = 0;          // counters that a draw has found without a tile, one bit each
+  int looking = 0;            // 1: the next request does not draw but asks for the values of all eight counters
   int live;                   // 1 in the wave that draws, until it has put the end marker in the ring (integers, not
                               // truth values, so that they stay in scalar registers)
-  int answer;                 // lane 0: the counter's value once the wave's memory operations have been waited for
+  int answer;                 // the counters' values once the wave's memory operations have been waited for
 
   TGG_DEV QueueDraw(const GemmParams& p_, Table& t_, int total_, int slab_k_, bool drawing)
-      : p(p_), t(t_), total(total_), slab_k(slab_k_), live(drawing ? 1 : 0) {}
+      : p(p_), t(t_), total(total_), slab_k(slab_k_), xq((gridDim.x & 7) == 0 ? (int)(blockIdx.x & 7) : 0), live(drawing ? 1 : 0) {}
 
   TGG_DEV int32_t& ring(int pos) { return reinterpret_cast<int32_t*>(t.scan_)[pos & (kRing - 1)]; }
   TGG_DEV bool spread() const { return (gridDim.x & 7) == 0; }  // eight counters; else one
-  TGG_DEV int counter() const { return spread() ? ((int)(blockIdx.x & 7) + victim) & 7 : 0; }
   TGG_DEV int wanted() { live = __builtin_amdgcn_readfirstlane(live); return ahead < kAhead ? live : 0; }
   // begin_slab has requested a slab of the tile (issued < slabs: there was one left)
   TGG_DEV void count(int issued, int slabs) { ahead -= (int)((uint32_t)(issued - slabs) >> 31); }
 
-  // n: the value drawn from the current counter
-  TGG_DEV void accept(int n) {
-    const int id = spread() ? sched_queue_id(n, counter(), (int)gridDim.x >> 3) : n;
-    if (id < total) {
-      const int per_group = (int)((p.m_total + BM - 1) / BM) * ((p.N + BN - 1) / BN);
-      const int rows = __builtin_amdgcn_readfirstlane(t.rows[t.tile0[id / per_group]]);
-      ring(drawn++) = id;
-      ahead += rows > 0 ? (rows + slab_k - 1) / slab_k : 1;  // an empty group's tile has one slab of nothing
-    } else if (++victim >= (spread() ? 8 : 1)) {
+  // the answer to a request (a value per lane)
+  TGG_DEV void accept(int value) {
+    const int R = (int)gridDim.x >> 3;
+    bool end = false;
+    if (__builtin_expect(looking, 0)) {
+      const int left = sched_queue_left(value, total, R) & ~exhausted;
+      looking = 0;
+      end = left == 0;
+      if (!end) xq = sched_queue_next(left, xq);
+    } else {
+      const int n = __builtin_amdgcn_readfirstlane(value);
+      const int id = spread() ? sched_queue_id(n, xq, R) : n;
+      if (id < total) {
+        const int per_group = (int)((p.m_total + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+        const int rows = __builtin_amdgcn_readfirstlane(t.rows[t.tile0[id / per_group]]);
+        ring(drawn++) = id;
+        ahead += rows > 0 ? (rows + slab_k - 1) / slab_k : 1;  // an empty group's tile has one slab of nothing
+      } else {
+        exhausted |= 1 << xq;
+        looking = spread();
+        end = !looking;
+      }
+    }
+    if (end) {
       ring(drawn++) = total;
       live = 0;
     }
   }
 
-  TGG_DEV void draw_now() {
-    int n = 0;
-    if (lane_id() == 0) n = atomicAdd(p.queue + counter(), 1);
-    accept(__builtin_amdgcn_readfirstlane(n));
+  // lane 0 draws from the current counter, or (looking) lanes 0-7 read one counter each
+  TGG_DEV int ask() {
+    const int lane = lane_id();
+    int value = 0;
+    // The address is made a lane's own: for one that the wave shares the compiler merges the lanes' additions and reads
+    // the result back on the spot, which is the wait that a request is to avoid.
+    int at = looking ? (lane & 7) : xq;
+    asm("" : "+v"(at));
+    if (lane < (looking ? 8 : 1)) value = __hip_atomic_fetch_add(p.queue + at, looking ? 0 : 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return value;
   }
+
+  TGG_DEV void draw_now() { accept(ask()); }
 
   TGG_DEV void first() { while (wanted()) draw_now(); }
 
-  // Requests a draw; `answer` is in flight until take().  A builtin, so that the compiler knows of the register in flight
-  // and waits wherever it might touch it.  The address is made a lane's own: for one that the wave shares the compiler
-  // merges the lanes' additions and reads the result back on the spot, which is the wait that this is to avoid.
-  TGG_DEV void request() {
-    int at = counter();
-    asm("" : "+v"(at));
-    if (lane_id() == 0) answer = __hip_atomic_fetch_add(p.queue + at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  // `answer` is in flight until take().  A builtin, so that the compiler knows of the register in flight and waits wherever it
+  // might touch it.
+  TGG_DEV void request() { answer = ask(); }
 
   // The drawing wave, after it has waited for all of its memory operations and in front of a workgroup barrier.
   TGG_DEV void take(int requested) {
     asm volatile("" : "+v"(answer));  // arrived: not to be read any earlier than here
-    if (__builtin_expect(requested, 0)) accept(__builtin_amdgcn_readfirstlane(answer));
+    if (__builtin_expect(requested, 0)) accept(answer);
     while (__builtin_expect(ahead <= 1 && live, 0)) draw_now();  // the next slab's request may ask for the next tile
   }
 };
