@@ -219,3 +219,45 @@ def test_four_wave_kernel_reads_no_accumulator_right_behind_its_multiply():
         pytest.skip("no device assembly in the build directory (the library was built elsewhere or not yet)")
     found = accumulator_reads_too_early(f.read_text())
     assert not found, f"{len(found)} reads too close behind the multiply, first: {found[0]}"
+
+
+# The weight-gradient kernel holds a work-queue draw that is in flight across K steps in v255 (see gemm_wgrad.hip).
+def stray_uses_of_v255(text: str):
+    stray, inside = [], False
+    for raw in text.splitlines():
+        line = raw.split(";")[0].strip()
+        if line.endswith(":") and not line.startswith("."):
+            inside = "gemm_wgrad_kernel" in line
+            continue
+        if not inside or not line or line.startswith("."):
+            continue
+        toks = [t.strip(",") for t in line.split()]
+        if not any(255 in _regs(t, "v") for t in toks[1:]):
+            continue
+        drawn = toks[0] == "global_atomic_add" and toks[1] == "v255" and toks[-1] == "sc0" and "v255" not in toks[2:]
+        taken = toks[0] == "v_readfirstlane_b32" and toks[2] == "v255"
+        if not (drawn or taken):
+            stray.append(line)
+    return stray
+
+
+def test_v255_scanner_on_snippets():
+    head = "_ZN3tgg17gemm_wgrad_kernelILi0EEEvNS_10GemmParamsE:\n"
+    assert stray_uses_of_v255(head + "global_atomic_add v255, v1, v2, s[4:5] sc0\nv_readfirstlane_b32 s3, v255\n") == []
+    assert len(stray_uses_of_v255(head + "v_mov_b32_e32 v255, v3\n")) == 1
+    assert len(stray_uses_of_v255(head + "ds_read_b128 v[252:255], v3\n")) == 1
+    assert len(stray_uses_of_v255(head + "global_atomic_add v255, v255, v2, s[4:5] sc0\n")) == 1
+    assert stray_uses_of_v255("other_kernel:\nv_mov_b32_e32 v255, v3\n") == []
+
+
+def test_weight_gradient_kernel_keeps_the_draw_in_flight_and_its_accumulators():
+    f = BUILD / "gemm_wgrad.gfx950.s"
+    if not f.exists():
+        pytest.skip("no device assembly in the build directory (the library was built elsewhere or not yet)")
+    text = f.read_text()
+    assert "gemm_wgrad_kernel" in text
+    stray = stray_uses_of_v255(text)
+    assert not stray, f"{len(stray)} compiler-generated uses of v255, first: {stray[0]}"
+    found = accumulator_reads_too_early(text.replace("gemm_wgrad_kernel", "gemm_w4_kernel"))
+    assert not found, f"{len(found)} reads too close behind the multiply, first: {found[0]}"
+    assert "scratch_" not in text  # a spilled value would be reloaded behind the copies

@@ -61,6 +61,8 @@ int launch_fast_16bit(const GemmParams& p, int dt, int layout, hipStream_t s);
 bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size);
 bool w4_decided_on_device(const GemmParams& p);
 int launch_w4_16bit(const GemmParams& p, int dt, int layout, hipStream_t s);
+bool wgrad_supported(const GemmParams& p, int dt, bool any_size);
+int launch_wgrad_16bit(const GemmParams& p, int dt, hipStream_t s);
 bool fast_quant_supported(const GemmParams& p, int dt, int layout);
 int launch_fast_16bit_quant(const GemmParams& p, int dt, int layout, hipStream_t s);
 void set_fast_variant(int v);
@@ -195,6 +197,7 @@ static int dispatch_16bit(const GemmParams& p, int dt, int layout, hipStream_t s
     q.wide_gate = 2;
     return launch_fast_16bit(q, dt, layout, s);
   }
+  if (!force_generic && four_wave && layout == 2 && wgrad_supported(p, dt, four_wave == 2)) return launch_wgrad_16bit(p, dt, s);
   if (!force_generic && fast_supported(p, dt, layout)) return launch_fast_16bit(p, dt, layout, s);
   return launch_generic_16bit(p, dt, layout, s);
 }

@@ -55,8 +55,8 @@
 //     than three multiplies after the multiply that wrote them (a multiply takes 16 cycles to issue and delivers
 //     within two more), except where a flush follows a tile directly: there the last row block's accumulators pass
 //     through a statement of idle cycles first.  Accumulators are never the target of a load.
-#include "fast_common.hpp"
 #include "launch.hpp"
+#include "w4_common.hpp"
 
 namespace tgg {
 
@@ -64,30 +64,6 @@ namespace {
 
 enum : int { W4_NT = 0, W4_NN = 1 };
 constexpr int BK4 = 64;
-
-template <int DT> TGG_DEV void mfma_acc(f32x4_t& acc, const i32x4_t& w, const i32x4_t& x) {
-  if (DT == DT_BF16) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(x));
-  else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(x));
-}
-
-// The same with a zero addend: the first K step of a tile starts its accumulators afresh
-template <int DT> TGG_DEV void mfma_new(f32x4_t& acc, const i32x4_t& w, const i32x4_t& x) {
-  if (DT == DT_BF16) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(w), "v"(x));
-  else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(acc) : "v"(w), "v"(x));
-}
-
-// 16-byte fragment of a K-contiguous operand
-template <int OFF> TGG_DEV void lds_read_b128(i32x4_t& dst, uint32_t addr) {
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF) : "memory");
-}
-// fragment of a token-row operand: two transposing 8-byte reads (K 0..3 and 4..7 of the lane's column)
-template <int OFF0, int OFF1> TGG_DEV void lds_read_tr(i32x4_t& dst, uint32_t addr) {
-  i32x2_t lo, hi;
-  asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%3\n\tds_read_b64_tr_b16 %1, %2 offset:%4"
-               : "=&v"(lo), "=&v"(hi) : "v"(addr), "n"(OFF0), "n"(OFF1) : "memory");
-  dst = __builtin_shufflevector(lo, hi, 0, 1, 2, 3);
-}
-#define TGG_TIE8(f) "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]), "+v"(f[6]), "+v"(f[7])
 
 struct W4Cfg {
   static constexpr int BM = 256, BN = 256, NWAVES = 4, THREADS = 256;

@@ -1,0 +1,462 @@
+// Four-wave bf16/fp16 K-grouped GEMM kernel for gfx950 (weight gradient): C[g] = A[tokens of g, :]^T . B[tokens of g, :],
+// A [Ktot, Mdim], B [Ktot, N], C [G, Mdim, N].
+//
+// One workgroup per CU, four waves, one per SIMD; tile 256x256, every wave owns a 128x128 block of 16x16x32 MFMA tiles with
+// its 256 accumulator registers in AGPRs (see gemm_w4.hip for why, and for the rules that the order of the instructions
+// follows).  A K step is 32 tokens, and so is a slab: 16 KB of A and 16 KB of B, token rows of 512 bytes, four slab buffers
+// in LDS.  Per K step q, per wave:
+//   64 multiplies on fragment set q % 2; meanwhile the 16 fragments of slab q + 1 are read into the other set (two
+//   transposing 8-byte reads each) and this wave's eight copies of slab q + 4 go straight to LDS, into the buffer of slab q;
+//   wait for the fragment reads and for this wave's copies of slab q + 2, workgroup barrier.
+// The copies have between two and three K steps to land, where two 64-token buffers leave them one or two: what
+// a launch with short segments waits for is memory (it writes 128 KB of output per tile, and loads queue behind stores).
+// Token rows are 512 bytes whatever the slab's depth, so that the shallow slabs cost no extra requests here (operands whose
+// rows run along K would fetch half lines), and a segment's last slab is padded to 32 tokens and not to 64.
+//
+// The epilogue rides on multiplies as in gemm_w4.hip: strips 0-3 of a wave's block are converted and stored between the
+// multiplies of the tile's last K step, strips 4-7 between those of the next tile's first, whose multiplies start from a
+// zero addend.  Against the eight-wave kernel (gemm_fast.hip, TN), outputs of 2048 x 1536 for 128 groups of 256 / 512 / 1024 tokens
+// on average: 318 / 476 / 798 -> 313 / 441 / 704 us (5120 tokens: 3434 -> 3042, 1.36 PFLOP/s); with 16 groups of 64 / 256 / 4096: 41 / 49 / 357 -> 32 / 46 / 322.
+// What bounds it: from about 512 tokens on the matrix pipe (0.73 us a K step with all CUs multiplying, 0.53 on a quarter of them,
+// i.e. power), 1.5 us a tile for the epilogue's conversions and LDS staging; below, memory: with 256 tokens a launch that stores nothing takes
+// 191 us and one that stores 300, where 1.04 GB at the copy rate would take 204 (reads that come from HBM wait behind the writes:
+// on 64 CUs, or with the operands in the memory-side cache, the stores cost nothing).  A tile has an even number of K steps, four at least (of nothing where the segment ends sooner: the
+// copy stream is four slabs ahead of the multiplies, so it is in the tile being multiplied or in the next one, and every
+// tile starts on the same parity).
+//
+// Tiles come from the work queue of sched.hpp (largest groups first, one counter per XCD) or, without one, from the
+// fixed walk.  Wave 0 draws: the request for the tile after the next goes out four K steps before a tile's end, and its answer, in
+// order with the copies, has arrived by the wait that ends the tile.  It sits in v255, which is named in the
+// instruction text because a value in flight across K steps must not be known to the compiler (tests/test_isa_hazards.py
+// scans the kept assembly for any other use).
+#include "launch.hpp"
+#include "w4_common.hpp"
+#include <utility>
+
+namespace tgg {
+
+namespace {
+
+struct WgradCfg {
+  static constexpr int BM = 256, BN = 256, THREADS = 256, KS = 32;
+  static constexpr int OP_BYTES = KS * 512, SLAB_BYTES = 2 * OP_BYTES, SLABS = 4;
+  static constexpr int EPI_PITCH = 4 * 32 + 16;         // epilogue staging; a piece: 16 rows x 64 outputs, row pitch in bytes
+  static constexpr int EPI_PIECE = 16 * EPI_PITCH;
+  static constexpr int EPI_WAVE_BYTES = 2 * EPI_PIECE;  // two pieces alternate
+  static constexpr int SCHED_OFF = SLABS * SLAB_BYTES;
+  static constexpr int NEXT_OFF = SCHED_OFF + (((int)sizeof(SchedTableT<kFastMaxGroups>) + 255) & ~255);  // drawn tile ids, two words
+  static constexpr int EPI_OFF = NEXT_OFF + 256;
+  static constexpr int SMEM_BYTES = EPI_OFF + 4 * EPI_WAVE_BYTES;
+  static_assert(SMEM_BYTES <= 160 * 1024, "LDS budget");
+};
+
+// Division of 32-bit values by a divisor that is fixed for the launch, on the scalar unit.  m = floor(2^32 / d) + 1: the
+// estimate n m / 2^32 is the quotient or one more for every 32-bit n.
+struct FixedDiv {
+  uint32_t d, m;
+  TGG_DEV explicit FixedDiv(int d_) : d((uint32_t)d_), m(d_ > 1 ? 0xffffffffu / (uint32_t)d_ + 1 : 0) {}
+  TGG_DEV uint32_t div(uint32_t n) const {
+    if (d == 1) return n;
+    const uint32_t q = __umulhi(n, m);
+    return q * d > n ? q - 1 : q;
+  }
+};
+
+// f(integral_constant<int, n>) for n = 0 .. 63: the gaps of a K step's multiplies
+template <class F, int... N> TGG_DEV void each_gap_of(const F& f, std::integer_sequence<int, N...>) { (f(std::integral_constant<int, N>()), ...); }
+template <class F> TGG_DEV void each_gap(const F& f) { each_gap_of(f, std::make_integer_sequence<int, 64>()); }
+
+template <int DT>
+__global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const GemmParams p) {
+  typedef WgradCfg C;
+  typedef Operand<256, false> Op;  // a slab of either operand: token rows of 512 bytes (here 32 of them)
+
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  auto& sched = *reinterpret_cast<SchedTableT<kFastMaxGroups>*>(smem + C::SCHED_OFF);
+  auto* const next_id = reinterpret_cast<volatile int32_t*>(smem + C::NEXT_OFF);
+  sched_init<C::BM>(p, sched);
+
+  const uint32_t smem_addr = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm0 = (wave >> 1) * 128, wn0 = (wave & 1) * 128;
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int a_ld = (int)p.m_total * 2, b_ld = p.N * 2;  // token row pitches in bytes
+
+  // Copy k (0..3) of an operand's slab by this wave is copy instruction wave + 4 k of the slab: token rows 2 (wave + 4 k), + 1.
+  int vo_a[4], vo_b[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    vo_a[k] = Op::lane_voff(lane, (wave + 4 * k) % Op::NPAT, a_ld) + (wave + 4 * k) * Op::RPI * a_ld;
+    vo_b[k] = Op::lane_voff(lane, (wave + 4 * k) % Op::NPAT, b_ld) + (wave + 4 * k) * Op::RPI * b_ld;
+  }
+  // LDS addresses of the fragment reads (gemm_fast.hip has the layout).  A slab buffer's number is (pair, parity): the parity
+  // goes into the instruction's offset, the pair is toggled in the address once in two K steps.
+  uint32_t a_rd[8], b_rd[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int e = l16 >> 2, c = l16 & 3, sw = (e * 4) ^ ((lg & 1) * 2), row = (lg * 8 + e) * 512 + (c & 1) * 8;
+    a_rd[i] = smem_addr + row + ((((wm0 + 16 * i) / 8 + (c >> 1)) ^ sw) << 4);
+    b_rd[i] = smem_addr + C::OP_BYTES + row + ((((wn0 + 16 * i) / 8 + (c >> 1)) ^ sw) << 4);
+  }
+
+  // ---- tiles -------------------------------------------------------------------------------------------------------
+  const int tiles_n = (p.N + C::BN - 1) / C::BN, tiles_m = (int)((p.m_total + C::BM - 1) / C::BM);
+  const int per_group = tiles_m * tiles_n, total = p.G * per_group;
+  const int nc = sched_chunk_width(tiles_n, p.n_chunk), full_chunks = tiles_n / nc, tail_width = tiles_n - full_chunks * nc;
+  const FixedDiv by_group(per_group), by_chunk(tiles_m * nc), by_nc(nc), by_tail(tail_width > 0 ? tail_width : 1);
+  const TileWalk walk64 = sched_walk(total, false);
+  const bool queued = p.queue != nullptr;
+  struct TileInfo {
+    int g, m0, n0;   // g = -1: there are no more tiles
+    int klen, steps; // tokens of the segment, K steps
+    int64_t k0;      // its first token
+  };
+  auto look_up = [&](int id) __attribute__((always_inline)) {
+    TileInfo t;
+    t.g = -1;
+    t.m0 = t.n0 = t.klen = t.steps = 0;
+    t.k0 = 0;
+    if (id < total) {
+      const int slot = (int)by_group.div((uint32_t)id), r = id - slot * per_group;
+      int c = (int)by_chunk.div((uint32_t)r);  // as sched_split
+      const bool tail = c >= full_chunks;
+      c = tail ? full_chunks : c;
+      const int width = tail ? tail_width : nc, q = r - c * tiles_m * nc;
+      const int mt = (int)(tail ? by_tail.div((uint32_t)q) : by_nc.div((uint32_t)q));
+      t.m0 = mt * C::BM;
+      t.n0 = (c * nc + q - mt * width) * C::BN;
+      t.g = __builtin_amdgcn_readfirstlane(sched.tile0[slot]);
+      t.klen = __builtin_amdgcn_readfirstlane(sched.rows[t.g]);
+      t.k0 = (int64_t)uniform64((uint64_t)sched.row0[t.g]);
+      const int steps = (t.klen + 2 * C::KS - 1) / (2 * C::KS) * 2;
+      t.steps = steps < C::SLABS ? C::SLABS : steps;
+    }
+    return t;
+  };
+  // The drawing wave.  A counter's value stands for a tile id (sched_queue_id); once it stands for none, the wave looks at
+  // all counters at once and goes on with one that has tiles left, if there is any.
+  const bool spread = (gridDim.x & 7) == 0;  // eight counters; else one
+  const int R = (int)gridDim.x >> 3;
+  const FixedDiv by_r(R > 0 ? R : 1);
+  int xq = spread ? (int)(blockIdx.x & 7) : 0;
+  auto id_of = [&](int n) __attribute__((always_inline)) {
+    if (!spread) return n;
+    const int pass = (int)by_r.div((uint32_t)n);
+    return (pass * 8 + ((pass & 1) ? 7 - xq : xq)) * R + n - pass * R;
+  };
+  int exhausted = 0;  // counters that a draw has found without a tile, one bit each
+  auto steal = [&]() __attribute__((always_inline)) {  // the next tile of another counter, `total` where there is none
+    while (spread) {  // eight rounds at most: a round ends the search or marks a counter
+      exhausted |= 1 << xq;
+      const int seen = lane < 8 ? __hip_atomic_load(p.queue + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+      const int left = sched_queue_left(seen, total, R) & ~exhausted;
+      if (left == 0) break;
+      xq = sched_queue_next(left, xq);
+      int n = 0;
+      if (lane == 0) n = atomicAdd(p.queue + xq, 1);
+      const int id = id_of(__builtin_amdgcn_readfirstlane(n));
+      if (id < total) return id;
+    }
+    return total;
+  };
+
+  // ---- the copy stream ---------------------------------------------------------------------------------------------
+  // The slabs of all of this workgroup's tiles form one sequence; the cursor is four slabs ahead of the multiplies.  Tokens
+  // beyond the segment read as zero through the descriptor's length.
+  struct Feed {
+    uint64_t a_base, b_base;  // the next slab
+    int rem;                  // tokens of the segment from there on
+    int a_off, b_off;         // the tile's columns within a token row, bytes
+    int left;                 // slabs of the tile still to be requested
+  };
+  auto feed_of = [&](const TileInfo& t) __attribute__((always_inline)) {
+    Feed f;
+    f.rem = t.klen;
+    f.left = t.g < 0 ? 0x7fffffff : t.steps;
+    f.a_off = t.m0 * 2;
+    f.b_off = t.n0 * 2;
+    f.a_base = (uint64_t)p.A + (uint64_t)(t.k0 * a_ld + f.a_off);
+    f.b_base = (uint64_t)p.B + (uint64_t)(t.k0 * b_ld + f.b_off);
+    return f;
+  };
+  Feed feed, nxt;
+  i32x4_t ra, rb;
+  auto rsrc = [&](uint64_t base, int bytes) __attribute__((always_inline)) {  // make_rsrc32 of values that are in scalar registers
+    return i32x4_t{(int)(uint32_t)base, (int)(uint32_t)(base >> 32) & 0xffff, bytes < 0 ? 0 : bytes, 0x00020000};
+  };
+  auto step_feed = [&]() __attribute__((always_inline)) {  // descriptors of the next slab; the cursor moves behind it
+    const bool wrap = feed.left == 0;
+    feed.a_base = wrap ? nxt.a_base : feed.a_base;
+    feed.b_base = wrap ? nxt.b_base : feed.b_base;
+    feed.rem = wrap ? nxt.rem : feed.rem;
+    feed.a_off = wrap ? nxt.a_off : feed.a_off;
+    feed.b_off = wrap ? nxt.b_off : feed.b_off;
+    feed.left = (wrap ? nxt.left : feed.left) - 1;
+    int rows = feed.rem < 0 ? 0 : feed.rem;
+    asm("" : "+s"(rows));  // two scalar instructions and not a vector one whose result would have to be read back
+    rows = rows > C::KS ? C::KS : rows;
+    ra = rsrc(feed.a_base, rows * a_ld - feed.a_off);
+    rb = rsrc(feed.b_base, rows * b_ld - feed.b_off);
+    feed.rem -= C::KS;
+    feed.a_base += (uint64_t)(C::KS * a_ld);
+    feed.b_base += (uint64_t)(C::KS * b_ld);
+  };
+  const uint32_t wave_buf = smem_addr + wave * 1024;  // copy `wave` of buffer 0's A slab
+  auto copy_m0 = [&](auto Kc, uint32_t buf) __attribute__((always_inline)) {
+    constexpr int k = decltype(Kc)::value;
+    asm volatile("s_add_u32 m0, %0, %1" : : "s"(buf), "n"((k >> 2) * C::OP_BYTES + (k & 3) * 4096) : "memory", "m0", "scc");
+  };
+  auto copy = [&](auto Kc) __attribute__((always_inline)) {
+    constexpr int k = decltype(Kc)::value;
+    const int v = k < 4 ? vo_a[k & 3] : vo_b[k & 3];
+    const i32x4_t r = k < 4 ? ra : rb;
+    asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(v), "s"(r) : "memory");
+  };
+
+  // ---- fragments and accumulators ------------------------------------------------------------------------------------
+  i32x4_t fa[2][8], fb[2][8];
+  f32x4_t acc[8][8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto toggle = [&](uint32_t& at) __attribute__((always_inline)) { asm volatile("v_xor_b32 %0, 0x10000, %0" : "+v"(at)); };
+  // read number q (0..15) of a slab's fragments: B's first, the next K step needs all of them at once; PAR: the slab's parity
+  auto read_frag = [&](auto PARc, auto Qc, i32x4_t (&sa)[8], i32x4_t (&sb)[8]) __attribute__((always_inline)) {
+    constexpr int Q = decltype(Qc)::value, off = decltype(PARc)::value * C::SLAB_BYTES;
+    if (Q < 8) lds_read_tr<off, off + 4 * 512>(sb[Q & 7], b_rd[Q & 7]);
+    else lds_read_tr<off, off + 4 * 512>(sa[Q & 7], a_rd[Q & 7]);
+  };
+
+  // ---- epilogue (see gemm_w4.hip, B as [G, K, N]): a lane owns row l16 and columns 16 j + 4 lg + (0..3) of block (i, j); a strip
+  // goes through the wave's LDS staging as two pieces of 64 columns and leaves as 16-byte stores of 128-byte row segments
+  i32x4_t pend_rs = make_rsrc32(0, 0);
+  int pend_cols = 0;
+  char* const stage = smem + C::EPI_OFF + wave * C::EPI_WAVE_BYTES;
+  struct EpiLane { char* wr; const char* rd; int off[2]; };
+  auto epi_lane = [&]() __attribute__((always_inline)) {
+    int el = lane;
+    asm volatile("" : "+v"(el));
+    EpiLane e;
+    e.wr = stage + (el & 15) * C::EPI_PITCH + (el >> 4) * 8;
+    e.rd = stage + (el >> 3) * C::EPI_PITCH + (el & 7) * 16;
+    const int off = ((el >> 3) * p.N + (el & 7) * 8) * 2, ch8 = (el & 7) * 8;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) e.off[h] = (64 * h + ch8 < pend_cols) ? off + 128 * h : kNoFetch;
+    return e;
+  };
+  auto epi_cvt = [&](const EpiLane& e, int i, int j) __attribute__((always_inline)) {
+    asm volatile("" : "+a"(acc[i][j]));
+    *(uint2*)(e.wr + (j >> 2) * C::EPI_PIECE + (j & 3) * 32) = pack4<DT>(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+    asm volatile("" ::: "memory");
+  };
+  auto epi_read = [&](const EpiLane& e, int h, i32x4_t (&v)[2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int it = 0; it < 2; ++it) v[it] = *(const i32x4_t*)(e.rd + h * C::EPI_PIECE + it * 8 * C::EPI_PITCH);
+    asm volatile("" ::: "memory");
+  };
+  auto epi_store = [&](const EpiLane& e, int i, int h, int it, const i32x4_t& v, bool between_multiplies) __attribute__((always_inline)) {
+    const int off = e.off[h] + (16 * i + 8 * it) * p.N * 2;
+    // wait states as in gemm_w4.hip: the data registers of a 16-byte store must not be overwritten within two
+    if (between_multiplies) asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 0" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
+    else asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 1" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
+  };
+  auto epi_flush = [&]() __attribute__((always_inline)) {  // strips 4-7 of the workgroup's last tile
+    asm volatile("s_nop 15\n\ts_nop 7" : "+a"(acc[7][0]), "+a"(acc[7][1]), "+a"(acc[7][2]), "+a"(acc[7][3]),
+                 "+a"(acc[7][4]), "+a"(acc[7][5]), "+a"(acc[7][6]), "+a"(acc[7][7]));
+    const EpiLane e = epi_lane();
+#pragma unroll
+    for (int i = 4; i < 8; ++i) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) epi_cvt(e, i, j);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        i32x4_t v[2];
+        epi_read(e, h, v);
+        epi_store(e, i, h, 0, v[0], false);
+        epi_store(e, i, h, 1, v[1], false);
+      }
+    }
+  };
+
+  // ---- prologue ------------------------------------------------------------------------------------------------------
+  typedef std::integral_constant<int, 0> I0;
+  typedef std::integral_constant<int, 1> I1;
+  typedef std::integral_constant<int, 2> I2;
+  typedef std::integral_constant<int, 16> W16;
+  typedef std::integral_constant<int, 32> W32;
+  typedef std::integral_constant<int, 48> W48;
+  bool live = queued && wave == 0;  // tiles are still being drawn
+  // requests the next tile's number; nothing may read v255 before the memory operations so far have been waited for
+  auto request = [&]() __attribute__((always_inline)) {
+    if (live && lane == 0) {
+      int32_t* const at = p.queue + xq;
+      asm volatile("global_atomic_add v255, %0, %1, %2 sc0" : : "v"(0), "v"(1), "s"(at) : "memory", "v255");
+    }
+  };
+  // takes the answer (it has arrived) and leaves the tile id for the other waves, in front of a barrier; pos: the tile's position
+  auto take = [&](int pos) __attribute__((always_inline)) {
+    if (live) {
+      int got;
+      asm volatile("v_readfirstlane_b32 %0, v255" : "=s"(got) : : "memory", "v255");
+      int id = id_of(got);
+      if (__builtin_expect(id >= total, 0)) {
+        id = steal();
+        live = id < total;
+      }
+      if (lane == 0) next_id[pos & 1] = id;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+  };
+  auto tile_at = [&](int pos) __attribute__((always_inline)) {
+    if (queued) return __builtin_amdgcn_readfirstlane(next_id[pos & 1]);
+    const int64_t id = walk64.first + (int64_t)pos * walk64.stride;
+    return id < walk64.end ? (int)id : total;
+  };
+  if (wave == 0 && lane < 2) next_id[lane] = total;  // what the other waves find once nothing is drawn any more
+  __syncthreads();
+  request();
+  wait_vmcnt<0>();
+  take(0);
+  __syncthreads();
+  TileInfo cur = look_up(tile_at(0)), following = cur;
+  feed = feed_of(cur);
+  nxt = feed;
+  request();
+#define TGG_WG_EACH8(f) f(0) f(1) f(2) f(3) f(4) f(5) f(6) f(7)
+  for (int s = 0; s < C::SLABS; ++s) {
+    step_feed();
+    const uint32_t buf = wave_buf + s * C::SLAB_BYTES;
+#define TGG_WG_P(c) copy_m0(std::integral_constant<int, c>(), buf); asm volatile("s_nop 0" ::: "memory"); copy(std::integral_constant<int, c>());
+    TGG_WG_EACH8(TGG_WG_P)
+#undef TGG_WG_P
+  }
+  wait_vmcnt<0>();
+  take(1);
+  __syncthreads();
+#define TGG_WG_RD(q) read_frag(I0(), std::integral_constant<int, q>(), fa[0], fb[0]);
+  TGG_WG_EACH8(TGG_WG_RD)
+  TGG_WG_RD(8) TGG_WG_RD(9) TGG_WG_RD(10) TGG_WG_RD(11) TGG_WG_RD(12) TGG_WG_RD(13) TGG_WG_RD(14) TGG_WG_RD(15)
+#undef TGG_WG_RD
+#undef TGG_WG_EACH8
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" : TGG_TIE8(fa[0]), TGG_TIE8(fb[0]) : : "memory");  // slab 0 is in registers: its buffer is free
+
+  uint32_t cp_off = 0;  // the slab buffer that the K step copies into
+  // One K step on fragment set CUR (the parity of the slab).  EPI 0: a tile's inner one, 1: its first, 2: its last, without the
+  // barrier.  WAIT: the memory operations that may be in flight at its end, see below.
+  auto kstep = [&](auto CURc, auto EPIc, auto WAITc) __attribute__((always_inline)) {
+    constexpr int CUR = decltype(CURc)::value, EPI = decltype(EPIc)::value, WAIT = decltype(WAITc)::value;
+    typedef std::integral_constant<int, CUR ^ 1> NextPar;
+    EpiLane e = {nullptr, nullptr, {0, 0}};
+    i32x4_t vv[2][2];
+    if (EPI) e = epi_lane();
+    const uint32_t buf = wave_buf + cp_off;
+    constexpr int EPI_S0 = EPI == 2 ? 0 : 4, EPI_G0 = EPI == 2 ? 4 : 0;
+    each_gap([&](auto Nc) __attribute__((always_inline)) {
+      constexpr int n = decltype(Nc)::value, i = n / 8, j = (i & 1) ? 7 - n % 8 : n % 8;  // snake order: one operand register changes per multiply
+      if constexpr (EPI != 0) {  // block bb of the half in the gap in front of multiply G0 + 7 bb / 4, as in gemm_w4.hip
+#pragma unroll
+        for (int bb = 0; bb < 32; ++bb) {
+          const int g = EPI_G0 + 7 * bb / 4, si = EPI_S0 + bb / 8, sj = (si & 1) ? 7 - bb % 8 : bb % 8;
+          if (g == n) epi_cvt(e, si, sj);
+          if ((bb & 3) == 3 && g == n) epi_read(e, sj >> 2, vv[(bb >> 2) & 1]);
+        }
+#pragma unroll
+        for (int bb = 3; bb < 32; bb += 4) {
+          const int g = EPI_G0 + 7 * bb / 4, si = EPI_S0 + bb / 8, sj = (si & 1) ? 7 - bb % 8 : bb % 8;
+          if (g + 2 == n) epi_store(e, si, sj >> 2, 0, vv[(bb >> 2) & 1][0], true);
+          if (g + 4 == n) epi_store(e, si, sj >> 2, 1, vv[(bb >> 2) & 1][1], true);
+        }
+      }
+      if constexpr (EPI == 1) mfma_new<DT>(acc[i][j], fb[CUR][j], fa[CUR][i]);
+      else mfma_acc<DT>(acc[i][j], fb[CUR][j], fa[CUR][i]);
+      if constexpr (n < 16) read_frag(NextPar(), Nc, fa[CUR ^ 1], fb[CUR ^ 1]);
+      if constexpr (n == 4) step_feed();
+      constexpr int c0 = n - 17;  // copies: m0 in one gap, the copy in the next, one every four multiplies
+      if constexpr (c0 >= 0 && c0 < 32 && c0 % 4 == 0) copy_m0(std::integral_constant<int, c0 / 4>(), buf);
+      if constexpr (c0 >= 0 && c0 < 32 && c0 % 4 == 1) copy(std::integral_constant<int, c0 / 4>());
+      if constexpr (CUR == 0 && c0 >= 0 && c0 < 32 && c0 % 4 == 2) toggle(a_rd[c0 / 4]);
+      if constexpr (CUR == 0 && c0 >= 0 && c0 < 32 && c0 % 4 == 3) toggle(b_rd[c0 / 4]);
+    });
+    cp_off = (cp_off + C::SLAB_BYTES) & (C::SLABS * C::SLAB_BYTES - 1);
+    // This wave's copies of slab q + 2, requested two K steps ago, have landed: younger are the sixteen copies of this K step and
+    // the one before, and their stores (sixteen in a tile's last K step and in the next tile's first; loads and stores complete in order).
+    asm volatile("s_waitcnt vmcnt(%16) lgkmcnt(0)" : TGG_TIE8(fa[CUR ^ 1]), TGG_TIE8(fb[CUR ^ 1]) : "n"(WAIT) : "memory", "v255");
+    if constexpr (EPI != 2) asm volatile("s_barrier" ::: "memory");
+  };
+
+  for (int pos = 0; cur.g >= 0; ++pos) {
+    following = look_up(tile_at(pos + 1));
+    nxt = feed_of(following);
+    if (cur.steps == 4) request();
+    kstep(I0(), I1(), W48());  // behind the last K step of the tile before; the launch's first three K steps find their slabs landed
+    kstep(I1(), I0(), W32());
+    for (int k = 4; k < cur.steps; k += 2) {
+      if (k + 2 >= cur.steps) request();  // four K steps before the answer is taken, no sooner: who draws late draws fairly
+      kstep(I0(), I0(), W16());
+      kstep(I1(), I0(), W16());
+    }
+    // what the tile's last K step, the next tile's first and a flush store
+    const int64_t rows_left = p.m_total - cur.m0 - wm0;
+    pend_rs = make_rsrc32((uint64_t)p.C + (uint64_t)((((int64_t)cur.g * p.m_total + cur.m0 + wm0) * (int64_t)p.N + cur.n0 + wn0) * 2),
+                          rows_left > 0 ? (int)(rows_left < 128 ? rows_left : 128) * p.N * 2 : 0);
+    pend_cols = p.N - cur.n0 - wn0;
+    kstep(I0(), I0(), W16());
+    kstep(I1(), I2(), W32());
+    take(pos + 2);
+    asm volatile("s_barrier" ::: "memory");
+    cur = following;
+  }
+  epi_flush();
+  if (queued && threadIdx.x == 0) sched_queue_finish(p.queue);
+  wait_vmcnt<0>();  // trailing zero-length copies still write LDS
+}
+
+template <int DT>
+int launch_wgrad(const GemmParams& p, hipStream_t s) {
+  static bool attr_set[64] = {false};
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  const bool listed = dev >= 0 && dev < 64;
+  auto kern = gemm_wgrad_kernel<DT>;
+  if (!listed || !attr_set[dev]) {
+    if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, WgradCfg::SMEM_BYTES) != hipSuccess)
+      return check_launch("hipFuncSetAttribute(gemm_wgrad)");
+    if (listed) attr_set[dev] = true;
+  }
+  int grid = num_cus();
+  if (p.grid_limit > 0 && p.grid_limit < grid) grid = p.grid_limit;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(WgradCfg::THREADS), WgradCfg::SMEM_BYTES, s, p);
+  return check_launch("gemm_wgrad");
+}
+
+}  // namespace
+
+// K-grouped launches of one and a half rounds of 256x256 tiles and more.  Smaller ones stay with the eight-wave kernel, which has
+// narrower tiles and draws a tile later, i.e. more evenly: half a round, 384 / 1024 tokens a group (512 x 1024, 16 groups) 25 / 55 us there
+// and 33 / 73 here; one and a half rounds (768 x 2048, 16 groups) 45 / 92 and 36 / 85.  Two more cases stay there: more groups than
+// this kernel has threads, whose table takes longer to make (300 groups of 264 x 520, 256 tokens: 98 against 113 us), and
+// launches of many rounds with around 128 tokens a group (128 groups of 1408 x 2816: 299 against 315 us; 64 tokens 209 / 208, 256 tokens
+// 416 / 408), where a tile is half padding here and both kernels wait for memory.
+bool wgrad_supported(const GemmParams& p, int dt, bool any_size) {
+  if (dt != DT_BF16 && dt != DT_F16) return false;
+  if (p.mode != MODE_KG && p.mode != MODE_KG_COUNT) return false;
+  if (p.G > WgradCfg::THREADS || (p.N & 7) != 0 || (p.m_total & 7) != 0) return false;
+  // token rows of a slab, and a wave's block of the output, within 32-bit offsets that stay below the out-of-range marker
+  if (p.m_total * 2 * 64 >= (1ll << 30) || (int64_t)p.N * 2 * 128 >= (1ll << 30)) return false;
+  const int64_t tiles_m = (p.m_total + 255) / 256, tiles_n = (p.N + 255) / 256;
+  if (p.G * tiles_m * tiles_n >= (1ll << 31)) return false;
+  if (any_size) return true;
+  int grid = num_cus();
+  if (p.grid_limit > 0 && p.grid_limit < grid) grid = p.grid_limit;
+  const int64_t tiles = p.G * tiles_m * tiles_n;
+  if (tiles >= 16 * (int64_t)grid && p.k_total > 96 * (int64_t)p.G && p.k_total < 192 * (int64_t)p.G) return false;
+  return 2 * tiles >= 3 * (int64_t)grid;
+}
+
+int launch_wgrad_16bit(const GemmParams& p, int dt, hipStream_t s) {
+  return dt == DT_BF16 ? launch_wgrad<DT_BF16>(p, s) : launch_wgrad<DT_F16>(p, s);
+}
+
+}  // namespace tgg
