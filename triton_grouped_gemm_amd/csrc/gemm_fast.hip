@@ -704,7 +704,7 @@ __global__ __launch_bounds__(CW::THREADS) void gemm_fast_auto_kernel(const GemmP
     static_assert(CS::THREADS == CW::THREADS && CS::SCHED_OFF == CW::SCHED_OFF && CS::SMEM_BYTES <= CW::SMEM_BYTES,
                   "the weight-streaming configuration shares the launch shape and the group table's place");
     static_assert(CW::THREADS >= kFastMaxGroups && CS::BM * 2 == CW::BM, "sched_init's half-height prefix is CS's");
-    stream = sched_short_tiles_pay<CW::BN>(p, sched);
+    stream = sched_short_tiles_pay<CW::BN>(p, sched, 10, 7);
   }
   if constexpr (!std::is_void<CS>::value) {
     // the four-wave kernel, launched in front of this one, has taken the launch (GemmParams::wide_gate)

@@ -606,7 +606,7 @@ __global__ __launch_bounds__(CW::THREADS) void gemm_fp8_auto_kernel(const GemmPa
     half_full = r >= 1 && r <= CW::BM / 2;
   }
   const int n_half_full = __syncthreads_count(half_full);
-  const bool stream = sched_short_tiles_pay<CW::BN>(p, sched);
+  const bool stream = sched_short_tiles_pay<CW::BN>(p, sched, 10, 7);
   const bool narrow = sched_num_tiles<CN::BM, CN::BN>(p, sched) <= (int64_t)gridDim.x;
   const bool sit_out = n_half_full * 8 >= sched.tile0[p.G];
   if (__builtin_expect(!narrow && !stream && !sit_out, 1))  // marked likely: the register allocator then favours this body's loops

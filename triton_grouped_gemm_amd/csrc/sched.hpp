@@ -265,23 +265,28 @@ TGG_HD int64_t sched_num_tiles(const GemmParams& p, const Table& t) {
 
 // Whether tiles of half the table's tile height pay for an M-grouped launch.  t.pad_ holds the tiles that the half
 // height cut has over the table's cut (sched_init leaves it there).  The persistent workgroups work in rounds (one
-// tile each per round), a half-height tile costs about 0.7 of a full one (measured over group counts 8-256 and
+// tile each per round), a half-height tile costs cost_half / cost_full of a full one (the eight-wave kernels: 0.7, measured over group counts 8-256 and
 // 64-2048 rows per group, for both operand widths), and what decides is whole rounds: a launch whose full-height
 // tiles just fit one round loses by going to two rounds of short tiles, whatever their number.
 template <int BN, class Table>
-__device__ __forceinline__ bool sched_short_tiles_pay(const GemmParams& p, const Table& t) {
+__device__ __forceinline__ bool sched_short_tiles_pay(const GemmParams& p, const Table& t, int cost_full, int cost_half) {
   const int64_t tiles_n = (p.N + BN - 1) / BN, wgs = gridDim.x;
   const int64_t rounds_full = ((int64_t)t.tile0[p.G] * tiles_n + wgs - 1) / wgs;
   const int64_t rounds_half = ((int64_t)(t.tile0[p.G] + t.pad_) * tiles_n + wgs - 1) / wgs;
-  return rounds_half * 7 <= rounds_full * 10;
+  return rounds_half * cost_half <= rounds_full * cost_full;
 }
 
-// Whether a launch of 256-row tiles is neither small enough for the narrow tiles (all of them fit one round of the
-// persistent workgroups) nor made of groups so small that 128-row tiles pay: the case in which the eight-wave kernels
-// run their BM x BN configuration.  t: a table built by sched_init<BM> with one thread per group.
+// Whether a launch that the four-wave kernel may take is its: 256-row tiles that are neither few enough for the narrow tiles (all
+// of them fit one round of the persistent workgroups) nor of groups so small that the eight-wave kernels' 128-row tiles pay.  Such
+// a tile costs three quarters of the four-wave kernel's.  Measured over 16-128 groups of 64-511 rows, seven
+// pairs of N and K, 357 launches, time of the four-wave kernel over the eight-wave kernels' by rounds of short over rounds of
+// full tiles: 1.0-1.1 1.08-1.19, 1.2-1.3 1.0-1.04, 1.4-1.5 0.93-0.99, 1.6 and more 0.91-0.97.  (With the 0.7 of
+// sched_short_tiles_pay for the eight-wave kernels' own 256-row tiles, ratios of 1.33-1.43 went to the slower side: 128
+// groups of 256 rows on average, N = 2048, K = 1536, B as [G, K, N]: 297 -> 270 us; N = 2048, K = 768: 165 -> 150 us.)
+// t: a table built by sched_init<BM> with one thread per group.
 template <int BM, int BN, class Table>
 __device__ __forceinline__ bool sched_wide_tiles_chosen(const GemmParams& p, const Table& t) {
-  return sched_num_tiles<BM, BN / 2>(p, t) > (int64_t)gridDim.x && !sched_short_tiles_pay<BN>(p, t);
+  return sched_num_tiles<BM, BN / 2>(p, t) > (int64_t)gridDim.x && !sched_short_tiles_pay<BN>(p, t, 4, 3);
 }
 
 // Tile order.  Consecutive tile ids are handed to workgroups that run at the same time on one XCD
