@@ -1,7 +1,8 @@
-"""The four-wave weight-gradient kernel (gemm_wgrad.hip) where it can go wrong: segments around its K step of 32 tokens, its
+"""The four-wave weight-gradient kernels.  16-bit (gemm_wgrad.hip) where it can go wrong: segments around its K step of 32 tokens, its
 step pairs and its shortest tile of four steps, outputs around its 256x256 tiles, fewer and more tiles than workgroups, workgroup
 counts with and without per-XCD queues.  Forced on every shape, against the eight-wave kernel bit for bit (both add
-up 32 tokens at a time in ascending order and round once) and against torch's fp32 product."""
+up 32 tokens at a time in ascending order and round once) and against torch's fp32 product.  FP8 (fp8_w4.hip): around its slab
+of 128 tokens and its shortest tile of two slabs."""
 import pytest
 import torch
 
@@ -63,3 +64,57 @@ def test_rows_beyond_a_segment_are_not_added_up():
     b[40 + 33:] = float("nan")
     out = _run(2, a, b, torch.tensor(sizes, device=dev, dtype=torch.int32), -1)
     assert bool((out[1] == 33).all()) and bool(torch.isinf(out[0]).all()) and bool(torch.isnan(out[2:]).all())
+
+
+def _run_fp8(four_wave, x, xs, y, ys, s, num_cu):
+    _native.set_option("four_wave", four_wave)
+    try:
+        (M, T), N, G = x.shape, y.shape[0], s.numel()
+        out = torch.full((G, M, N), float("nan"), device=x.device, dtype=torch.bfloat16)
+        code = {torch.float8_e4m3fn: _native.E4M3, torch.float8_e5m2: _native.E5M2}
+        _native.call("tgg_k_grouped_gemm_fp8_channel_queued", x.data_ptr(), xs.data_ptr(), y.data_ptr(), ys.data_ptr(), out.data_ptr(), s.data_ptr(),
+                     G, M, N, T, code[x.dtype], code[y.dtype], num_cu, _native.work_queue(x.device, None).data_ptr(), _native.stream_of(x))
+        return out
+    finally:
+        _native.set_option("four_wave", 1)
+
+
+@pytest.mark.parametrize("fx, fy", [(torch.float8_e4m3fn, torch.float8_e4m3fn), (torch.float8_e5m2, torch.float8_e4m3fn),
+                                    (torch.float8_e4m3fn, torch.float8_e5m2), (torch.float8_e5m2, torch.float8_e5m2)])
+@pytest.mark.parametrize("num_cu", [-1, 8, 7])
+@pytest.mark.parametrize("sizes, M, N, spare", [
+    ([0, 16, 112, 128, 144, 240, 256, 272, 384, 400, 0, 640], 256, 256, 0),  # every segment length at a single full tile
+    ([0, 16, 112, 128, 144, 240, 256, 272, 384, 400, 0, 640], 5, 520, 48),   # five rows, a ragged third column tile, codes behind the last segment
+    ([304, 0, 16, 1008], 263, 248, 0),
+    ([0, 0], 300, 256, 16),
+    ([2048], 776, 1544, 0),
+    ([128] * 256, 40, 136, 0),
+])
+def test_fp8_weight_gradient_kernel_at_its_edges(fx, fy, num_cu, sizes, M, N, spare):
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(len(sizes) + M)
+    T = sum(sizes) + spare
+    x = (torch.randn(M, T, device=dev, generator=gen) * 8).to(fx)
+    y = (torch.randn(N, T, device=dev, generator=gen) * 8).to(fy)
+    xs, ys = (torch.rand(len(sizes), n, device=dev, generator=gen) + 0.5 for n in (M, N))
+    s = torch.tensor(sizes, dtype=torch.int32, device=dev)
+    out = _run_fp8(1, x, xs, y, ys, s, num_cu)
+    assert torch.equal(out.view(torch.int16), _run_fp8(0, x, xs, y, ys, s, num_cu).view(torch.int16))  # the eight-wave kernel's bits
+    at = 0
+    for g, n in enumerate(sizes):
+        ref = (x[:, at:at + n].float() @ y[:, at:at + n].float().t()) * xs[g][:, None] * ys[g][None, :]
+        # one rounding to bf16; 2e-3 of the largest for products that one multiply instruction truncates (below 2^-13 of its largest) and the sum's order
+        assert bool(((out[g].float() - ref).abs() <= ref.abs() * 2.0 ** -8 * 1.02 + 2e-3 * ref.abs().max()).all()), f"group {g}"
+        at += n
+    assert int(_native.work_queue(dev, None).abs().sum()) == 0
+
+
+def test_fp8_codes_of_other_segments_are_not_added_up():
+    dev = torch.device("cuda:0")
+    s = torch.tensor([48, 32, 80], dtype=torch.int32, device=dev)
+    x, y = torch.ones(300, 160, device=dev), torch.ones(264, 160, device=dev)
+    x[:, :48] = float("nan")
+    y[:, 80:] = float("nan")
+    one = lambda n: torch.ones(3, n, device=dev)
+    out = _run_fp8(1, x.to(torch.float8_e4m3fn), one(300), y.to(torch.float8_e4m3fn), one(264), s, -1)
+    assert bool((out[1] == 32).all()) and bool(torch.isnan(out[0]).all()) and bool(torch.isnan(out[2]).all())

@@ -221,17 +221,23 @@ def test_four_wave_kernel_reads_no_accumulator_right_behind_its_multiply():
     assert not found, f"{len(found)} reads too close behind the multiply, first: {found[0]}"
 
 
-# The weight-gradient kernel holds a work-queue draw that is in flight across K steps in v255 (see gemm_wgrad.hip).
-def stray_uses_of_v255(text: str):
-    stray, inside = [], False
+# The K-grouped four-wave kernels hold a work-queue draw that is in flight across K steps in v255 (KgDraw, w4_common.hpp).
+_K_GROUPED = {"gemm_wgrad": "gemm_wgrad_kernel", "fp8_w4": "fp8_w4_kernel"}  # source file, kernel
+
+
+def _kernel_lines(text: str, kernel: str):
+    inside = False
     for raw in text.splitlines():
         line = raw.split(";")[0].strip()
         if line.endswith(":") and not line.startswith("."):
-            inside = "gemm_wgrad_kernel" in line
-            continue
-        if not inside or not line or line.startswith("."):
-            continue
-        toks = [t.strip(",") for t in line.split()]
+            inside = kernel in line
+        elif inside and line and not line.startswith("."):
+            yield line, [t.strip(",") for t in line.split()]
+
+
+def stray_uses_of_v255(text: str, kernel: str):
+    stray = []
+    for line, toks in _kernel_lines(text, kernel):
         if not any(255 in _regs(t, "v") for t in toks[1:]):
             continue
         drawn = toks[0] == "global_atomic_add" and toks[1] == "v255" and toks[-1] == "sc0" and "v255" not in toks[2:]
@@ -243,21 +249,52 @@ def stray_uses_of_v255(text: str):
 
 def test_v255_scanner_on_snippets():
     head = "_ZN3tgg17gemm_wgrad_kernelILi0EEEvNS_10GemmParamsE:\n"
-    assert stray_uses_of_v255(head + "global_atomic_add v255, v1, v2, s[4:5] sc0\nv_readfirstlane_b32 s3, v255\n") == []
-    assert len(stray_uses_of_v255(head + "v_mov_b32_e32 v255, v3\n")) == 1
-    assert len(stray_uses_of_v255(head + "ds_read_b128 v[252:255], v3\n")) == 1
-    assert len(stray_uses_of_v255(head + "global_atomic_add v255, v255, v2, s[4:5] sc0\n")) == 1
-    assert stray_uses_of_v255("other_kernel:\nv_mov_b32_e32 v255, v3\n") == []
+    found = lambda code, at=head: stray_uses_of_v255(at + code, "gemm_wgrad_kernel")
+    assert found("global_atomic_add v255, v1, v2, s[4:5] sc0\nv_readfirstlane_b32 s3, v255\n") == []
+    assert len(found("v_mov_b32_e32 v255, v3\n")) == 1
+    assert len(found("ds_read_b128 v[252:255], v3\n")) == 1
+    assert len(found("global_atomic_add v255, v255, v2, s[4:5] sc0\n")) == 1
+    assert found("v_mov_b32_e32 v255, v3\n", "other_kernel:\n") == []
 
 
-def test_weight_gradient_kernel_keeps_the_draw_in_flight_and_its_accumulators():
-    f = BUILD / "gemm_wgrad.gfx950.s"
+# Their fragment reads are inline assembly as well, and those of fp8_w4.hip are in flight across groups of multiplies and across the
+# slab loop: nothing may touch a register that a read is still to fill.  LDS operations complete in order, so a wait
+# for lgkmcnt(n) leaves the n youngest in flight.
+def uses_of_reads_in_flight(text: str, kernel: str):
+    bad, flight = [], []
+    for line, toks in _kernel_lines(text, kernel):
+        if toks[0] == "s_waitcnt":
+            m = re.search(r"lgkmcnt\((\d+)\)", line)
+            if m:
+                flight = flight[max(0, len(flight) - int(m.group(1))):]
+            continue
+        used = set().union(*[_regs(t, "v") for t in toks[1:]]) if len(toks) > 1 else set()
+        if used & set().union(set(), *flight):
+            bad.append(line)
+        if toks[0].startswith("ds_"):
+            flight.append(_regs(toks[1], "v") if toks[0].startswith("ds_read") else set())
+    return bad
+
+
+def test_reads_in_flight_scanner_on_snippets():
+    found = lambda code: uses_of_reads_in_flight("fp8_w4_kernel:\n" + code, "fp8_w4_kernel")
+    two = "ds_read_b128 v[0:3], v9\nds_read_b128 v[4:7], v9 offset:16\n"
+    assert len(found(two + "v_mov_b32_e32 v20, v2\n")) == 1
+    assert found(two + "s_waitcnt lgkmcnt(1)\nv_mov_b32_e32 v20, v2\n") == []
+    assert len(found(two + "s_waitcnt lgkmcnt(1)\nv_mov_b32_e32 v5, v20\n")) == 1
+    assert len(found(two + "s_waitcnt vmcnt(0)\nv_add_u32_e32 v21, v7, v20\n")) == 1
+    assert found(two + "s_waitcnt vmcnt(3) lgkmcnt(0)\nv_add_u32_e32 v21, v7, v0\n") == []
+
+
+@pytest.mark.parametrize("stem", sorted(_K_GROUPED))
+def test_k_grouped_four_wave_kernels(stem):
+    f, kernel = BUILD / f"{stem}.gfx950.s", _K_GROUPED[stem]
     if not f.exists():
         pytest.skip("no device assembly in the build directory (the library was built elsewhere or not yet)")
     text = f.read_text()
-    assert "gemm_wgrad_kernel" in text
-    stray = stray_uses_of_v255(text)
-    assert not stray, f"{len(stray)} compiler-generated uses of v255, first: {stray[0]}"
-    found = accumulator_reads_too_early(text.replace("gemm_wgrad_kernel", "gemm_w4_kernel"))
-    assert not found, f"{len(found)} reads too close behind the multiply, first: {found[0]}"
+    assert kernel in text
+    for what, found in (("uses of v255", stray_uses_of_v255(text, kernel)),
+                        ("uses of a register that an LDS read is to fill", uses_of_reads_in_flight(text, kernel)),
+                        ("accumulator reads too close behind the multiply", accumulator_reads_too_early(text.replace(kernel, "gemm_w4_kernel")))):
+        assert not found, f"{len(found)} {what}, first: {found[0]}"
     assert "scratch_" not in text  # a spilled value would be reloaded behind the copies

@@ -24,14 +24,10 @@
 // copy stream is four slabs ahead of the multiplies, so it is in the tile being multiplied or in the next one, and every
 // tile starts on the same parity).
 //
-// Tiles come from the work queue of sched.hpp (largest groups first, one counter per XCD) or, without one, from the
-// fixed walk.  Wave 0 draws: the request for the tile after the next goes out four K steps before a tile's end, and its answer, in
-// order with the copies, has arrived by the wait that ends the tile.  It sits in v255, which is named in the
-// instruction text because a value in flight across K steps must not be known to the compiler (tests/test_isa_hazards.py
-// scans the kept assembly for any other use).
+// Tiles come from KgDraw (w4_common.hpp); the request for the tile after the next goes out four K steps before a tile's end, and its
+// answer, in order with the copies, has arrived by the wait that ends the tile.
 #include "launch.hpp"
 #include "w4_common.hpp"
-#include <utility>
 
 namespace tgg {
 
@@ -50,22 +46,6 @@ struct WgradCfg {
   static_assert(SMEM_BYTES <= 160 * 1024, "LDS budget");
 };
 
-// Division of 32-bit values by a divisor that is fixed for the launch, on the scalar unit.  m = floor(2^32 / d) + 1: the
-// estimate n m / 2^32 is the quotient or one more for every 32-bit n.
-struct FixedDiv {
-  uint32_t d, m;
-  TGG_DEV explicit FixedDiv(int d_) : d((uint32_t)d_), m(d_ > 1 ? 0xffffffffu / (uint32_t)d_ + 1 : 0) {}
-  TGG_DEV uint32_t div(uint32_t n) const {
-    if (d == 1) return n;
-    const uint32_t q = __umulhi(n, m);
-    return q * d > n ? q - 1 : q;
-  }
-};
-
-// f(integral_constant<int, n>) for n = 0 .. 63: the gaps of a K step's multiplies
-template <class F, int... N> TGG_DEV void each_gap_of(const F& f, std::integer_sequence<int, N...>) { (f(std::integral_constant<int, N>()), ...); }
-template <class F> TGG_DEV void each_gap(const F& f) { each_gap_of(f, std::make_integer_sequence<int, 64>()); }
-
 template <int DT>
 __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const GemmParams p) {
   typedef WgradCfg C;
@@ -73,7 +53,6 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
 
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   auto& sched = *reinterpret_cast<SchedTableT<kFastMaxGroups>*>(smem + C::SCHED_OFF);
-  auto* const next_id = reinterpret_cast<volatile int32_t*>(smem + C::NEXT_OFF);
   sched_init<C::BM>(p, sched);
 
   const uint32_t smem_addr = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
@@ -100,65 +79,11 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
     b_rd[i] = smem_addr + C::OP_BYTES + row + ((((wn0 + 16 * i) / 8 + (c >> 1)) ^ sw) << 4);
   }
 
-  // ---- tiles -------------------------------------------------------------------------------------------------------
-  const int tiles_n = (p.N + C::BN - 1) / C::BN, tiles_m = (int)((p.m_total + C::BM - 1) / C::BM);
-  const int per_group = tiles_m * tiles_n, total = p.G * per_group;
-  const int nc = sched_chunk_width(tiles_n, p.n_chunk), full_chunks = tiles_n / nc, tail_width = tiles_n - full_chunks * nc;
-  const FixedDiv by_group(per_group), by_chunk(tiles_m * nc), by_nc(nc), by_tail(tail_width > 0 ? tail_width : 1);
-  const TileWalk walk64 = sched_walk(total, false);
-  const bool queued = p.queue != nullptr;
-  struct TileInfo {
-    int g, m0, n0;   // g = -1: there are no more tiles
-    int klen, steps; // tokens of the segment, K steps
-    int64_t k0;      // its first token
-  };
-  auto look_up = [&](int id) __attribute__((always_inline)) {
-    TileInfo t;
-    t.g = -1;
-    t.m0 = t.n0 = t.klen = t.steps = 0;
-    t.k0 = 0;
-    if (id < total) {
-      const int slot = (int)by_group.div((uint32_t)id), r = id - slot * per_group;
-      int c = (int)by_chunk.div((uint32_t)r);  // as sched_split
-      const bool tail = c >= full_chunks;
-      c = tail ? full_chunks : c;
-      const int width = tail ? tail_width : nc, q = r - c * tiles_m * nc;
-      const int mt = (int)(tail ? by_tail.div((uint32_t)q) : by_nc.div((uint32_t)q));
-      t.m0 = mt * C::BM;
-      t.n0 = (c * nc + q - mt * width) * C::BN;
-      t.g = __builtin_amdgcn_readfirstlane(sched.tile0[slot]);
-      t.klen = __builtin_amdgcn_readfirstlane(sched.rows[t.g]);
-      t.k0 = (int64_t)uniform64((uint64_t)sched.row0[t.g]);
-      const int steps = (t.klen + 2 * C::KS - 1) / (2 * C::KS) * 2;
-      t.steps = steps < C::SLABS ? C::SLABS : steps;
-    }
-    return t;
-  };
-  // The drawing wave.  A counter's value stands for a tile id (sched_queue_id); once it stands for none, the wave looks at
-  // all counters at once and goes on with one that has tiles left, if there is any.
-  const bool spread = (gridDim.x & 7) == 0;  // eight counters; else one
-  const int R = (int)gridDim.x >> 3;
-  const FixedDiv by_r(R > 0 ? R : 1);
-  int xq = spread ? (int)(blockIdx.x & 7) : 0;
-  auto id_of = [&](int n) __attribute__((always_inline)) {
-    if (!spread) return n;
-    const int pass = (int)by_r.div((uint32_t)n);
-    return (pass * 8 + ((pass & 1) ? 7 - xq : xq)) * R + n - pass * R;
-  };
-  int exhausted = 0;  // counters that a draw has found without a tile, one bit each
-  auto steal = [&]() __attribute__((always_inline)) {  // the next tile of another counter, `total` where there is none
-    while (spread) {  // eight rounds at most: a round ends the search or marks a counter
-      exhausted |= 1 << xq;
-      const int seen = lane < 8 ? __hip_atomic_load(p.queue + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-      const int left = sched_queue_left(seen, total, R) & ~exhausted;
-      if (left == 0) break;
-      xq = sched_queue_next(left, xq);
-      int n = 0;
-      if (lane == 0) n = atomicAdd(p.queue + xq, 1);
-      const int id = id_of(__builtin_amdgcn_readfirstlane(n));
-      if (id < total) return id;
-    }
-    return total;
+  const KgTiles<SchedTableT<kFastMaxGroups>> tiles(p, sched);
+  KgDraw draw(p, reinterpret_cast<int32_t*>(smem + C::NEXT_OFF), tiles.total, wave, lane);
+  auto steps_of = [&](const KgTile& t) __attribute__((always_inline)) {
+    const int steps = (t.klen + 2 * C::KS - 1) / (2 * C::KS) * 2;
+    return steps < C::SLABS ? C::SLABS : steps;
   };
 
   // ---- the copy stream ---------------------------------------------------------------------------------------------
@@ -170,10 +95,10 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
     int a_off, b_off;         // the tile's columns within a token row, bytes
     int left;                 // slabs of the tile still to be requested
   };
-  auto feed_of = [&](const TileInfo& t) __attribute__((always_inline)) {
+  auto feed_of = [&](const KgTile& t) __attribute__((always_inline)) {
     Feed f;
     f.rem = t.klen;
-    f.left = t.g < 0 ? 0x7fffffff : t.steps;
+    f.left = t.g < 0 ? 0x7fffffff : steps_of(t);
     f.a_off = t.m0 * 2;
     f.b_off = t.n0 * 2;
     f.a_base = (uint64_t)p.A + (uint64_t)(t.k0 * a_ld + f.a_off);
@@ -287,43 +212,15 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
   typedef std::integral_constant<int, 16> W16;
   typedef std::integral_constant<int, 32> W32;
   typedef std::integral_constant<int, 48> W48;
-  bool live = queued && wave == 0;  // tiles are still being drawn
-  // requests the next tile's number; nothing may read v255 before the memory operations so far have been waited for
-  auto request = [&]() __attribute__((always_inline)) {
-    if (live && lane == 0) {
-      int32_t* const at = p.queue + xq;
-      asm volatile("global_atomic_add v255, %0, %1, %2 sc0" : : "v"(0), "v"(1), "s"(at) : "memory", "v255");
-    }
-  };
-  // takes the answer (it has arrived) and leaves the tile id for the other waves, in front of a barrier; pos: the tile's position
-  auto take = [&](int pos) __attribute__((always_inline)) {
-    if (live) {
-      int got;
-      asm volatile("v_readfirstlane_b32 %0, v255" : "=s"(got) : : "memory", "v255");
-      int id = id_of(got);
-      if (__builtin_expect(id >= total, 0)) {
-        id = steal();
-        live = id < total;
-      }
-      if (lane == 0) next_id[pos & 1] = id;
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    }
-  };
-  auto tile_at = [&](int pos) __attribute__((always_inline)) {
-    if (queued) return __builtin_amdgcn_readfirstlane(next_id[pos & 1]);
-    const int64_t id = walk64.first + (int64_t)pos * walk64.stride;
-    return id < walk64.end ? (int)id : total;
-  };
-  if (wave == 0 && lane < 2) next_id[lane] = total;  // what the other waves find once nothing is drawn any more
   __syncthreads();
-  request();
+  draw.request();
   wait_vmcnt<0>();
-  take(0);
+  draw.take(0);
   __syncthreads();
-  TileInfo cur = look_up(tile_at(0)), following = cur;
+  KgTile cur = tiles.look_up(draw.tile_at(0)), following = cur;
   feed = feed_of(cur);
   nxt = feed;
-  request();
+  draw.request();
 #define TGG_WG_EACH8(f) f(0) f(1) f(2) f(3) f(4) f(5) f(6) f(7)
   for (int s = 0; s < C::SLABS; ++s) {
     step_feed();
@@ -333,7 +230,7 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
 #undef TGG_WG_P
   }
   wait_vmcnt<0>();
-  take(1);
+  draw.take(1);
   __syncthreads();
 #define TGG_WG_RD(q) read_frag(I0(), std::integral_constant<int, q>(), fa[0], fb[0]);
   TGG_WG_EACH8(TGG_WG_RD)
@@ -353,7 +250,7 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
     if (EPI) e = epi_lane();
     const uint32_t buf = wave_buf + cp_off;
     constexpr int EPI_S0 = EPI == 2 ? 0 : 4, EPI_G0 = EPI == 2 ? 4 : 0;
-    each_gap([&](auto Nc) __attribute__((always_inline)) {
+    for_each<64>([&](auto Nc) __attribute__((always_inline)) {
       constexpr int n = decltype(Nc)::value, i = n / 8, j = (i & 1) ? 7 - n % 8 : n % 8;  // snake order: one operand register changes per multiply
       if constexpr (EPI != 0) {  // block bb of the half in the gap in front of multiply G0 + 7 bb / 4, as in gemm_w4.hip
 #pragma unroll
@@ -387,13 +284,14 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
   };
 
   for (int pos = 0; cur.g >= 0; ++pos) {
-    following = look_up(tile_at(pos + 1));
+    following = tiles.look_up(draw.tile_at(pos + 1));
     nxt = feed_of(following);
-    if (cur.steps == 4) request();
+    const int steps = steps_of(cur);
+    if (steps == 4) draw.request();
     kstep(I0(), I1(), W48());  // behind the last K step of the tile before; the launch's first three K steps find their slabs landed
     kstep(I1(), I0(), W32());
-    for (int k = 4; k < cur.steps; k += 2) {
-      if (k + 2 >= cur.steps) request();  // four K steps before the answer is taken, no sooner: who draws late draws fairly
+    for (int k = 4; k < steps; k += 2) {
+      if (k + 2 >= steps) draw.request();  // four K steps before the answer is taken, no sooner: who draws late draws fairly
       kstep(I0(), I0(), W16());
       kstep(I1(), I0(), W16());
     }
@@ -404,12 +302,12 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
     pend_cols = p.N - cur.n0 - wn0;
     kstep(I0(), I0(), W16());
     kstep(I1(), I2(), W32());
-    take(pos + 2);
+    draw.take(pos + 2);
     asm volatile("s_barrier" ::: "memory");
     cur = following;
   }
   epi_flush();
-  if (queued && threadIdx.x == 0) sched_queue_finish(p.queue);
+  draw.finish();
   wait_vmcnt<0>();  // trailing zero-length copies still write LDS
 }
 
