@@ -162,22 +162,27 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
   };
 
   // A slab takes 128 bytes of rows that lie far apart, one line of each, which HBM serves slowly and late.  So once in two slabs the
-  // rows' next two lines are touched (one word of each, into a sink in LDS) and wait in L2 when they are copied.  The
+  // rows' next two lines are touched (one word of each, into a sink in LDS) and wait in L2 when they are copied, the first two of a
+  // tile at the start of the tile before.  The
   // workgroups of an XCD that run together share their panels (the tiles of a run of 32 neighbours: nc columns by 32 / nc rows),
   // and each touches its part of them only: all of it by everybody costs more than it gains.
   const int rows_a = (C::BM + tiles.nc - 1) / tiles.nc, parts_b = tiles.nc < 32 ? 32 / tiles.nc : 1, rows_b = (C::BN + parts_b - 1) / parts_b;
-  int touch_a = kNoFetch, touch_b = kNoFetch;
-  auto aim_touch = [&](const KgTile& t) __attribute__((always_inline)) {
+  struct Part { int a, b; };  // the lane's offsets, kNoFetch beyond the workgroup's part
+  auto part_of = [&](const KgTile& t) __attribute__((always_inline)) {
     const int mt = t.m0 >> 8, nt = t.n0 >> 8, part_a = nt - (int)tiles.by_nc.div((uint32_t)nt) * tiles.nc, part_b = mt % parts_b;
     const int thread = wave * 64 + lane;
-    touch_a = thread < rows_a ? (part_a * rows_a + thread) * ld : kNoFetch;
-    touch_b = thread < rows_b ? (part_b * rows_b + thread) * ld : kNoFetch;
+    return Part{thread < rows_a ? (part_a * rows_a + thread) * ld : kNoFetch, thread < rows_b ? (part_b * rows_b + thread) * ld : kNoFetch};
   };
-  auto touch = [&](const i32x4_t& r, int v0, int ahead) __attribute__((always_inline)) {
-    const int off = koff + ahead, v = off < feed.klen ? v0 : kNoFetch;
+  auto touch = [&](const i32x4_t& r, int v0, int off, int klen) __attribute__((always_inline)) {
+    const int v = off < klen ? v0 : kNoFetch;
     const uint32_t at = smem_addr + C::SINK_OFF + wave * 256;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" : : "s"(at), "v"(v), "s"(r), "s"(off) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, %3 offen lds" : : "s"(at), "v"(v), "s"(r), "s"(off) : "memory", "m0");
   };
+  auto touch_two = [&](const Feed& f, const Part& part, int off) __attribute__((always_inline)) {  // the lines at off and behind
+    if (wave * 64 < rows_a) { touch(f.ra, part.a, off, f.klen); touch(f.ra, part.a, off + C::KS, f.klen); }
+    if (wave * 64 < rows_b) { touch(f.rb, part.b, off, f.klen); touch(f.rb, part.b, off + C::KS, f.klen); }
+  };
+  Part part = {kNoFetch, kNoFetch};
   // ---- fragments and accumulators ----------------------------------------------------------------------------------------------
   i32x8_t fa[8], fb[8];
   f32x4_t acc[8][8];
@@ -317,10 +322,7 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
       if constexpr (n >= 32 && n % 2 == 0) copy_m0(TGG_F8_I((n - 32) / 2));
       if constexpr (n >= 32 && n % 2 == 1) copy(TGG_F8_I((n - 33) / 2));
       if constexpr (n == 63) {
-        if ((koff & C::KS) == 0) {
-          if (wave * 64 < rows_a) { touch(feed.ra, touch_a, C::KS); touch(feed.ra, touch_a, 2 * C::KS); }
-          if (wave * 64 < rows_b) { touch(feed.rb, touch_b, C::KS); touch(feed.rb, touch_b, 2 * C::KS); }
-        }
+        if ((koff & C::KS) == 0) touch_two(feed, part, koff + C::KS);
       }
       if constexpr (EPI == 1 && n < 32) epi_gap(Nc, TGG_F8_I(4));
       if constexpr (EPI == 2 && n >= 32) epi_gap(TGG_F8_I(n - 32), TGG_F8_I(0));
@@ -334,7 +336,8 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
   for (int pos = 0; cur.g >= 0; ++pos) {
     following = tiles.look_up(draw.tile_at(pos + 1));
     nxt = feed_of(following);
-    aim_touch(cur);
+    touch_two(nxt, part_of(following), 0);
+    part = part_of(cur);
     const int steps = steps_of(cur);
     if (steps == 2) draw.request();
     // the launch's first slab finds the slab behind it landed; later first slabs have the sixteen stores of row blocks 4-7 behind the copies

@@ -15,12 +15,12 @@
 //
 // The epilogue rides on multiplies as in gemm_w4.hip: strips 0-3 of a wave's block are converted and stored between the
 // multiplies of the tile's last K step, strips 4-7 between those of the next tile's first, whose multiplies start from a
-// zero addend.  Against the eight-wave kernel (gemm_fast.hip, TN), outputs of 2048 x 1536 for 128 groups of 256 / 512 / 1024 tokens
-// on average: 318 / 476 / 798 -> 313 / 441 / 704 us (5120 tokens: 3434 -> 3042, 1.36 PFLOP/s); with 16 groups of 64 / 256 / 4096: 41 / 49 / 357 -> 32 / 46 / 322.
-// What bounds it: from about 512 tokens on the matrix pipe (0.73 us a K step with all CUs multiplying, 0.53 on a quarter of them,
-// i.e. power), 1.5 us a tile for the epilogue's conversions and LDS staging; below, memory: with 256 tokens a launch that stores nothing takes
-// 191 us and one that stores 300, where 1.04 GB at the copy rate would take 204 (reads that come from HBM wait behind the writes:
-// on 64 CUs, or with the operands in the memory-side cache, the stores cost nothing).  A tile has an even number of K steps, four at least (of nothing where the segment ends sooner: the
+// zero addend.  Against the eight-wave kernel (gemm_fast.hip, TN), 128 groups of 2048 x 1536 with 64 /
+// 128 / 256 / 512 / 1024 tokens on average, operands in no cache: 190 / 237 / 325 / 488 / 815 -> 179 / 212 / 287 / 432 / 721 us (5120 tokens:
+// 3434 -> 3042, 1.36 PFLOP/s).  What bounds it: from about 512 tokens on the matrix pipe (0.73 us a K step with all CUs multiplying,
+// 0.53 on a quarter of them, i.e. power) and 1.5 us a tile for the epilogue's conversions and LDS staging; below, memory (256 tokens: 1.04 GB,
+// 204 us at the copy rate): reads that come from HBM wait behind the writes, so the next tile's are requested a tile ahead (below).
+// A tile has an even number of K steps, four at least (of nothing where the segment ends sooner: the
 // copy stream is four slabs ahead of the multiplies, so it is in the tile being multiplied or in the next one, and every
 // tile starts on the same parity).
 //
@@ -42,7 +42,9 @@ struct WgradCfg {
   static constexpr int SCHED_OFF = SLABS * SLAB_BYTES;
   static constexpr int NEXT_OFF = SCHED_OFF + (((int)sizeof(SchedTableT<kFastMaxGroups>) + 255) & ~255);  // drawn tile ids, two words
   static constexpr int EPI_OFF = NEXT_OFF + 256;
-  static constexpr int SMEM_BYTES = EPI_OFF + 4 * EPI_WAVE_BYTES;
+  static constexpr int SINK_OFF = EPI_OFF + 4 * EPI_WAVE_BYTES;  // where touched lines' words go, 256 bytes a wave
+  static constexpr int SMEM_BYTES = SINK_OFF + 4 * 256;
+  static constexpr int TOUCH = 256;  // tokens of the next tile that are touched
   static_assert(SMEM_BYTES <= 160 * 1024, "LDS budget");
 };
 
@@ -139,6 +141,28 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
     asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(v), "s"(r) : "memory");
   };
 
+  // While a tile is multiplied and the one before it is stored, the next tile's lines are brought into L2: one word of each of its
+  // first 256 tokens' lines (four per token row and operand) goes into a sink in LDS.  The workgroups of an XCD that run
+  // together share their panels (the tiles of a run of 32 neighbours: nc columns by 32 / nc rows), and each touches its part of
+  // them only.  128 groups of 2048 x 1536, 64 / 128 / 256 / 512 tokens, operands in no cache: 201 / 243 / 312 / 450 -> 179 / 212 / 287 / 432 us.
+  // Touched during the tile's own K steps (a few slabs ahead of the copies) the lines come hardly sooner than the copies (313 us with 256 tokens) and
+  // long segments lose 2 %; the next tile's touched two K steps later: 200 / 226 / 292 / 441.
+  const int sharers_b = tiles.nc < 32 ? 32 / tiles.nc : 1;
+  const int lines_a = (4 * C::TOUCH + tiles.nc - 1) / tiles.nc, lines_b = (4 * C::TOUCH + sharers_b - 1) / sharers_b;
+  auto touch = [&](uint64_t base, int off, int klen, int ld, int part, int lines) __attribute__((always_inline)) {
+    const i32x4_t r = make_rsrc32(base, (klen < C::TOUCH ? klen : C::TOUCH) * ld - off);
+    const uint32_t at = smem_addr + C::SINK_OFF + wave * 256;
+    for (int n0 = wave * 64; n0 < lines; n0 += C::THREADS) {
+      const int n = n0 + lane, line = part * lines + n;
+      const int v = n < lines ? (line >> 2) * ld + (line & 3) * 128 : kNoFetch;
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, 0 offen lds" : : "s"(at), "v"(v), "s"(r) : "memory", "m0");
+    }
+  };
+  auto touch_tile = [&](const KgTile& t, const Feed& f) __attribute__((always_inline)) {
+    const int mt = t.m0 >> 8, nt = t.n0 >> 8;
+    touch(f.a_base, f.a_off, t.klen, a_ld, nt - (int)tiles.by_nc.div((uint32_t)nt) * tiles.nc, lines_a);
+    touch(f.b_base, f.b_off, t.klen, b_ld, mt % sharers_b, lines_b);
+  };
   // ---- fragments and accumulators ------------------------------------------------------------------------------------
   i32x4_t fa[2][8], fb[2][8];
   f32x4_t acc[8][8];
@@ -286,6 +310,7 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
   for (int pos = 0; cur.g >= 0; ++pos) {
     following = tiles.look_up(draw.tile_at(pos + 1));
     nxt = feed_of(following);
+    touch_tile(following, nxt);
     const int steps = steps_of(cur);
     if (steps == 4) draw.request();
     kstep(I0(), I1(), W48());  // behind the last K step of the tile before; the launch's first three K steps find their slabs landed
@@ -333,10 +358,8 @@ int launch_wgrad(const GemmParams& p, hipStream_t s) {
 
 // K-grouped launches of one and a half rounds of 256x256 tiles and more.  Smaller ones stay with the eight-wave kernel, which has
 // narrower tiles and draws a tile later, i.e. more evenly: half a round, 384 / 1024 tokens a group (512 x 1024, 16 groups) 25 / 55 us there
-// and 33 / 73 here; one and a half rounds (768 x 2048, 16 groups) 45 / 92 and 36 / 85.  Two more cases stay there: more groups than
-// this kernel has threads, whose table takes longer to make (300 groups of 264 x 520, 256 tokens: 98 against 113 us), and
-// launches of many rounds with around 128 tokens a group (128 groups of 1408 x 2816: 299 against 315 us; 64 tokens 209 / 208, 256 tokens
-// 416 / 408), where a tile is half padding here and both kernels wait for memory.
+// and 33 / 73 here; one and a half rounds (768 x 2048, 16 groups) 45 / 92 and 36 / 85.  More groups
+// than this kernel has threads stay there too: their table takes longer to make (300 groups of 264 x 520, 256 tokens: 98 against 113 us).
 bool wgrad_supported(const GemmParams& p, int dt, bool any_size) {
   if (dt != DT_BF16 && dt != DT_F16) return false;
   if (p.mode != MODE_KG && p.mode != MODE_KG_COUNT) return false;
@@ -348,9 +371,7 @@ bool wgrad_supported(const GemmParams& p, int dt, bool any_size) {
   if (any_size) return true;
   int grid = num_cus();
   if (p.grid_limit > 0 && p.grid_limit < grid) grid = p.grid_limit;
-  const int64_t tiles = p.G * tiles_m * tiles_n;
-  if (tiles >= 16 * (int64_t)grid && p.k_total > 96 * (int64_t)p.G && p.k_total < 192 * (int64_t)p.G) return false;
-  return 2 * tiles >= 3 * (int64_t)grid;
+  return 2 * p.G * tiles_m * tiles_n >= 3 * (int64_t)grid;
 }
 
 int launch_wgrad_16bit(const GemmParams& p, int dt, hipStream_t s) {
