@@ -102,7 +102,7 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
 
   // ---- the copy stream -------------------------------------------------------------------------------------------------------
   // The cursor is two slabs ahead of the multiplies.  A tile's windows (descriptors) are fixed, the offset along K travels in the copies'
-  // scalar offset, which the windows' range check leaves out; chunks beyond the tile's range along K are not fetched.
+  // scalar offset, which the windows' range check counts in; chunks beyond the tile's range along K are not fetched.
   const KgTiles<SchedTableT<kFastMaxGroups>> tiles(p, sched);
   KgDraw draw(p, reinterpret_cast<int32_t*>(smem + C::NEXT_OFF), tiles.total, wave, lane);
   auto steps_of = [&](const KgTile& t) __attribute__((always_inline)) {

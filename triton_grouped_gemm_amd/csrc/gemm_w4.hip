@@ -1,5 +1,5 @@
 // Four-wave bf16/fp16 grouped GEMM kernel for gfx950: the large-problem path of the M-grouped and masked entry points
-// (B as [G, N, K], or as [G, K, N] with N a multiple of 256).
+// (B as [G, N, K] or as [G, K, N]).
 //
 // One workgroup per CU, four waves, one per SIMD; tile 256x256, K slab 64; every wave owns a 128x128 block of
 // 16x16x32 MFMA tiles with its 256 accumulator registers in AGPRs.  Against the eight-wave kernel (gemm_fast.hip,
@@ -41,7 +41,7 @@
 //
 // Headline shape (G = 128, M = 655360, N = 1536, K = 2048), same box: 3.03 ms against 3.30 ms for the eight-wave
 // kernel; K = 768 shape 1.77 against 1.97 ms; masked decode (G = 128, up to 512 rows per group, N = 4096, K = 1536)
-// 0.51 against 0.56 ms.  Large M-grouped launches with K a multiple of 128 take this kernel (w4_supported); masked
+// 0.51 against 0.56 ms.  Large M-grouped launches take this kernel (w4_supported); masked
 // launches of that size enqueue it together with the eight-wave kernel and the counts decide on the device which of
 // the two runs (GemmParams::wide_gate); everything else goes to the eight-wave kernels.
 //
@@ -86,11 +86,14 @@ struct W4Cfg {
 // of the copy stream and the barriers going).  Worth 2 % where a quarter of the tiles have at most 128 rows (masked
 // decode); where nearly every tile is full the branch per K step costs the others 1 %, and such a wave multiplies
 // the zeros its windows deliver.
-template <int DT, int LAYOUT, bool SIT_OUT>
+// TAIL: K is any multiple of 8 from 192 on, and N, for B as [G, K, N], any multiple of 8.  A tile's last slabs are cut short (or
+// added, for an even number of four at least): lanes whose chunk of a K-contiguous row starts at or beyond K get an out-of-range
+// offset, and token rows beyond K lie behind the window's end.  An instantiation of its own: the plain one needs no mask.
+template <int DT, int LAYOUT, bool SIT_OUT, bool TAIL>
 __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParams p) {
   typedef W4Cfg C;
   constexpr int S_OFF = 0, D_OFF = C::A_BYTES;  // the operands' places in a slab buffer
-  constexpr bool B_KMAJOR = LAYOUT == W4_NT;  // NN: B is [G, K, N], its slab 64 token rows of 512 bytes (N a multiple of 256)
+  constexpr bool B_KMAJOR = LAYOUT == W4_NT;  // NN: B is [G, K, N], its slab 64 token rows of 512 bytes
   typedef Operand<C::BM, true> Op;            // the A slab, and B's when K-contiguous: 256 rows of 128 bytes
   typedef Operand<C::BN, B_KMAJOR> OpB;
 
@@ -108,10 +111,11 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
   const int wm0 = (wave >> 1) * 128, wn0 = (wave & 1) * 128;
   const int l16 = lane & 15, lg = lane >> 4;
 
-  const int ld = p.K * 2;  // row pitch of A and of B in bytes; K is a multiple of 128 (w4_supported)
+  const int ld = p.K * 2;  // row pitch of A and of B in bytes; K is a multiple of 128 (w4_supported) unless TAIL
+  const int kt_all = TAIL ? max(4, (p.K + 2 * BK4 - 1) / (2 * BK4) * 2) : p.K / BK4;  // slabs per tile
   // Copy k (0..7) of an operand's slab by this wave is copy instruction wave + 4 k of the slab: rows 8 (wave + 4 k) ...
   // + 7.  Its per-lane source offset within the tile's window is fixed for the launch; the slab's offset along K
-  // travels in the instruction's scalar offset, which the range check of the window (its valid rows) leaves out.
+  // travels in the instruction's scalar offset, which the range check of the window counts in: rows behind the valid ones stay behind its end.
   int vo[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) vo[k] = Op::lane_voff(lane, wave % Op::NPAT, ld) + (wave + 4 * k) * Op::RPI * ld;
@@ -161,9 +165,9 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
     const int n_left = p.N - t.n0;
     w.rs = make_rsrc32((uint64_t)p.A + (uint64_t)(t.row0 * ld), live ? t.rows * ld : 0);  // only the tile's valid rows
     if (B_KMAJOR) w.rd = make_rsrc32((uint64_t)p.B + (uint64_t)(((int64_t)t.g * p.N + t.n0) * ld), live ? (n_left < C::BN ? n_left : C::BN) * ld : 0);
-    // NN: the tile's 256 columns of the group's K rows; N is a multiple of 256 (w4_supported), so every 512-byte row
-    // segment lies inside its row, and the scalar offset of a slab (which the range check leaves out) stays below K rows
-    else w.rd = make_rsrc32((uint64_t)p.B + (uint64_t)(((int64_t)t.g * p.K * p.N + t.n0) * 2), live ? p.K * ld_b : 0);
+    // NN: the tile's 256 columns of the group's K rows, to the end of the last one.  What a row segment reads beyond its row are the
+    // next row's first columns, for outputs that are not stored.
+    else w.rd = make_rsrc32((uint64_t)p.B + (uint64_t)(((int64_t)t.g * p.K * p.N + t.n0) * 2), live ? p.K * ld_b - t.n0 * 2 : 0);
     return w;
   };
   const TileWalk walk64 = sched_walk(num_tiles, p.tile_split != 0);
@@ -196,11 +200,13 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
   "v208", "v209", "v210", "v211", "v212", "v213", "v214", "v215", "v216", "v217", "v218", "v219", "v220", "v221", "v222", "v223", "v224", "v225", "v226", "v227", \
   "v228", "v229", "v230", "v231", "v232", "v233", "v234", "v235", "v236", "v237", "v238", "v239", "v240", "v241", "v242", "v243", "v244", "v245", "v246", "v247", \
   "v248", "v249", "v250", "v251", "v252", "v253", "v254", "v255"
+  int mask_s = 0, mask_d = 0;  // TAIL: kNoFetch in the lanes whose chunk of the cursor's slab lies beyond K
+  const int chunk_off = Op::lane_chunk(lane, wave % Op::NPAT) * 16;
   const uint32_t s_wr = smem_addr + S_OFF + wave * 1024 + lane * 16;  // LDS address of this lane's 16 bytes of A copy 0 (buffer 0)
   // A chunk k of the slab at offset koff of window ra -> register set SET
   auto load_s = [&](auto Kc, auto SETc, const i32x4_t& ra, int koff) __attribute__((always_inline))  {
     constexpr int k = decltype(Kc)::value, kq = k + 8 * decltype(SETc)::value;
-    const int v = vo[k];
+    const int v = TAIL ? vo[k] | mask_s : vo[k];
 #define TGG_W4_F(lo, hi) asm volatile("buffer_load_dwordx4 v[" lo ":" hi "], %0, %1, %2 offen" : : "v"(v), "s"(ra), "s"(koff) : "memory", TGG_W4_GA_CLOBBER);
     TGG_W4_GA(kq, TGG_W4_F)
 #undef TGG_W4_F
@@ -220,7 +226,7 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
   };
   auto copy_d = [&](auto Kc, const i32x4_t& rb, int koff, bool spaced) __attribute__((always_inline))  {
     constexpr int k = decltype(Kc)::value;
-    const int v = vo_b[k];
+    const int v = TAIL && B_KMAJOR ? vo_b[k] | mask_d : vo_b[k];
     if (spaced) asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" : : "v"(v), "s"(rb), "s"(koff) : "memory");
     else asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" : : "v"(v), "s"(rb), "s"(koff) : "memory");
   };
@@ -302,9 +308,9 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
     const int off = e.off[h] + (16 * i + 8 * it) * p.N * 2;
     // Two wait states must pass before a 16-byte store's data registers may be overwritten, and the compiler, which
     // considers them free after this statement, reuses them at once: between multiplies the multiply that follows is
-    // one wait state, the flush has none.  No wait states in front: the descriptor sits in scalar registers since the
+    // one wait state (TAIL: a mask may come between them), the flush has none.  No wait states in front: the descriptor sits in scalar registers since the
     // end of the tile.  Both hazards are checked on the kept assembly (tests/test_isa_hazards.py).
-    if (between_multiplies) asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 0" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
+    if (between_multiplies && !TAIL) asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 0" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
     else asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 1" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
   };
   // NT: no staging.  A lane holds rows 16 i + 4 lg + r (r = 0..3) of column 8 l16 + j of the wave's block in
@@ -328,7 +334,7 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
     i32x4_t v;
     v[0] = (int)x.x; v[1] = (int)x.y; v[2] = (int)y.x; v[3] = (int)y.y;
     const int off = lane_off + (16 * i + r) * p.N * 2;
-    if (between_multiplies) asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 0" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
+    if (between_multiplies && !TAIL) asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 0" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
     else asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 1" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
   };
   // everything that is pending, without multiplies to hide it under
@@ -377,20 +383,22 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
   int koff_s, koff_d;
   Win nxt;
   Tile nxt_tile;
-  const int k_bytes = row_bytes;  // a tile's extent along K in bytes: where a cursor moves on to the next tile
+  const int k_bytes = TAIL ? __builtin_amdgcn_readfirstlane(kt_all * 128) : row_bytes;  // a tile's extent along K in bytes: where a cursor moves on to the next tile
   auto advance_s = [&]() __attribute__((always_inline))  {
     const bool wrap = koff_s + 128 == k_bytes;
     koff_s = wrap ? 0 : koff_s + 128;
 #pragma unroll
     for (int q = 0; q < 3; ++q) rs_c[q] = wrap ? nxt.rs[q] : rs_c[q];
+    if (TAIL) mask_s = koff_s + chunk_off >= row_bytes ? kNoFetch : 0;
   };
   const int d_step = B_KMAJOR ? 128 : __builtin_amdgcn_readfirstlane(64 * ld_b);         // B's slab offset per slab ...
-  const int d_bytes = B_KMAJOR ? k_bytes : __builtin_amdgcn_readfirstlane(p.K * ld_b);   // ... and where it reaches the next tile
+  const int d_bytes = B_KMAJOR ? k_bytes : __builtin_amdgcn_readfirstlane((TAIL ? kt_all * BK4 : p.K) * ld_b);   // ... and where it reaches the next tile
   auto advance_d = [&]() __attribute__((always_inline))  {
     const bool wrap = koff_d + d_step == d_bytes;
     koff_d = wrap ? 0 : koff_d + d_step;
 #pragma unroll
     for (int q = 0; q < 3; ++q) rd_c[q] = wrap ? nxt.rd[q] : rd_c[q];
+    if (TAIL && B_KMAJOR) mask_d = koff_d + chunk_off >= row_bytes ? kNoFetch : 0;
   };
 
   // One K step: 64 multiplies on fragment set CUR (when MUL); the 16 fragments of K step NKS of the slab at nb_off go
@@ -516,8 +524,11 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
 #undef TGG_W4_P3
   koff_s = 3 * 128;  // at least four slabs per tile (w4_supported): both cursors are still in the first tile
   koff_d = 2 * d_step;
+  if (TAIL) {
+    mask_s = koff_s + chunk_off >= row_bytes ? kNoFetch : 0;
+    if (B_KMAJOR) mask_d = koff_d + chunk_off >= row_bytes ? kNoFetch : 0;
+  }
   kstep(I1(), I0(), No(), I0(), 0u, I0(), 0u, I0(), 0u);  // reads K step 0 of buffer 0 into set 0, multiplies nothing, waits for everything
-  const int kt_all = p.K / BK4;
 
   for (int tile_id = walk.first; tile_id < walk.end; tile_id += walk.stride) {
     const bool active = wm0 < cur.rows && cur.n0 + wn0 < p.N;  // this wave's block of the tile has rows and columns
@@ -565,13 +576,13 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
 #undef TGG_W4_GA_CLOBBER
 }
 
-template <int DT, int LAYOUT, bool SIT_OUT>
+template <int DT, int LAYOUT, bool SIT_OUT, bool TAIL>
 int launch_w4(const GemmParams& p, hipStream_t s) {
   static bool attr_set[64] = {false};
   int dev = 0;
   (void)hipGetDevice(&dev);
   const bool listed = dev >= 0 && dev < 64;
-  auto kern = gemm_w4_kernel<DT, LAYOUT, SIT_OUT>;
+  auto kern = gemm_w4_kernel<DT, LAYOUT, SIT_OUT, TAIL>;
   if (!listed || !attr_set[dev]) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, W4Cfg::SMEM_BYTES) != hipSuccess)
       return check_launch("hipFuncSetAttribute(gemm_w4)");
@@ -583,23 +594,36 @@ int launch_w4(const GemmParams& p, hipStream_t s) {
   return check_launch("gemm_w4");
 }
 
+// see TAIL
+bool needs_tail(const GemmParams& p, int layout) { return p.K % 128 != 0 || p.K < 256 || (layout == W4_NN && (p.N & 255) != 0); }
+
 }  // namespace
 
-// Whether 256-row tiles pay depends on the group sizes, which only the device knows.  With 512 rows and more per group on
-// average they do; a masked launch (counts anywhere up to its row stride) or an M-grouped one with smaller groups is
-// enqueued together with the eight-wave kernel, and the two decide from the sizes which of them runs.
-bool w4_decided_on_device(const GemmParams& p) {
-  return p.mode == MODE_MASKED || p.m_total < 512 * (int64_t)p.G;
+// More than two rounds of 256x256 tiles whatever the group sizes turn out to be: at least ceil(m_total / 256) row tiles.
+static bool w4_large(const GemmParams& p) {
+  int grid = num_cus();
+  if (p.grid_limit > 0 && p.grid_limit < grid) grid = p.grid_limit;
+  return ((p.m_total + 255) / 256) * ((p.N + 127) / 128) > 4 * (int64_t)grid;
 }
 
-// The four-wave kernel takes M-grouped launches (rows contiguous or padded) whose tile count is large whatever the
-// group sizes turn out to be: at least ceil(m_total / 256) row tiles.  Smaller launches stay with the eight-wave
-// kernels, which choose narrower tiles on the device.
+// Whether 256-row tiles pay depends on the group sizes, which only the device knows.  With 512 rows and more per group on
+// average they do; a masked launch (counts anywhere up to its row stride), one with smaller groups or one of fewer rounds is
+// enqueued together with the eight-wave kernel, and the two decide from the sizes which of them runs.
+bool w4_decided_on_device(const GemmParams& p) {
+  return p.mode == MODE_MASKED || p.m_total < 512 * (int64_t)p.G || !w4_large(p);
+}
+
+// The four-wave kernel takes large M-grouped and masked launches, and M-grouped ones of 128 rows and more per group whose likely tiles
+// (every group's last one half full) cost two rounds of K = 2048 or more.  Of those, and of large ones with a tail, drawn at random with operands
+// in no cache, it takes 0.89-0.98 of the eight-wave kernel's time with the launch that returns (4 us) in it: 64 groups of 313 rows
+// on average, N = 1416, K = 2056, [K, N]: 198 -> 194 us; 32 of 1635, N = 1536, K = 3208: 549 -> 487; 8 of 1700, N = 3296, K = 1256:
+// 136 -> 123.  Where the sizes then choose the eight-wave kernel they lose the 4 us (32 of 263, N = 3072, K = 2880: 203 -> 209).
+// Smaller launches stay with the eight-wave kernels, which choose narrower tiles on the device.
 bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   if (dt != DT_BF16 && dt != DT_F16) return false;
   if (layout != W4_NT && layout != W4_NN) return false;
-  // NN: every 512-byte row segment of a tile must lie inside its row of B, and a group's B within 2 GiB
-  if (layout == W4_NN && ((p.N & 255) != 0 || (int64_t)p.K * p.N * 2 >= (1ll << 31))) return false;
+  // NN: a group's B, with the rows that the tail may add, within 2 GiB
+  if (layout == W4_NN && ((int64_t)p.K + 128) * p.N * 2 >= (1ll << 31)) return false;
   if (p.mode != MODE_MG && p.mode != MODE_MG_PAD && p.mode != MODE_MASKED) return false;
   // launches whose groups may be small are decided on the device (w4_decided_on_device), by a predicate that needs
   // one thread of this kernel per group
@@ -608,23 +632,35 @@ bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   if ((p.N & 7) != 0 || p.K < 8 || (p.K & 7) != 0) return false;
   if ((int64_t)p.K * 2 * 256 >= (1ll << 30)) return false;
   if ((int64_t)p.N * 2 * 128 >= (1ll << 30)) return false;  // a wave's block of the output within the epilogue's 32-bit offsets, out-of-range marker included
-  if (p.K % 128 != 0 || p.K < 256) return false;  // an even number of 64-deep slabs per tile, four at least
+  if (p.K < 192) return false;  // the first three slabs of a tile are whole
+  if (p.mode == MODE_MASKED && layout == W4_NN && needs_tail(p, layout)) return false;  // waves that sit tiles out, cut windows and transposing reads together do not fit the registers
   if (any_size) return true;
+  // a short K spends more on the slab that makes the tail's number even than the eight-wave kernel loses (4 groups of 13000 rows, N = 3096,
+  // K = 512, [K, N]: 195 us there, 202 here; 16 of 1200, N = 3072, K = 536: 79 and 81)
+  if (needs_tail(p, layout) && p.K < 768) return false;
+  if (w4_large(p)) return true;
+  if (p.mode == MODE_MASKED || p.m_total < 128 * (int64_t)p.G) return false;
   int grid = num_cus();
   if (p.grid_limit > 0 && p.grid_limit < grid) grid = p.grid_limit;
-  const int64_t row_tiles = (p.m_total + 255) / 256;
-  const int64_t narrow_tiles = row_tiles * ((p.N + 127) / 128);
-  return narrow_tiles > 4 * (int64_t)grid;
+  const int64_t likely_tiles_2 = (2 * ((p.m_total + 255) / 256) + p.G) * ((p.N + 255) / 256);
+  return likely_tiles_2 * p.K >= 2 * 4096 * (int64_t)grid;
+}
+
+template <int DT, int LAYOUT>
+int launch_w4_layout(const GemmParams& p, hipStream_t s) {
+  const bool sit_out = p.mode == MODE_MASKED;
+  if (needs_tail(p, LAYOUT)) {
+    if constexpr (LAYOUT == W4_NT) {
+      if (sit_out) return launch_w4<DT, LAYOUT, true, true>(p, s);
+    }
+    return launch_w4<DT, LAYOUT, false, true>(p, s);
+  }
+  return sit_out ? launch_w4<DT, LAYOUT, true, false>(p, s) : launch_w4<DT, LAYOUT, false, false>(p, s);
 }
 
 int launch_w4_16bit(const GemmParams& p, int dt, int layout, hipStream_t s) {
-  const bool sit_out = p.mode == MODE_MASKED;
-  if (layout == W4_NT) {
-    if (dt == DT_BF16) return sit_out ? launch_w4<DT_BF16, W4_NT, true>(p, s) : launch_w4<DT_BF16, W4_NT, false>(p, s);
-    return sit_out ? launch_w4<DT_F16, W4_NT, true>(p, s) : launch_w4<DT_F16, W4_NT, false>(p, s);
-  }
-  if (dt == DT_BF16) return sit_out ? launch_w4<DT_BF16, W4_NN, true>(p, s) : launch_w4<DT_BF16, W4_NN, false>(p, s);
-  return sit_out ? launch_w4<DT_F16, W4_NN, true>(p, s) : launch_w4<DT_F16, W4_NN, false>(p, s);
+  if (layout == W4_NT) return dt == DT_BF16 ? launch_w4_layout<DT_BF16, W4_NT>(p, s) : launch_w4_layout<DT_F16, W4_NT>(p, s);
+  return dt == DT_BF16 ? launch_w4_layout<DT_BF16, W4_NN>(p, s) : launch_w4_layout<DT_F16, W4_NN>(p, s);
 }
 
 }  // namespace tgg
