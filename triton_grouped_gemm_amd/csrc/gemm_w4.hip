@@ -614,10 +614,11 @@ bool w4_decided_on_device(const GemmParams& p) {
 }
 
 // The four-wave kernel takes large M-grouped and masked launches, and M-grouped ones of 128 rows and more per group whose likely tiles
-// (every group's last one half full) cost two rounds of K = 2048 or more.  Of those, and of large ones with a tail, drawn at random with operands
+// (every group's last one half full) cost two rounds of K = 2048 or more and would not be chosen for 128-row tiles
+// (sched_wide_tiles_chosen).  Of those, and of large ones with a tail, drawn at random with operands
 // in no cache, it takes 0.89-0.98 of the eight-wave kernel's time with the launch that returns (4 us) in it: 64 groups of 313 rows
 // on average, N = 1416, K = 2056, [K, N]: 198 -> 194 us; 32 of 1635, N = 1536, K = 3208: 549 -> 487; 8 of 1700, N = 3296, K = 1256:
-// 136 -> 123.  Where the sizes then choose the eight-wave kernel they lose the 4 us (32 of 263, N = 3072, K = 2880: 203 -> 209).
+// 136 -> 123.  Where the sizes choose the eight-wave kernel after all they lose the 4 us.
 // Smaller launches stay with the eight-wave kernels, which choose narrower tiles on the device.
 bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   if (dt != DT_BF16 && dt != DT_F16) return false;
@@ -642,8 +643,10 @@ bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   if (p.mode == MODE_MASKED || p.m_total < 128 * (int64_t)p.G) return false;
   int grid = num_cus();
   if (p.grid_limit > 0 && p.grid_limit < grid) grid = p.grid_limit;
-  const int64_t likely_tiles_2 = (2 * ((p.m_total + 255) / 256) + p.G) * ((p.N + 255) / 256);
-  return likely_tiles_2 * p.K >= 2 * 4096 * (int64_t)grid;
+  const int64_t tiles_n = (p.N + 255) / 256;
+  const int64_t full_2 = (2 * ((p.m_total + 255) / 256) + p.G) * tiles_n, half_2 = (2 * ((p.m_total + 127) / 128) + p.G) * tiles_n;  // twice the likely tiles
+  const int64_t rounds_full = (full_2 + 2 * grid - 1) / (2 * grid), rounds_half = (half_2 + 2 * grid - 1) / (2 * grid);
+  return full_2 * p.K >= 2 * 4096 * (int64_t)grid && rounds_half * 3 > rounds_full * 4;
 }
 
 template <int DT, int LAYOUT>
