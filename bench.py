@@ -46,31 +46,35 @@ PEAK_HBM_GBS = 8000.0
 # printed only while the hash of that source set still equals the stamp below; after any change to those files it
 # is null until the counters are read again (python bench.py --print-traffic-stamps prints the current hashes).
 MEASURED_TRAFFIC_GB = {
-    "bf16_m_grouped_gateup_nt": (11.38, "gemm16"),
-    "bf16_m_grouped_gateup_nn": (9.9, "gemm16"),
-    "bf16_m_grouped_gateup_fp8_out": (10.74, "gemm16"),
-    "bf16_m_grouped_down_nt": (5.24, "gemm16"),
-    "bf16_m_grouped_down_nn": (5.33, "gemm16"),
+    "bf16_m_grouped_gateup_nt": (11.67, "gemm16"),
+    "bf16_m_grouped_gateup_nn": (10.08, "gemm16"),
+    "bf16_m_grouped_gateup_fp8_out": (10.63, "gemm16"),
+    "bf16_m_grouped_down_nt": (5.19, "gemm16"),
+    "bf16_m_grouped_down_nn": (5.4, "gemm16"),
     "bf16_masked_decode": (2.47, "gemm16"),
-    "bf16_k_grouped_wgrad": (28.75, "gemm16"),
-    "fp8_block_m_grouped": (24.84, "gemm8"),
-    "fp8_channel_m_grouped": (26.96, "gemm8"),
-    "fp8_channel_k_grouped": (16.78, "gemm8"),
+    "bf16_k_grouped_wgrad": (28.64, "wgrad16"),
+    "fp8_block_m_grouped": (25.7, "gemm8"),
+    "fp8_channel_m_grouped": (27.08, "gemm8"),
+    "fp8_channel_k_grouped": (34.96, "wgrad8"),
     "quant_trans128": (8.12, "quant"),
     "quant_token128": (8.2, "quant"),
     "moe_permute": (3.06, "permute"),      # the row mover (the sort kernels move < 1 % of that)
     "moe_unpermute": (3.07, "permute"),
 }
 TRAFFIC_SOURCES = {
-    "gemm16": ("common.hpp", "sched.hpp", "fast_common.hpp", "gemm_fast.hip", "gemm_w4.hip"),
+    "gemm16": ("common.hpp", "sched.hpp", "fast_common.hpp", "gemm_fast.hip", "gemm_w4.hip", "w4_common.hpp"),
+    "wgrad16": ("common.hpp", "sched.hpp", "fast_common.hpp", "w4_common.hpp", "gemm_wgrad.hip"),
     "gemm8": ("common.hpp", "sched.hpp", "fast_common.hpp", "gemm_fp8.hip"),
+    "wgrad8": ("common.hpp", "sched.hpp", "fast_common.hpp", "w4_common.hpp", "fp8_w4.hip"),
     "quant": ("common.hpp", "sched.hpp", "quant.hip"),
     "permute": ("moe_permute.hip",),
 }
 TRAFFIC_STAMPS = {  # sha256 over the source set's files, first 16 hex digits, at the time of the counter runs
-    "gemm16": "f2a0e05e5afc8cad",
-    "gemm8": "54cd90ab5497d50e",
-    "quant": "8debad0aae3b9696",
+    "gemm16": "c010d7390f3df54c",
+    "wgrad16": "6a12e4b6dc8f5c5a",
+    "gemm8": "d31401691561dfe5",
+    "wgrad8": "c69a9cd153d25608",
+    "quant": "38349f034b203fad",
     "permute": "f5951f56ef17868f",
 }
 
