@@ -70,11 +70,11 @@ TRAFFIC_SOURCES = {
     "permute": ("moe_permute.hip",),
 }
 TRAFFIC_STAMPS = {  # sha256 over the source set's files, first 16 hex digits, at the time of the counter runs
-    "gemm16": "c010d7390f3df54c",
-    "wgrad16": "6a12e4b6dc8f5c5a",
-    "gemm8": "d31401691561dfe5",
-    "wgrad8": "c69a9cd153d25608",
-    "quant": "38349f034b203fad",
+    "gemm16": "7d9935c4d9fdc77a",
+    "wgrad16": "ea0cce726744fea9",
+    "gemm8": "6cb661a67b4db873",
+    "wgrad8": "3c25bf5057f1827b",
+    "quant": "3244157566b79278",
     "permute": "f5951f56ef17868f",
 }
 

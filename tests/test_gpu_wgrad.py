@@ -118,3 +118,20 @@ def test_fp8_codes_of_other_segments_are_not_added_up():
     one = lambda n: torch.ones(3, n, device=dev)
     out = _run_fp8(1, x.to(torch.float8_e4m3fn), one(300), y.to(torch.float8_e4m3fn), one(264), s, -1)
     assert bool((out[1] == 32).all()) and bool(torch.isnan(out[0]).all()) and bool(torch.isnan(out[2]).all())
+
+
+@pytest.mark.parametrize("sizes, T", [([48, 40, 72], 160), ([160, 7], 160), ([96, 80], 160), ([16, 33, 111], 160)])
+def test_fp8_counts_that_are_no_multiples_of_16(sizes, T):
+    """Exactly one of the two enqueued kernels computes: odd counts, odd counts that the axis' end clips away or to a multiple of 16."""
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(T + sizes[0])
+    x = (torch.randn(300, T, device=dev, generator=gen) * 8).to(torch.float8_e4m3fn)
+    y = (torch.randn(264, T, device=dev, generator=gen) * 8).to(torch.float8_e4m3fn)
+    one = lambda n: torch.ones(len(sizes), n, device=dev)
+    out = _run_fp8(1, x, one(300), y, one(264), torch.tensor(sizes, dtype=torch.int32, device=dev), -1)
+    at = 0
+    for g, n in enumerate(sizes):
+        end = min(T, at + n)
+        ref = x[:, at:end].float() @ y[:, at:end].float().t()
+        assert bool(((out[g].float() - ref).abs() <= ref.abs() * 2.0 ** -8 * 1.02 + 2e-3 * ref.abs().max()).all()), f"group {g}"
+        at = end

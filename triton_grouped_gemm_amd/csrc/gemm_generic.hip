@@ -140,6 +140,7 @@ template <int TA, int TB, bool A_KMAJOR, bool B_KMAJOR, int EPI, int OUT>
 __global__ __launch_bounds__(GTHREADS) void gemm_generic_kernel(const GemmParams p) {
   __shared__ GenericSmem sm;
   constexpr int ESA = ElemSize<TA>::v, ESB = ElemSize<TB>::v;
+  if (sched_kg_gate_shut(p)) return;
   sched_init<GBM>(p, sm.sched);
   if (!sched_kg_gate_open(p, sm.sched)) return;
   const int64_t num_tiles = sched_num_tiles<GBM, GBN>(p, sm.sched);
