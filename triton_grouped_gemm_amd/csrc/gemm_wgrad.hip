@@ -48,7 +48,10 @@ struct WgradCfg {
   static_assert(SMEM_BYTES <= 160 * 1024, "LDS budget");
 };
 
-template <int DT>
+// NT: see store_b128.  128 groups of 2048 x N, operands in no cache, 32 / 128 / 256 / 1024 tokens a group: N = 1544 non-temporal 463 / 456 /
+// 444 / 888 us, else 202 / 236 / 314 / 823 (the eight-wave kernel, non-temporal: 435 / 392 / 400 / 967); N = 1552 379 / 374 / 357 / 855 and 199 / 231 /
+// 310 / 814; N = 1568, whole 64 bytes, 184 / 194 / 306 / 800 and 188 / 227 / 310 / 811; N = 1536 146 / 167 / 252 / 688 and 165 / 191 / 272 / 703.
+template <int DT, bool NT>
 __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const GemmParams p) {
   typedef WgradCfg C;
   typedef Operand<256, false> Op;  // a slab of either operand: token rows of 512 bytes (here 32 of them)
@@ -207,9 +210,8 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
   };
   auto epi_store = [&](const EpiLane& e, int i, int h, int it, const i32x4_t& v, bool between_multiplies) __attribute__((always_inline)) {
     const int off = e.off[h] + (16 * i + 8 * it) * p.N * 2;
-    // wait states as in gemm_w4.hip: the data registers of a 16-byte store must not be overwritten within two
-    if (between_multiplies) asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 0" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
-    else asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 1" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
+    if (between_multiplies) store_b128<NT, 0>(v, off, pend_rs);  // the multiply that follows is the second wait state
+    else store_b128<NT, 1>(v, off, pend_rs);
   };
   auto epi_flush = [&]() __attribute__((always_inline)) {  // strips 4-7 of the workgroup's last tile
     asm volatile("s_nop 15\n\ts_nop 7" : "+a"(acc[7][0]), "+a"(acc[7][1]), "+a"(acc[7][2]), "+a"(acc[7][3]),
@@ -336,13 +338,13 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
   wait_vmcnt<0>();  // trailing zero-length copies still write LDS
 }
 
-template <int DT>
+template <int DT, bool NT>
 int launch_wgrad(const GemmParams& p, hipStream_t s) {
   static bool attr_set[64] = {false};
   int dev = 0;
   (void)hipGetDevice(&dev);
   const bool listed = dev >= 0 && dev < 64;
-  auto kern = gemm_wgrad_kernel<DT>;
+  auto kern = gemm_wgrad_kernel<DT, NT>;
   if (!listed || !attr_set[dev]) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, WgradCfg::SMEM_BYTES) != hipSuccess)
       return check_launch("hipFuncSetAttribute(gemm_wgrad)");
@@ -375,7 +377,8 @@ bool wgrad_supported(const GemmParams& p, int dt, bool any_size) {
 }
 
 int launch_wgrad_16bit(const GemmParams& p, int dt, hipStream_t s) {
-  return dt == DT_BF16 ? launch_wgrad<DT_BF16>(p, s) : launch_wgrad<DT_F16>(p, s);
+  if (rows_of_whole_64_bytes(p)) return dt == DT_BF16 ? launch_wgrad<DT_BF16, true>(p, s) : launch_wgrad<DT_F16, true>(p, s);
+  return dt == DT_BF16 ? launch_wgrad<DT_BF16, false>(p, s) : launch_wgrad<DT_F16, false>(p, s);
 }
 
 }  // namespace tgg

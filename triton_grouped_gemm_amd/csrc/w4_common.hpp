@@ -30,6 +30,16 @@ template <int OFF0, int OFF1> TGG_DEV void lds_read_tr(i32x4_t& dst, uint32_t ad
 }
 #define TGG_TIE8(f) "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]), "+v"(f[6]), "+v"(f[7])
 
+// A 16-byte output store of a lane and the wait states behind it (two must pass before the data registers may be overwritten).
+// NT: non-temporal, for rows that begin on a multiple of 64 bytes.  Elsewhere the ends of a row segment share a line
+// with the segments beside it, which are stored a few multiplies apart; non-temporal, such a line goes out piece by piece, which costs
+// memory-bound launches up to half their time, while lines that stay in L2 are completed there first (figures: gemm_wgrad.hip).
+inline bool rows_of_whole_64_bytes(const GemmParams& p) { return p.N % 32 == 0 && ((uintptr_t)p.C & 63) == 0; }
+template <bool NT, int NOP> TGG_DEV void store_b128(const i32x4_t& v, int off, const i32x4_t& rs) {
+  if constexpr (NT) asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop %3" : : "v"(v), "v"(off), "s"(rs), "n"(NOP) : "memory");
+  else asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen\n\ts_nop %3" : : "v"(v), "v"(off), "s"(rs), "n"(NOP) : "memory");
+}
+
 // Division of 32-bit values by a divisor that is fixed for the launch, on the scalar unit.  m = floor(2^32 / d) + 1: the
 // estimate n m / 2^32 is the quotient or one more for every 32-bit n.
 struct FixedDiv {
