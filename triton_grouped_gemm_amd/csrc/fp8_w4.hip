@@ -163,7 +163,7 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
 
   // A slab takes 128 bytes of rows that lie far apart, one line of each, which HBM serves slowly and late.  So once in two slabs the
   // rows' next two lines are touched (one word of each, into a sink in LDS) and wait in L2 when they are copied, the first two of a
-  // tile at the start of the tile before.  The
+  // tile at the start of the tile before, the next two when the copies, a slab and a half before the tile, have come to its second.  The
   // workgroups of an XCD that run together share their panels (the tiles of a run of 32 neighbours: nc columns by 32 / nc rows),
   // and each touches its part of them only: all of it by everybody costs more than it gains.
   const int rows_a = (C::BM + tiles.nc - 1) / tiles.nc, parts_b = tiles.nc < 32 ? 32 / tiles.nc : 1, rows_b = (C::BN + parts_b - 1) / parts_b;
@@ -322,7 +322,8 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
       if constexpr (n >= 32 && n % 2 == 0) copy_m0(TGG_F8_I((n - 32) / 2));
       if constexpr (n >= 32 && n % 2 == 1) copy(TGG_F8_I((n - 33) / 2));
       if constexpr (n == 63) {
-        if ((koff & C::KS) == 0) touch_two(feed, part, koff + C::KS);
+        // the first two lines of a tile have been touched before, and its last slab requests the next tile's second
+        if (EPI != 2 && (koff & C::KS) != 0) touch_two(feed, part, koff + C::KS);
       }
       if constexpr (EPI == 1 && n < 32) epi_gap(Nc, TGG_F8_I(4));
       if constexpr (EPI == 2 && n >= 32) epi_gap(TGG_F8_I(n - 32), TGG_F8_I(0));
@@ -351,6 +352,7 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
                           rows_left > 0 ? (int)(rows_left < 128 ? rows_left : 128) * p.N * 2 : 0);
     pend_cols = p.N - cur.n0 - wn0;
     slab(I2(), I0(), pos);
+    touch_two(feed, part_of(following), 2 * C::KS);
     cur = following;
   }
   epi_flush();
