@@ -164,9 +164,12 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
   // A slab takes 128 bytes of rows that lie far apart, one line of each, which HBM serves slowly and late.  So once in two slabs the
   // rows' next two lines are touched (one word of each, into a sink in LDS) and wait in L2 when they are copied, the first two of a
   // tile at the start of the tile before, the next two when the copies, a slab and a half before the tile, have come to its second.  The
-  // workgroups of an XCD that run together share their panels (the tiles of a run of 32 neighbours: nc columns by 32 / nc rows),
-  // and each touches its part of them only: all of it by everybody costs more than it gains.
-  const int rows_a = (C::BM + tiles.nc - 1) / tiles.nc, parts_b = tiles.nc < 32 ? 32 / tiles.nc : 1, rows_b = (C::BN + parts_b - 1) / parts_b;
+  // workgroups of an XCD that run together share their panels (the tiles of a run of 32 neighbours: nc columns by 32 / nc rows, or as
+  // many as a group has), and each touches its part of them only: all of it by everybody costs more than it gains, and so does
+  // a panel that nobody shares (outputs of a single column or row of tiles: 51 groups of 1316 x 208, 2900 tokens 125 -> 117 us, 2 of 208 x 4648, 8500
+  // tokens 251 -> 230; parts for 32 / nc rows where a group has fewer: 71 of 1334 x 488, 2600 tokens 270 -> 262).
+  const int parts_b = max(1, min(tiles.tiles_m, 32 / tiles.nc));
+  const int rows_a = tiles.nc > 1 ? (C::BM + tiles.nc - 1) / tiles.nc : 0, rows_b = parts_b > 1 ? (C::BN + parts_b - 1) / parts_b : 0;
   struct Part { int a, b; };  // the lane's offsets, kNoFetch beyond the workgroup's part
   auto part_of = [&](const KgTile& t) __attribute__((always_inline)) {
     const int mt = t.m0 >> 8, nt = t.n0 >> 8, part_a = nt - (int)tiles.by_nc.div((uint32_t)nt) * tiles.nc, part_b = mt % parts_b;
