@@ -62,7 +62,7 @@ bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size);
 bool w4_decided_on_device(const GemmParams& p);
 int launch_w4_16bit(const GemmParams& p, int dt, int layout, hipStream_t s);
 bool wgrad_supported(const GemmParams& p, int dt, bool any_size);
-bool fp8_w4_supported(const GemmParams& p);
+bool fp8_w4_supported(const GemmParams& p, bool any_size);
 int launch_fp8_w4(const GemmParams& p, int ta, int tb, hipStream_t s);
 int launch_wgrad_16bit(const GemmParams& p, int dt, hipStream_t s);
 bool fast_quant_supported(const GemmParams& p, int dt, int layout);
@@ -424,7 +424,7 @@ int tgg_k_grouped_gemm_fp8_channel_queued(const void* x, const float* xs, const 
     // The tuned kernel needs every token count to be a multiple of 16 and only the device knows the counts: both
     // kernels are enqueued, each reads the counts first and exactly one of them runs (the other returns at once).
     p.kg_gate = 1;
-    if (g_four_wave.load() && fp8_w4_supported(p)) {
+    if (const int four_wave = g_four_wave.load(); four_wave && fp8_w4_supported(p, four_wave == 2)) {
       if (int e = launch_fp8_w4(p, fmt_a, fmt_b, (hipStream_t)stream)) return e;
     } else if (int e = launch_fast_fp8_channel(p, fmt_a, fmt_b, TGG_BF16, (hipStream_t)stream)) {
       return e;

@@ -385,14 +385,17 @@ int launch_cfg(const GemmParams& p, hipStream_t s) {
 
 }  // namespace
 
-// Every K-grouped launch that its table and offsets allow: with operands that are not in a cache, 16 shapes of 512 x 1024 to 3072 x 4096
-// for 4-128 groups of 128-4096 tokens take 0.74-1.03 of the eight-wave kernel's time.
-bool fp8_w4_supported(const GemmParams& p) {
+// What its table and offsets allow, but for outputs of a single column of tiles over long segments, which wait for the rows of A, shared by
+// nobody, and get them no sooner here.  650 random launches of 64-6144 columns and 16-16000 tokens a group, operands in no cache: 0.94 of the
+// eight-wave kernel's time in the mean (0.69-1.11) with N > 256, 0.95 with N <= 256 and fewer than 1000 tokens, 1.04 with 1000 and more
+// (0.89-1.16: 89 groups of 1850 x 136, 2100 tokens 183 us and 157 there, 4 of 4251 x 144, 1400 tokens 46 and 41).
+bool fp8_w4_supported(const GemmParams& p, bool any_size) {
   if (p.mode != MODE_KG_COUNT) return false;
   if (p.G > Fp8W4Cfg::THREADS || (p.N & 7) != 0 || (p.k_total & 15) != 0) return false;
   // a tile's window of either operand, and a wave's block of the output, within 32-bit offsets below the out-of-range marker
   if (p.k_total * 256 >= (1ll << 30) || (int64_t)p.N * 2 * 128 >= (1ll << 30)) return false;
-  return p.G * ((p.m_total + 255) / 256) * (((int64_t)p.N + 255) / 256) < (1ll << 31);
+  if (p.G * ((p.m_total + 255) / 256) * (((int64_t)p.N + 255) / 256) >= (1ll << 31)) return false;
+  return any_size || p.N > Fp8W4Cfg::BN || p.k_total < 1000 * (int64_t)p.G;
 }
 
 int launch_fp8_w4(const GemmParams& p, int ta, int tb, hipStream_t s) {
