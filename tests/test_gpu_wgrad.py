@@ -54,6 +54,19 @@ def test_weight_gradient_kernel_at_its_edges(dtype, num_cu, sizes, M, N):
     assert int(_native.work_queue(dev, None).abs().sum()) == 0  # handed back zeroed
 
 
+@pytest.mark.parametrize("M, N", [(2 ** 21 - 8, 8), (2 ** 21, 8), (2 ** 22, 8), (8, 2 ** 21 - 8), (8, 2 ** 21), (8, 2 ** 22)])
+def test_token_rows_that_are_too_long_for_the_touched_window(M, N):
+    """256 touched token rows have to lie below 1 GiB, the offset of what is not fetched: longer ones stay with the eight-wave kernel."""
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(M + N)
+    a, b = (torch.randn(40, n, device=dev, generator=gen).bfloat16() for n in (M, N))
+    s = torch.tensor([33, 7], dtype=torch.int32, device=dev)
+    out = _run(2, a, b, s, -1)
+    assert torch.equal(out.view(torch.int16), _run(0, a, b, s, -1).view(torch.int16))
+    ref = a[33:].float().t() @ b[33:].float()
+    assert bool(((out[1].float() - ref).abs() <= ref.abs() * 2.0 ** -8 * 1.02 + 2e-6 * ref.abs().max()).all())
+
+
 def test_rows_beyond_a_segment_are_not_added_up():
     """Infinities and NaN in the tokens of the neighbouring groups, and in columns beside a ragged tile, stay where they are."""
     dev = torch.device("cuda:0")

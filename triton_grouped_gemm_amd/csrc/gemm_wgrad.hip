@@ -46,6 +46,7 @@ struct WgradCfg {
   static constexpr int SMEM_BYTES = SINK_OFF + 4 * 256;
   static constexpr int TOUCH = 256;  // tokens of the next tile that are touched
   static_assert(SMEM_BYTES <= 160 * 1024, "LDS budget");
+  static_assert(TOUCH >= KS && TOUCH >= BM / 2, "wgrad_supported bounds the slab's and the stores' windows by the touched rows'");
 };
 
 // NT: see store_b128.  128 groups of 2048 x N, operands in no cache, 32 / 128 / 256 / 1024 tokens a group: N = 1544 non-temporal 463 / 456 /
@@ -366,8 +367,9 @@ bool wgrad_supported(const GemmParams& p, int dt, bool any_size) {
   if (dt != DT_BF16 && dt != DT_F16) return false;
   if (p.mode != MODE_KG && p.mode != MODE_KG_COUNT) return false;
   if (p.G > WgradCfg::THREADS || (p.N & 7) != 0 || (p.m_total & 7) != 0) return false;
-  // token rows of a slab, and a wave's block of the output, within 32-bit offsets that stay below the out-of-range marker
-  if (p.m_total * 2 * 64 >= (1ll << 30) || (int64_t)p.N * 2 * 128 >= (1ll << 30)) return false;
+  // the token rows of either operand that are touched (a slab has fewer), and a wave's block of the output, within 32-bit offsets that stay
+  // below the out-of-range marker
+  if (p.m_total * 2 * WgradCfg::TOUCH >= (1ll << 30) || (int64_t)p.N * 2 * WgradCfg::TOUCH >= (1ll << 30)) return false;
   const int64_t tiles_m = (p.m_total + 255) / 256, tiles_n = (p.N + 255) / 256;
   if (p.G * tiles_m * tiles_n >= (1ll << 31)) return false;
   if (any_size) return true;
