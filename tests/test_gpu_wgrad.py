@@ -54,6 +54,34 @@ def test_weight_gradient_kernel_at_its_edges(dtype, num_cu, sizes, M, N):
     assert int(_native.work_queue(dev, None).abs().sum()) == 0  # handed back zeroed
 
 
+@pytest.mark.parametrize("queued", [True, False])
+@pytest.mark.parametrize("num_cu", [-1, 64, 8])
+@pytest.mark.parametrize("tokens", [31, 32, 63, 64, 95, 96])
+@pytest.mark.parametrize("N", [256, 264])
+def test_short_segments_by_the_default_route(queued, num_cu, tokens, N):
+    """Either side of the lines between the two kernels (wgrad_supported), on launches large enough for the four-wave one."""
+    dev = torch.device("cuda:0")
+    G, M = 70, 1544
+    sizes = [tokens + (g % 3 - 1) * 20 for g in range(G - 1)]
+    sizes.append(tokens * G - sum(sizes))
+    gen = torch.Generator(device=dev).manual_seed(tokens)
+    a, b = (torch.randn(tokens * G, n, device=dev, generator=gen).bfloat16() for n in (M, N))
+    s = torch.tensor(sizes, dtype=torch.int32, device=dev)
+
+    def run(four_wave):
+        out = torch.full((G, M, N), float("nan"), device=dev, dtype=torch.bfloat16)
+        _native.set_option("four_wave", four_wave)
+        try:
+            _native.call("tgg_k_grouped_gemm_sizes", a.data_ptr(), b.data_ptr(), out.data_ptr(), s.data_ptr(), 0, G, M, N, tokens * G, _native.BF16,
+                         num_cu, _native.work_queue(dev, None).data_ptr() if queued else 0, _native.stream_of(a))
+        finally:
+            _native.set_option("four_wave", 1)
+        return out.view(torch.int16)
+    out = run(1)
+    assert torch.equal(out, run(0)) and torch.equal(out, run(2))
+    assert not bool(torch.isnan(out.view(torch.bfloat16)).any())
+
+
 @pytest.mark.parametrize("M, N", [(2 ** 21 - 8, 8), (2 ** 21, 8), (2 ** 22, 8), (8, 2 ** 21 - 8), (8, 2 ** 21), (8, 2 ** 22)])
 def test_token_rows_that_are_too_long_for_the_touched_window(M, N):
     """256 touched token rows have to lie below 1 GiB, the offset of what is not fetched: longer ones stay with the eight-wave kernel."""

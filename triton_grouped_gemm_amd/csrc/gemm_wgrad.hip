@@ -363,6 +363,10 @@ int launch_wgrad(const GemmParams& p, hipStream_t s) {
 // narrower tiles and draws a tile later, i.e. more evenly: half a round, 384 / 1024 tokens a group (512 x 1024, 16 groups) 25 / 55 us there
 // and 33 / 73 here; one and a half rounds (768 x 2048, 16 groups) 45 / 92 and 36 / 85.  More groups
 // than this kernel has threads stay there too: their table takes longer to make (300 groups of 264 x 520, 256 tokens: 98 against 113 us).
+// So do short segments where few workgroups run or no queue evens them out: a tile has four K steps at least here, one slab there, which is
+// hidden while memory is the bound.  Time of this kernel over the eight-wave kernel's, 1600 random launches of 2-400 tokens a group: a queue and 64 CUs
+// 1.05 below 64 tokens (100 and 128 CUs 1.0, all 0.8); no queue and 64-128 CUs 1.07-1.2 below 96 tokens, more of them 1.04 below 32 where N is a multiple
+// of 32 (0.7 elsewhere).  128 groups of 1536 x 2816, 15 tokens, 64 CUs, no queue: 652 -> 491 us.
 bool wgrad_supported(const GemmParams& p, int dt, bool any_size) {
   if (dt != DT_BF16 && dt != DT_F16) return false;
   if (p.mode != MODE_KG && p.mode != MODE_KG_COUNT) return false;
@@ -375,6 +379,8 @@ bool wgrad_supported(const GemmParams& p, int dt, bool any_size) {
   if (any_size) return true;
   int grid = num_cus();
   if (p.grid_limit > 0 && p.grid_limit < grid) grid = p.grid_limit;
+  const int64_t tokens = p.k_total / p.G;
+  if (p.queue ? 4 * grid <= num_cus() && tokens < 64 : 2 * grid <= num_cus() ? tokens < 96 : tokens < 32 && rows_of_whole_64_bytes(p)) return false;
   return 2 * p.G * tiles_m * tiles_n >= 3 * (int64_t)grid;
 }
 
