@@ -1,6 +1,7 @@
 """The four-wave kernel's instantiation for any K and N (gemm_w4.hip, TAIL) where it can go wrong: K around its slab of 64, its pairs
 of slabs and its least of 192; N around its 256 columns with B as [G, K, N].  Forced on every shape, against the shape-agnostic
-kernel bit for bit (both add up 32 values of K at a time in ascending order and round once)."""
+kernel bit for bit (both add up 32 values of K at a time in ascending order and round once).  At the end the launches that reach it, and
+the plain instantiation, by the default route: alone, and enqueued together with the eight-wave kernel with sizes that choose either."""
 import pytest
 import torch
 
@@ -34,15 +35,16 @@ def test_any_k_and_n(dtype, num_cu, K, N, trans_b):
     assert torch.equal(_with("four_wave", 2, 1, run), _with("force_generic", 1, 0, run))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("K", [200, 264, 392])
-def test_masked_with_a_tail(K):
+def test_masked_with_a_tail(K, dtype):
     dev = torch.device("cuda:0")
     torch.manual_seed(K)
     s = torch.tensor([256, 0, 100, 129], dtype=torch.int32, device=dev)
-    a, b = torch.randn(4 * 256, K, device=dev).bfloat16(), torch.randn(4, 520, K, device=dev).bfloat16()
+    a, b = torch.randn(4 * 256, K, device=dev).to(dtype), torch.randn(4, 520, K, device=dev).to(dtype)
 
     def run():
-        out = torch.zeros(4 * 256, 520, device=dev, dtype=torch.bfloat16)
+        out = torch.zeros(4 * 256, 520, device=dev, dtype=dtype)
         m_grouped_gemm_masked(a, b, out, s, 256)
         return out
     assert torch.equal(_with("four_wave", 2, 1, run), _with("force_generic", 1, 0, run))
@@ -59,3 +61,69 @@ def test_what_lies_beyond_a_tail_is_not_added_up(trans_b):
     s = torch.tensor(sizes, dtype=torch.int32, device=dev)
     out = _with("four_wave", 2, 1, lambda: m_grouped_gemm(a, b, s, trans_b))
     assert bool((out[70:130] == K).all())
+
+
+CUS = 8  # workgroups of the launches below: small ones then have the rounds of tiles of large ones
+
+
+def _chosen(sizes, N):
+    """What the sizes decide where both kernels are enqueued (sched_wide_tiles_chosen): True = the four-wave kernel."""
+    full, half = (sum(-(-n // h) for n in sizes) for h in (256, 128))
+    tiles_n = -(-N // 256)
+    return full * -(-N // 128) > CUS and -(-half * tiles_n // CUS) * 3 > -(-full * tiles_n // CUS) * 4
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("trans_b, N, K", [(True, 1032, 776), (False, 1032, 768), (False, 1024, 904), (True, 1024, 1024)])
+@pytest.mark.parametrize("case, sizes, wide", [
+    ("alone", [1500, 2, 1301, 1397], None),                                     # 512 rows a group and more, more than four rounds: the four-wave kernel alone
+    ("small groups", [500, 513, 480, 300, 0, 700, 511, 300, 896], True),
+    ("small groups", [470] + [40] * 8, False),                                  # groups that fill a fraction of the operand, in 128-row tiles
+    ("few rounds", [330, 255, 180], True),                                      # at most four rounds, of a long K
+    ("few rounds", [100, 0, 40], False),                                        # the same operand with few rows: narrow tiles
+])
+def test_the_default_route(dtype, trans_b, N, K, case, sizes, wide):
+    dev = torch.device("cuda:0")
+    G, rows = len(sizes), 4200
+    if case == "few rounds":
+        rows, K = 768 if N > 1024 else 1024, K + 1024
+        assert -(-rows // 256) * -(-N // 128) <= 4 * CUS  # and gemm_w4.hip's likely tiles: 9 / 2 or 11 / 2 rows of them, two rounds of K = 2048
+    if wide is not None:
+        assert _chosen(sizes, N) == wide
+    gen = torch.Generator(device=dev).manual_seed(K + rows)
+    a = torch.randn(rows, K, device=dev, generator=gen).to(dtype)
+    b = (torch.randn(G, *((N, K) if trans_b else (K, N)), device=dev, generator=gen) * K ** -0.5).to(dtype)
+    s = torch.tensor(sizes, dtype=torch.int32, device=dev)
+
+    def run():
+        out = torch.full((rows, N), float("nan"), device=dev, dtype=dtype)
+        _native.call("tgg_m_grouped_gemm", a.data_ptr(), b.data_ptr(), out.data_ptr(), s.data_ptr(), 0, G, rows, N, K, int(trans_b),
+                     _native.BF16 if dtype == torch.bfloat16 else _native.F16, CUS, _native.stream_of(a))
+        return out
+    out = run()
+    assert torch.equal(out.view(torch.int16), _with("four_wave", 0, 1, run).view(torch.int16))
+    assert torch.equal(out.view(torch.int16), _with("force_generic", 1, 0, run).view(torch.int16))
+    assert not bool(torch.isnan(out[:sum(sizes)]).any()) and bool(torch.isnan(out[sum(sizes):]).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("masked, wide", [([512, 300, 511, 0, 400], True), ([40, 128, 0, 99, 128], False)])
+def test_the_default_route_of_masked_launches_with_a_tail(dtype, masked, wide):
+    dev = torch.device("cuda:0")
+    N, K, slots = 1032, 904, 512
+    assert _chosen(masked, N) == wide
+    gen = torch.Generator(device=dev).manual_seed(K)
+    a = torch.randn(len(masked) * slots, K, device=dev, generator=gen).to(dtype)
+    b = (torch.randn(len(masked), N, K, device=dev, generator=gen) * K ** -0.5).to(dtype)
+    s = torch.tensor(masked, dtype=torch.int32, device=dev)
+
+    def run():
+        out = torch.full((len(masked) * slots, N), float("nan"), device=dev, dtype=dtype)
+        _native.call("tgg_m_grouped_gemm_masked", a.data_ptr(), b.data_ptr(), out.data_ptr(), s.data_ptr(), 0, len(masked), slots, len(masked) * slots, N, K,
+                     1, _native.BF16 if dtype == torch.bfloat16 else _native.F16, CUS, _native.stream_of(a))
+        return out
+    out = run()
+    assert torch.equal(out.view(torch.int16), _with("force_generic", 1, 0, run).view(torch.int16))
+    for g, n in enumerate(masked):
+        block = out[g * slots:(g + 1) * slots]
+        assert not bool(torch.isnan(block[:n]).any()) and bool(torch.isnan(block[n:]).all())
