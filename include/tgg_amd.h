@@ -251,21 +251,27 @@ int tgg_debug_queue_order(int grid, int draws, int32_t* out);
  * once, atomically, so a thread that changes one while another thread launches decides only which value that launch
  * sees; returns 1 for an unknown key):
  *   "force_generic" 0/1  route every GEMM through the shape-agnostic kernel
- *   "variant"       int  tile configuration of the tuned kernels (16-bit, and FP8 M-grouped): 0 (default) = chosen per launch on the
+ *   "variant"       int  tile configuration of the eight-wave kernels (16-bit, and FP8 M-grouped): 0 (default) = chosen per launch on the
  *                        device from the group sizes -- 256x128 when all such tiles fit one round of the persistent
  *                        workgroups; otherwise, for 16-bit M-grouped / masked and FP8 M-grouped launches, the
  *                        weight-streaming configuration (128x256 tiles, three weight slab buffers) when its rounds of
  *                        the persistent workgroups, at 0.7 of a 256-row tile's cost each, are no more than those of
  *                        the 256x256 tiles (groups of up to about 200 rows on average); 256x256 otherwise; 1 = always 256x128; 2 = always 256x256; 4 = always the weight-streaming
  *                        configuration (16-bit NT / NN, FP8 M-grouped)
- *   "four_wave"     int  16-bit M-grouped / masked NT (or NN with N a multiple of 256), K a multiple of 128 (at least 256): 1 (default) = the four-wave
- *                        kernel (128x128 per wave) on large launches (more than four rounds of 256x128 tiles; masked
- *                        launches and M-grouped ones with fewer than 512 rows per group on average enqueue both
- *                        kernels, which decide on the device from the sizes which of them runs), 0 = eight-wave
- *                        kernels only, 2 = the four-wave kernel on every launch it can take, whatever the sizes
+ *   "four_wave"     int  the four-wave kernels (128x128 per wave), all for N (16-bit: and K, at least 192, or Mdim) a multiple of 8 and up to 256
+ *                        groups (512 where a launch is not decided on the device): 1 (default) = where they are the faster ones; 0 =
+ *                        eight-wave kernels only; 2 = on every launch that they can take, whatever the sizes.  By default:
+ *                        16-bit M-grouped / masked: launches of more than four rounds of 256x128 tiles, and smaller M-grouped ones of at
+ *                        least 128 rows per group whose likely tiles cost two rounds of K = 2048; K from 768 on where it is no multiple of 128
+ *                        or N is none of 256 with trans_b = 0 (masked launches with trans_b = 0 need both multiples).  Masked
+ *                        launches, those with fewer than 512 rows per group on average and the smaller ones enqueue both kernels,
+ *                        which decide on the device from the sizes which of them runs;
+ *                        16-bit K-grouped: launches of one and a half rounds of 256x256 tiles and more, but for segments of less than 32-96
+ *                        tokens on few workgroups or without a queue;
+ *                        FP8 K-grouped: all but outputs of up to 256 columns with 1000 tokens a group and more
  *   "tile_split"    0/1  M-grouped tuned kernels: per-XCD contiguous tile ranges (default 1) or interleaved sweeps
  *   "n_chunk"       int  column tiles per chunk of the tile order (0 = automatic, at most eight)
- *   "store_nt"      0/1  write the output with non-temporal stores (default 1)
+ *   "store_nt"      0/1  eight-wave kernels: write the output with non-temporal stores (default 1)
  *   "kg_second_launch" 0/1  tgg_k_grouped_gemm_fp8_channel enqueues the tuned kernel and the shape-agnostic kernel, and
  *                        each decides on the device from the token counts whether it runs (tuned: all counts multiples
  *                        of 16); 0 leaves the second one out, so a test can see what the tuned kernel does alone */

@@ -98,14 +98,14 @@ struct GemmParams {
   int tile_split;         // tuned kernels: 1 = per-XCD contiguous tile ranges (see sched_walk)
   int n_chunk;            // column tiles per chunk of the tile order, 0 = automatic (see sched_tile)
   int32_t* queue;         // K-grouped tuned kernels: tile-id counter in device memory (zero at launch), or null = static walk
-  int store_nt;           // tuned kernels: 1 = non-temporal output stores
+  int store_nt;           // eight-wave kernels: 1 = non-temporal output stores
   // FP8 K-grouped by token counts: the tuned kernel copies 16-byte chunks, so it needs every count (hence every
   // segment start) to be a multiple of 16; the shape-agnostic kernel takes anything.  Only the device knows the
   // counts, so both kernels are launched and each looks at the counts first: 1 = run only if all counts are
   // multiples of 16 (tuned), 2 = run only if one is not (shape-agnostic), 0 = always run.
   int kg_gate;
-  // 16-bit launches that the four-wave kernel could take but whose groups may be small (masked; M-grouped with fewer
-  // than 512 rows per group on average): it pays only where the eight-wave kernels would choose their 256x256 tiles,
+  // 16-bit launches that the four-wave kernel could take but whose groups may be small or few (w4_decided_on_device): it pays only
+  // where its 256x256 tiles are neither so few that narrow ones fit one round nor dearer than 128-row tiles,
   // which depends on the sizes, and only the device knows them.  Both kernels are
   // launched and each evaluates the same predicate on its group table first (sched_wide_tiles_chosen):
   // 1 = run only if it holds (four-wave), 2 = run only if it does not (eight-wave), 0 = always run.

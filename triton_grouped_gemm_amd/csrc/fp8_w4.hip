@@ -168,6 +168,9 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
   // many as a group has), and each touches its part of them only: all of it by everybody costs more than it gains, and so does
   // a panel that nobody shares (outputs of a single column or row of tiles: 51 groups of 1316 x 208, 2900 tokens 125 -> 117 us, 2 of 208 x 4648, 8500
   // tokens 251 -> 230; parts for 32 / nc rows where a group has fewer: 71 of 1334 x 488, 2600 tokens 270 -> 262).
+  // Rows a multiple of many KB apart crowd into few sets of L2, and touched lines leave it again before they are copied: 128 groups of 3072 x 4096,
+  // 5120 tokens each, 655360 codes a row: 6161 us, untouched 6185, with twice the traffic; 655744 a row: 5658 and 6201.  32 groups, 1024 tokens
+  // on average, 32768 a row: 435 and 461; 32896: 403 and 455.
   const int parts_b = max(1, min(tiles.tiles_m, 32 / tiles.nc));
   const int rows_a = tiles.nc > 1 ? (C::BM + tiles.nc - 1) / tiles.nc : 0, rows_b = parts_b > 1 ? (C::BN + parts_b - 1) / parts_b : 0;
   struct Part { int a, b; };  // the lane's offsets, kNoFetch beyond the workgroup's part

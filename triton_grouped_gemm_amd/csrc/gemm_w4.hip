@@ -100,7 +100,7 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   auto& sched = *reinterpret_cast<SchedTableT<kFastMaxGroups>*>(smem + C::SCHED_OFF);
   sched_init<C::BM>(p, sched);
-  // a launch that only pays where the eight-wave kernels would choose 256x256 tiles as well (GemmParams::wide_gate):
+  // a launch that pays only with sizes for 256x256 tiles (GemmParams::wide_gate):
   // the same predicate on the same table decides there that the eight-wave launch behind this one has nothing to do
   if (p.wide_gate == 1 && !sched_wide_tiles_chosen<C::BM, C::BN>(p, sched)) return;
   const int num_tiles = (int)sched_num_tiles<C::BM, C::BN>(p, sched);
@@ -608,17 +608,18 @@ static bool w4_large(const GemmParams& p) {
 
 // Whether 256-row tiles pay depends on the group sizes, which only the device knows.  With 512 rows and more per group on
 // average they do; a masked launch (counts anywhere up to its row stride), one with smaller groups or one of fewer rounds is
-// enqueued together with the eight-wave kernel, and the two decide from the sizes which of them runs.
+// enqueued together with the eight-wave kernel, and the two decide from the sizes which of them runs.  The average is that of the operand:
+// where the groups of a large launch fill a twentieth of it, this kernel alone takes 1.1 of the eight-wave kernel's time (up to 1.33; a fifth
+// of it 0.98, all 0.93: 200 random launches with a tail).  Decided on the device as well these would take 1.08, 1.01 and 0.94.
 bool w4_decided_on_device(const GemmParams& p) {
   return p.mode == MODE_MASKED || p.m_total < 512 * (int64_t)p.G || !w4_large(p);
 }
 
 // The four-wave kernel takes large M-grouped and masked launches, and M-grouped ones of 128 rows and more per group whose likely tiles
 // (every group's last one half full) cost two rounds of K = 2048 or more and would not be chosen for 128-row tiles
-// (sched_wide_tiles_chosen).  Of those, and of large ones with a tail, drawn at random with operands
-// in no cache, it takes 0.89-0.98 of the eight-wave kernel's time with the launch that returns (4 us) in it: 64 groups of 313 rows
-// on average, N = 1416, K = 2056, [K, N]: 198 -> 194 us; 32 of 1635, N = 1536, K = 3208: 549 -> 487; 8 of 1700, N = 3296, K = 1256:
-// 136 -> 123.  Where the sizes choose the eight-wave kernel after all they lose the 4 us.
+// (sched_wide_tiles_chosen).  Of 574 of those, drawn at random with operands in no cache, 554 were its by their sizes as well and
+// took 0.91 of the eight-wave kernel's time (0.92 with a tail, 0.85-1.01) with the launch that returns in it; 20 were not and lost 4-6 us, 1.03.
+// Large ones with a tail: 0.93.  32 groups of 1635 rows, N = 1536, K = 3208: 549 -> 487 us; 8 of 1700, N = 3296, K = 1256: 136 -> 123.
 // Smaller launches stay with the eight-wave kernels, which choose narrower tiles on the device.
 bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   if (dt != DT_BF16 && dt != DT_F16) return false;
