@@ -94,6 +94,7 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
   typedef W4Cfg C;
   constexpr int S_OFF = 0, D_OFF = C::A_BYTES;  // the operands' places in a slab buffer
   constexpr bool B_KMAJOR = LAYOUT == W4_NT;  // NN: B is [G, K, N], its slab 64 token rows of 512 bytes
+  static_assert(!(SIT_OUT && TAIL), "masked launches with a tail are the eight-wave kernels' (w4_supported)");
   typedef Operand<C::BM, true> Op;            // the A slab, and B's when K-contiguous: 256 rows of 128 bytes
   typedef Operand<C::BN, B_KMAJOR> OpB;
 
@@ -635,7 +636,9 @@ bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   if ((int64_t)p.K * 2 * 256 >= (1ll << 30)) return false;
   if ((int64_t)p.N * 2 * 128 >= (1ll << 30)) return false;  // a wave's block of the output within the epilogue's 32-bit offsets, out-of-range marker included
   if (p.K < 192) return false;  // the first three slabs of a tile are whole
-  if (p.mode == MODE_MASKED && layout == W4_NN && needs_tail(p, layout)) return false;  // waves that sit tiles out, cut windows and transposing reads together do not fit the registers
+  // masked launches with a tail: the launch that returns costs more than this kernel gains (120 random ones from K = 776 on, counts up to 0.05-0.4 of the
+  // slots 1.035 of the eight-wave kernels' time alone, up to 0.7 and all of them 0.995)
+  if (p.mode == MODE_MASKED && needs_tail(p, layout)) return false;
   if (any_size) return true;
   // a short K spends more on the slab that makes the tail's number even than the eight-wave kernel loses (4 groups of 13000 rows, N = 3096,
   // K = 512, [K, N]: 195 us there, 202 here; 16 of 1200, N = 3072, K = 536: 79 and 81)
@@ -652,14 +655,8 @@ bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
 
 template <int DT, int LAYOUT>
 int launch_w4_layout(const GemmParams& p, hipStream_t s) {
-  const bool sit_out = p.mode == MODE_MASKED;
-  if (needs_tail(p, LAYOUT)) {
-    if constexpr (LAYOUT == W4_NT) {
-      if (sit_out) return launch_w4<DT, LAYOUT, true, true>(p, s);
-    }
-    return launch_w4<DT, LAYOUT, false, true>(p, s);
-  }
-  return sit_out ? launch_w4<DT, LAYOUT, true, false>(p, s) : launch_w4<DT, LAYOUT, false, false>(p, s);
+  if (needs_tail(p, LAYOUT)) return launch_w4<DT, LAYOUT, false, true>(p, s);
+  return p.mode == MODE_MASKED ? launch_w4<DT, LAYOUT, true, false>(p, s) : launch_w4<DT, LAYOUT, false, false>(p, s);
 }
 
 int launch_w4_16bit(const GemmParams& p, int dt, int layout, hipStream_t s) {
