@@ -643,6 +643,9 @@ bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   // a short K spends more on the slab that makes the tail's number even than the eight-wave kernel loses (4 groups of 13000 rows, N = 3096,
   // K = 512, [K, N]: 195 us there, 202 here; 16 of 1200, N = 3072, K = 536: 79 and 81)
   if (needs_tail(p, layout) && p.K < 768) return false;
+  // and so does, up to K = 1024, the launch that returns where only N is cut, whose slabs the eight-wave kernel has whole as well (17 random ones 1.014 of
+  // its time alone, up to 1.07; K = 1152-1500 0.995; K no multiple of 128: 0.98)
+  if (layout == W4_NN && p.K % 128 == 0 && p.K <= 1024 && needs_tail(p, layout) && w4_decided_on_device(p)) return false;
   if (w4_large(p)) return true;
   if (p.mode == MODE_MASKED || p.m_total < 128 * (int64_t)p.G) return false;
   int grid = num_cus();
