@@ -704,11 +704,11 @@ __global__ __launch_bounds__(CW::THREADS) void gemm_fast_auto_kernel(const GemmP
     static_assert(CS::THREADS == CW::THREADS && CS::SCHED_OFF == CW::SCHED_OFF && CS::SMEM_BYTES <= CW::SMEM_BYTES,
                   "the weight-streaming configuration shares the launch shape and the group table's place");
     static_assert(CW::THREADS >= kFastMaxGroups && CS::BM * 2 == CW::BM, "sched_init's half-height prefix is CS's");
-    stream = sched_short_tiles_pay<CW::BN>(p, sched, 10, 7);
-  }
-  if constexpr (!std::is_void<CS>::value) {
-    // the four-wave kernel, launched in front of this one, has taken the launch (GemmParams::wide_gate)
+    // the four-wave kernel, launched in front of this one, has taken the launch (GemmParams::wide_gate).  Asked before `stream` is known: the other
+    // order makes the compiler spill scalars in the narrow tiles' loop ([K, N], 4 groups of 325 rows, N = 3072, K = 4096: 80.4 us, this one 76.7; 8 of
+    // 300, N = 1024, K = 2048: 45.3 and 44.4)
     if (p.wide_gate == 2 && sched_wide_tiles_chosen<CW::BM, CW::BN>(p, sched)) return;
+    stream = sched_short_tiles_pay<CW::BN>(p, sched, 10, 7);
   }
   if (__builtin_expect(sched_num_tiles<CN::BM, CN::BN>(p, sched) > (int64_t)gridDim.x, 1)) {
     if constexpr (!std::is_void<CS>::value) {
