@@ -105,17 +105,31 @@ TGG_HD void sched_order_groups_serial(const GemmParams& p, Table& t) {
   for (int g = 0; g < p.G; ++g) t.tile0[sched_group_rank(t, p.G, g)] = g;
 }
 
+// Inclusive prefix sum over the wave's lanes, by moves between lanes inside the vector unit: within a row of sixteen first, then
+// the rows' totals.  (Exchanges through LDS take six dependent round trips of over a hundred cycles instead.)
+TGG_DEV int64_t sched_wave_scan(int64_t v) {
+#define TGG_SCAN_STEP(ctrl, rows) \
+  { \
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, ctrl, rows, 0xf, false); \
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)((uint64_t)v >> 32), ctrl, rows, 0xf, false); \
+    v += (int64_t)(((uint64_t)hi << 32) | lo); \
+  }
+  TGG_SCAN_STEP(0x111, 0xf)  // row_shr:1, 2, 4, 8: lanes whose source lies in front of the row add the zero
+  TGG_SCAN_STEP(0x112, 0xf)
+  TGG_SCAN_STEP(0x114, 0xf)
+  TGG_SCAN_STEP(0x118, 0xf)
+  TGG_SCAN_STEP(0x142, 0xa)  // row_bcast:15: a row's last lane to the next row, into rows 1 and 3
+  TGG_SCAN_STEP(0x143, 0xc)  // row_bcast:31: lane 31 to rows 2 and 3
+#undef TGG_SCAN_STEP
+  return v;
+}
+
 // Exclusive prefix sum over the workgroup's threads (in thread order) and the total; all threads must call it.
-// Wave-wide scan by lane exchange, the waves' totals through the table's scratch words.
+// Wave-wide scans, the waves' totals through the table's scratch words.
 template <class Table>
 TGG_DEV int64_t sched_block_scan(int64_t v, Table& t, int64_t& total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = ((int)blockDim.x + 63) >> 6;
-  int64_t inc = v;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int64_t o = __shfl_up(inc, d, 64);
-    if (lane >= d) inc += o;
-  }
+  const int64_t inc = sched_wave_scan(v);
   if (lane == 63) t.scan_[wave] = inc;
   __syncthreads();
   int64_t base = 0, tot = 0;
