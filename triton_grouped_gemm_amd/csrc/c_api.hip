@@ -24,6 +24,9 @@ static std::atomic<int> g_n_chunk{0};
 static std::atomic<int> g_kg_second_launch{1};
 static std::atomic<int> g_four_wave{1};  // 0 = eight-wave kernels only, 1 = four-wave kernel on large M-grouped NT launches (default), 2 = on every launch it can take
 
+static std::atomic<int> g_variant{0};  // as given to set_fast_variant and set_fp8_variant
+static std::atomic<int> g_deep{1};  // 0 = never the deep-ring kernel, 1 = on launches of few tiles (default), 2 = on every launch it can take
+
 int set_error(const char* fmt, ...) {
   va_list ap;
   va_start(ap, fmt);
@@ -58,6 +61,8 @@ int launch_scales_transpose(const float*, float*, int64_t, int, hipStream_t);
 int launch_cvt_fp8(const float*, void*, int64_t, int, hipStream_t);
 bool fast_supported(const GemmParams& p, int dt, int layout);
 int launch_fast_16bit(const GemmParams& p, int dt, int layout, hipStream_t s);
+bool deep_supported(const GemmParams& p, int dt, int layout, bool any_size);
+int launch_deep_16bit(const GemmParams& p, int dt, int layout, hipStream_t s);
 bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size);
 bool w4_decided_on_device(const GemmParams& p);
 int launch_w4_16bit(const GemmParams& p, int dt, int layout, hipStream_t s);
@@ -190,6 +195,10 @@ static GemmParams params_fp8_block(const void* Aq, const float* sa, const void* 
 
 static int dispatch_16bit(const GemmParams& p, int dt, int layout, hipStream_t s) {
   const int force_generic = g_force_generic.load(), four_wave = g_four_wave.load();
+  // a configuration of the other kernels that has been asked for stays what runs
+  if (const int deep = g_deep.load(); !force_generic && (deep == 2 || (deep == 1 && four_wave == 1 && g_variant.load() == 0)) &&
+                                      deep_supported(p, dt, layout, deep == 2))
+    return launch_deep_16bit(p, dt, layout, s);
   if (!force_generic && four_wave && w4_supported(p, dt, layout, four_wave == 2)) {
     if (!w4_decided_on_device(p) || four_wave == 2) return launch_w4_16bit(p, dt, layout, s);
     // whether 256-row tiles pay depends on the sizes; both kernels look at them and exactly one runs
@@ -745,10 +754,11 @@ int tgg_debug_row_tiles(const int64_t* sizes, int G, int mode, int64_t m_total, 
 
 int tgg_set_option(const char* key, int value) {
   if (key && strcmp(key, "force_generic") == 0) { g_force_generic = value != 0; return 0; }
-  if (key && strcmp(key, "variant") == 0) { set_fast_variant(value); set_fp8_variant(value); return 0; }
+  if (key && strcmp(key, "variant") == 0) { g_variant = value; set_fast_variant(value); set_fp8_variant(value); return 0; }
   if (key && strcmp(key, "tile_split") == 0) { g_tile_split = value != 0; return 0; }
   if (key && strcmp(key, "n_chunk") == 0) { g_n_chunk = value < 0 ? 0 : value; return 0; }
   if (key && strcmp(key, "kg_second_launch") == 0) { g_kg_second_launch = value != 0; return 0; }
+  if (key && strcmp(key, "deep") == 0) { g_deep = value < 0 ? 0 : (value > 2 ? 2 : value); return 0; }
   if (key && strcmp(key, "four_wave") == 0) { g_four_wave = value < 0 ? 0 : (value > 2 ? 2 : value); return 0; }
   if (key && strcmp(key, "store_nt") == 0) { g_store_nt = value != 0; return 0; }
   return set_error("unknown option '%s'", key ? key : "(null)");

@@ -77,7 +77,8 @@ constexpr int kSlabRowBytes = 128;  // a slab holds 128 bytes of every K-contigu
 //   !KMAJOR: 64 token rows of ROWS*2 bytes.  A copy instruction covers 1024 / (ROWS*2) token rows;
 //           chunk c of token row k sits at slot c ^ ((k % 4) * 4) ^ ((k / 8 % 2) * 2): the transposing fragment
 //           read of a wave touches token rows 8 g + e (g = 0..3, e = 0..3) at the same columns, and this spreads
-//           them over all banks.
+//           them over all banks.  Token rows of 128 bytes (ROWS = 64) take turns in the halves of the banks by
+//           themselves: chunk c sits at slot c ^ ((k / 2 % 2) * 4) ^ ((k / 8 % 2) * 2).
 template <int ROWS, bool KMAJOR> struct Operand {
   static constexpr int SLAB_BYTES = ROWS * kSlabRowBytes;
   static constexpr int NI = SLAB_BYTES / 1024;                 // copy instructions per slab
@@ -86,12 +87,14 @@ template <int ROWS, bool KMAJOR> struct Operand {
   static constexpr int RPI = 1024 / ROW_BYTES;                 // LDS rows per copy instruction
   static constexpr int NPAT = KMAJOR ? 2 : (RPI >= 16 ? 1 : 16 / RPI);  // swizzle patterns over instructions
 
+  static TGG_DEV int token_swizzle(int k) { return (CPR == 8 ? (k / 2 % 2) * 4 : (k % 4) * 4) ^ ((k / 8 % 2) * 2); }
+
   // byte offset (from the slab's first byte in global memory) fetched by `lane` of a copy
   // instruction with swizzle pattern `pat`; ld = bytes between consecutive global rows.
   static TGG_DEV int lane_voff(int lane, int pat, int ld) {
     const int r_local = lane / CPR, slot = lane % CPR;
     const int r = pat * RPI + r_local;  // row index modulo the swizzle period
-    const int sw = KMAJOR ? (r / 2) % 8 : ((r % 4) * 4) ^ ((r / 8 % 2) * 2);
+    const int sw = KMAJOR ? (r / 2) % 8 : token_swizzle(r);
     return r_local * ld + ((slot ^ sw) << 4);
   }
   // K-contiguous rows only: which 16-byte chunk of its row (0..7) that lane fetches
