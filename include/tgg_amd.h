@@ -83,6 +83,18 @@ int tgg_k_grouped_gemm_queued(const void* A, const void* B, void* C, const int32
 int tgg_k_grouped_gemm_sizes(const void* A, const void* B, void* C, const void* sizes, int sizes_i64, int G, int Mdim,
                              int N, int64_t Ktot, int dtype, int num_cu, int32_t* queue, void* stream);
 
+/* Launches of few outputs over many tokens, cut along K: a segment is computed in parts whose fp32 sums go to a workspace, and a second kernel adds
+ * them up in order and rounds once (which parts, the device decides from the sizes: the same sizes give the same bits).  split_bytes: how much
+ * workspace such a launch wants, 0 where cutting does not pay (fp8: 0 for the 16-bit entry point, 1 for the FP8 one).  The _split entry points are
+ * tgg_k_grouped_gemm_sizes and tgg_k_grouped_gemm_fp8_channel_queued with that workspace (16-byte aligned, in use until the call's kernels are done;
+ * null, or smaller than asked for: as without).  The reference has no counterpart. */
+int tgg_k_grouped_split_bytes(int G, int Mdim, int N, int64_t Ktot, int fp8, int num_cu, int64_t* bytes);
+int tgg_k_grouped_gemm_split(const void* A, const void* B, void* C, const void* sizes, int sizes_i64, int G, int Mdim, int N,
+                             int64_t Ktot, int dtype, int num_cu, int32_t* queue, void* workspace, int64_t workspace_bytes, void* stream);
+int tgg_k_grouped_gemm_fp8_channel_split(const void* x, const float* xs, const void* y, const float* ys, void* out,
+                                         const int32_t* tokens, int G, int M, int N, int64_t Ktot, int fmt_a, int fmt_b,
+                                         int num_cu, int32_t* queue, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* C = (Aq . Bq[g]^T) * a_scale[r] * b_scale[g*N+n].  Replaces gmm_fp8_act_per_channel_w_per_expert
  * (gemm/FP8/m_grouped_gemm_channel_expert.py:139-198). */
 int tgg_m_grouped_gemm_fp8_channel(const void* Aq, const float* a_scale, const void* Bq, const float* b_scale,
@@ -269,6 +281,7 @@ int tgg_debug_queue_order(int grid, int draws, int32_t* out);
  *                        16-bit K-grouped: launches of one and a half rounds of 256x256 tiles and more, but for segments of less than 32-96
  *                        tokens on few workgroups or without a queue;
  *                        FP8 K-grouped: all but outputs of up to 256 columns with 1000 tokens a group and more
+ *   "kg_split"      0/1  K-grouped launches may be cut along K where the caller brings a workspace (default 1)
  *   "deep"          int  the kernel for launches of few tiles (16-bit M-grouped / padded / placed / masked, up to 256 groups; 64x64, 64x128 or
  *                        128x128 tiles, chosen on the device from the sizes): 1 (default) = launches whose 128x128 tiles fit one round of
  *                        the workgroups, unless "variant" or "four_wave" asks for another kernel; 0 = never; 2 = on every launch that it can take

@@ -30,6 +30,9 @@ SIGNATURES = {
     "tgg_k_grouped_gemm": [_P, _P, _P, _P, _P, _I, _I, _I, _L, _I, _I, _P],
     "tgg_k_grouped_gemm_queued": [_P, _P, _P, _P, _P, _I, _I, _I, _L, _I, _I, _P, _P],
     "tgg_k_grouped_gemm_sizes": [_P, _P, _P, _P, _I, _I, _I, _I, _L, _I, _I, _P, _P],
+    "tgg_k_grouped_split_bytes": [_I, _I, _I, _L, _I, _I, _P],
+    "tgg_k_grouped_gemm_split": [_P, _P, _P, _P, _I, _I, _I, _I, _L, _I, _I, _P, _P, _L, _P],
+    "tgg_k_grouped_gemm_fp8_channel_split": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _L, _I, _I, _I, _P, _P, _L, _P],
     "tgg_m_grouped_gemm_fp8_channel": [_P, _P, _P, _P, _P, _P, _I, _I, _L, _I, _I, _I, _I, _I, _I, _P],
     "tgg_k_grouped_gemm_fp8_channel": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _L, _I, _I, _I, _P],
     "tgg_k_grouped_gemm_fp8_channel_queued": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _L, _I, _I, _I, _P, _P],
@@ -142,6 +145,13 @@ def work_queue(device: torch.device, queue: Optional[torch.Tensor] = None) -> to
     if q is None:
         q = _work_queues[key] = torch.zeros(QUEUE_WORDS, dtype=torch.int32, device=device)
     return q
+
+
+def split_workspace(groups: int, m: int, n: int, k_total: int, fp8: bool, num_cu: int, device: torch.device) -> Optional[torch.Tensor]:
+    """The workspace of a K-grouped launch that is to be cut along K, None where it is not (include/tgg_amd.h)."""
+    need = ctypes.c_int64()
+    call("tgg_k_grouped_split_bytes", groups, m, n, k_total, int(fp8), num_cu, ctypes.addressof(need))
+    return torch.empty(need.value, dtype=torch.uint8, device=device) if need.value else None
 
 
 def ptr(t) -> int:

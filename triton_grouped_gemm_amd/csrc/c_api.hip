@@ -22,6 +22,7 @@ static std::atomic<int> g_tile_split{1};
 static std::atomic<int> g_store_nt{1};
 static std::atomic<int> g_n_chunk{0};
 static std::atomic<int> g_kg_second_launch{1};
+static std::atomic<int> g_kg_split{1};
 static std::atomic<int> g_four_wave{1};  // 0 = eight-wave kernels only, 1 = four-wave kernel on large M-grouped NT launches (default), 2 = on every launch it can take
 
 static std::atomic<int> g_variant{0};  // as given to set_fast_variant and set_fp8_variant
@@ -68,8 +69,11 @@ bool w4_decided_on_device(const GemmParams& p);
 int launch_w4_16bit(const GemmParams& p, int dt, int layout, hipStream_t s);
 bool wgrad_supported(const GemmParams& p, int dt, bool any_size);
 bool fp8_w4_supported(const GemmParams& p, bool any_size);
+int64_t wgrad_split_bytes(const GemmParams& p, int dt);
+int64_t fp8_w4_split_bytes(const GemmParams& p);
 int launch_fp8_w4(const GemmParams& p, int ta, int tb, hipStream_t s);
 int launch_wgrad_16bit(const GemmParams& p, int dt, hipStream_t s);
+int kg_split_slots(const GemmParams& p);
 bool fast_quant_supported(const GemmParams& p, int dt, int layout);
 int launch_fast_16bit_quant(const GemmParams& p, int dt, int layout, hipStream_t s);
 void set_fast_variant(int v);
@@ -193,6 +197,13 @@ static GemmParams params_fp8_block(const void* Aq, const float* sa, const void* 
   return p;
 }
 
+// Lends a K-grouped launch the caller's workspace, where it is to be cut along K and the workspace has the room
+static void lend_workspace(GemmParams& p, int64_t need, void* workspace, int64_t bytes) {
+  if (need <= 0 || !workspace || bytes < need) return;
+  p.split_ws = (float*)workspace;
+  p.split_slots = kg_split_slots(p);
+}
+
 static int dispatch_16bit(const GemmParams& p, int dt, int layout, hipStream_t s) {
   const int force_generic = g_force_generic.load(), four_wave = g_four_wave.load();
   // a configuration of the other kernels that has been asked for stays what runs
@@ -208,7 +219,7 @@ static int dispatch_16bit(const GemmParams& p, int dt, int layout, hipStream_t s
     q.wide_gate = 2;
     return launch_fast_16bit(q, dt, layout, s);
   }
-  if (!force_generic && four_wave && layout == 2 && wgrad_supported(p, dt, four_wave == 2)) return launch_wgrad_16bit(p, dt, s);
+  if (!force_generic && four_wave && layout == 2 && (p.split_ws || wgrad_supported(p, dt, four_wave == 2))) return launch_wgrad_16bit(p, dt, s);
   if (!force_generic && fast_supported(p, dt, layout)) return launch_fast_16bit(p, dt, layout, s);
   return launch_generic_16bit(p, dt, layout, s);
 }
@@ -398,6 +409,33 @@ int tgg_k_grouped_gemm_sizes(const void* A, const void* B, void* C, const void* 
   return dispatch_16bit(p, dtype, 2, (hipStream_t)stream);
 }
 
+int tgg_k_grouped_split_bytes(int G, int Mdim, int N, int64_t Ktot, int fp8, int num_cu, int64_t* bytes) {
+  if (!bytes) return set_error("null result pointer");
+  *bytes = 0;
+  if (G < 1 || Mdim < 1 || N < 1 || Ktot < 0 || g_force_generic.load() || g_four_wave.load() != 1 || g_variant.load() != 0 || !g_kg_split.load()) return 0;
+  if (fp8) {
+    GemmParams p = params_fp8_k_channel(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, G, Mdim, N, Ktot, num_cu, nullptr);
+    if ((Ktot & 15) == 0 && fast_fp8_supported(p, false)) *bytes = fp8_w4_split_bytes(p);
+  } else {
+    *bytes = wgrad_split_bytes(params_k_grouped_sizes(nullptr, nullptr, nullptr, nullptr, 0, G, Mdim, N, Ktot, num_cu, nullptr), DT_BF16);
+  }
+  return 0;
+}
+
+int tgg_k_grouped_gemm_split(const void* A, const void* B, void* C, const void* sizes, int sizes_i64, int G, int Mdim, int N,
+                             int64_t Ktot, int dtype, int num_cu, int32_t* queue, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (int e = check_common(A, B, C, sizes, G, N, TGG_MAX_GROUPS)) return e;
+  if (Mdim < 1 || Ktot < 0) return set_error("bad Mdim=%d or Ktot=%lld", Mdim, (long long)Ktot);
+  if (dtype != TGG_BF16 && dtype != TGG_F16) return set_error("data type code %d not supported", dtype);
+  if ((Mdim & 7) || (N & 7)) return set_error("Mdim and N must be multiples of 8 (16-byte rows), got %d, %d", Mdim, N);
+  if (!aligned16(workspace)) return set_error("the workspace must be 16-byte aligned");
+  GemmParams p = params_k_grouped_sizes(A, B, C, sizes, sizes_i64, G, Mdim, N, Ktot, num_cu, queue);
+  int64_t need = 0;
+  if (int e = tgg_k_grouped_split_bytes(G, Mdim, N, Ktot, 0, num_cu, &need)) return e;
+  lend_workspace(p, need, workspace, workspace_bytes);
+  return dispatch_16bit(p, dtype, 2, (hipStream_t)stream);
+}
+
 static bool is_fp8(int f) { return f == TGG_E4M3 || f == TGG_E5M2; }
 
 int tgg_m_grouped_gemm_fp8_channel(const void* Aq, const float* a_scale, const void* Bq, const float* b_scale,
@@ -423,23 +461,34 @@ int tgg_k_grouped_gemm_fp8_channel(const void* x, const float* xs, const void* y
 int tgg_k_grouped_gemm_fp8_channel_queued(const void* x, const float* xs, const void* y, const float* ys, void* out,
                                           const int32_t* tokens, int G, int M, int N, int64_t Ktot, int fmt_a,
                                           int fmt_b, int num_cu, int32_t* queue, void* stream) {
+  return tgg_k_grouped_gemm_fp8_channel_split(x, xs, y, ys, out, tokens, G, M, N, Ktot, fmt_a, fmt_b, num_cu, queue, nullptr, 0, stream);
+}
+
+int tgg_k_grouped_gemm_fp8_channel_split(const void* x, const float* xs, const void* y, const float* ys, void* out,
+                                         const int32_t* tokens, int G, int M, int N, int64_t Ktot, int fmt_a, int fmt_b,
+                                         int num_cu, int32_t* queue, void* workspace, int64_t workspace_bytes, void* stream) {
   if (int e = check_common(x, y, out, tokens, G, N)) return e;
   if (!xs || !ys) return set_error("null scale pointer");
   if (M < 1 || Ktot < 0) return set_error("bad M=%d or Ktot=%lld", M, (long long)Ktot);
   if (!is_fp8(fmt_a) || !is_fp8(fmt_b)) return set_error("fp8 format codes must be E4M3 or E5M2");
   if (Ktot & 15) return set_error("Ktot must be a multiple of 16 for fp8 operands, got %lld", (long long)Ktot);
+  if (!aligned16(workspace)) return set_error("the workspace must be 16-byte aligned");
   GemmParams p = params_fp8_k_channel(x, xs, y, ys, out, tokens, G, M, N, Ktot, num_cu, queue);
+  int64_t need = 0;
+  if (int e = workspace ? tgg_k_grouped_split_bytes(G, M, N, Ktot, 1, num_cu, &need) : 0) return e;
+  lend_workspace(p, need, workspace, workspace_bytes);
   if (!g_force_generic.load() && fast_fp8_supported(p, false)) {
     // The tuned kernel needs every token count to be a multiple of 16 and only the device knows the counts: both
     // kernels are enqueued, each reads the counts first and exactly one of them runs (the other returns at once).
     p.kg_gate = 1;
-    if (const int four_wave = g_four_wave.load(); four_wave && fp8_w4_supported(p, four_wave == 2)) {
+    if (const int four_wave = g_four_wave.load(); four_wave && (p.split_ws || fp8_w4_supported(p, four_wave == 2))) {
       if (int e = launch_fp8_w4(p, fmt_a, fmt_b, (hipStream_t)stream)) return e;
     } else if (int e = launch_fast_fp8_channel(p, fmt_a, fmt_b, TGG_BF16, (hipStream_t)stream)) {
       return e;
     }
     if (!g_kg_second_launch.load()) return 0;
     p.kg_gate = 2;
+    p.split_ws = nullptr;
   }
   return launch_generic_fp8_channel(p, fmt_a, fmt_b, TGG_BF16, (hipStream_t)stream);
 }
@@ -758,6 +807,7 @@ int tgg_set_option(const char* key, int value) {
   if (key && strcmp(key, "tile_split") == 0) { g_tile_split = value != 0; return 0; }
   if (key && strcmp(key, "n_chunk") == 0) { g_n_chunk = value < 0 ? 0 : value; return 0; }
   if (key && strcmp(key, "kg_second_launch") == 0) { g_kg_second_launch = value != 0; return 0; }
+  if (key && strcmp(key, "kg_split") == 0) { g_kg_split = value != 0; return 0; }
   if (key && strcmp(key, "deep") == 0) { g_deep = value < 0 ? 0 : (value > 2 ? 2 : value); return 0; }
   if (key && strcmp(key, "four_wave") == 0) { g_four_wave = value < 0 ? 0 : (value > 2 ? 2 : value); return 0; }
   if (key && strcmp(key, "store_nt") == 0) { g_store_nt = value != 0; return 0; }

@@ -98,6 +98,8 @@ struct GemmParams {
   int tile_split;         // tuned kernels: 1 = per-XCD contiguous tile ranges (see sched_walk)
   int n_chunk;            // column tiles per chunk of the tile order, 0 = automatic (see sched_tile)
   int32_t* queue;         // K-grouped tuned kernels: tile-id counter in device memory (zero at launch), or null = static walk
+  float* split_ws;        // K-grouped four-wave kernels: workspace for the parts of segments cut along K (kg_split.hpp), or null
+  int split_slots;        // how many parts it has room for
   int store_nt;           // eight-wave kernels: 1 = non-temporal output stores
   // FP8 K-grouped by token counts: the tuned kernel copies 16-byte chunks, so it needs every count (hence every
   // segment start) to be a multiple of 16; the shape-agnostic kernel takes anything.  Only the device knows the

@@ -29,7 +29,7 @@
 // random ones: what bounds it is how fast 128-byte lines of distant rows come from HBM and L2, not power.  Without the touches
 // (below) 466 and 1474 us.
 #include "launch.hpp"
-#include "w4_common.hpp"
+#include "kg_split.hpp"
 
 namespace tgg {
 
@@ -42,7 +42,8 @@ struct Fp8W4Cfg {
   static constexpr int NEXT_OFF = SCHED_OFF + (((int)sizeof(SchedTableT<kFastMaxGroups>) + 255) & ~255);
   static constexpr int SCALE_OFF = NEXT_OFF + 256;  // the tile's row scales, then its column scales
   static constexpr int SINK_OFF = SCALE_OFF + (BM + BN) * 4;  // where touched lines' words go, 256 bytes a wave
-  static constexpr int SMEM_BYTES = SINK_OFF + 4 * 256;
+  static constexpr int META_OFF = SINK_OFF + 4 * 256;  // launches cut along K: what the table's entries are
+  static constexpr int SMEM_BYTES = META_OFF + kFastMaxGroups * 4;
   static_assert(STAGE_BYTES == 0x10000, "the slab buffers alternate by one address bit");
   static_assert(SMEM_BYTES <= 160 * 1024, "LDS budget");
 };
@@ -61,8 +62,11 @@ template <int OFF> TGG_DEV void read_frag8(i32x8_t& dst, uint32_t at0, uint32_t 
   dst = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-// FA / FB: 0 = e4m3fn, 1 = e5m2 (format codes of the f8f6f4 multiply)
-template <int FA, int FB, int OUT>
+typedef SplitCost<128, 2, 18, 8> Fp8SplitCost;
+
+// FA / FB: 0 = e4m3fn, 1 = e5m2 (format codes of the f8f6f4 multiply).  SPLIT: segments may be cut along K, see gemm_wgrad.hip; the
+// kernel that adds the parts up applies the scales.
+template <int FA, int FB, int OUT, bool SPLIT>
 __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmParams p) {
   typedef Fp8W4Cfg C;
   typedef Operand<256, true> Op;  // a slab of either operand: 256 rows of 128 bytes
@@ -70,7 +74,13 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   auto& sched = *reinterpret_cast<SchedTableT<kFastMaxGroups>*>(smem + C::SCHED_OFF);
   sched_init<C::BM>(p, sched);
-  if (!sched_kg_gate_open(p, sched)) return;
+  if (!sched_kg_gate_open(p, sched)) {
+    if (SPLIT && blockIdx.x == 0 && (int)threadIdx.x < p.G) reinterpret_cast<int32_t*>(p.split_ws)[2 * threadIdx.x + 1] = 0;  // there are no parts
+    return;
+  }
+  int32_t* const meta = SPLIT ? reinterpret_cast<int32_t*>(smem + C::META_OFF) : nullptr;
+  int groups = p.G;
+  if constexpr (SPLIT) groups = __builtin_amdgcn_readfirstlane(split_plan<Fp8SplitCost>(p, sched, meta, (int)((p.m_total + 255) / 256) * ((p.N + 255) / 256)));
 
   const uint32_t smem_addr = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
   const int lane = lane_id();
@@ -103,7 +113,7 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
   // ---- the copy stream -------------------------------------------------------------------------------------------------------
   // The cursor is two slabs ahead of the multiplies.  A tile's windows (descriptors) are fixed, the offset along K travels in the copies'
   // scalar offset, which the windows' range check counts in; chunks beyond the tile's range along K are not fetched.
-  const KgTiles<SchedTableT<kFastMaxGroups>> tiles(p, sched);
+  const KgTiles<SchedTableT<kFastMaxGroups>> tiles(p, sched, groups, meta);
   KgDraw draw(p, reinterpret_cast<int32_t*>(smem + C::NEXT_OFF), tiles.total, wave, lane);
   auto steps_of = [&](const KgTile& t) __attribute__((always_inline)) {
     const int steps = (t.klen + C::KS - 1) / C::KS;
@@ -355,9 +365,12 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
     }
     const int64_t rows_left = p.m_total - cur.m0 - wm0;
     pend_rs = make_rsrc32((uint64_t)p.C + (uint64_t)((((int64_t)cur.g * p.m_total + cur.m0 + wm0) * (int64_t)p.N + cur.n0 + wn0) * 2),
-                          rows_left > 0 ? (int)(rows_left < 128 ? rows_left : 128) * p.N * 2 : 0);
+                          rows_left > 0 && (!SPLIT || cur.slot < 0) ? (int)(rows_left < 128 ? rows_left : 128) * p.N * 2 : 0);
     pend_cols = p.N - cur.n0 - wn0;
     slab(I2(), I0(), pos);
+    if constexpr (SPLIT) {
+      if (cur.slot >= 0) store_part(acc, p.split_ws, (int64_t)cur.slot * tiles.per_group + (cur.m0 >> 8) * ((p.N + 255) >> 8) + (cur.n0 >> 8), wave, lane);
+    }
     touch_two(feed, part_of(following), 2 * C::KS);
     cur = following;
   }
@@ -368,13 +381,13 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
 #undef TGG_F8_EACH16
 }
 
-template <int FA, int FB, int OUT>
+template <int FA, int FB, int OUT, bool SPLIT>
 int launch_cfg(const GemmParams& p, hipStream_t s) {
   static bool attr_set[64] = {false};
   int dev = 0;
   (void)hipGetDevice(&dev);
   const bool listed = dev >= 0 && dev < 64;
-  auto kern = fp8_w4_kernel<FA, FB, OUT>;
+  auto kern = fp8_w4_kernel<FA, FB, OUT, SPLIT>;
   if (!listed || !attr_set[dev]) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Fp8W4Cfg::SMEM_BYTES) != hipSuccess)
       return check_launch("hipFuncSetAttribute(fp8_w4)");
@@ -401,9 +414,18 @@ bool fp8_w4_supported(const GemmParams& p, bool any_size) {
   return any_size || p.N > Fp8W4Cfg::BN || p.k_total < 1000 * (int64_t)p.G;
 }
 
+int64_t fp8_w4_split_bytes(const GemmParams& p) { return fp8_w4_supported(p, true) ? split_bytes(p, 4000, 16000) : 0; }
+
+template <bool SPLIT>
+static int launch_formats(const GemmParams& p, int ta, int tb, hipStream_t s) {
+  if (ta == DT_E4M3) return tb == DT_E4M3 ? launch_cfg<0, 0, DT_BF16, SPLIT>(p, s) : launch_cfg<0, 1, DT_BF16, SPLIT>(p, s);
+  return tb == DT_E4M3 ? launch_cfg<1, 0, DT_BF16, SPLIT>(p, s) : launch_cfg<1, 1, DT_BF16, SPLIT>(p, s);
+}
+
 int launch_fp8_w4(const GemmParams& p, int ta, int tb, hipStream_t s) {
-  if (ta == DT_E4M3) return tb == DT_E4M3 ? launch_cfg<0, 0, DT_BF16>(p, s) : launch_cfg<0, 1, DT_BF16>(p, s);
-  return tb == DT_E4M3 ? launch_cfg<1, 0, DT_BF16>(p, s) : launch_cfg<1, 1, DT_BF16>(p, s);
+  if (!p.split_ws) return launch_formats<false>(p, ta, tb, s);
+  if (int e = launch_formats<true>(p, ta, tb, s)) return e;
+  return launch_split_sum<DT_BF16, true>(p, s);
 }
 
 }  // namespace tgg

@@ -27,7 +27,7 @@
 // Tiles come from KgDraw (w4_common.hpp); the request for the tile after the next goes out four K steps before a tile's end, and its
 // answer, in order with the copies, has arrived by the wait that ends the tile.
 #include "launch.hpp"
-#include "w4_common.hpp"
+#include "kg_split.hpp"
 
 namespace tgg {
 
@@ -43,16 +43,21 @@ struct WgradCfg {
   static constexpr int NEXT_OFF = SCHED_OFF + (((int)sizeof(SchedTableT<kFastMaxGroups>) + 255) & ~255);  // drawn tile ids, two words
   static constexpr int EPI_OFF = NEXT_OFF + 256;
   static constexpr int SINK_OFF = EPI_OFF + 4 * EPI_WAVE_BYTES;  // where touched lines' words go, 256 bytes a wave
-  static constexpr int SMEM_BYTES = SINK_OFF + 4 * 256;
+  static constexpr int META_OFF = SINK_OFF + 4 * 256;  // launches cut along K: what the table's entries are
+  static constexpr int SMEM_BYTES = META_OFF + kFastMaxGroups * 4;
   static constexpr int TOUCH = 256;  // tokens of the next tile that are touched
   static_assert(SMEM_BYTES <= 160 * 1024, "LDS budget");
   static_assert(TOUCH >= KS && TOUCH >= BM / 2, "wgrad_supported bounds the slab's and the stores' windows by the touched rows'");
 };
 
+typedef SplitCost<64, 3, 20, 8> WgradSplitCost;
+
 // NT: see store_b128.  128 groups of 2048 x N, operands in no cache, 32 / 128 / 256 / 1024 tokens a group: N = 1544 non-temporal 463 / 456 /
 // 444 / 888 us, else 202 / 236 / 314 / 823 (the eight-wave kernel, non-temporal: 435 / 392 / 400 / 967); N = 1552 379 / 374 / 357 / 855 and 199 / 231 /
 // 310 / 814; N = 1568, whole 64 bytes, 184 / 194 / 306 / 800 and 188 / 227 / 310 / 811; N = 1536 146 / 167 / 252 / 688 and 165 / 191 / 272 / 703.
-template <int DT, bool NT>
+// SPLIT: segments may be cut along K (kg_split.hpp).  An instantiation of its own: tiles of parts leave as fp32 behind their last K step
+// (they are long), and the plain one needs no look at what a tile is.
+template <int DT, bool NT, bool SPLIT>
 __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const GemmParams p) {
   typedef WgradCfg C;
   typedef Operand<256, false> Op;  // a slab of either operand: token rows of 512 bytes (here 32 of them)
@@ -60,6 +65,9 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   auto& sched = *reinterpret_cast<SchedTableT<kFastMaxGroups>*>(smem + C::SCHED_OFF);
   sched_init<C::BM>(p, sched);
+  int32_t* const meta = SPLIT ? reinterpret_cast<int32_t*>(smem + C::META_OFF) : nullptr;
+  int groups = p.G;
+  if constexpr (SPLIT) groups = __builtin_amdgcn_readfirstlane(split_plan<WgradSplitCost>(p, sched, meta, (int)((p.m_total + 255) / 256) * ((p.N + 255) / 256)));
 
   const uint32_t smem_addr = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
   const int lane = lane_id();
@@ -85,7 +93,7 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
     b_rd[i] = smem_addr + C::OP_BYTES + row + ((((wn0 + 16 * i) / 8 + (c >> 1)) ^ sw) << 4);
   }
 
-  const KgTiles<SchedTableT<kFastMaxGroups>> tiles(p, sched);
+  const KgTiles<SchedTableT<kFastMaxGroups>> tiles(p, sched, groups, meta);
   KgDraw draw(p, reinterpret_cast<int32_t*>(smem + C::NEXT_OFF), tiles.total, wave, lane);
   auto steps_of = [&](const KgTile& t) __attribute__((always_inline)) {
     const int steps = (t.klen + 2 * C::KS - 1) / (2 * C::KS) * 2;
@@ -326,10 +334,13 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
     // what the tile's last K step, the next tile's first and a flush store
     const int64_t rows_left = p.m_total - cur.m0 - wm0;
     pend_rs = make_rsrc32((uint64_t)p.C + (uint64_t)((((int64_t)cur.g * p.m_total + cur.m0 + wm0) * (int64_t)p.N + cur.n0 + wn0) * 2),
-                          rows_left > 0 ? (int)(rows_left < 128 ? rows_left : 128) * p.N * 2 : 0);
+                          rows_left > 0 && (!SPLIT || cur.slot < 0) ? (int)(rows_left < 128 ? rows_left : 128) * p.N * 2 : 0);
     pend_cols = p.N - cur.n0 - wn0;
     kstep(I0(), I0(), W16());
     kstep(I1(), I2(), W32());
+    if constexpr (SPLIT) {
+      if (cur.slot >= 0) store_part(acc, p.split_ws, (int64_t)cur.slot * tiles.per_group + (cur.m0 >> 8) * ((p.N + 255) >> 8) + (cur.n0 >> 8), wave, lane);
+    }
     draw.take(pos + 2);
     asm volatile("s_barrier" ::: "memory");
     cur = following;
@@ -339,13 +350,13 @@ __global__ __launch_bounds__(WgradCfg::THREADS) void gemm_wgrad_kernel(const Gem
   wait_vmcnt<0>();  // trailing zero-length copies still write LDS
 }
 
-template <int DT, bool NT>
+template <int DT, bool NT, bool SPLIT>
 int launch_wgrad(const GemmParams& p, hipStream_t s) {
   static bool attr_set[64] = {false};
   int dev = 0;
   (void)hipGetDevice(&dev);
   const bool listed = dev >= 0 && dev < 64;
-  auto kern = gemm_wgrad_kernel<DT, NT>;
+  auto kern = gemm_wgrad_kernel<DT, NT, SPLIT>;
   if (!listed || !attr_set[dev]) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, WgradCfg::SMEM_BYTES) != hipSuccess)
       return check_launch("hipFuncSetAttribute(gemm_wgrad)");
@@ -384,9 +395,19 @@ bool wgrad_supported(const GemmParams& p, int dt, bool any_size) {
   return 2 * p.G * tiles_m * tiles_n >= 3 * (int64_t)grid;
 }
 
+int64_t wgrad_split_bytes(const GemmParams& p, int dt) { return wgrad_supported(p, dt, true) ? split_bytes(p, 2000, 6400) : 0; }
+
+int kg_split_slots(const GemmParams& p) { return split_room(p).slots; }
+
 int launch_wgrad_16bit(const GemmParams& p, int dt, hipStream_t s) {
-  if (rows_of_whole_64_bytes(p)) return dt == DT_BF16 ? launch_wgrad<DT_BF16, true>(p, s) : launch_wgrad<DT_F16, true>(p, s);
-  return dt == DT_BF16 ? launch_wgrad<DT_BF16, false>(p, s) : launch_wgrad<DT_F16, false>(p, s);
+  if (p.split_ws) {
+    const bool whole = rows_of_whole_64_bytes(p);
+    if (int e = dt == DT_BF16 ? (whole ? launch_wgrad<DT_BF16, true, true>(p, s) : launch_wgrad<DT_BF16, false, true>(p, s))
+                              : (whole ? launch_wgrad<DT_F16, true, true>(p, s) : launch_wgrad<DT_F16, false, true>(p, s))) return e;
+    return dt == DT_BF16 ? launch_split_sum<DT_BF16, false>(p, s) : launch_split_sum<DT_F16, false>(p, s);
+  }
+  if (rows_of_whole_64_bytes(p)) return dt == DT_BF16 ? launch_wgrad<DT_BF16, true, false>(p, s) : launch_wgrad<DT_F16, true, false>(p, s);
+  return dt == DT_BF16 ? launch_wgrad<DT_BF16, false, false>(p, s) : launch_wgrad<DT_F16, false, false>(p, s);
 }
 
 }  // namespace tgg

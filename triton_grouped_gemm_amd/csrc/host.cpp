@@ -189,10 +189,15 @@ PyObject* k_grouped_gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   {
     const Unlocked unlocked;
     c = at::empty({g, m, n}, a.options());
-    rc = tgg_k_grouped_gemm_sizes(a.data_ptr(), b.data_ptr(), c.data_ptr(), sizes.data_ptr(), is64(sizes), (int)g, (int)m, (int)n, kt,
-                                  dt, (int)num_cu, (int32_t*)queue.data_ptr(), stream());
+    at::Tensor workspace;  // of launches that are cut along K; the allocator keeps it for the stream's next ones
+    int64_t bytes = 0;
+    rc = tgg_k_grouped_split_bytes((int)g, (int)m, (int)n, kt, 0, (int)num_cu, &bytes);
+    if (bytes > 0) workspace = at::empty({bytes}, a.options().dtype(at::kByte));
+    if (rc == 0)
+      rc = tgg_k_grouped_gemm_split(a.data_ptr(), b.data_ptr(), c.data_ptr(), sizes.data_ptr(), is64(sizes), (int)g, (int)m, (int)n, kt, dt,
+                                    (int)num_cu, (int32_t*)queue.data_ptr(), bytes > 0 ? workspace.data_ptr() : nullptr, bytes, stream());
   }
-  return done("tgg_k_grouped_gemm_sizes", rc, c);
+  return done("tgg_k_grouped_gemm_split", rc, c);
   END_HANDLE_TH_ERRORS
 }
 

@@ -60,6 +60,7 @@ template <int N, class F> TGG_DEV void for_each(const F& f) { for_each_of(f, std
 // values fixed for the launch done on the scalar unit.
 struct KgTile {
   int g, m0, n0;  // g = -1: there are no more tiles
+  int slot;       // launches cut along K (kg_split.hpp): the part's place in the workspace, -1: the group is in one part
   int klen;       // tokens of the segment
   int64_t k0;     // its first token
 };
@@ -69,14 +70,16 @@ struct KgTiles {
   const Table& t;
   int tiles_m, nc, full_chunks, tail_width, per_group, total;
   FixedDiv by_group, by_chunk, by_nc, by_tail;
-  TGG_DEV KgTiles(const GemmParams& p, const Table& t_)
+  const int32_t* meta;  // launches cut along K: what part an entry of the table is, else null
+  TGG_DEV KgTiles(const GemmParams& p, const Table& t_, int groups, const int32_t* meta_)
       : t(t_), tiles_m((int)((p.m_total + 255) / 256)), nc(sched_chunk_width((p.N + 255) / 256, p.n_chunk)),
         full_chunks((p.N + 255) / 256 / nc), tail_width((p.N + 255) / 256 - full_chunks * nc), per_group(tiles_m * ((p.N + 255) / 256)),
-        total(p.G * per_group), by_group(per_group), by_chunk(tiles_m * nc), by_nc(nc), by_tail(tail_width > 0 ? tail_width : 1) {}
+        total(groups * per_group), by_group(per_group), by_chunk(tiles_m * nc), by_nc(nc), by_tail(tail_width > 0 ? tail_width : 1), meta(meta_) {}
   TGG_DEV KgTile look_up(int id) const {
     KgTile r;
     r.g = -1;
     r.m0 = r.n0 = r.klen = 0;
+    r.slot = -1;
     r.k0 = 0;
     if (id < total) {
       const int slot = (int)by_group.div((uint32_t)id), at = id - slot * per_group;
@@ -90,6 +93,11 @@ struct KgTiles {
       r.g = __builtin_amdgcn_readfirstlane(t.tile0[slot]);
       r.klen = __builtin_amdgcn_readfirstlane(t.rows[r.g]);
       r.k0 = (int64_t)uniform64((uint64_t)t.row0[r.g]);
+      if (meta) {
+        const int part = __builtin_amdgcn_readfirstlane(meta[r.g]);
+        r.g = part & 0xffff;
+        r.slot = (part >> 16) - 1;
+      }
     }
     return r;
   }

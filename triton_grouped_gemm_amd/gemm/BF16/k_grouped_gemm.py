@@ -66,9 +66,11 @@ def k_grouped_gemm(A: Tensor, B: Tensor, size_per_group: Tensor, group_start: Op
     if group_start is None or group_end is None:
         # the kernel makes the segments' starts itself (five launches of 5 us when torch makes them)
         sizes = size_per_group.contiguous()
-        _native.call("tgg_k_grouped_gemm_sizes", A.data_ptr(), B.data_ptr(), C.data_ptr(), sizes.data_ptr(),
+        workspace = _native.split_workspace(num_groups, M_DIM, N_DIM, K_TOTAL, False, int(numSM), A.device)
+        _native.call("tgg_k_grouped_gemm_split", A.data_ptr(), B.data_ptr(), C.data_ptr(), sizes.data_ptr(),
                      int(sizes.dtype == torch.int64), num_groups, M_DIM, N_DIM, K_TOTAL, _dtype_code(A.dtype),
-                     int(numSM), queue.data_ptr(), _native.stream_of(A))
+                     int(numSM), queue.data_ptr(), _native.ptr(workspace), 0 if workspace is None else workspace.numel(),
+                     _native.stream_of(A))
         return C
     group_start = group_start.to(device=A.device, dtype=torch.int32).contiguous()
     group_end = group_end.to(device=A.device, dtype=torch.int32).contiguous()

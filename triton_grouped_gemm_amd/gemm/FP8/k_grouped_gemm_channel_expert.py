@@ -45,8 +45,9 @@ def matmul(x_fp8: Tensor, x_scale: Tensor, y_fp8: Tensor, y_scale: Tensor, token
     output = torch.empty((num_groups, M, N), dtype=torch.bfloat16, device=x_fp8.device)
     # tile-id counter of the kernel's work queue (a tile costs what its group has tokens; see include/tgg_amd.h)
     queue = _native.work_queue(x_fp8.device, queue)
-    _native.call("tgg_k_grouped_gemm_fp8_channel_queued", x_fp8.data_ptr(), xs.data_ptr(), y_fp8.data_ptr(),
+    workspace = _native.split_workspace(num_groups, M, N, K, True, -1, x_fp8.device)
+    _native.call("tgg_k_grouped_gemm_fp8_channel_split", x_fp8.data_ptr(), xs.data_ptr(), y_fp8.data_ptr(),
                  ys.data_ptr(), output.data_ptr(), tokens.data_ptr(), num_groups, M, N, K,
                  _FMT.get(int(dtype_a), _native.E5M2), _FMT.get(int(dtype_b), _native.E5M2), -1, queue.data_ptr(),
-                 _native.stream_of(x_fp8))
+                 _native.ptr(workspace), 0 if workspace is None else workspace.numel(), _native.stream_of(x_fp8))
     return output
