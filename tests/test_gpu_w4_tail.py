@@ -127,3 +127,19 @@ def test_the_default_route_of_masked_launches(dtype, K, masked, wide):
     for g, n in enumerate(masked):
         block = out[g * slots:(g + 1) * slots]
         assert not bool(torch.isnan(block[:n]).any()) and bool(torch.isnan(block[n:]).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("num_cu", [8, 3, 1])  # full and half tiles in every order, in one workgroup
+@pytest.mark.parametrize("K", [256, 320, 512])
+@pytest.mark.parametrize("N, trans_b", [(520, True), (512, False), (264, False)])
+@pytest.mark.parametrize("sizes", [[128, 1, 64, 65], [129, 384, 16, 200, 300, 127, 640], [256, 17, 256, 0, 385]])
+def test_half_tiles(dtype, num_cu, K, N, trans_b, sizes):
+    """Tiles of at most 128 rows beside full ones: 64 rows per wave row, a part of them or none."""
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(K + N)
+    s = torch.tensor(sizes, dtype=torch.int32, device=dev)
+    a = torch.randn(sum(sizes), K, device=dev, generator=gen).to(dtype)
+    b = (torch.randn(len(sizes), *((N, K) if trans_b else (K, N)), device=dev, generator=gen) * K ** -0.5).to(dtype)
+    run = lambda: m_grouped_gemm(a, b, s, trans_b, numSM=num_cu)
+    assert torch.equal(_with("four_wave", 2, 1, run), _with("force_generic", 1, 0, run))

@@ -298,3 +298,41 @@ def test_k_grouped_four_wave_kernels(stem):
                         ("accumulator reads too close behind the multiply", accumulator_reads_too_early(text.replace(kernel, "gemm_w4_kernel")))):
         assert not found, f"{len(found)} {what}, first: {found[0]}"
     assert "scratch_" not in text  # a spilled value would be reloaded behind the copies
+
+
+# The four-wave kernel names its fragments (v[64:191]), staged chunks (v[192:255]) and accumulators (all AGPRs) in the text of its own statements;
+# the compiler, which knows nothing of what they hold, must not use any of them itself.
+def compiler_uses_of_named_registers(text: str):
+    stray, inside, ours = [], False, False
+    for raw in text.splitlines():
+        if "#ASMSTART" in raw or "#ASMEND" in raw:
+            ours = "#ASMSTART" in raw
+            continue
+        line = raw.split(";")[0].strip()
+        if line.endswith(":") and not line.startswith("."):
+            inside = "gemm_w4_kernel" in line
+            continue
+        if not inside or ours or not line or line.startswith("."):
+            continue
+        toks = [t.strip(",") for t in line.split()[1:]]
+        if any(_regs(t, "a") or any(r >= 64 for r in _regs(t, "v")) for t in toks):
+            stray.append(line)
+    return stray
+
+
+def test_named_register_scanner_on_snippets():
+    head = "_ZN3tgg14gemm_w4_kernelILi0ELi0EEEvNS_10GemmParamsE:\n"
+    assert compiler_uses_of_named_registers(head + "v_mov_b32_e32 v63, v3\n") == []
+    assert compiler_uses_of_named_registers(head + ";#ASMSTART\nds_read_b128 v[64:67], v3 offset:0\n;#ASMEND\n") == []
+    assert len(compiler_uses_of_named_registers(head + "v_mov_b32_e32 v64, v3\n")) == 1
+    assert len(compiler_uses_of_named_registers(head + "v_accvgpr_write_b32 a0, v3\n")) == 1
+    assert len(compiler_uses_of_named_registers(head + "v_mov_b64_e32 v[62:63], v[190:191]\n")) == 1
+    assert compiler_uses_of_named_registers("other_kernel:\nv_mov_b32_e32 v200, v3\n") == []
+
+
+def test_four_wave_kernel_leaves_its_named_registers_alone():
+    f = BUILD / "gemm_w4.gfx950.s"
+    if not f.exists():
+        pytest.skip("no device assembly in the build directory (the library was built elsewhere or not yet)")
+    stray = compiler_uses_of_named_registers(f.read_text())
+    assert not stray, f"{len(stray)} compiler-generated uses, first: {stray[0]}"

@@ -28,6 +28,12 @@
 // the LDS writes cost more than that copy would.  The slabs of all of a workgroup's tiles form one stream; each
 // of the two cursors carries the buffer descriptor of its tile's window and an offset along K.
 //
+// A tile of at most 128 rows (a group's last one, mostly) is a half tile: the two wave rows take 64 rows each, four row blocks per wave, and a K step is 32
+// multiplies; its results leave behind its last K step.  So that a wave's fragments may lie elsewhere in the two kinds, all fragments and
+// accumulators are named registers.  Before, the zeros that such a tile's windows deliver were multiplied (masked launches: waves without rows
+// sat the tile out).  128 groups, 32768 rows, same box: N = 1536, K = 2048 274 -> 265 us, as [K, N] N = 2048, K = 1536 287 -> 278; 32 groups,
+// 16384 rows, N = 2048, K = 2880 220 -> 215; headline and masked decode the same.
+//
 // The epilogue rides on multiplies: the upper half of a wave's block is converted and stored between the multiplies
 // of the tile's last K step, the lower half between those of the next tile's first K step, whose multiplies start
 // from a zero addend instead of the accumulators (see "epilogue" below).  With B as [G, N, K] the results never pass
@@ -46,12 +52,11 @@
 // the two runs (GemmParams::wide_gate); everything else goes to the eight-wave kernels.
 //
 // What the compiler does not know about assembly statements, and how it is handled here:
-//   * a fragment read's result arrives later: every register a read targets passes through the wait statement
-//     ("+v") before a multiply may use it;
+//   * fragments and accumulators are named in the instruction text and waited for by the K step's wait statement; the compiler's own allocation
+//     is kept below them (amdgpu_num_vgpr; tests/test_isa_hazards.py scans the kept assembly for any other use);
 //   * the A chunks are in flight across loop iterations and paths that join: their registers (v[192:255]) are named
-//     in the instruction text and listed as clobbered, the compiler never holds a value in them
-//     (tests/test_isa_hazards.py scans the kept assembly for any other use);
-//   * the multiplies write AGPRs: compiled code (the epilogue's conversions) reads a block's accumulators no sooner
+//     in the instruction text too;
+//   * the multiplies write AGPRs: the epilogue's conversions read a block's accumulators no sooner
 //     than three multiplies after the multiply that wrote them (a multiply takes 16 cycles to issue and delivers
 //     within two more), except where a flush follows a tile directly: there the last row block's accumulators pass
 //     through a statement of idle cycles first.  Accumulators are never the target of a load.
@@ -64,6 +69,43 @@ namespace {
 
 enum : int { W4_NT = 0, W4_NN = 1 };
 constexpr int BK4 = 64;
+
+#define TGG_W4_ACC_CLOBBER "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", "a10", "a11", "a12", "a13", "a14", "a15", "a16", "a17", "a18", "a19", "a20", "a21", \
+  "a22", "a23", "a24", "a25", "a26", "a27", "a28", "a29", "a30", "a31", "a32", "a33", "a34", "a35", "a36", "a37", "a38", "a39", "a40", "a41", "a42", "a43", \
+  "a44", "a45", "a46", "a47", "a48", "a49", "a50", "a51", "a52", "a53", "a54", "a55", "a56", "a57", "a58", "a59", "a60", "a61", "a62", "a63", "a64", "a65", \
+  "a66", "a67", "a68", "a69", "a70", "a71", "a72", "a73", "a74", "a75", "a76", "a77", "a78", "a79", "a80", "a81", "a82", "a83", "a84", "a85", "a86", "a87", \
+  "a88", "a89", "a90", "a91", "a92", "a93", "a94", "a95", "a96", "a97", "a98", "a99", "a100", "a101", "a102", "a103", "a104", "a105", "a106", "a107", "a108", "a109", \
+  "a110", "a111", "a112", "a113", "a114", "a115", "a116", "a117", "a118", "a119", "a120", "a121", "a122", "a123", "a124", "a125", "a126", "a127", "a128", "a129", "a130", "a131", \
+  "a132", "a133", "a134", "a135", "a136", "a137", "a138", "a139", "a140", "a141", "a142", "a143", "a144", "a145", "a146", "a147", "a148", "a149", "a150", "a151", "a152", "a153", \
+  "a154", "a155", "a156", "a157", "a158", "a159", "a160", "a161", "a162", "a163", "a164", "a165", "a166", "a167", "a168", "a169", "a170", "a171", "a172", "a173", "a174", "a175", \
+  "a176", "a177", "a178", "a179", "a180", "a181", "a182", "a183", "a184", "a185", "a186", "a187", "a188", "a189", "a190", "a191", "a192", "a193", "a194", "a195", "a196", "a197", \
+  "a198", "a199", "a200", "a201", "a202", "a203", "a204", "a205", "a206", "a207", "a208", "a209", "a210", "a211", "a212", "a213", "a214", "a215", "a216", "a217", "a218", "a219", \
+  "a220", "a221", "a222", "a223", "a224", "a225", "a226", "a227", "a228", "a229", "a230", "a231", "a232", "a233", "a234", "a235", "a236", "a237", "a238", "a239", "a240", "a241", \
+  "a242", "a243", "a244", "a245", "a246", "a247", "a248", "a249", "a250", "a251", "a252", "a253", "a254", "a255"
+#define TGG_W4_I(k) std::integral_constant<int, (k)>()
+
+// Registers by number (see "fragments and accumulators"): FA, FB the fragments' first VGPR, AT the accumulators' first AGPR.
+template <int DT, bool FRESH, int AT, int X, int Y> TGG_DEV void acc_mfma() {
+  if constexpr (DT == DT_BF16 && FRESH) asm volatile("v_mfma_f32_16x16x32_bf16 a[%c0:%c1], v[%c2:%c3], v[%c4:%c5], 0" : : "n"(AT), "n"(AT + 3), "n"(X), "n"(X + 3), "n"(Y), "n"(Y + 3));
+  else if constexpr (DT == DT_BF16) asm volatile("v_mfma_f32_16x16x32_bf16 a[%c0:%c1], v[%c2:%c3], v[%c4:%c5], a[%c0:%c1]" : : "n"(AT), "n"(AT + 3), "n"(X), "n"(X + 3), "n"(Y), "n"(Y + 3));
+  else if constexpr (FRESH) asm volatile("v_mfma_f32_16x16x32_f16 a[%c0:%c1], v[%c2:%c3], v[%c4:%c5], 0" : : "n"(AT), "n"(AT + 3), "n"(X), "n"(X + 3), "n"(Y), "n"(Y + 3));
+  else asm volatile("v_mfma_f32_16x16x32_f16 a[%c0:%c1], v[%c2:%c3], v[%c4:%c5], a[%c0:%c1]" : : "n"(AT), "n"(AT + 3), "n"(X), "n"(X + 3), "n"(Y), "n"(Y + 3));
+}
+template <int V, int OFF> TGG_DEV void frag_read_b128(uint32_t addr) {
+  asm volatile("ds_read_b128 v[%c1:%c2], %0 offset:%c3" : : "v"(addr), "n"(V), "n"(V + 3), "n"(OFF) : "memory");
+}
+template <int V, int OFF0, int OFF1> TGG_DEV void frag_read_tr(uint32_t addr) {  // two transposing 8-byte reads (K 0..3 and 4..7 of the lane's column)
+  asm volatile("ds_read_b64_tr_b16 v[%c1:%c2], %0 offset:%c5\n\tds_read_b64_tr_b16 v[%c3:%c4], %0 offset:%c6"
+               : : "v"(addr), "n"(V), "n"(V + 1), "n"(V + 2), "n"(V + 3), "n"(OFF0), "n"(OFF1) : "memory");
+}
+template <int AT> TGG_DEV float acc_read() {
+  float v;
+  asm volatile("v_accvgpr_read_b32 %0, a%c1" : "=v"(v) : "n"(AT));
+  return v;
+}
+template <int AT> TGG_DEV void acc_zero() {
+  asm volatile("v_accvgpr_write_b32 a%c0, 0\n\tv_accvgpr_write_b32 a%c1, 0\n\tv_accvgpr_write_b32 a%c2, 0\n\tv_accvgpr_write_b32 a%c3, 0" : : "n"(AT), "n"(AT + 1), "n"(AT + 2), "n"(AT + 3));
+}
 
 struct W4Cfg {
   static constexpr int BM = 256, BN = 256, NWAVES = 4, THREADS = 256;
@@ -82,19 +124,14 @@ struct W4Cfg {
 // A is the operand that takes the long way through registers ("staged", s), B is copied straight to LDS ("direct",
 // d).  Staging B instead makes no difference even where the weights are what streams from memory (masked decode:
 // 0.526 ms either way).
-// SIT_OUT: a wave whose block of a tile has no rows or no columns multiplies nothing in that tile (it keeps its share
-// of the copy stream and the barriers going).  Worth 2 % where a quarter of the tiles have at most 128 rows (masked
-// decode); where nearly every tile is full the branch per K step costs the others 1 %, and such a wave multiplies
-// the zeros its windows deliver.
 // TAIL: K is any multiple of 8 from 192 on, and N, for B as [G, K, N], any multiple of 8.  A tile's last slabs are cut short (or
 // added, for an even number of four at least): lanes whose chunk of a K-contiguous row starts at or beyond K get an out-of-range
 // offset, and token rows beyond K lie behind the window's end.  An instantiation of its own: the plain one needs no mask.
-template <int DT, int LAYOUT, bool SIT_OUT, bool TAIL>
-__global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParams p) {
+template <int DT, int LAYOUT, bool TAIL>
+__global__ __launch_bounds__(W4Cfg::THREADS) __attribute__((amdgpu_num_vgpr(64))) void gemm_w4_kernel(const GemmParams p) {
   typedef W4Cfg C;
   constexpr int S_OFF = 0, D_OFF = C::A_BYTES;  // the operands' places in a slab buffer
   constexpr bool B_KMAJOR = LAYOUT == W4_NT;  // NN: B is [G, K, N], its slab 64 token rows of 512 bytes
-  static_assert(!(SIT_OUT && TAIL), "masked launches with a tail are the eight-wave kernels' (w4_supported)");
   typedef Operand<C::BM, true> Op;            // the A slab, and B's when K-contiguous: 256 rows of 128 bytes
   typedef Operand<C::BN, B_KMAJOR> OpB;
 
@@ -109,39 +146,40 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
   const uint32_t smem_addr = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm0 = (wave >> 1) * 128, wn0 = (wave & 1) * 128;
+  const int wave_m = wave >> 1, wn0 = (wave & 1) * 128;
   const int l16 = lane & 15, lg = lane >> 4;
 
   const int ld = p.K * 2;  // row pitch of A and of B in bytes; K is a multiple of 128 (w4_supported) unless TAIL
   const int kt_all = TAIL ? max(4, (p.K + 2 * BK4 - 1) / (2 * BK4) * 2) : p.K / BK4;  // slabs per tile
   // Copy k (0..7) of an operand's slab by this wave is copy instruction wave + 4 k of the slab: rows 8 (wave + 4 k) ...
-  // + 7.  Its per-lane source offset within the tile's window is fixed for the launch; the slab's offset along K
-  // travels in the instruction's scalar offset, which the range check of the window counts in: rows behind the valid ones stay behind its end.
-  int vo[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) vo[k] = Op::lane_voff(lane, wave % Op::NPAT, ld) + (wave + 4 * k) * Op::RPI * ld;
+  // + 7.  The per-lane source offset of copy 0 within the tile's window is fixed for the launch; the others' distance from it and the slab's offset along
+  // K travel in the instruction's scalar offset, which the range check of the window counts in: rows behind the valid ones stay behind its end.
+  const int vo = Op::lane_voff(lane, wave % Op::NPAT, ld) + wave * Op::RPI * ld;
   static_assert(Op::NPAT == 2, "the swizzle pattern of copy wave + 4 k is that of copy wave");
   // NN: B's copies have offsets of their own (two token rows of 512 bytes per copy, row pitch 2 N)
   const int ld_b = (B_KMAJOR ? p.K : p.N) * 2;
   // NT: B's rows land in LDS permuted: LDS row 128 h + 16 j + c of the slab (column block j of a wave's half h, lane
   // column c of the multiply) holds column 128 h + 8 c + j of the tile, so that a lane's results of the eight column
   // blocks are eight neighbouring outputs of a row and leave as one 16-byte store without passing through LDS.
-  int vo_b[8];
+  // LDS row 8 (wave + 4 k) + lane / 8: h = k / 4, j = 2 (k % 4) + wave / 2, c = 8 (wave % 2) + lane / 8
+  // (NN: two swizzle patterns, of the even and the odd copies)
+  int vo_b[B_KMAJOR ? 1 : 2];
+  if (B_KMAJOR) {
+    vo_b[0] = Op::lane_voff(lane, wave % Op::NPAT, ld) + (8 * (8 * (wave & 1) + lane / Op::CPR) + (wave >> 1) - lane / Op::CPR) * ld;
+  } else {
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    if (B_KMAJOR) {
-      const int r_local = lane / Op::CPR;  // LDS row 8 (wave + 4 k) + r_local: h = k / 4, j = 2 (k % 4) + wave / 2, c = 8 (wave % 2) + r_local
-      const int col = 128 * (k >> 2) + 8 * (8 * (wave & 1) + r_local) + 2 * (k & 3) + (wave >> 1);
-      vo_b[k] = Op::lane_voff(lane, wave % Op::NPAT, ld) + (col - r_local) * ld;
-    } else {
-      vo_b[k] = OpB::lane_voff(lane, (wave + 4 * k) % OpB::NPAT, ld_b) + (wave + 4 * k) * OpB::RPI * ld_b;
-    }
+    for (int k = 0; k < (B_KMAJOR ? 1 : 2); ++k) vo_b[k] = OpB::lane_voff(lane, (wave + 4 * k) % OpB::NPAT, ld_b) + wave * OpB::RPI * ld_b;
   }
+  static_assert(B_KMAJOR || OpB::NPAT == 8, "the swizzle pattern of copy wave + 4 k is that of copy wave or of copy wave + 4");
+  const int row_a = __builtin_amdgcn_readfirstlane(ld), row_b = __builtin_amdgcn_readfirstlane(ld_b);
+  auto far_a = [&](int k) __attribute__((always_inline)) { return 4 * Op::RPI * k * row_a; };  // copy k's distance from copy 0
+  auto far_b = [&](int k) __attribute__((always_inline)) { return (B_KMAJOR ? 128 * (k >> 2) + 2 * (k & 3) : 4 * OpB::RPI * k) * row_b; };
 
   // LDS addresses of the fragment reads relative to a slab buffer (see gemm_fast.hip for the layout)
   uint32_t a_rd[2], b_rd[B_KMAJOR ? 2 : 8];
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks) a_rd[ks] = smem_addr + (wm0 + l16) * 128 + (((4 * ks + lg) ^ ((l16 / 2) % 8)) << 4);
+  auto set_a_rd = [&](int ks, const Tile& t) __attribute__((always_inline)) {  // for a tile's fragments of K step ks: the wave's rows are those of its height
+    a_rd[ks] = smem_addr + (wave_m * (t.rows <= C::BM / 2 ? 64 : 128) + l16) * 128 + (((4 * ks + lg) ^ ((l16 / 2) % 8)) << 4);
+  };
   if (B_KMAJOR) {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) b_rd[ks] = smem_addr + C::A_BYTES + (wn0 + l16) * 128 + (((4 * ks + lg) ^ ((l16 / 2) % 8)) << 4);
@@ -188,10 +226,7 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
     return true;
   };
 
-  // The staged A chunks live in v[192:255] (two sets of eight), named in the instruction text: a value that is in
-  // flight across loop iterations must not be known to the compiler, which would move it between registers (before
-  // it has arrived) wherever two paths join.  The compiler's own allocation ends below v192 (checked on the kept
-  // assembly by the tests).
+  // The staged A chunks live in v[192:255] (two sets of eight), named in the instruction text like all fragments and accumulators.
 #define TGG_W4_GA(c, f) \
   if (c == 0) { f("224", "227") } else if (c == 1) { f("228", "231") } else if (c == 2) { f("232", "235") } else if (c == 3) { f("236", "239") } \
   else if (c == 4) { f("240", "243") } else if (c == 5) { f("244", "247") } else if (c == 6) { f("248", "251") } else if (c == 7) { f("252", "255") } \
@@ -207,8 +242,8 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
   // A chunk k of the slab at offset koff of window ra -> register set SET
   auto load_s = [&](auto Kc, auto SETc, const i32x4_t& ra, int koff) __attribute__((always_inline))  {
     constexpr int k = decltype(Kc)::value, kq = k + 8 * decltype(SETc)::value;
-    const int v = TAIL ? vo[k] | mask_s : vo[k];
-#define TGG_W4_F(lo, hi) asm volatile("buffer_load_dwordx4 v[" lo ":" hi "], %0, %1, %2 offen" : : "v"(v), "s"(ra), "s"(koff) : "memory", TGG_W4_GA_CLOBBER);
+    const int v = TAIL ? vo | mask_s : vo, off = koff + far_a(k);
+#define TGG_W4_F(lo, hi) asm volatile("buffer_load_dwordx4 v[" lo ":" hi "], %0, %1, %2 offen" : : "v"(v), "s"(ra), "s"(off) : "memory", TGG_W4_GA_CLOBBER);
     TGG_W4_GA(kq, TGG_W4_F)
 #undef TGG_W4_F
   };
@@ -225,39 +260,35 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
     constexpr int k = decltype(Kc)::value;
     asm volatile("s_add_u32 m0, %0, %1" : : "s"(buf_addr), "n"(D_OFF + 4 * k * 1024) : "memory", "m0", "scc");
   };
-  auto copy_d = [&](auto Kc, const i32x4_t& rb, int koff, bool spaced) __attribute__((always_inline))  {
+  auto copy_d = [&](auto Kc, const i32x4_t& rb, int koff) __attribute__((always_inline))  {
     constexpr int k = decltype(Kc)::value;
-    const int v = TAIL && B_KMAJOR ? vo_b[k] | mask_d : vo_b[k];
-    if (spaced) asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" : : "v"(v), "s"(rb), "s"(koff) : "memory");
-    else asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" : : "v"(v), "s"(rb), "s"(koff) : "memory");
+    const int v = TAIL && B_KMAJOR ? vo_b[0] | mask_d : vo_b[B_KMAJOR ? 0 : k & 1], off = koff + far_b(k);
+    // (the staged chunks' registers are listed here too: the compiler must not hold a value in them in a K step without loads either)
+    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" : : "v"(v), "s"(rb), "s"(off) : "memory", TGG_W4_GA_CLOBBER);
   };
   // a slab's A copy k straight to LDS (prologue only)
   auto copy_direct = [&](auto Kc, auto ISBc, const i32x4_t& ra, int koff, uint32_t buf_addr) __attribute__((always_inline))  {
     constexpr int k = decltype(Kc)::value;
-    const int v = decltype(ISBc)::value ? vo_b[k] : vo[k];
+    const int v = decltype(ISBc)::value ? vo_b[B_KMAJOR ? 0 : k & 1] : vo, off = koff + (decltype(ISBc)::value ? far_b(k) : far_a(k));
     asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds"
-                 : : "s"(buf_addr), "n"(4 * k * 1024), "v"(v), "s"(ra), "s"(koff) : "memory", "m0", "scc");
+                 : : "s"(buf_addr), "n"(4 * k * 1024), "v"(v), "s"(ra), "s"(off) : "memory", "m0", "scc");
   };
   const uint32_t wave_buf = smem_addr + wave * 1024;  // copy `wave` of buffer 0's A slab
 
   // ---- fragments and accumulators --------------------------------------------------------------------------------
-  i32x4_t fa[2][8], fb[2][8];
-  f32x4_t acc[8][8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // All of them are named in the instruction text: block (i, j)'s accumulators a[32 i + 4 j : + 3], A's fragment i of set s v[64 + 32 s + 4 i : + 3], B's
+  // fragment j v[128 + 32 s + 4 j : + 3].  Full and half tiles leave and find different parts of them in use, and where such
+  // paths join the compiler moves what it knows of from register to register.  Its own allocation ends below v64 (amdgpu_num_vgpr)
+  // and has no AGPR (they are clobbered at every K step's end; tests/test_isa_hazards.py looks at the kept assembly).
+  for_each<64>([&](auto Bc) __attribute__((always_inline)) { acc_zero<4 * decltype(Bc)::value>(); });
 
-  // read number q (0..15) of the fragments of K step KS of the slab at byte offset `buf_off`: B fragments first
+  // read number q (0..15) of the fragments of K step KS of the slab at byte offset `buf_off`, into set SET: B fragments first
   // (the next step needs all of them at once), then A fragments in the order of use
-  auto read_frag = [&](auto KSc, auto Qc, i32x4_t (&sa)[8], i32x4_t (&sb)[8], uint32_t buf_off) {
-    constexpr int KS = decltype(KSc)::value, Q = decltype(Qc)::value;
-    if (Q < 8) {
-      if (B_KMAJOR) lds_read_b128<Q * 2048>(sb[Q], b_rd[B_KMAJOR ? KS : 0] + buf_off);
-      else lds_read_tr<KS * 32 * (C::BN * 2), KS * 32 * (C::BN * 2) + 4 * (C::BN * 2)>(sb[Q], b_rd[B_KMAJOR ? 0 : (Q < 8 ? Q : 0)] + buf_off);
-    } else {
-      lds_read_b128<(Q - 8) * 2048>(sa[Q - 8], a_rd[KS] + buf_off);
-    }
+  auto read_frag = [&](auto KSc, auto Qc, auto SETc, uint32_t buf_off) __attribute__((always_inline)) {
+    constexpr int KS = decltype(KSc)::value, Q = decltype(Qc)::value, SET = 32 * decltype(SETc)::value;
+    if constexpr (Q < 8 && B_KMAJOR) frag_read_b128<128 + SET + 4 * Q, Q * 2048>(b_rd[KS] + buf_off);
+    else if constexpr (Q < 8) frag_read_tr<128 + SET + 4 * Q, KS * 32 * (C::BN * 2), KS * 32 * (C::BN * 2) + 4 * (C::BN * 2)>(b_rd[Q] + buf_off);
+    else frag_read_b128<64 + SET + 4 * (Q - 8), (Q - 8) * 2048>(a_rd[KS] + buf_off);
   };
   // ---- epilogue ------------------------------------------------------------------------------------------------------
   // With one wave per SIMD nothing else would keep the matrix pipe busy while a wave converts and stores its 128x128
@@ -294,9 +325,9 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
     return e;
   };
   // block (i, j) -> staging piece j / 4; not before this point in the instruction stream
-  auto epi_cvt = [&](const EpiLane& e, int i, int j) __attribute__((always_inline))  {
-    asm volatile("" : "+a"(acc[i][j]));
-    *(uint2*)(e.wr + (j >> 2) * C::EPI_PIECE + (j & 3) * 32) = pack4<DT>(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+  auto epi_cvt = [&](const EpiLane& e, auto Ic, auto Jc) __attribute__((always_inline))  {
+    constexpr int j = decltype(Jc)::value, at = 32 * decltype(Ic)::value + 4 * j;
+    *(uint2*)(e.wr + (j >> 2) * C::EPI_PIECE + (j & 3) * 32) = pack4<DT>(acc_read<at>(), acc_read<at + 1>(), acc_read<at + 2>(), acc_read<at + 3>());
     asm volatile("" ::: "memory");
   };
   auto epi_read = [&](const EpiLane& e, int h, i32x4_t (&v)[2]) {
@@ -323,11 +354,11 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
     return col < pend_cols ? ((el >> 4) * 4 * p.N + col) * 2 : kNoFetch;
   };
   // outputs 4 h .. 4 h + 3 of the lane's eight in row r of strip i, converted; not before this point in the instruction stream
-  auto epi_half_t = [&](int i, int r, int h) __attribute__((always_inline))  {
-    asm volatile("" : "+a"(acc[i][4 * h]), "+a"(acc[i][4 * h + 1]), "+a"(acc[i][4 * h + 2]), "+a"(acc[i][4 * h + 3]));
+  auto epi_half_t = [&](auto Ic, auto Rc, auto Hc) __attribute__((always_inline))  {
+    constexpr int at = 32 * decltype(Ic)::value + 16 * decltype(Hc)::value + decltype(Rc)::value;
     uint2 x;
-    x.x = pack2<DT>(acc[i][4 * h][r], acc[i][4 * h + 1][r]);
-    x.y = pack2<DT>(acc[i][4 * h + 2][r], acc[i][4 * h + 3][r]);
+    x.x = pack2<DT>(acc_read<at>(), acc_read<at + 4>());
+    x.y = pack2<DT>(acc_read<at + 8>(), acc_read<at + 12>());
     asm volatile("" : "+v"(x.x), "+v"(x.y));
     return x;
   };
@@ -338,27 +369,23 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
     if (between_multiplies && !TAIL) asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 0" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
     else asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 1" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
   };
-  // everything that is pending, without multiplies to hide it under
-  auto epi_flush = [&]() __attribute__((always_inline))  {
-    if (pending) {
-      // the last row block's multiplies may have just been issued: give them time before compiled code reads the registers
-      asm volatile("s_nop 15\n\ts_nop 7" : "+a"(acc[7][0]), "+a"(acc[7][1]), "+a"(acc[7][2]), "+a"(acc[7][3]),
-                   "+a"(acc[7][4]), "+a"(acc[7][5]), "+a"(acc[7][6]), "+a"(acc[7][7]));
-      if (B_KMAJOR) {
-        const int lane_off = epi_lane_t();
-#pragma unroll
-        for (int i = 4; i < 8; ++i)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const uint2 x = epi_half_t(i, r, 0), y = epi_half_t(i, r, 1);
-            epi_store_t(lane_off, i, r, x, y, false);
-          }
-      }
+  // strips S0 .. S0 + 3 without multiplies to hide them under
+  auto epi_strips = [&](auto S0c) __attribute__((always_inline))  {
+    constexpr int S0 = decltype(S0c)::value;
+    // the last row block's multiplies may have just been issued: give them time before the registers are read
+    asm volatile("s_nop 15\n\ts_nop 7" : : : "memory");
+    if constexpr (B_KMAJOR) {
+      const int lane_off = epi_lane_t();
+      for_each<16>([&](auto Uc) __attribute__((always_inline)) {
+        constexpr int i = S0 + decltype(Uc)::value / 4, r = decltype(Uc)::value % 4;
+        const uint2 x = epi_half_t(TGG_W4_I(i), TGG_W4_I(r), TGG_W4_I(0)), y = epi_half_t(TGG_W4_I(i), TGG_W4_I(r), TGG_W4_I(1));
+        epi_store_t(lane_off, i, r, x, y, false);
+      });
+    } else {
       const EpiLane e = epi_lane();
-#pragma unroll
-      for (int i = B_KMAJOR ? 8 : 4; i < 8; ++i) {  // the first four strips left during the tile's last K step
-#pragma unroll
-        for (int j = 0; j < 8; ++j) epi_cvt(e, i, j);
+      for_each<4>([&](auto Qc) __attribute__((always_inline)) {
+        constexpr int i = S0 + decltype(Qc)::value;
+        for_each<8>([&](auto Jc) __attribute__((always_inline)) { epi_cvt(e, TGG_W4_I(i), Jc); });
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           i32x4_t v[2];
@@ -366,8 +393,12 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
           epi_store(e, i, h, 0, v[0], false);
           epi_store(e, i, h, 1, v[1], false);
         }
-      }
+      });
     }
+  };
+  // what a full tile has left pending
+  auto epi_flush = [&]() __attribute__((always_inline))  {
+    if (pending) epi_strips(std::integral_constant<int, 4>());
     pending = false;
     pend_rs[2] = 0;
   };
@@ -378,6 +409,9 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
   typedef std::integral_constant<int, 2> I2;
   typedef std::integral_constant<bool, true> Yes;
   typedef std::integral_constant<bool, false> No;
+  typedef std::integral_constant<int, 3> I3;
+  typedef std::integral_constant<int, 4> I4;
+  typedef std::integral_constant<int, 8> I8;
 
   // the two cursors of the copy stream and the tile after the one being multiplied
   i32x4_t rs_c, rd_c;
@@ -417,11 +451,16 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
   // ROLE 2: second K step: the B copies of the slab two ahead, into the buffer at cp_addr.
   // EPI 1: the first K step of a tile -- multiplies start from zero, strips 4-7 of the tile before are stored between
   //        them.  EPI 2: the last K step of a tile -- strips 0-3 are stored between its multiplies.
-  auto kstep = [&](auto CURc, auto NKSc, auto MULc, auto ROLEc, uint32_t nb_off, auto EPIc, uint32_t wr_addr, auto SETc, uint32_t cp_addr) __attribute__((always_inline))  {
-    constexpr int CUR = decltype(CURc)::value, NKS = decltype(NKSc)::value, ROLE = decltype(ROLEc)::value;
-    constexpr bool MUL = decltype(MULc)::value;
-    constexpr int EPI = decltype(EPIc)::value;
-    static_assert(!EPI || MUL, "the epilogue rides on a multiplying K step");
+  // NS: row blocks of the tile per wave, eight, or four in a tile of at most 128 rows (no epilogue rides on its 32 multiplies; EPI 3:
+  // they start from zero).  RD: fragments of A to read for the next K step.
+  auto kstep = [&](auto CURc, auto NKSc, auto NSc, auto RDc, auto ROLEc, uint32_t nb_off, auto EPIc, uint32_t wr_addr, auto SETc, uint32_t cp_addr) __attribute__((always_inline))  {
+    constexpr int CUR = decltype(CURc)::value, NKS = decltype(NKSc)::value, ROLE = decltype(ROLEc)::value, NS = decltype(NSc)::value, RD = decltype(RDc)::value;
+    constexpr bool MUL = NS > 0;
+    constexpr int EPI = decltype(EPIc)::value == 3 ? 0 : decltype(EPIc)::value;
+    constexpr bool FRESH = decltype(EPIc)::value == 1 || decltype(EPIc)::value == 3;
+    static_assert(!EPI || NS == 8, "the epilogue rides on the multiplies of a full tile");
+    constexpr int G1 = NS == 4 ? 8 + RD : 16, D1 = NS == 4 ? 2 : 4, L1 = NS == 4 ? 1 : 2;  // LDS writes: first gap, distance, distance of the reload behind
+    constexpr int G2 = 16, D2 = NS == 4 ? 2 : 5;                                             // copies likewise
     EpiLane e = {nullptr, nullptr, {0, 0}};
     i32x4_t vv[2][2];
     if (EPI && !B_KMAJOR) e = epi_lane();
@@ -437,64 +476,53 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
     // multiply that completed it and before the one that starts it afresh; a piece (four blocks) is read back in the
     // gap of its last block and stored two and four gaps later.
     constexpr int EPI_S0 = EPI == 2 ? 0 : 4, EPI_G0 = EPI == 2 ? 4 : 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        const int j = (i & 1) ? 7 - jj : jj;  // snake order: one operand register changes per multiply
-        if (EPI && B_KMAJOR) {
-          const int gap = i * 8 + jj;
-#pragma unroll
-          for (int u = 0; u < 16; ++u) {
-            if (EPI_T0 + 3 * u == gap) ex = epi_half_t(EPI_S0 + u / 4, u % 4, 0);
-            if (EPI_T0 + 3 * u + 1 == gap) { const uint2 ey = epi_half_t(EPI_S0 + u / 4, u % 4, 1); epi_store_t(lane_off, EPI_S0 + u / 4, u % 4, ex, ey, true); }
+    for_each<(NS == 4 ? 32 : 64)>([&](auto Nc) __attribute__((always_inline)) {
+      constexpr int n = decltype(Nc)::value, i = n / 8, j = (i & 1) ? 7 - n % 8 : n % 8;  // snake order: one operand register changes per multiply
+      if constexpr (EPI != 0 && B_KMAJOR) {
+        constexpr int u = (n - EPI_T0) / 3;
+        if constexpr (n >= EPI_T0 && u < 16) {
+          if constexpr ((n - EPI_T0) % 3 == 0) ex = epi_half_t(TGG_W4_I(EPI_S0 + u / 4), TGG_W4_I(u % 4), TGG_W4_I(0));
+          if constexpr ((n - EPI_T0) % 3 == 1) {
+            const uint2 ey = epi_half_t(TGG_W4_I(EPI_S0 + u / 4), TGG_W4_I(u % 4), TGG_W4_I(1));
+            epi_store_t(lane_off, EPI_S0 + u / 4, u % 4, ex, ey, true);
           }
-        }
-        if (EPI && !B_KMAJOR) {
-          const int gap = i * 8 + jj;
-#pragma unroll
-          for (int bb = 0; bb < 32; ++bb) {
-            const int g = EPI_G0 + 7 * bb / 4, si = EPI_S0 + bb / 8, sj = (si & 1) ? 7 - bb % 8 : bb % 8;
-            if (g == gap) epi_cvt(e, si, sj);
-            if ((bb & 3) == 3 && g == gap) epi_read(e, sj >> 2, vv[(bb >> 2) & 1]);
-          }
-#pragma unroll
-          for (int bb = 3; bb < 32; bb += 4) {
-            const int g = EPI_G0 + 7 * bb / 4, si = EPI_S0 + bb / 8, sj = (si & 1) ? 7 - bb % 8 : bb % 8;
-            if (g + 2 == gap) epi_store(e, si, sj >> 2, 0, vv[(bb >> 2) & 1][0], true);
-            if (g + 4 == gap) epi_store(e, si, sj >> 2, 1, vv[(bb >> 2) & 1][1], true);
-          }
-        }
-        if (EPI == 1) {
-          if (B_KMAJOR) mfma_new<DT>(acc[i][j], fa[CUR][i], fb[CUR][j]);
-          else mfma_new<DT>(acc[i][j], fb[CUR][j], fa[CUR][i]);
-        } else if (MUL) {
-          if (B_KMAJOR) mfma_acc<DT>(acc[i][j], fa[CUR][i], fb[CUR][j]);
-          else mfma_acc<DT>(acc[i][j], fb[CUR][j], fa[CUR][i]);
-        }
-        const int n = i * 8 + jj;
-#define TGG_W4_RD(q) if (n == q) read_frag(std::integral_constant<int, NKS>(), std::integral_constant<int, q>(), fa[CUR ^ 1], fb[CUR ^ 1], nb_off);
-        TGG_W4_RD(0) TGG_W4_RD(1) TGG_W4_RD(2) TGG_W4_RD(3) TGG_W4_RD(4) TGG_W4_RD(5) TGG_W4_RD(6) TGG_W4_RD(7)
-        TGG_W4_RD(8) TGG_W4_RD(9) TGG_W4_RD(10) TGG_W4_RD(11) TGG_W4_RD(12) TGG_W4_RD(13) TGG_W4_RD(14) TGG_W4_RD(15)
-#undef TGG_W4_RD
-        if (ROLE == 1) {
-#define TGG_W4_ST(c) if (n == 16 + 4 * c) write_s(std::integral_constant<int, c>(), SETc, wr_addr); \
-                     if (n == 18 + 4 * c) { load_s(std::integral_constant<int, c>(), SETc, rs_c, koff_s); if (!MUL) __builtin_amdgcn_s_sleep(1); }
-          TGG_W4_ST(0) TGG_W4_ST(1) TGG_W4_ST(2) TGG_W4_ST(3) TGG_W4_ST(4) TGG_W4_ST(5) TGG_W4_ST(6) TGG_W4_ST(7)
-#undef TGG_W4_ST
-          if (n == 52) advance_s();
-        }
-        if (ROLE == 2) {
-#define TGG_W4_CP(c) if (n == 16 + 5 * c) copy_d_m0(std::integral_constant<int, c>(), cp_addr); \
-                     if (n == 17 + 5 * c) { copy_d(std::integral_constant<int, c>(), rd_c, koff_d, MUL); if (!MUL) __builtin_amdgcn_s_sleep(1); }
-          TGG_W4_CP(0) TGG_W4_CP(1) TGG_W4_CP(2) TGG_W4_CP(3) TGG_W4_CP(4) TGG_W4_CP(5) TGG_W4_CP(6) TGG_W4_CP(7)
-#undef TGG_W4_CP
-          if (n == 56) advance_d();
         }
       }
-    if (ROLE == 2) asm volatile("s_waitcnt lgkmcnt(0)" : TGG_TIE8(fa[CUR ^ 1]), TGG_TIE8(fb[CUR ^ 1]) : : "memory");
-    else if (ROLE == 1) asm volatile("s_waitcnt vmcnt(%16) lgkmcnt(0)" : TGG_TIE8(fa[CUR ^ 1]), TGG_TIE8(fb[CUR ^ 1]) : "n"(EPI ? 24 : 8) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : TGG_TIE8(fa[CUR ^ 1]), TGG_TIE8(fb[CUR ^ 1]) : : "memory");
+      if constexpr (EPI != 0 && !B_KMAJOR) {
+        for_each<32>([&](auto Bc) __attribute__((always_inline)) {
+          constexpr int bb = decltype(Bc)::value, g = EPI_G0 + 7 * bb / 4, si = EPI_S0 + bb / 8, sj = (si & 1) ? 7 - bb % 8 : bb % 8;
+          if constexpr (g == n) epi_cvt(e, TGG_W4_I(si), TGG_W4_I(sj));
+          if constexpr ((bb & 3) == 3 && g == n) epi_read(e, sj >> 2, vv[(bb >> 2) & 1]);
+        });
+        for_each<32>([&](auto Bc) __attribute__((always_inline)) {
+          constexpr int bb = decltype(Bc)::value, g = EPI_G0 + 7 * bb / 4, si = EPI_S0 + bb / 8, sj = (si & 1) ? 7 - bb % 8 : bb % 8;
+          if constexpr ((bb & 3) == 3 && g + 2 == n) epi_store(e, si, sj >> 2, 0, vv[(bb >> 2) & 1][0], true);
+          if constexpr ((bb & 3) == 3 && g + 4 == n) epi_store(e, si, sj >> 2, 1, vv[(bb >> 2) & 1][1], true);
+        });
+      }
+      if constexpr (MUL) {
+        constexpr int fa = 64 + 32 * CUR + 4 * i, fb = 128 + 32 * CUR + 4 * j;
+        if constexpr (B_KMAJOR) acc_mfma<DT, FRESH, 32 * i + 4 * j, fa, fb>();
+        else acc_mfma<DT, FRESH, 32 * i + 4 * j, fb, fa>();
+      }
+      if constexpr (n < 8 + RD) read_frag(TGG_W4_I(NKS), Nc, TGG_W4_I(CUR ^ 1), nb_off);
+      if constexpr (ROLE == 1) {
+        constexpr int w = n - G1, l = n - G1 - L1;
+        if constexpr (w >= 0 && w % D1 == 0 && w / D1 < 8) write_s(TGG_W4_I(w / D1), SETc, wr_addr);
+        if constexpr (l >= 0 && l % D1 == 0 && l / D1 < 8) load_s(TGG_W4_I(l / D1), SETc, rs_c, koff_s);
+      }
+      if constexpr (ROLE == 2) {
+        constexpr int m = n - G2, c = n - G2 - 1;
+        if constexpr (m >= 0 && m % D2 == 0 && m / D2 < 8) copy_d_m0(TGG_W4_I(m / D2), cp_addr);
+        if constexpr (c >= 0 && c % D2 == 0 && c / D2 < 8) copy_d(TGG_W4_I(c / D2), rd_c, koff_d);
+      }
+    });
+    if constexpr (ROLE == 1) advance_s();
+    if constexpr (ROLE == 2) advance_d();
+    __builtin_amdgcn_sched_barrier(0);  // the scalar work sits in front of the wait and not in the gaps behind it
+    if constexpr (ROLE == 2) asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory", TGG_W4_ACC_CLOBBER);
+    else if constexpr (ROLE == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(EPI ? 24 : 8) : "memory", TGG_W4_ACC_CLOBBER);
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : : : "memory", TGG_W4_ACC_CLOBBER);
   };
 
   // ---- prologue: slab 0 lands in buffer 0, slabs 1 and 2 are requested, the first fragments are read -----------------
@@ -529,42 +557,64 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
     mask_s = koff_s + chunk_off >= row_bytes ? kNoFetch : 0;
     if (B_KMAJOR) mask_d = koff_d + chunk_off >= row_bytes ? kNoFetch : 0;
   }
-  kstep(I1(), I0(), No(), I0(), 0u, I0(), 0u, I0(), 0u);  // reads K step 0 of buffer 0 into set 0, multiplies nothing, waits for everything
+  set_a_rd(0, cur);
+  set_a_rd(1, cur);
+  kstep(I1(), I0(), I0(), I8(), I0(), 0u, I0(), 0u, I0(), 0u);  // reads K step 0 of buffer 0 into set 0, multiplies nothing, waits for everything
 
   for (int tile_id = walk.first; tile_id < walk.end; tile_id += walk.stride) {
+    const bool half = cur.rows <= C::BM / 2;  // a tile of at most 128 rows: 64 per wave, half the multiplies
+    const int wm0 = wave_m * (half ? 64 : 128);
     const bool active = wm0 < cur.rows && cur.n0 + wn0 < p.N;  // this wave's block of the tile has rows and columns
-    const bool mul = !SIT_OUT || active;
-    if (!mul) epi_flush();  // no multiplies in this tile to hide the pending stores under
-    // one slab; FIRST: the tile's first, whose first K step starts the accumulators afresh and carries the epilogue;
-    // PAR: parity of the slab = its LDS buffer; the A chunks of the next slab wait in register set 1 - PAR
-    auto slab = [&](auto EPc, auto PARc) __attribute__((always_inline)) {
-      typedef std::integral_constant<int, decltype(EPc)::value == 1 ? 1 : 0> Ep0;  // the tile's first slab: its first K step carries strips 4-7 of the tile before
-      typedef std::integral_constant<int, decltype(EPc)::value == 2 ? 2 : 0> Ep1;  // the tile's last slab: its second K step carries strips 0-3
-      constexpr int PAR = decltype(PARc)::value;
+    const int rows_left = cur.rows - wm0, most = half ? 64 : 128;
+    const i32x4_t out_rs = make_rsrc32((uint64_t)p.C + (uint64_t)(((cur.row0 + wm0) * (int64_t)p.N + cur.n0 + wn0) * 2),
+                                       active ? (rows_left < most ? rows_left : most) * p.N * 2 : 0);
+    const int out_cols = __builtin_amdgcn_readfirstlane(active ? p.N - cur.n0 - wn0 : 0);
+    // One slab.  EP: 1 the first of a full tile, whose first K step starts the accumulators afresh and carries strips 4-7 of the tile before,
+    // 2 the last of a full tile, whose second K step carries strips 0-3, 3 the first of a half tile; PAR: parity of the slab = its LDS buffer; the A
+    // chunks of the next slab wait in register set 1 - PAR.  RD: fragments of A to read for the slab behind.
+    auto slab = [&](auto NSc, auto EPc, auto PARc, auto RDc) __attribute__((always_inline)) {
+      constexpr int EP = decltype(EPc)::value, PAR = decltype(PARc)::value;
+      typedef std::integral_constant<int, EP == 1 || EP == 3 ? EP : 0> Ep0;
+      typedef std::integral_constant<int, EP == 2 ? 2 : 0> Ep1;
       typedef std::integral_constant<int, 1 - PAR> SetN;
       constexpr uint32_t cur_off = PAR * C::STAGE_BYTES, nxt_off = C::STAGE_BYTES - cur_off;
-      if (mul) kstep(I0(), I1(), Yes(), I1(), cur_off, Ep0(), s_wr + nxt_off, SetN(), 0u);
-      else kstep(I0(), I1(), No(), I1(), cur_off, I0(), s_wr + nxt_off, SetN(), 0u);
+      kstep(I0(), I1(), NSc, NSc, I1(), cur_off, Ep0(), s_wr + nxt_off, SetN(), 0u);
       // set 1 is complete, this wave has read all it needs of the current slab, its copies of the next slab have landed
       asm volatile("s_barrier" ::: "memory");
-      if (mul) kstep(I1(), I0(), Yes(), I2(), nxt_off, Ep1(), 0u, I0(), wave_buf + cur_off);
-      else kstep(I1(), I0(), No(), I2(), nxt_off, I0(), 0u, I0(), wave_buf + cur_off);
+      kstep(I1(), I0(), NSc, RDc, I2(), nxt_off, Ep1(), 0u, I0(), wave_buf + cur_off);
     };
-    slab(I1(), I0());  // an even number of slabs per tile, at least four: every tile starts in buffer 0
-    slab(I0(), I1());
-    for (int kt = 4; kt < kt_all; kt += 2) {
-      slab(I0(), I0());
-      slab(I0(), I1());
+    if (__builtin_expect(half, 0)) {
+      epi_flush();
+      slab(I4(), I3(), I0(), I4());  // an even number of slabs per tile, at least four: every tile starts in buffer 0
+      slab(I4(), I0(), I1(), I4());
+      for (int kt = 4; kt < kt_all; kt += 2) {
+        slab(I4(), I0(), I0(), I4());
+        slab(I4(), I0(), I1(), I4());
+      }
+      slab(I4(), I0(), I0(), I4());
+      set_a_rd(0, nxt_tile);
+      slab(I4(), I0(), I1(), I8());
+      pend_rs = out_rs;
+      pend_cols = out_cols;
+      epi_strips(I0());
+      pend_rs[2] = 0;
+    } else {
+      slab(I8(), I1(), I0(), I8());
+      slab(I8(), I0(), I1(), I8());
+      for (int kt = 4; kt < kt_all; kt += 2) {
+        slab(I8(), I0(), I0(), I8());
+        slab(I8(), I0(), I1(), I8());
+      }
+      // what the tile's last K step, the next tile's first K step and a flush store: nothing for a wave whose block of
+      // the tile has no rows or no columns
+      pend_rs = out_rs;
+      pend_cols = out_cols;
+      pending = true;
+      slab(I8(), I0(), I0(), I8());
+      set_a_rd(0, nxt_tile);
+      slab(I8(), I2(), I1(), I8());
     }
-    // what the tile's last K step, the next tile's first K step and a flush store: nothing for a wave whose block of
-    // the tile has no rows or no columns
-    const int rows_left = cur.rows - wm0;
-    pend_rs = make_rsrc32((uint64_t)p.C + (uint64_t)(((cur.row0 + wm0) * (int64_t)p.N + cur.n0 + wn0) * 2),
-                          active ? (rows_left < 128 ? rows_left : 128) * p.N * 2 : 0);
-    pend_cols = __builtin_amdgcn_readfirstlane(active ? p.N - cur.n0 - wn0 : 0);
-    pending = mul;  // a wave that sat the tile out has flushed and leaves nothing behind
-    slab(I0(), I0());
-    slab(I2(), I1());
+    set_a_rd(1, nxt_tile);
     // both cursors are in the next tile by now: it becomes the current one, and the one after it is looked up
     cur = nxt_tile;
     const bool more = tile_at(tile_id + 2 * walk.stride, nxt_tile);
@@ -577,13 +627,13 @@ __global__ __launch_bounds__(W4Cfg::THREADS) void gemm_w4_kernel(const GemmParam
 #undef TGG_W4_GA_CLOBBER
 }
 
-template <int DT, int LAYOUT, bool SIT_OUT, bool TAIL>
+template <int DT, int LAYOUT, bool TAIL>
 int launch_w4(const GemmParams& p, hipStream_t s) {
   static bool attr_set[64] = {false};
   int dev = 0;
   (void)hipGetDevice(&dev);
   const bool listed = dev >= 0 && dev < 64;
-  auto kern = gemm_w4_kernel<DT, LAYOUT, SIT_OUT, TAIL>;
+  auto kern = gemm_w4_kernel<DT, LAYOUT, TAIL>;
   if (!listed || !attr_set[dev]) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, W4Cfg::SMEM_BYTES) != hipSuccess)
       return check_launch("hipFuncSetAttribute(gemm_w4)");
@@ -607,14 +657,13 @@ static bool w4_large(const GemmParams& p) {
   return ((p.m_total + 255) / 256) * ((p.N + 127) / 128) > 4 * (int64_t)grid;
 }
 
-// Whether 256-row tiles pay depends on the group sizes, which only the device knows.  With 512 rows and more per group on
-// average they do; a masked launch (counts anywhere up to its row stride), one with smaller groups or one of fewer rounds is
-// enqueued together with the eight-wave kernel, and the two decide from the sizes which of them runs.  The average is that of the operand:
-// where the groups of a large launch fill a twentieth of it, this kernel alone takes 1.1 of the eight-wave kernel's time (up to 1.33; a fifth
-// of it 0.98, all 0.93: 200 random launches with a tail).  Decided on the device as well these would take 1.08, 1.01 and 0.94.
-bool w4_decided_on_device(const GemmParams& p) {
-  return p.mode == MODE_MASKED || p.m_total < 512 * (int64_t)p.G || !w4_large(p);
-}
+// Whether 256-row tiles pay depends on the group sizes, which only the device knows.  With 200 rows and more per group on
+// average they do: of 130 random launches decided on the device (Dirichlet groups, more than two rounds and fewer) none of those took longer by this
+// kernel alone (0.85-1.00, 0.98 in the mean: the launch that returns is 4-6 us), while below, 84-184 rows, it was 0.85-1.13.  Smaller groups, and masked
+// launches (counts anywhere up to the row stride), are enqueued together with the eight-wave kernel, and the two decide from the sizes which
+// of them runs.  The average is that of the operand: where the groups fill a twentieth of it, this kernel alone takes 1.1 of the eight-wave kernel's
+// time (up to 1.33; a fifth of it 0.98: 200 random launches with a tail, before half tiles).
+bool w4_decided_on_device(const GemmParams& p) { return p.mode == MODE_MASKED || p.m_total < 200 * (int64_t)p.G; }
 
 // The four-wave kernel takes large M-grouped and masked launches, and M-grouped ones of 128 rows and more per group whose likely tiles
 // (every group's last one half full) cost two rounds of K = 2048 or more and would not be chosen for 128-row tiles
@@ -658,8 +707,7 @@ bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
 
 template <int DT, int LAYOUT>
 int launch_w4_layout(const GemmParams& p, hipStream_t s) {
-  if (needs_tail(p, LAYOUT)) return launch_w4<DT, LAYOUT, false, true>(p, s);
-  return p.mode == MODE_MASKED ? launch_w4<DT, LAYOUT, true, false>(p, s) : launch_w4<DT, LAYOUT, false, false>(p, s);
+  return needs_tail(p, LAYOUT) ? launch_w4<DT, LAYOUT, true>(p, s) : launch_w4<DT, LAYOUT, false>(p, s);
 }
 
 int launch_w4_16bit(const GemmParams& p, int dt, int layout, hipStream_t s) {
