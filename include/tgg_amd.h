@@ -159,6 +159,11 @@ int tgg_per_block_cast_to_fp8(const void* x, void* codes, float* scales, int bat
  * streams (sa_mn_major = 1). */
 int tgg_scales_to_mn_major(const float* in, float* out, int64_t M, int kblocks, void* stream);
 
+/* Rows of a contiguous (padded) layout, sum over groups of sizes[g] (as int32) rounded up to block_m, which the reference reads back to the host
+ * (gemm/deep_gemm_ops.py:49-51), written by the GPU to page-locked host memory: host[0] = the total, then host[1] = 1.  The caller clears
+ * host[1] first and may wait for the word instead of for a copy and an event (8-byte aligned, coherent, in use until the word is set). */
+int tgg_padded_total(const void* sizes, int sizes_i64, int G, int64_t block_m, int64_t* host, void* stream);
+
 /* Element-wise fp32 -> fp8 code with the conversion the quantizers use (test hook for the
  * `.to(torch.float8_*)` casts of the recipes above). */
 int tgg_cvt_f32_to_fp8(const float* in, void* out, int64_t n, int fmt, void* stream);

@@ -58,6 +58,7 @@ int num_cus() {
 int launch_trans_quant128(const void*, void*, float*, const GemmParams&, int64_t, void*, int, hipStream_t);
 int launch_token_cast128(const void*, void*, float*, int64_t, int, int, int, hipStream_t);
 int launch_block_cast128(const void*, void*, float*, int, int, int, int, hipStream_t);
+int launch_padded_total(const void*, int, int, int64_t, int64_t*, hipStream_t);
 int launch_scales_transpose(const float*, float*, int64_t, int, hipStream_t);
 int launch_cvt_fp8(const float*, void*, int64_t, int, hipStream_t);
 bool fast_supported(const GemmParams& p, int dt, int layout);
@@ -564,6 +565,12 @@ int tgg_scales_to_mn_major(const float* in, float* out, int64_t M, int kblocks, 
   if (!in || !out) return set_error("null pointer");
   if (M < 0 || kblocks < 0 || (M + 63) / 64 >= (1ll << 24)) return set_error("bad M=%lld or kblocks=%d", (long long)M, kblocks);
   return launch_scales_transpose(in, out, M, kblocks, (hipStream_t)stream);
+}
+
+int tgg_padded_total(const void* sizes, int sizes_i64, int G, int64_t block_m, int64_t* host, void* stream) {
+  if (!sizes || !host) return set_error("null pointer");
+  if (G < 1 || block_m < 1 || ((uintptr_t)host & 7)) return set_error("bad G=%d or block_m=%lld, or misaligned result", G, (long long)block_m);
+  return launch_padded_total(sizes, sizes_i64, G, block_m, host, (hipStream_t)stream);
 }
 
 int tgg_cvt_f32_to_fp8(const float* in, void* out, int64_t n, int fmt, void* stream) {

@@ -476,6 +476,28 @@ int launch_block_cast128(const void* x, void* codes, float* scales, int batch, i
   return check_launch("block_cast128");
 }
 
+// Sum of the sizes, each taken as int32 and rounded up to block_m (floor division, also of negative ones), to host memory that the
+// GPU writes over the bus: the total, then the word that says it is there.
+__global__ __launch_bounds__(64) void padded_total_kernel(const void* sizes, int is64, int G, int64_t block_m, int64_t* host) {
+  int64_t sum = 0;
+  for (int g = threadIdx.x; g < G; g += 64) {
+    const int64_t v = is64 ? (int64_t)(int32_t)((const int64_t*)sizes)[g] : (int64_t)((const int32_t*)sizes)[g];
+    const int64_t up = v + block_m - 1;
+    sum += (up >= 0 ? up / block_m : -((block_m - 1 - up) / block_m)) * block_m;
+  }
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) sum += __shfl_xor(sum, d, 64);
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(host, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(host + 1, (int64_t)1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+int launch_padded_total(const void* sizes, int is64, int G, int64_t block_m, int64_t* host, hipStream_t s) {
+  hipLaunchKernelGGL(padded_total_kernel, dim3(1), dim3(64), 0, s, sizes, is64, G, block_m, host);
+  return check_launch("padded_total");
+}
+
 int launch_scales_transpose(const float* in, float* out, int64_t rows, int cols, hipStream_t s) {
   if (rows == 0 || cols == 0) return 0;
   hipLaunchKernelGGL(scales_transpose_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(256), 0, s, in, out, rows, cols);
