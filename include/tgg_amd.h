@@ -287,7 +287,7 @@ int tgg_debug_queue_order(int grid, int draws, int32_t* out);
  *                        tokens on few workgroups or without a queue;
  *                        FP8 K-grouped: all but outputs of up to 256 columns with 1000 tokens a group and more
  *   "kg_split"      0/1  K-grouped launches may be cut along K where the caller brings a workspace (default 1)
- *   "deep"          int  the kernel for launches of few tiles (16-bit M-grouped / padded / placed / masked, up to 256 groups; 64x64, 64x128 or
+ *   "deep"          int  the kernel for launches of few tiles (16-bit M-grouped / padded / placed / masked, FP8 per-channel M-grouped, up to 256 groups; 64x64, 64x128 or
  *                        128x128 tiles, chosen on the device from the sizes): 1 (default) = launches whose 128x128 tiles fit one round of
  *                        the workgroups, unless "variant" or "four_wave" asks for another kernel; 0 = never; 2 = on every launch that it can take
  *   "tile_split"    0/1  M-grouped tuned kernels: per-XCD contiguous tile ranges (default 1) or interleaved sweeps

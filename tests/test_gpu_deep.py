@@ -95,3 +95,29 @@ def test_the_default_route(sizes, rows, N, K, trans_b):
         total = sum(-(-n // 128) * 128 for n in sizes) or 128
         check(total, padded, lambda a, out: _native.call("tgg_m_grouped_gemm_padded", a.data_ptr(), b.data_ptr(), out.data_ptr(), s.data_ptr(), 1, G,
                                                          total, N, K, 128, _native.BF16, -1, _native.stream_of(a)))
+
+
+@pytest.mark.parametrize("act, weight", [(torch.float8_e4m3fn, torch.float8_e4m3fn), (torch.float8_e5m2, torch.float8_e4m3fn), (torch.float8_e4m3fn, torch.float8_e5m2),
+                                         (torch.float8_e5m2, torch.float8_e5m2)])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("num_cu", [-1, 16, 3])
+@pytest.mark.parametrize("K", [16, 128, 144, 512, 1040, 2048])  # 1 to 16 slabs
+@pytest.mark.parametrize("sizes, N", [([63, 0, 64, 65, 1, 129], 136), ([300, 0, 127], 520), ([5], 8), ([0, 40], 200)])
+def test_fp8_per_channel(act, weight, out_dtype, num_cu, K, sizes, N):
+    """Against the eight-wave kernel bit for bit: the same multiplies in the same order along K, the same scaling."""
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(K + N)
+    G, M = len(sizes), sum(sizes)
+    a, b = torch.randn(M, K, device=dev, generator=gen).mul_(40).to(act), torch.randn(G, N, K, device=dev, generator=gen).mul_(40).to(weight)
+    sa, sb = torch.rand(M, device=dev, generator=gen), torch.rand(G, N, device=dev, generator=gen).mul_(1e-3)
+    s = torch.tensor(sizes, dtype=torch.int32, device=dev)
+    code = {torch.float8_e4m3fn: _native.E4M3, torch.float8_e5m2: _native.E5M2}
+
+    def run():
+        out = torch.full((M + 3, N), float("nan"), device=dev, dtype=out_dtype)
+        _native.call("tgg_m_grouped_gemm_fp8_channel", a.data_ptr(), sa.data_ptr(), b.data_ptr(), sb.data_ptr(), out.data_ptr(), s.data_ptr(), 0, G, M, N, K,
+                     code[act], code[weight], _native.DTYPE_CODE[out_dtype], num_cu, _native.stream_of(a))
+        return out.view(torch.int16)
+    out = _with("deep", 2, 1, run)
+    assert torch.equal(out, _with("deep", 0, 1, run)) and torch.equal(out, run())
+    assert not bool(torch.isnan(out.view(out_dtype)[:M]).any()) and bool(torch.isnan(out.view(out_dtype)[M:]).all())

@@ -65,6 +65,8 @@ bool fast_supported(const GemmParams& p, int dt, int layout);
 int launch_fast_16bit(const GemmParams& p, int dt, int layout, hipStream_t s);
 bool deep_supported(const GemmParams& p, int dt, int layout, bool any_size);
 int launch_deep_16bit(const GemmParams& p, int dt, int layout, hipStream_t s);
+bool deep_fp8_supported(const GemmParams& p, bool any_size);
+int launch_deep_fp8(const GemmParams& p, int ta, int tb, int out_dt, hipStream_t s);
 bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size);
 bool w4_decided_on_device(const GemmParams& p);
 int launch_w4_16bit(const GemmParams& p, int dt, int layout, hipStream_t s);
@@ -449,6 +451,9 @@ int tgg_m_grouped_gemm_fp8_channel(const void* Aq, const float* a_scale, const v
   if (K & 15) return set_error("K must be a multiple of 16 for fp8 operands, got %d", K);
   if (M == 0) return 0;
   const GemmParams p = params_fp8_channel(Aq, a_scale, Bq, b_scale, C, sizes, sizes_i64, G, M, N, K, num_cu);
+  if (const int deep = g_deep.load(); !g_force_generic.load() && (deep == 2 || (deep == 1 && g_variant.load() == 0)) &&
+                                      (out_dtype == TGG_BF16 || out_dtype == TGG_F16) && deep_fp8_supported(p, deep == 2))
+    return launch_deep_fp8(p, fmt_a, fmt_b, out_dtype, (hipStream_t)stream);
   if (!g_force_generic.load() && fast_fp8_supported(p, false)) return launch_fast_fp8_channel(p, fmt_a, fmt_b, out_dtype, (hipStream_t)stream);
   return launch_generic_fp8_channel(p, fmt_a, fmt_b, out_dtype, (hipStream_t)stream);
 }

@@ -19,6 +19,8 @@
 // 320 rows, N = 512, K = 256 (64 tiles of 64x64): 10.0 -> 7.1 us, of which 4.5 are the host's; 4 of 768, N = 856, K = 2048 (168): 34 -> 17; 8 of
 // 1086, N = 2048, K = 4072 (208 of 128x128): 96 -> 55; 16 of 1280, N = 1024, K = 512 (160 of 64x128): 14.3 -> 10.3.  In launches of several
 // rounds a small tile's operands cost more than its fit gains (128 groups, 32768 rows, N = 1536, K = 2048: 256 us by the larger tiles, 381 here).
+// FP8 with per-channel scales, 100 random launches of up to 8192 rows: 0.62 of the eight-wave kernel's time (0.42-0.87), the same bits.  4 groups of 270
+// rows, N = 2048, K = 4096: 35 -> 16 us; 16 of 3393, N = 768, K = 768: 16.1 -> 12.7.
 #include "launch.hpp"
 #include "w4_common.hpp"
 
@@ -26,7 +28,7 @@ namespace tgg {
 
 namespace {
 
-enum : int { DEEP_NT = 0, DEEP_NN = 1 };
+enum : int { DEEP_NT = 0, DEEP_NN = 1, DEEP_FP8 = 2 };  // FP8: NT, K-contiguous codes, per-row and per-(group, column) scales
 constexpr int BKD = 64;
 
 template <int BM_, int BN_, int ST_>
@@ -53,10 +55,16 @@ TGG_DEV void copy_slab_b128(const i32x4_t& rsrc, uint32_t lds_addr, int voff, in
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" : : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(koff) : "memory", "m0");
 }
 
-// The whole kernel but for the group table, which the caller has built for tiles of C::BM rows.
-template <class C, int DT, int LAYOUT>
+// The whole kernel but for the group table, which the caller has built for tiles of C::BM rows.  DT: the outputs' type, and unless FP8 the operands';
+// FA / FB: FP8, 0 = e4m3fn, 1 = e5m2 (format codes of the f8f6f4 multiply).
+// FP8: a slab is 128 bytes of every row as well, but its multiplies take all 128 values at once (32 per lane: 16-byte chunks lg and lg + 4 of a row,
+// see gemm_fp8.hip).  The two steps of a slab are the two halves of the wave's row blocks; the second one goes column block by
+// column block, and the next slab's fragment takes the place of the one that has been used.
+template <class C, int DT, int LAYOUT, int FA, int FB>
 TGG_DEV void gemm_deep_body(const GemmParams& p) {
-  constexpr bool B_KMAJOR = LAYOUT == DEEP_NT;
+  constexpr bool FP8 = LAYOUT == DEEP_FP8;
+  constexpr bool B_KMAJOR = LAYOUT != DEEP_NN;
+  constexpr int ES = FP8 ? 1 : 2, KS = BKD * 2 / ES;  // bytes of an operand's value, values of a slab row
   typedef Operand<C::BM, true> OpA;
   typedef Operand<C::BN, B_KMAJOR> OpB;
   static_assert(C::NWAVES % OpA::NPAT == 0 && C::NWAVES % OpB::NPAT == 0, "a wave's copies share one swizzle pattern");
@@ -72,8 +80,8 @@ TGG_DEV void gemm_deep_body(const GemmParams& p) {
   const int wm0 = (wave >> 1) * (C::BM / 2), wn0 = (wave & 1) * (C::BN / 2);
   const int l16 = lane & 15, lg = lane >> 4;
 
-  const int ld = p.K * 2, ld_b = (B_KMAJOR ? p.K : p.N) * 2;
-  const int kt_n = (p.K + BKD - 1) / BKD;
+  const int ld = p.K * ES, ld_b = (B_KMAJOR ? p.K : p.N) * ES;
+  const int kt_n = (p.K + KS - 1) / KS;
   // Source offsets of this wave's copies within the tile's window.  NT: B's rows land permuted, LDS row 16 TN h + 16 j + c of the slab
   // holds column 16 TN h + TN c + j of the tile, so that a lane's results of the TN column blocks are neighbouring outputs of a row.
   int vo_a[C::CA], vo_b[C::CB];
@@ -90,7 +98,7 @@ TGG_DEV void gemm_deep_body(const GemmParams& p) {
     }
   }
   // K tail: lanes whose chunk of a K-contiguous row starts at or beyond K fetch nothing in a tile's last slab
-  const int tail_chunks = (p.K % BKD) / 8;
+  const int tail_chunks = (p.K % KS) * ES / 16;
   const int tail = tail_chunks != 0 && OpA::lane_chunk(lane, wave % OpA::NPAT) >= tail_chunks ? kNoFetch : 0;
 
   // LDS offsets of the fragment reads, relative to a slab buffer
@@ -165,6 +173,7 @@ TGG_DEV void gemm_deep_body(const GemmParams& p) {
   };
 
   i32x4_t fa[2][C::TM], fb[2][C::TN];
+  i32x8_t fa8[C::TM], fb8[C::TN];  // FP8
   f32x4_t acc[C::TM][C::TN];
   auto clear = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -198,6 +207,48 @@ TGG_DEV void gemm_deep_body(const GemmParams& p) {
       }
     __builtin_amdgcn_sched_barrier(0);
   };
+  // ---- FP8 ----
+  auto frag8 = [&](const char* s, const int (&at)[2], int block) __attribute__((always_inline)) -> i32x8_t {
+    const i32x4_t lo = *(const i32x4_t*)(s + at[0] + block * 16 * 128), hi = *(const i32x4_t*)(s + at[1] + block * 16 * 128);
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  auto read8_a = [&](const char* s, int half) __attribute__((always_inline)) {
+    if constexpr (FP8) {
+#pragma unroll
+      for (int i = half * C::TM / 2; i < (half + 1) * C::TM / 2; ++i) fa8[i] = frag8(s, a_rd, i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto read8_b = [&](const char* s, int j) __attribute__((always_inline)) {
+    if constexpr (FP8) fb8[j] = frag8(s, b_rd, j);
+  };
+  // Half a slab's multiplies: row blocks of `half`; copies k0 .. k0 + NC / 2 - 1 go out between them.  The second half reads the next slab's
+  // fragments of B (at `next`) behind the last use of this one's.
+  auto step8 = [&](int half, int k0, uint32_t copy_buf, const char* next) __attribute__((always_inline)) {
+    if constexpr (FP8) {
+      constexpr int HM = C::TM / 2, SP = HM * C::TN / (C::NC / 2);
+      static_assert(SP >= 1, "half a slab's copies go out during half its multiplies");
+#pragma unroll
+      for (int j = 0; j < C::TN; ++j) {
+#pragma unroll
+        for (int ii = 0; ii < HM; ++ii) {
+          const int i = half * HM + ((j & 1) ? HM - 1 - ii : ii), n = j * HM + ii;
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fa8[i], fb8[j], acc[i][j], FA, FB, 0, 0, 0, 0);
+          if (n % SP == 0 && n / SP < C::NC / 2) {
+            __builtin_amdgcn_sched_barrier(0);
+            copy_k(k0 + n / SP, copy_buf);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        if (half == 1) {
+          __builtin_amdgcn_sched_barrier(0);
+          read8_b(next, j);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
   seek();
 #pragma unroll 1
   for (int s = 0; s < C::ST - 1; ++s) {
@@ -210,14 +261,25 @@ TGG_DEV void gemm_deep_body(const GemmParams& p) {
   clear();
   wait_vmcnt<(C::ST - 2) * C::NC + C::NC / 2>();
   __syncthreads();
-  read(0, smem, 0);
+  if constexpr (FP8) {
+    read8_a(smem, 0);
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j) read8_b(smem, j);
+  } else {
+    read(0, smem, 0);
+  }
   int buf = 0, prev = (C::ST - 1) * C::STAGE_BYTES;  // byte offsets of the current slab's buffer and the one before it
   for (int tile_id = w_first; tile_id < w_end; tile_id += w_stride) {
     const Tile cur = tile_id == seen_id ? seen : sched_tile<C::BM, C::BN>(p, sched, tile_id);
     for (int kt = 0; kt < kt_n; ++kt) {
       const int nxt = buf == (C::ST - 1) * C::STAGE_BYTES ? 0 : buf + C::STAGE_BYTES;
-      read(1, smem + buf, 1);
-      step(0, C::NC / 2, smem_addr + prev);
+      if constexpr (FP8) {
+        read8_a(smem + buf, 1);
+        step8(0, C::NC / 2, smem_addr + prev, nullptr);
+      } else {
+        read(1, smem + buf, 1);
+        step(0, C::NC / 2, smem_addr + prev);
+      }
       advance();
       // this wave's copies of the next slab have landed (a tile's stores, younger than those copies for ST - 2 slabs, may be in flight as well),
       // and it has read all it needs of this one
@@ -225,8 +287,13 @@ TGG_DEV void gemm_deep_body(const GemmParams& p) {
       else wait_vmcnt<(C::ST - 2) * C::NC>();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __syncthreads();
-      read(0, smem + nxt, 0);
-      step(1, 0, smem_addr + buf);
+      if constexpr (FP8) {
+        read8_a(smem + nxt, 0);
+        step8(1, 0, smem_addr + buf, smem + nxt);
+      } else {
+        read(0, smem + nxt, 0);
+        step(1, 0, smem_addr + buf);
+      }
       prev = buf;
       buf = nxt;
     }
@@ -240,10 +307,21 @@ TGG_DEV void gemm_deep_body(const GemmParams& p) {
     const int e16 = el & 15, eg = el >> 4;
     if (B_KMAJOR) {
       const int off0 = C::TN * e16 < cols ? (4 * eg * p.N + C::TN * e16) * 2 : kNoFetch;
+      float cs[C::TN];
+      if constexpr (FP8) {  // the scales of the lane's columns; those of its rows block by block
+#pragma unroll
+        for (int j = 0; j < C::TN; ++j) cs[j] = C::TN * e16 < cols ? p.scale_n[(int64_t)cur.g * p.N + cur.n0 + wn0 + C::TN * e16 + j] : 0.f;
+      }
 #pragma unroll
       for (int i = 0; i < C::TM; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
+          if constexpr (FP8) {
+            const int row = wm0 + 16 * i + 4 * eg + r;
+            const float rs = row < cur.rows ? p.scale_m[cur.row0 + row] : 0.f;
+#pragma unroll
+            for (int j = 0; j < C::TN; ++j) acc[i][j][r] = acc[i][j][r] * rs * cs[j];
+          }
           const int off = off0 + (16 * i + r) * p.N * 2;
           if constexpr (C::TN == 4) {
             const uint2 v = pack4<DT>(acc[i][0][r], acc[i][1][r], acc[i][2][r], acc[i][3][r]);
@@ -276,7 +354,7 @@ TGG_DEV void gemm_deep_body(const GemmParams& p) {
 }
 
 // The tile height of the table is 128; the small tiles take the half-height cut that sched_init leaves.
-template <int DT, int LAYOUT>
+template <int DT, int LAYOUT, int FA = 0, int FB = 0>
 __global__ __launch_bounds__(256) void gemm_deep_kernel(const GemmParams p) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   auto& sched = *reinterpret_cast<SchedTableT<kFastMaxGroups>*>(smem + kDeepSchedOff);
@@ -289,21 +367,21 @@ __global__ __launch_bounds__(256) void gemm_deep_kernel(const GemmParams p) {
   auto rounds = [&](int64_t tiles) { return (int)((tiles + wgs - 1) / wgs); };
   const int small = rounds((int64_t)rows64 * cols64) * 16, mid = rounds((int64_t)rows64 * cols128) * 24, wide = rounds((int64_t)rows128 * cols128) * 32;
   if (wide <= mid && wide < small) {
-    gemm_deep_body<Wide, DT, LAYOUT>(p);
+    gemm_deep_body<Wide, DT, LAYOUT, FA, FB>(p);
   } else {
     sched_use_half_height(p, sched, half_tile0);
-    if (small <= mid) gemm_deep_body<Small, DT, LAYOUT>(p);
-    else gemm_deep_body<Mid, DT, LAYOUT>(p);
+    if (small <= mid) gemm_deep_body<Small, DT, LAYOUT, FA, FB>(p);
+    else gemm_deep_body<Mid, DT, LAYOUT, FA, FB>(p);
   }
 }
 
-template <int DT, int LAYOUT>
+template <int DT, int LAYOUT, int FA = 0, int FB = 0>
 int launch_deep(const GemmParams& p, hipStream_t s) {
   static bool attr_set[64] = {false};
   int dev = 0;
   (void)hipGetDevice(&dev);
   const bool listed = dev >= 0 && dev < 64;
-  auto kern = gemm_deep_kernel<DT, LAYOUT>;
+  auto kern = gemm_deep_kernel<DT, LAYOUT, FA, FB>;
   if (!listed || !attr_set[dev]) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kDeepSmemBytes) != hipSuccess)
       return check_launch("hipFuncSetAttribute(gemm_deep)");
@@ -320,6 +398,16 @@ int launch_deep(const GemmParams& p, hipStream_t s) {
 // Launches whose 128x128 tiles fit one round of the workgroups: for certain, or with a fifth to spare by the likely number of row tiles (a
 // group's last one half full, one at least).  More rounds of small tiles lose to the larger tiles' kernels: 8 groups of 4096 rows, N = 1536,
 // K = 2048 (432 tiles): 34 us there, 52 here; at 252 tiles 32.6 and 31.0.  Masked launches: counts anywhere up to the slots, so for certain only.
+static bool few_tiles(const GemmParams& p) {
+  int grid = num_cus();
+  if (p.grid_limit > 0 && p.grid_limit < grid) grid = p.grid_limit;
+  const int64_t cols = (p.N + 127) / 128;
+  if (p.mode == MODE_MASKED) return p.G * ((p.m_stride + 127) / 128) * cols <= grid;
+  const int64_t used = p.m_total < p.G ? p.m_total : p.G;  // groups that can have rows
+  const int64_t most = (p.m_total + 127 * used) / 128, half_full = p.m_total / 128 + used / 2, likely = half_full > used ? half_full : used;
+  return most * cols <= grid || 5 * likely * cols <= 4 * grid;
+}
+
 bool deep_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   if (dt != DT_BF16 && dt != DT_F16) return false;
   if (layout != DEEP_NT && layout != DEEP_NN) return false;
@@ -328,14 +416,24 @@ bool deep_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   if ((p.N & 7) != 0 || p.K < 8 || (p.K & 7) != 0) return false;
   if ((int64_t)p.K * 2 * 128 >= (1ll << 30) || (int64_t)p.N * 2 * 128 >= (1ll << 30)) return false;
   if (layout == DEEP_NN && ((int64_t)p.K + 64) * p.N * 2 >= (1ll << 30)) return false;
-  if (any_size) return true;
-  int grid = num_cus();
-  if (p.grid_limit > 0 && p.grid_limit < grid) grid = p.grid_limit;
-  const int64_t cols = (p.N + 127) / 128;
-  if (p.mode == MODE_MASKED) return p.G * ((p.m_stride + 127) / 128) * cols <= grid;
-  const int64_t used = p.m_total < p.G ? p.m_total : p.G;  // groups that can have rows
-  const int64_t most = (p.m_total + 127 * used) / 128, half_full = p.m_total / 128 + used / 2, likely = half_full > used ? half_full : used;
-  return most * cols <= grid || 5 * likely * cols <= 4 * grid;
+  return any_size || few_tiles(p);
+}
+
+// The same for FP8 operands with per-channel scales.
+bool deep_fp8_supported(const GemmParams& p, bool any_size) {
+  if (p.mode != MODE_MG || p.G > 256 || (p.N & 7) != 0 || p.K < 16 || (p.K & 15) != 0) return false;
+  if ((int64_t)p.K * 128 >= (1ll << 30) || (int64_t)p.N * 2 * 128 >= (1ll << 30)) return false;
+  return any_size || few_tiles(p);
+}
+
+template <int FA, int FB>
+static int launch_deep_fp8_out(const GemmParams& p, int out_dt, hipStream_t s) {
+  return out_dt == DT_F16 ? launch_deep<DT_F16, DEEP_FP8, FA, FB>(p, s) : launch_deep<DT_BF16, DEEP_FP8, FA, FB>(p, s);
+}
+
+int launch_deep_fp8(const GemmParams& p, int ta, int tb, int out_dt, hipStream_t s) {
+  if (ta == DT_E4M3) return tb == DT_E4M3 ? launch_deep_fp8_out<0, 0>(p, out_dt, s) : launch_deep_fp8_out<0, 1>(p, out_dt, s);
+  return tb == DT_E4M3 ? launch_deep_fp8_out<1, 0>(p, out_dt, s) : launch_deep_fp8_out<1, 1>(p, out_dt, s);
 }
 
 int launch_deep_16bit(const GemmParams& p, int dt, int layout, hipStream_t s) {
