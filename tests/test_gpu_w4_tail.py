@@ -130,7 +130,7 @@ def test_the_default_route_of_masked_launches(dtype, K, masked, wide):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("num_cu", [8, 3, 1])  # full and half tiles in every order, in one workgroup
+@pytest.mark.parametrize("num_cu", [8, 3, 1, 32, 64])  # full and half tiles in every order, in one workgroup; last rounds cut into half tiles
 @pytest.mark.parametrize("K", [256, 320, 512])
 @pytest.mark.parametrize("N, trans_b", [(520, True), (512, False), (264, False)])
 @pytest.mark.parametrize("sizes", [[128, 1, 64, 65], [129, 384, 16, 200, 300, 127, 640], [256, 17, 256, 0, 385]])

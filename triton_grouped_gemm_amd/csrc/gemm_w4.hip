@@ -152,9 +152,16 @@ __global__ __launch_bounds__(W4Cfg::THREADS) __attribute__((amdgpu_num_vgpr(64))
   const int ld = p.K * 2;  // row pitch of A and of B in bytes; K is a multiple of 128 (w4_supported) unless TAIL
   const int kt_all = TAIL ? max(4, (p.K + 2 * BK4 - 1) / (2 * BK4) * 2) : p.K / BK4;  // slabs per tile
   // Copy k (0..7) of an operand's slab by this wave is copy instruction wave + 4 k of the slab: rows 8 (wave + 4 k) ...
-  // + 7.  The per-lane source offset of copy 0 within the tile's window is fixed for the launch; the others' distance from it and the slab's offset along
-  // K travel in the instruction's scalar offset, which the range check of the window counts in: rows behind the valid ones stay behind its end.
-  const int vo = Op::lane_voff(lane, wave % Op::NPAT, ld) + wave * Op::RPI * ld;
+  // + 7.  Its per-lane source offset within the tile's window is fixed for the launch and kept in a register; the slab's offset along K travels in the
+  // instruction's scalar offset, which the range check of the window counts in: rows behind the valid ones stay behind its end.  One register for all
+  // copies, with their distances from the first added to the scalar offset in front of each, costs 1.5 % of a launch (64 groups, 126593 rows, N = 4096,
+  // K = 3072: 2.43 against 2.38 ms); the empty statements keep the compiler from computing the offsets anew instead.
+  int vo[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    vo[k] = Op::lane_voff(lane, wave % Op::NPAT, ld) + (wave + 4 * k) * Op::RPI * ld;
+    asm volatile("" : "+v"(vo[k]));
+  }
   static_assert(Op::NPAT == 2, "the swizzle pattern of copy wave + 4 k is that of copy wave");
   // NN: B's copies have offsets of their own (two token rows of 512 bytes per copy, row pitch 2 N)
   const int ld_b = (B_KMAJOR ? p.K : p.N) * 2;
@@ -162,18 +169,13 @@ __global__ __launch_bounds__(W4Cfg::THREADS) __attribute__((amdgpu_num_vgpr(64))
   // column c of the multiply) holds column 128 h + 8 c + j of the tile, so that a lane's results of the eight column
   // blocks are eight neighbouring outputs of a row and leave as one 16-byte store without passing through LDS.
   // LDS row 8 (wave + 4 k) + lane / 8: h = k / 4, j = 2 (k % 4) + wave / 2, c = 8 (wave % 2) + lane / 8
-  // (NN: two swizzle patterns, of the even and the odd copies)
-  int vo_b[B_KMAJOR ? 1 : 2];
-  if (B_KMAJOR) {
-    vo_b[0] = Op::lane_voff(lane, wave % Op::NPAT, ld) + (8 * (8 * (wave & 1) + lane / Op::CPR) + (wave >> 1) - lane / Op::CPR) * ld;
-  } else {
+  int vo_b[8];
 #pragma unroll
-    for (int k = 0; k < (B_KMAJOR ? 1 : 2); ++k) vo_b[k] = OpB::lane_voff(lane, (wave + 4 * k) % OpB::NPAT, ld_b) + wave * OpB::RPI * ld_b;
+  for (int k = 0; k < 8; ++k) {
+    vo_b[k] = B_KMAJOR ? Op::lane_voff(lane, wave % Op::NPAT, ld) + (8 * (8 * (wave & 1) + lane / Op::CPR) + (wave >> 1) - lane / Op::CPR + 128 * (k >> 2) + 2 * (k & 3)) * ld
+                       : OpB::lane_voff(lane, (wave + 4 * k) % OpB::NPAT, ld_b) + (wave + 4 * k) * OpB::RPI * ld_b;
+    asm volatile("" : "+v"(vo_b[k]));
   }
-  static_assert(B_KMAJOR || OpB::NPAT == 8, "the swizzle pattern of copy wave + 4 k is that of copy wave or of copy wave + 4");
-  const int row_a = __builtin_amdgcn_readfirstlane(ld), row_b = __builtin_amdgcn_readfirstlane(ld_b);
-  auto far_a = [&](int k) __attribute__((always_inline)) { return 4 * Op::RPI * k * row_a; };  // copy k's distance from copy 0
-  auto far_b = [&](int k) __attribute__((always_inline)) { return (B_KMAJOR ? 128 * (k >> 2) + 2 * (k & 3) : 4 * OpB::RPI * k) * row_b; };
 
   // LDS addresses of the fragment reads relative to a slab buffer (see gemm_fast.hip for the layout)
   uint32_t a_rd[2], b_rd[B_KMAJOR ? 2 : 8];
@@ -211,11 +213,27 @@ __global__ __launch_bounds__(W4Cfg::THREADS) __attribute__((amdgpu_num_vgpr(64))
   };
   const TileWalk walk64 = sched_walk(num_tiles, p.tile_split != 0);
   struct { int first, end, stride; } walk = {(int)walk64.first, (int)walk64.end, (int)walk64.stride};
+  // A last round of at most half an XCD's workgroups is cut into half tiles, one each: tile ids from tail_first on count halves there.  The launch
+  // ends with the time of a half tile in place of a whole one (8 groups, 11560 rows, N = 1536, K = 4096: 169 -> 153 us; 128 groups, 32768 rows,
+  // N = 1536, K = 2048: 259 -> 250).  A longer last round is left whole: cut, it would be more than one half tile for some workgroup, as long as the whole.
+  int tail_first = walk.end;
+  if (p.tile_split != 0 && (gridDim.x & 7) == 0) {
+    const int per_xcd = (int)gridDim.x >> 3, begin = walk.first - (int)(blockIdx.x >> 3), rest = (walk.end - begin) % per_xcd;
+    if (2 * rest <= per_xcd) {
+      tail_first = walk.end - rest;
+      walk.end = tail_first + 2 * rest;
+    }
+  }
   const int row_bytes = __builtin_amdgcn_readfirstlane(ld);
   int hint_g = -1;
   auto tile_at = [&](int id, Tile& t) __attribute__((always_inline))  {  // false: the walk has ended
     if (id >= walk.end) { t.g = 0; t.row0 = 0; t.rows = 0; t.n0 = 0; t.k0 = t.k1 = 0; return false; }
-    const Tile v = sched_tile<C::BM, C::BN>(p, sched, id, hint_g);
+    Tile v = sched_tile<C::BM, C::BN>(p, sched, id < tail_first ? id : tail_first + ((id - tail_first) >> 1), hint_g);
+    if (id >= tail_first) {  // rows 0 .. 127 of the tile or those behind, if any
+      const int at = ((id - tail_first) & 1) * (C::BM / 2), left = v.rows - at;
+      v.row0 += at;
+      v.rows = left < 0 ? 0 : (left < C::BM / 2 ? left : C::BM / 2);
+    }
     // the same in every lane; in scalar registers, so that what depends on it branches as a wave
     t.g = __builtin_amdgcn_readfirstlane(v.g);
     t.row0 = (int64_t)uniform64((uint64_t)v.row0);
@@ -242,8 +260,8 @@ __global__ __launch_bounds__(W4Cfg::THREADS) __attribute__((amdgpu_num_vgpr(64))
   // A chunk k of the slab at offset koff of window ra -> register set SET
   auto load_s = [&](auto Kc, auto SETc, const i32x4_t& ra, int koff) __attribute__((always_inline))  {
     constexpr int k = decltype(Kc)::value, kq = k + 8 * decltype(SETc)::value;
-    const int v = TAIL ? vo | mask_s : vo, off = koff + far_a(k);
-#define TGG_W4_F(lo, hi) asm volatile("buffer_load_dwordx4 v[" lo ":" hi "], %0, %1, %2 offen" : : "v"(v), "s"(ra), "s"(off) : "memory", TGG_W4_GA_CLOBBER);
+    const int v = TAIL ? vo[k] | mask_s : vo[k];
+#define TGG_W4_F(lo, hi) asm volatile("buffer_load_dwordx4 v[" lo ":" hi "], %0, %1, %2 offen" : : "v"(v), "s"(ra), "s"(koff) : "memory", TGG_W4_GA_CLOBBER);
     TGG_W4_GA(kq, TGG_W4_F)
 #undef TGG_W4_F
   };
@@ -262,16 +280,16 @@ __global__ __launch_bounds__(W4Cfg::THREADS) __attribute__((amdgpu_num_vgpr(64))
   };
   auto copy_d = [&](auto Kc, const i32x4_t& rb, int koff) __attribute__((always_inline))  {
     constexpr int k = decltype(Kc)::value;
-    const int v = TAIL && B_KMAJOR ? vo_b[0] | mask_d : vo_b[B_KMAJOR ? 0 : k & 1], off = koff + far_b(k);
+    const int v = TAIL && B_KMAJOR ? vo_b[k] | mask_d : vo_b[k];
     // (the staged chunks' registers are listed here too: the compiler must not hold a value in them in a K step without loads either)
-    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" : : "v"(v), "s"(rb), "s"(off) : "memory", TGG_W4_GA_CLOBBER);
+    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" : : "v"(v), "s"(rb), "s"(koff) : "memory", TGG_W4_GA_CLOBBER);
   };
   // a slab's A copy k straight to LDS (prologue only)
   auto copy_direct = [&](auto Kc, auto ISBc, const i32x4_t& ra, int koff, uint32_t buf_addr) __attribute__((always_inline))  {
     constexpr int k = decltype(Kc)::value;
-    const int v = decltype(ISBc)::value ? vo_b[B_KMAJOR ? 0 : k & 1] : vo, off = koff + (decltype(ISBc)::value ? far_b(k) : far_a(k));
+    const int v = decltype(ISBc)::value ? vo_b[k] : vo[k];
     asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds"
-                 : : "s"(buf_addr), "n"(4 * k * 1024), "v"(v), "s"(ra), "s"(off) : "memory", "m0", "scc");
+                 : : "s"(buf_addr), "n"(4 * k * 1024), "v"(v), "s"(ra), "s"(koff) : "memory", "m0", "scc");
   };
   const uint32_t wave_buf = smem_addr + wave * 1024;  // copy `wave` of buffer 0's A slab
 
@@ -419,21 +437,31 @@ __global__ __launch_bounds__(W4Cfg::THREADS) __attribute__((amdgpu_num_vgpr(64))
   Win nxt;
   Tile nxt_tile;
   const int k_bytes = TAIL ? __builtin_amdgcn_readfirstlane(kt_all * 128) : row_bytes;  // a tile's extent along K in bytes: where a cursor moves on to the next tile
-  auto advance_s = [&]() __attribute__((always_inline))  {
-    const bool wrap = koff_s + 128 == k_bytes;
-    koff_s = wrap ? 0 : koff_s + 128;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) rs_c[q] = wrap ? nxt.rs[q] : rs_c[q];
-    if (TAIL) mask_s = koff_s + chunk_off >= row_bytes ? kNoFetch : 0;
+  // A cursor moves on to the next slab in four parts, one to a gap between two multiplies: where all of them stand in one gap the matrix pipe idles.
+  bool wrap = false;
+  auto advance_s = [&](int part) __attribute__((always_inline))  {
+    __builtin_amdgcn_sched_barrier(0);
+    if (part == 0) {
+      wrap = koff_s + 128 == k_bytes;
+      koff_s = wrap ? 0 : koff_s + 128;
+    } else {
+      rs_c[part - 1] = wrap ? nxt.rs[part - 1] : rs_c[part - 1];
+      if (TAIL && part == 3) mask_s = koff_s + chunk_off >= row_bytes ? kNoFetch : 0;
+    }
+    __builtin_amdgcn_sched_barrier(0);
   };
   const int d_step = B_KMAJOR ? 128 : __builtin_amdgcn_readfirstlane(64 * ld_b);         // B's slab offset per slab ...
   const int d_bytes = B_KMAJOR ? k_bytes : __builtin_amdgcn_readfirstlane((TAIL ? kt_all * BK4 : p.K) * ld_b);   // ... and where it reaches the next tile
-  auto advance_d = [&]() __attribute__((always_inline))  {
-    const bool wrap = koff_d + d_step == d_bytes;
-    koff_d = wrap ? 0 : koff_d + d_step;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) rd_c[q] = wrap ? nxt.rd[q] : rd_c[q];
-    if (TAIL && B_KMAJOR) mask_d = koff_d + chunk_off >= row_bytes ? kNoFetch : 0;
+  auto advance_d = [&](int part) __attribute__((always_inline))  {
+    __builtin_amdgcn_sched_barrier(0);
+    if (part == 0) {
+      wrap = koff_d + d_step == d_bytes;
+      koff_d = wrap ? 0 : koff_d + d_step;
+    } else {
+      rd_c[part - 1] = wrap ? nxt.rd[part - 1] : rd_c[part - 1];
+      if (TAIL && B_KMAJOR && part == 3) mask_d = koff_d + chunk_off >= row_bytes ? kNoFetch : 0;
+    }
+    __builtin_amdgcn_sched_barrier(0);
   };
 
   // One K step: 64 multiplies on fragment set CUR (when MUL); the 16 fragments of K step NKS of the slab at nb_off go
@@ -510,16 +538,21 @@ __global__ __launch_bounds__(W4Cfg::THREADS) __attribute__((amdgpu_num_vgpr(64))
         constexpr int w = n - G1, l = n - G1 - L1;
         if constexpr (w >= 0 && w % D1 == 0 && w / D1 < 8) write_s(TGG_W4_I(w / D1), SETc, wr_addr);
         if constexpr (l >= 0 && l % D1 == 0 && l / D1 < 8) load_s(TGG_W4_I(l / D1), SETc, rs_c, koff_s);
+        constexpr int part = n - (NS == 4 ? 28 : 56);  // behind the last load
+        if constexpr (part >= 0 && part < 4) advance_s(part);
       }
       if constexpr (ROLE == 2) {
         constexpr int m = n - G2, c = n - G2 - 1;
         if constexpr (m >= 0 && m % D2 == 0 && m / D2 < 8) copy_d_m0(TGG_W4_I(m / D2), cp_addr);
         if constexpr (c >= 0 && c % D2 == 0 && c / D2 < 8) copy_d(TGG_W4_I(c / D2), rd_c, koff_d);
+        if constexpr (NS == 4) {
+          if constexpr (n == 31) for_each<4>([&](auto Pc) __attribute__((always_inline)) { advance_d(decltype(Pc)::value); });
+        } else {
+          constexpr int part = n - 56;
+          if constexpr (part >= 0 && part < 4) advance_d(part);
+        }
       }
     });
-    if constexpr (ROLE == 1) advance_s();
-    if constexpr (ROLE == 2) advance_d();
-    __builtin_amdgcn_sched_barrier(0);  // the scalar work sits in front of the wait and not in the gaps behind it
     if constexpr (ROLE == 2) asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory", TGG_W4_ACC_CLOBBER);
     else if constexpr (ROLE == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(EPI ? 24 : 8) : "memory", TGG_W4_ACC_CLOBBER);
     else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : : : "memory", TGG_W4_ACC_CLOBBER);
