@@ -281,7 +281,7 @@ int tgg_debug_queue_order(int grid, int draws, int32_t* out);
  *                        16-bit M-grouped / masked: launches of more than four rounds of 256x128 tiles, and smaller M-grouped ones of at
  *                        least 128 rows per group whose likely tiles cost two rounds of K = 2048; K from 768 on where it is no multiple of 128
  *                        or N is none of 256 with trans_b = 0 (masked launches need both multiples).  Masked
- *                        launches, those with fewer than 512 rows per group on average and the smaller ones enqueue both kernels,
+ *                        launches and those with fewer than 200 rows per group on average enqueue both kernels,
  *                        which decide on the device from the sizes which of them runs;
  *                        16-bit K-grouped: launches of one and a half rounds of 256x256 tiles and more, but for segments of less than 32-96
  *                        tokens on few workgroups or without a queue;
