@@ -143,3 +143,23 @@ def test_half_tiles(dtype, num_cu, K, N, trans_b, sizes):
     b = (torch.randn(len(sizes), *((N, K) if trans_b else (K, N)), device=dev, generator=gen) * K ** -0.5).to(dtype)
     run = lambda: m_grouped_gemm(a, b, s, trans_b, numSM=num_cu)
     assert torch.equal(_with("four_wave", 2, 1, run), _with("force_generic", 1, 0, run))
+
+
+@pytest.mark.parametrize("trans_b", [True, False])
+@pytest.mark.parametrize("N, K, sizes, num_cu", [
+    (512, 768, [1, 1023, 256], 8),        # more than 1.15 rounds of likely tiles, of one group mostly
+    (256, 776, [400, 0, 800], 8),         # a tail, too short for it
+    (264, 1032, [500, 130, 138], 8),      # one that is long enough; N cut as well
+    (256, 768, [400, 3, 797], 8),         # 0.81 of a round
+    (256, 896, [256, 767, 1], 8),         # 0.69 of one
+    (256, 768, [512, 0, 1, 511] * 75, -1),  # more groups than threads
+])
+def test_mid_size_launches(trans_b, N, K, sizes, num_cu):
+    """Launches on both sides of the lines between the four-wave and the eight-wave kernels: the same bits."""
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(N + K)
+    s = torch.tensor(sizes, dtype=torch.int32, device=dev)
+    a = torch.randn(sum(sizes), K, device=dev, generator=gen).to(torch.bfloat16)
+    b = (torch.randn(len(sizes), *((N, K) if trans_b else (K, N)), device=dev, generator=gen) * K ** -0.5).to(torch.bfloat16)
+    run = lambda: _with("deep", 0, 1, lambda: m_grouped_gemm(a, b, s, trans_b, numSM=num_cu))
+    assert torch.equal(run(), _with("force_generic", 1, 0, run))
