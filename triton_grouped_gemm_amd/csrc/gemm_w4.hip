@@ -736,7 +736,7 @@ bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   const int64_t full_2 = (2 * ((p.m_total + 255) / 256) + p.G) * tiles_n, half_2 = (2 * ((p.m_total + 127) / 128) + p.G) * tiles_n;  // twice the likely tiles
   const int64_t rounds_full = (full_2 + 2 * grid - 1) / (2 * grid), rounds_half = (half_2 + 2 * grid - 1) / (2 * grid);
   // Launches with 256 rows a group and more run on this kernel alone from 1.15 rounds of likely tiles on, and from 0.7 to 0.9 of one: 218 random ones 0.90 of
-  // the eight-wave kernel's time (0.79-1.11, five of them above 1.01; 8 groups of 2925 rows, N = 2048, K = 2048: 93 -> 83 us; 32 of 557, N = 840, K = 512: 35 -> 28).  Around
+  // the eight-wave kernel's time (0.79-1.11, five of them above 1.01; 8 groups of 2925 rows, N = 2048, K = 2048: 93 -> 83 us; 16 of 1725, N = 768, K = 2816: 148 -> 124).  Around
   // half a round and one the eight-wave kernel's narrower tiles just fit where these just don't: 42 at 0.48-0.7 rounds 1.00 (up to 1.28), 29 at
   // 0.9-1.15 0.96 (up to 1.15); with 200-256 rows a group 31 launches 1.01 (up to 1.31); K = 512, or up to 1000 with a tail: 0.98, up to 1.2.
   if (p.m_total >= 256 * (int64_t)p.G && p.K >= (needs_tail(p, layout) ? 1024 : 768) &&
