@@ -264,6 +264,12 @@ int tgg_debug_generic_extents(int kind, const int64_t* sizes, const int32_t* row
  * together list every id once and each of them in growing order. */
 int tgg_debug_queue_order(int grid, int draws, int32_t* out);
 
+/* Test hook, host only: what a 16-bit launch of these sizes enqueues under the present options: *route = 0 the shape-agnostic kernel, 1 the
+ * eight-wave kernels, 2 the four-wave kernel, 3 both of these, one of which the group sizes choose on the device, 4 the kernel for few tiles,
+ * 5 the four-wave weight-gradient kernel.  Modes as in tgg_debug_tile_order (0, 1, 2; 4 K-grouped without a queue or workspace, K unused).  The reference
+ * chooses by architecture and autotuning (gemm/BF16/m_grouped_gemm_TMA.py:25-52). */
+int tgg_debug_route_16bit(int mode, int G, int64_t m_total, int64_t aux, int N, int K, int trans_b, int num_cu, int32_t* route);
+
 /* Library controls (process-wide test and tuning hooks, not a per-call interface: every launch reads each option
  * once, atomically, so a thread that changes one while another thread launches decides only which value that launch
  * sees; returns 1 for an unknown key):

@@ -207,24 +207,33 @@ static void lend_workspace(GemmParams& p, int64_t need, void* workspace, int64_t
   p.split_slots = kg_split_slots(p);
 }
 
+// What a 16-bit launch enqueues.  A configuration of the other kernels that has been asked for stays what runs.
+enum Route16 : int { ROUTE_GENERIC = 0, ROUTE_EIGHT_WAVE = 1, ROUTE_FOUR_WAVE = 2, ROUTE_FOUR_OR_EIGHT = 3, ROUTE_DEEP = 4, ROUTE_WGRAD = 5 };
+static Route16 route_16bit(const GemmParams& p, int dt, int layout) {
+  if (g_force_generic.load()) return ROUTE_GENERIC;
+  const int four_wave = g_four_wave.load(), deep = g_deep.load();
+  if ((deep == 2 || (deep == 1 && four_wave == 1 && g_variant.load() == 0)) && deep_supported(p, dt, layout, deep == 2)) return ROUTE_DEEP;
+  if (four_wave && w4_supported(p, dt, layout, four_wave == 2))
+    return !w4_decided_on_device(p) || four_wave == 2 ? ROUTE_FOUR_WAVE : ROUTE_FOUR_OR_EIGHT;
+  if (four_wave && layout == 2 && (p.split_ws || wgrad_supported(p, dt, four_wave == 2))) return ROUTE_WGRAD;
+  return fast_supported(p, dt, layout) ? ROUTE_EIGHT_WAVE : ROUTE_GENERIC;
+}
+
 static int dispatch_16bit(const GemmParams& p, int dt, int layout, hipStream_t s) {
-  const int force_generic = g_force_generic.load(), four_wave = g_four_wave.load();
-  // a configuration of the other kernels that has been asked for stays what runs
-  if (const int deep = g_deep.load(); !force_generic && (deep == 2 || (deep == 1 && four_wave == 1 && g_variant.load() == 0)) &&
-                                      deep_supported(p, dt, layout, deep == 2))
-    return launch_deep_16bit(p, dt, layout, s);
-  if (!force_generic && four_wave && w4_supported(p, dt, layout, four_wave == 2)) {
-    if (!w4_decided_on_device(p) || four_wave == 2) return launch_w4_16bit(p, dt, layout, s);
-    // whether 256-row tiles pay depends on the sizes; both kernels look at them and exactly one runs
-    GemmParams q = p;
-    q.wide_gate = 1;
-    if (int e = launch_w4_16bit(q, dt, layout, s)) return e;
-    q.wide_gate = 2;
-    return launch_fast_16bit(q, dt, layout, s);
+  switch (route_16bit(p, dt, layout)) {
+    case ROUTE_DEEP: return launch_deep_16bit(p, dt, layout, s);
+    case ROUTE_FOUR_WAVE: return launch_w4_16bit(p, dt, layout, s);
+    case ROUTE_FOUR_OR_EIGHT: {  // whether 256-row tiles pay depends on the sizes; both kernels look at them and exactly one runs
+      GemmParams q = p;
+      q.wide_gate = 1;
+      if (int e = launch_w4_16bit(q, dt, layout, s)) return e;
+      q.wide_gate = 2;
+      return launch_fast_16bit(q, dt, layout, s);
+    }
+    case ROUTE_WGRAD: return launch_wgrad_16bit(p, dt, s);
+    case ROUTE_EIGHT_WAVE: return launch_fast_16bit(p, dt, layout, s);
+    default: return launch_generic_16bit(p, dt, layout, s);
   }
-  if (!force_generic && four_wave && layout == 2 && (p.split_ws || wgrad_supported(p, dt, four_wave == 2))) return launch_wgrad_16bit(p, dt, s);
-  if (!force_generic && fast_supported(p, dt, layout)) return launch_fast_16bit(p, dt, layout, s);
-  return launch_generic_16bit(p, dt, layout, s);
 }
 
 }  // namespace tgg
@@ -771,6 +780,20 @@ int tgg_debug_queue_order(int grid, int draws, int32_t* out) {
   if (draws < 0) return set_error("negative number of draws");
   for (int xq = 0; xq < 8; ++xq)
     for (int n = 0; n < draws; ++n) out[(int64_t)xq * draws + n] = sched_queue_id(n, xq, grid >> 3);
+  return 0;
+}
+
+int tgg_debug_route_16bit(int mode, int G, int64_t m_total, int64_t aux, int N, int K, int trans_b, int num_cu, int32_t* route) {
+  if (!route) return set_error("null pointer");
+  if (G < 1 || G > TGG_MAX_GROUPS || m_total < 1 || N < 1) return set_error("bad G=%d, m_total=%lld or N=%d", G, (long long)m_total, N);
+  GemmParams p;
+  if (mode == MODE_MG) p = params_m_grouped(nullptr, nullptr, nullptr, nullptr, 0, G, m_total, N, K, trans_b, num_cu);
+  else if (mode == MODE_MG_PAD) p = params_padded(nullptr, nullptr, nullptr, nullptr, 0, nullptr, G, m_total, N, K, (int)aux, num_cu);
+  else if (mode == MODE_MASKED) p = params_masked(nullptr, nullptr, nullptr, nullptr, 0, G, aux, m_total, N, K, trans_b, num_cu);
+  else if (mode == MODE_KG_COUNT) p = params_k_grouped_sizes(nullptr, nullptr, nullptr, nullptr, 0, G, (int)m_total, N, aux, num_cu, nullptr);
+  else return set_error("mode %d", mode);
+  const int layout = mode == MODE_KG_COUNT ? 2 : (mode == MODE_MG_PAD || trans_b ? 0 : 1);
+  *route = route_16bit(p, TGG_BF16, layout);
   return 0;
 }
 

@@ -710,9 +710,11 @@ bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   // NN: a group's B, with the rows that the tail may add, within 2 GiB
   if (layout == W4_NN && ((int64_t)p.K + 128) * p.N * 2 >= (1ll << 31)) return false;
   if (p.mode != MODE_MG && p.mode != MODE_MG_PAD && p.mode != MODE_MASKED) return false;
-  // launches whose groups may be small are decided on the device (w4_decided_on_device), by a predicate that needs
-  // one thread of this kernel per group
-  if (w4_decided_on_device(p) && p.G > W4Cfg::THREADS) return false;
+  // Launches whose groups may be small are decided on the device (w4_decided_on_device), by a predicate that needs
+  // one thread of this kernel per group.  With more groups than threads one of them makes the whole table, 0.12-0.2 us a group, which
+  // the eight-wave kernels' 512 threads do together: 367 groups of 256 rows, N = 512, K = 768 106 us there, 171 here; with 512 rows and more per group it is
+  // a few percent of a launch and this kernel is the faster one all the same.
+  if (p.G > W4Cfg::THREADS && (w4_decided_on_device(p) || p.m_total < 512 * (int64_t)p.G)) return false;
   if (p.q_fmt != 0 || p.G > kFastMaxGroups) return false;
   if ((p.N & 7) != 0 || p.K < 8 || (p.K & 7) != 0) return false;
   if ((int64_t)p.K * 2 * 256 >= (1ll << 30)) return false;
