@@ -285,10 +285,9 @@ int tgg_debug_route_16bit(int mode, int G, int64_t m_total, int64_t aux, int N, 
  *                        groups (512 where a launch is not decided on the device): 1 (default) = where they are the faster ones; 0 =
  *                        eight-wave kernels only; 2 = on every launch that they can take, whatever the sizes.  By default:
  *                        16-bit M-grouped / masked: launches of more than four rounds of 256x128 tiles, and smaller M-grouped ones of at
- *                        least 128 rows per group whose likely tiles cost two rounds of K = 2048, or of at least 256 whose likely tiles are
- *                        1.15 rounds and more or 0.7-0.9 of one (K from 768 on, 1024 with a tail); K from 768 on where it is no multiple of 128
+ *                        least 128 rows per group whose likely tiles cost two rounds of K = 2048; K from 768 on where it is no multiple of 128
  *                        or N is none of 256 with trans_b = 0 (masked launches need both multiples).  Masked
- *                        launches and those with fewer than 200 rows per group on average enqueue both kernels,
+ *                        launches, those with fewer than 512 rows per group on average and the smaller ones enqueue both kernels,
  *                        which decide on the device from the sizes which of them runs;
  *                        16-bit K-grouped: launches of one and a half rounds of 256x256 tiles and more, but for segments of less than 32-96
  *                        tokens on few workgroups or without a queue;

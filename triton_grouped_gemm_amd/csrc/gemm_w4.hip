@@ -690,13 +690,15 @@ static bool w4_large(const GemmParams& p) {
   return ((p.m_total + 255) / 256) * ((p.N + 127) / 128) > 4 * (int64_t)grid;
 }
 
-// Whether 256-row tiles pay depends on the group sizes, which only the device knows.  With 200 rows and more per group on
-// average they do: of 130 random launches decided on the device (Dirichlet groups, more than two rounds and fewer) none of those took longer by this
-// kernel alone (0.85-1.00, 0.98 in the mean: the launch that returns is 4-6 us), while below, 84-184 rows, it was 0.85-1.13.  Smaller groups, and masked
-// launches (counts anywhere up to the row stride), are enqueued together with the eight-wave kernel, and the two decide from the sizes which
-// of them runs.  The average is that of the operand: where the groups fill a twentieth of it, this kernel alone takes 1.1 of the eight-wave kernel's
-// time (up to 1.33; a fifth of it 0.98: 200 random launches with a tail, before half tiles).
-bool w4_decided_on_device(const GemmParams& p) { return p.mode == MODE_MASKED || p.m_total < 200 * (int64_t)p.G; }
+// Whether 256-row tiles pay depends on the group sizes, which only the device knows.  With 512 rows and more per group on
+// average they do; a masked launch (counts anywhere up to its row stride), one with smaller groups or one of fewer rounds is
+// enqueued together with the eight-wave kernel, and the two decide from the sizes which of them runs.  The average is that of the operand, whose rows the
+// groups may own in part only (a buffer of fixed size, a padded layout of small groups).  Filled whole, launches of 200-511 rows a group take 0.95 of the
+// eight-wave kernel's time by this kernel alone and 0.97 decided on the device; filled to a tenth and less 1.05-1.14 alone (15 random ones, up to
+// 1.21).  Large ones of longer groups 0.93-0.98 alone, however much of them is filled (56 random ones, a fiftieth to the whole).
+bool w4_decided_on_device(const GemmParams& p) {
+  return p.mode == MODE_MASKED || p.m_total < 512 * (int64_t)p.G || !w4_large(p);
+}
 
 // The four-wave kernel takes large M-grouped and masked launches, and M-grouped ones of 128 rows and more per group whose likely tiles
 // (every group's last one half full) cost two rounds of K = 2048 or more and would not be chosen for 128-row tiles
@@ -710,11 +712,10 @@ bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   // NN: a group's B, with the rows that the tail may add, within 2 GiB
   if (layout == W4_NN && ((int64_t)p.K + 128) * p.N * 2 >= (1ll << 31)) return false;
   if (p.mode != MODE_MG && p.mode != MODE_MG_PAD && p.mode != MODE_MASKED) return false;
-  // Launches whose groups may be small are decided on the device (w4_decided_on_device), by a predicate that needs
-  // one thread of this kernel per group.  With more groups than threads one of them makes the whole table, 0.12-0.2 us a group, which
-  // the eight-wave kernels' 512 threads do together: 367 groups of 256 rows, N = 512, K = 768 106 us there, 171 here; with 512 rows and more per group it is
-  // a few percent of a launch and this kernel is the faster one all the same.
-  if (p.G > W4Cfg::THREADS && (w4_decided_on_device(p) || p.m_total < 512 * (int64_t)p.G)) return false;
+  // launches whose groups may be small are decided on the device (w4_decided_on_device), by a predicate that needs
+  // one thread of this kernel per group; besides, with more groups than threads one of them makes the whole table, 0.12-0.2 us a group, which the eight-wave
+  // kernels' 512 threads do together (367 groups of 256 rows, N = 512, K = 768: 106 us there, 171 here)
+  if (w4_decided_on_device(p) && p.G > W4Cfg::THREADS) return false;
   if (p.q_fmt != 0 || p.G > kFastMaxGroups) return false;
   if ((p.N & 7) != 0 || p.K < 8 || (p.K & 7) != 0) return false;
   if ((int64_t)p.K * 2 * 256 >= (1ll << 30)) return false;
@@ -737,12 +738,9 @@ bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {
   const int64_t tiles_n = (p.N + 255) / 256;
   const int64_t full_2 = (2 * ((p.m_total + 255) / 256) + p.G) * tiles_n, half_2 = (2 * ((p.m_total + 127) / 128) + p.G) * tiles_n;  // twice the likely tiles
   const int64_t rounds_full = (full_2 + 2 * grid - 1) / (2 * grid), rounds_half = (half_2 + 2 * grid - 1) / (2 * grid);
-  // Launches with 256 rows a group and more run on this kernel alone from 1.15 rounds of likely tiles on, and from 0.7 to 0.9 of one: 218 random ones 0.90 of
-  // the eight-wave kernel's time (0.79-1.11, five of them above 1.01; 8 groups of 2925 rows, N = 2048, K = 2048: 93 -> 83 us; 16 of 1725, N = 768, K = 2816: 148 -> 124).  Around
-  // half a round and one the eight-wave kernel's narrower tiles just fit where these just don't: 42 at 0.48-0.7 rounds 1.00 (up to 1.28), 29 at
-  // 0.9-1.15 0.96 (up to 1.15); with 200-256 rows a group 31 launches 1.01 (up to 1.31); K = 512, or up to 1000 with a tail: 0.98, up to 1.2.
-  if (p.m_total >= 256 * (int64_t)p.G && p.K >= (needs_tail(p, layout) ? 1024 : 768) &&
-      (20 * full_2 >= 23 * 2 * grid || (10 * full_2 >= 7 * 2 * grid && 10 * full_2 <= 9 * 2 * grid))) return true;
+  // (Fewer rounds are no safe choice: launches of 256 rows a group and more take 0.91 of the eight-wave kernel's time from 1.15 rounds of likely tiles on
+  // and from 0.7 to 0.9 of one where the groups fill the operand, but 1.03 with half of it filled, up to 1.24, and 1.1 with a tenth, up to 1.29: its narrower
+  // tiles fit what is left.  Decided on the device they would pay 4 us for 30-100.)
   return full_2 * p.K >= 2 * 4096 * (int64_t)grid && rounds_half * 3 > rounds_full * 4;
 }
 
