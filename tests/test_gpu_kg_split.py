@@ -89,6 +89,61 @@ def test_fp8(fa, fb, m, n, sizes, runs_tuned):
     assert torch.equal(out, fp8_k_grouped(x, xs.t(), y, ys.t(), s, m, n, total, G, 1 if fa == torch.float8_e4m3fn else 2, 1 if fb == torch.float8_e4m3fn else 2))
 
 
+def _planned_parts(sizes, m, n, unit, tile, part, cost, cus=256):
+    """split_plan's choice in Python integers: how many parts each group is cut into."""
+    up = lambda a, b: -(-a // b)
+    per_group = up(m, 256) * up(n, 256)
+    steps = [up(k, unit) for k in sizes]
+    share = up(sum(steps) * per_group, cus)
+    ranked = sorted(steps, reverse=True)
+    uncut = max([share] + [(t + 1) * ranked[t * cus // per_group] for t in range(256) if t * cus // per_group < len(sizes)])
+    best, chosen = None, None
+    if uncut > share + cost + tile:
+        for t in range(256):
+            c = max(8, share * (64 + t % 64) >> (8 - t // 64))
+            parts = [1 if k <= c else up(k, c) for k in steps]
+            length = [k if q == 1 else up(k, q) for k, q in zip(steps, parts)]
+            slots = sum(q for q in parts if q > 1)
+            long = [(q, k) for q, k, x in zip(parts, steps, length) if 2 * x > c]
+            n_long, sum_long = sum(q for q, _ in long), sum(k for _, k in long)
+            expected = up(n_long * per_group, cus) * sum_long // n_long if n_long else 0
+            expected = max(expected, share, max(length))
+            expected += up(sum(parts) * per_group, cus) * tile + up(slots * per_group * part, cus) + cost
+            if 0 < slots <= 2 * cus // per_group and sum(parts) <= 512 and expected + expected // 12 < uncut + up(len(sizes) * per_group, cus) * tile:
+                if best is None or expected < best:
+                    best, chosen = expected, parts
+    return chosen or [1] * len(sizes)
+
+
+@pytest.mark.parametrize("m, n, sizes", [
+    (264, 264, [2560] * 200),                                   # equal ones: nothing is cut
+    (256, 128, [37000] * 3 + [1500] * 61 + [49000, 49000, 1] + [6400] * 63),  # runs of equals, across the lanes of a wave
+    (264, 520, [4000 + 640 * (g % 7) for g in range(90)]),
+    (128, 128, [(2909 * g * g) % 9000 for g in range(130)]),    # hardly two alike
+    (64, 256, [0] * 64 + [1000000] + [3000] * 190 + [400000]),  # every thread's group
+    (2304, 1152, [130, 40000, 64]),
+])
+def test_the_plan(m, n, sizes):
+    """The device's plan, which takes a group at a time from lanes' registers, runs of equals at once and divides by reciprocals, against the plan's
+    definition: how many parts each group is in; and the result, exact."""
+    dev = torch.device("cuda:0")
+    assert torch.cuda.get_device_properties(dev).multi_processor_count == 256
+    G, total = len(sizes), sum(sizes)
+    gen = torch.Generator(device=dev).manual_seed(G)
+    a, b = (torch.randint(-1, 2, (total, w), device=dev, generator=gen).bfloat16() for w in (m, n))
+    s = torch.tensor(sizes, dtype=torch.int32, device=dev)
+    need = _cut(G, m, n, total, False)
+    assert need > 0
+    workspace, c = torch.empty(need, dtype=torch.uint8, device=dev), torch.full((G, m, n), float("nan"), device=dev, dtype=torch.bfloat16)
+    _native.call("tgg_k_grouped_gemm_split", a.data_ptr(), b.data_ptr(), c.data_ptr(), s.data_ptr(), 0, G, m, n, total, _native.BF16, -1,
+                 _native.work_queue(dev).data_ptr(), workspace.data_ptr(), need, _native.stream_of(a))
+    assert _parts(workspace, G) == _planned_parts(sizes, m, n, 64, 3, 20, 8)  # WgradSplitCost
+    at = 0
+    for g, k in enumerate(sizes):
+        assert torch.equal(c[g], (a[at:at + k].float().t() @ b[at:at + k].float()).bfloat16()), g
+        at += k
+
+
 def test_what_is_not_cut():
     assert _cut(128, 2048, 1536, 32768, False) == 0   # many tiles, short segments
     assert _cut(4, 256, 256, 4096, False) == 0        # short segments

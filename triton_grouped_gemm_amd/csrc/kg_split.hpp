@@ -18,6 +18,17 @@ template <int U, int TILE_COST, int PART_COST, int SUM_COST> struct SplitCost {
   static constexpr int U_TOKENS = U, TILE = TILE_COST, PART = PART_COST, SUM = SUM_COST;
 };
 
+// ceil(a / b) for 0 <= a < 2^26 and 1 <= b < 2^26, by a reciprocal and its corrections: an integer division is four times as many instructions, and
+// a plan makes one for every group.  The estimate is off by less than 2^-21 of the quotient and one; its remainder over b makes that one at most.
+TGG_DEV int split_div_up(int a, int b) {
+  const float r = __builtin_amdgcn_rcpf((float)b);
+  const int x = a + b - 1;
+  int q = (int)((float)x * r);
+  q += (int)((float)(x - q * b) * r);
+  const int left = x - q * b;
+  return q + (left >= b ? 1 : 0) - (left < 0 ? 1 : 0);
+}
+
 // The smallest of the workgroup's values (256 threads, all of which must call this).
 template <class Table>
 TGG_DEV int64_t split_block_min(int64_t v, Table& t) {
@@ -41,9 +52,13 @@ TGG_DEV int64_t split_block_min(int64_t v, Table& t) {
 // that is what an uncut launch is expected to take.  Part lengths: the best of 256 candidates, one per thread, from a
 // quarter of an even share to four of them; expected are an even share or the rounds that the tiles of more than half that length make;
 // a cut is made for a twelfth of the time at least.
+// Every candidate is a look at all groups, and every workgroup makes the plan.  With a read from LDS and two integer divisions per group that took 0.16 us a group in front
+// of the launch; with the groups in lanes' registers, runs of equal ones counted at once and the divisions by reciprocals (the same plan) 0.01-0.08.
+// 53 groups of 376 x 1192, 2180 tokens each (nothing to cut) 189 -> 180 us, 173 by a launch that does not ask; 200 of 264 x 264, 512000 tokens, equal 284 -> 250,
+// unequal 323 -> 270; 108 of 80 x 136, 3738 tokens 175 -> 102.
 template <class Cost, class Table>
 TGG_DEV int split_plan(const GemmParams& p, Table& t, int32_t* meta, int tiles_per_group) {
-  const int tid = threadIdx.x, G = p.G, P = (int)gridDim.x;
+  const int tid = threadIdx.x, lane = lane_id(), G = p.G, P = (int)gridDim.x;
   constexpr int U = Cost::U_TOKENS, kNever = 0x3fffffff;
   const int my_rows = tid < G ? t.rows[tid] : 0;
   const int my_steps = (my_rows + U - 1) / U;
@@ -61,16 +76,33 @@ TGG_DEV int split_plan(const GemmParams& p, Table& t, int32_t* meta, int tiles_p
     const int e = tid >> 6, f = tid & 63;
     int c = (int)(((int64_t)share * (64 + f)) >> (8 - e));
     if (c < 8) c = 8;
-    int parts = 0, slots = 0, longest = 0, n_long = 0, sum_long = 0;
-    for (int g = 0; g < G; ++g) {
-      const int steps = (t.rows[g] + U - 1) / U;
-      const int n = steps <= c ? 1 : (steps + c - 1) / c;
-      const int len = n == 1 ? steps : (steps + n - 1) / n;
-      parts += n;
-      slots += n > 1 ? n : 0;
+    const FixedDiv by_c(c);
+    const int c_least = __builtin_amdgcn_readfirstlane(c);  // of the wave's candidates
+    int parts = 0, slots = 0, longest = 0, n_long = 0, sum_long = 0, run = 0, seen = 0;
+    auto count = [&]() __attribute__((always_inline)) {  // `run` groups of `seen` steps
+      int n = 1, len = seen;
+      if (seen > c_least && seen > c) {
+        n = (int)by_c.div((uint32_t)(seen + c - 1));
+        len = split_div_up(seen, n);
+        slots += n * run;
+      }
+      parts += n * run;
       longest = len > longest ? len : longest;
-      if (2 * len > c) { n_long += n; sum_long += steps; }
+      if (2 * len > c) { n_long += n * run; sum_long += seen * run; }
+    };
+    for (int g0 = 0; g0 < G; g0 += 64) {  // a lane's group each, then one after the other from the lanes' registers
+      const int mine = g0 + lane < G ? (t.rows[g0 + lane] + U - 1) / U : 0, in = G - g0 < 64 ? G - g0 : 64;
+      for (int i = 0; i < in; ++i) {
+        const int steps = __builtin_amdgcn_readlane(mine, i);
+        if (steps != seen) {  // (uniform)
+          count();
+          seen = steps;
+          run = 0;
+        }
+        ++run;
+      }
     }
+    count();
     const int64_t tiles = (int64_t)parts * tiles_per_group, rounds_long = ((int64_t)n_long * tiles_per_group + P - 1) / P;
     int64_t expected = n_long > 0 ? rounds_long * sum_long / n_long : 0;
     if (expected < share) expected = share;
@@ -202,8 +234,11 @@ inline SplitRoom split_room(const GemmParams& p) {
 // out to need no cut.  `gain`, in tokens: what a cut has to save for its parts to be written and added up.  With equal groups it saves what the
 // last round of tiles lacks; with groups as a Dirichlet(1) draw deals them the largest has about ln G + 0.6 times the average, and
 // the launch takes as long as that one.  The first alone decides where the launch is short, lest equal groups pay for nothing.
-// 220 random launches (half of them of equal groups), time with a cut offered over without: 16 bits, from 2000 tokens on 0.2-0.9, below 0.7-1.5; FP8,
-// from 4000 on 0.2-0.95, below 0.7-1.2; unequal groups in launches of 6400 (FP8 16000) tokens and more 0.4-1.0, equal ones there up to 1.03.
+// The host does not know the sizes, so what unequal groups gain equal ones pay for.  Time with a cut offered over without, 800 random launches of 1-256
+// groups: unequal ones 0.31 in the mean (16 bits, up to 1.04) and 0.29 (FP8, up to 1.02).  Equal ones 0.47 and 0.38 with up to 64 groups, 0.84 and 0.81 with 24-256; those in
+// which the device finds nothing to cut pay 7 us, 1.01-1.06 in launches of 160 us and more.  Dearer is that what is not cut runs on the four-wave kernel also where the eight-wave
+// one would be the faster: equal groups, 16 bits, few narrow tiles and a gain of 2000-3000 tokens up to 1.24 (108 groups of 80 x 136, 3738 tokens: 83 -> 102 us; unequal ones
+// of that class 0.38-0.53), FP8, up to 256 columns, 1.02-1.17 (34 of 2080 x 96, 6524 tokens: 199 -> 234; unequal ones 0.48).
 inline int64_t split_bytes(const GemmParams& p, int64_t gain, int64_t long_enough) {
   int grid = num_cus();
   if (p.grid_limit > 0 && p.grid_limit < grid) grid = p.grid_limit;
