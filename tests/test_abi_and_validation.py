@@ -203,3 +203,14 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(_native, "LIB_PATH", tmp_path / "libtgg_amd.so")
     with pytest.raises(RuntimeError, match="no non-HIP fallback"):
         _native.load()
+
+
+def test_no_memory_for_a_workspace_is_no_error(monkeypatch):
+    """A K-grouped launch that may be cut along K runs uncut where the allocator has no workspace for it."""
+    args = (16, 768, 768, 131072, False, -1, torch.device("cpu"))
+    assert _native.split_workspace(*args).numel() > 1 << 20
+
+    def full(*_, **__):
+        raise torch.OutOfMemoryError("no memory left")
+    monkeypatch.setattr(torch, "empty", full)
+    assert _native.split_workspace(*args) is None

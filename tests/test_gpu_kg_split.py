@@ -2,6 +2,7 @@
 one another, lengths that do not divide, few workgroups, fp16 and both FP8 formats.  Integer inputs whose sums fp32 holds exactly, so
 that any way of adding them up gives the oracle's bits; then random ones against 64-bit sums."""
 import ctypes
+import gc
 
 import pytest
 import torch
@@ -169,3 +170,42 @@ def test_a_cut_call_can_be_captured():
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("path", ["native", "python", "fp8"])
+def test_a_call_without_memory_for_its_workspace(path):
+    """A launch that may be cut along K wants up to 128 MiB; where the allocator has no more to give it runs uncut, as it did before there was a cut."""
+    dev = torch.device("cuda:0")
+    G, m, n, total = 4, 256, 256, 32768
+    assert _cut(G, m, n, total, path == "fp8") > 100 << 20
+    gen = torch.Generator(device=dev).manual_seed(1)
+    s = torch.tensor([20000, 4768, 8000, 0], dtype=torch.int32, device=dev)
+    if path == "fp8":
+        x, y = (torch.randn(w, total, device=dev, generator=gen).to(torch.float8_e4m3fn) for w in (m, n))
+        xs, ys = (torch.rand(G, w, device=dev, generator=gen).t() for w in (m, n))
+        run = lambda: fp8_k_grouped(x, xs, y, ys, s, m, n, total, G)
+    else:
+        a, b = (torch.randn(total, w, device=dev, generator=gen).bfloat16() for w in (m, n))
+        if path == "python":  # the native call path takes plain tensors only
+            s = torch.stack([s, s], 1)[:, 0]
+        run = lambda: k_grouped_gemm(a, b, s)
+    _native.set_option("kg_split", 0)
+    try:
+        uncut = run()
+    finally:
+        _native.set_option("kg_split", 1)
+    cut = run()
+    assert path == "fp8" or not torch.equal(cut, uncut)  # with room it is summed in another order (the rounding hides that for these FP8 sums)
+    del cut
+    torch.cuda.synchronize()
+    gc.collect()
+    torch.cuda.empty_cache()
+    limit = (torch.cuda.memory_reserved(dev) + (16 << 20)) / torch.cuda.get_device_properties(dev).total_memory
+    torch.cuda.set_per_process_memory_fraction(limit, dev)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(100 << 20, dtype=torch.uint8, device=dev)
+        out = run()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    assert torch.equal(out, uncut)

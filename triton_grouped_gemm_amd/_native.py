@@ -150,10 +150,16 @@ def work_queue(device: torch.device, queue: Optional[torch.Tensor] = None) -> to
 
 
 def split_workspace(groups: int, m: int, n: int, k_total: int, fp8: bool, num_cu: int, device: torch.device) -> Optional[torch.Tensor]:
-    """The workspace of a K-grouped launch that is to be cut along K, None where it is not (include/tgg_amd.h)."""
+    """The workspace of a K-grouped launch that is to be cut along K (include/tgg_amd.h); None where it is not, or where there is no memory
+    for one: the launch then runs uncut, only longer."""
     need = ctypes.c_int64()
     call("tgg_k_grouped_split_bytes", groups, m, n, k_total, int(fp8), num_cu, ctypes.addressof(need))
-    return torch.empty(need.value, dtype=torch.uint8, device=device) if need.value else None
+    if not need.value:
+        return None
+    try:
+        return torch.empty(need.value, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def ptr(t) -> int:

@@ -196,7 +196,13 @@ PyObject* k_grouped_gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     at::Tensor workspace;  // of launches that are cut along K; the allocator keeps it for the stream's next ones
     int64_t bytes = 0;
     rc = tgg_k_grouped_split_bytes((int)g, (int)m, (int)n, kt, 0, (int)num_cu, &bytes);
-    if (bytes > 0) workspace = at::empty({bytes}, a.options().dtype(at::kByte));
+    if (bytes > 0) {
+      try {
+        workspace = at::empty({bytes}, a.options().dtype(at::kByte));
+      } catch (const c10::OutOfMemoryError&) {  // it runs without one as well, only longer
+        bytes = 0;
+      }
+    }
     if (rc == 0)
       rc = tgg_k_grouped_gemm_split(a.data_ptr(), b.data_ptr(), c.data_ptr(), sizes.data_ptr(), is64(sizes), (int)g, (int)m, (int)n, kt, dt,
                                     (int)num_cu, (int32_t*)queue.data_ptr(), bytes > 0 ? workspace.data_ptr() : nullptr, bytes, stream());
