@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from triton_grouped_gemm_amd import _native
+from triton_grouped_gemm_amd.gemm.deep_gemm_ops import m_grouped_bf16_nt_contiguous
 from triton_grouped_gemm_amd.gemm.layout import round_up_to_alignment
 
 pytestmark = pytest.mark.gpu
@@ -22,3 +23,12 @@ def test_padded_total(dtype, block_m, groups):
     _native.call("tgg_padded_total", on_gpu.data_ptr(), int(dtype == torch.int64), groups, block_m, word.data_ptr(), _native.stream_of(on_gpu))
     torch.cuda.synchronize()
     assert word.tolist() == [int(round_up_to_alignment(sizes.to(torch.int32), block_m).sum()), 1]
+
+
+def test_no_groups():
+    """The reference's check comes first: rows where there are no groups for them are a ValueError, small as the call may be."""
+    dev = torch.device("cuda:0")
+    a, b = torch.zeros(128, 64, dtype=torch.bfloat16, device=dev), torch.zeros(0, 128, 64, dtype=torch.bfloat16, device=dev)
+    out = torch.zeros(128, 128, dtype=torch.bfloat16, device=dev)
+    with pytest.raises(ValueError, match="expected M=0, got M=128"):
+        m_grouped_bf16_nt_contiguous(a, b, torch.zeros(0, dtype=torch.int32, device=dev), out=out)

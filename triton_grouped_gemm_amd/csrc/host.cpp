@@ -405,8 +405,10 @@ class PaddedTotal {
   int rc_ = 0;
 };
 
-// Whether a GEMM is over within some 30 us: its products, and the weights of the groups that can have rows.
+// Whether a GEMM is over within some 30 us: its products, and the weights of the groups that can have rows.  (No groups: no sizes to sum either, the
+// total of 0 is the other way's, with its errors.)
 bool brief_gemm(int64_t m, int64_t n, int64_t k, int64_t groups, int64_t block_m, int64_t element_bytes) {
+  if (groups < 1) return false;
   const int64_t used = std::min(groups, (m + block_m - 1) / block_m);
   return 2.0 * m * n * k * element_bytes <= 4e10 && (double)used * n * k * element_bytes <= 1.5e8;
 }
