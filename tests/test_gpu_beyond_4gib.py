@@ -81,9 +81,15 @@ def test_k_grouped_bf16_operand_beyond_4gib(dev):
     b = workloads.randn_bf16((M, Nd), 1.0, 304, dev)
     assert a.numel() * 2 > 1 << 32
     sizes = torch.tensor(SIZES, dtype=torch.int32, device=dev)
-    out, ref = _tuned_and_generic(lambda: k_grouped_gemm(a, b, sizes))
-    assert out.shape == (len(SIZES), Md, Nd) and torch.equal(out, ref)
-    assert torch.count_nonzero(out[1]) == 0
+    cut = k_grouped_gemm(a, b, sizes)  # along K, in parts on both sides of the mark: other sums than the shape-agnostic kernel's, so held against 64 bits only
+    _native.set_option("kg_split", 0)
+    try:
+        out, ref = _tuned_and_generic(lambda: k_grouped_gemm(a, b, sizes))
+    finally:
+        _native.set_option("kg_split", 1)
+    assert out.shape == cut.shape == (len(SIZES), Md, Nd) and torch.equal(out, ref)
+    assert not torch.equal(out, cut)
+    assert torch.count_nonzero(out[1]) == 0 and torch.count_nonzero(cut[1]) == 0
     start = 0
     for g, n in enumerate(SIZES):
         if n:
@@ -91,12 +97,15 @@ def test_k_grouped_bf16_operand_beyond_4gib(dev):
             # covers the fp32 accumulation of that many products
             ref64 = a[start:start + n, :256].double().t() @ b[start:start + n].double()
             assert _half_ulp_ok(out[g, :256], ref64, slack=2e-5), f"group {g}"
+            assert _half_ulp_ok(cut[g, :256], ref64, slack=2e-5), f"group {g}, cut"
+            # the other rows: either result is its 64-bit sum within that bound, so they differ by no more than twice it
+            assert _half_ulp_ok(cut[g], out[g].float(), slack=4e-5 + 2.0 ** -8), f"group {g}, cut"
         start += n
     # the three-token group, wholly beyond the mark, pins which rows went where
     s3 = sum(SIZES[:3])
     assert s3 > MARK
     exact = a[s3:s3 + 3].float().t() @ b[s3:s3 + 3].float()
-    assert _half_ulp_ok(out[3], exact)
+    assert _half_ulp_ok(out[3], exact) and _half_ulp_ok(cut[3], exact)
 
 
 def test_masked_bf16_operand_beyond_4gib(dev):

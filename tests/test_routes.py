@@ -47,3 +47,16 @@ def test_the_rows_of_an_operand_do_not_say_how_many_the_groups_own(trans_b, k, g
 def test_masked_launches_are_decided_on_the_device(k, expected):
     assert route(MASKED, 128, 128 * 512, 4096, k, aux=512) == expected
     assert route(MASKED, 128, 128 * 4096, 4096, k, aux=4096) == expected
+
+
+def _split_bytes(groups, m, n, tokens, fp8):
+    need = ctypes.c_int64(-1)
+    _native.call("tgg_k_grouped_split_bytes", groups, m, n, tokens, int(fp8), -1, ctypes.addressof(need))
+    return need.value
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_the_size_of_the_operands_does_not_decide_whether_segments_are_cut(fp8):
+    """A launch of few outputs is cut along K however many tokens there are, also where an operand has 2^31 values and more."""
+    for tokens in (1 << 17, 1 << 19, 1 << 20, 1 << 21):
+        assert _split_bytes(5, 2048, 256, tokens, fp8) > 0, tokens

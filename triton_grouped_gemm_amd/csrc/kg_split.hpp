@@ -245,8 +245,6 @@ inline int64_t split_bytes(const GemmParams& p, int64_t gain, int64_t long_enoug
   const int64_t tiles = p.G * ((p.m_total + 255) / 256) * ((p.N + 255) / 256), tokens = p.k_total / p.G;
   const SplitRoom room = split_room(p);
   if (room.slots < 2 || tiles > 4 * grid) return 0;
-  // operands beyond 2^31 values keep the one sum a segment whose bits are held against the shape-agnostic kernel's there
-  if (p.k_total * (p.m_total > p.N ? p.m_total : p.N) >= (1ll << 31)) return 0;
   const int64_t rounds = (tiles + grid - 1) / grid, share = tokens * tiles / grid, equal = rounds * tokens - share;
   int log2_g = 0;
   while ((2 << log2_g) <= p.G) ++log2_g;
