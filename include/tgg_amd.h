@@ -84,7 +84,9 @@ int tgg_k_grouped_gemm_sizes(const void* A, const void* B, void* C, const void* 
                              int N, int64_t Ktot, int dtype, int num_cu, int32_t* queue, void* stream);
 
 /* Launches of few outputs over many tokens, cut along K: a segment is computed in parts whose fp32 sums go to a workspace, and a second kernel adds
- * them up in order and rounds once (which parts, the device decides from the sizes: the same sizes give the same bits).  split_bytes: how much
+ * them up in order and rounds once (which parts, the device decides from the sizes and the number of workgroups: the
+ * same sizes on the same GPU with the same num_cu give the same bits; another num_cu, or a call without a workspace, may round otherwise, and the entry points that take
+ * segment bounds sum every segment in one piece).  split_bytes: how much
  * workspace such a launch wants, 0 where cutting does not pay (fp8: 0 for the 16-bit entry point, 1 for the FP8 one).  The _split entry points are
  * tgg_k_grouped_gemm_sizes and tgg_k_grouped_gemm_fp8_channel_queued with that workspace (16-byte aligned, in use until the call's kernels are done;
  * null, or smaller than asked for: as without).  The reference has no counterpart. */

@@ -90,6 +90,28 @@ def test_fp8(fa, fb, m, n, sizes, runs_tuned):
     assert torch.equal(out, fp8_k_grouped(x, xs.t(), y, ys.t(), s, m, n, total, G, 1 if fa == torch.float8_e4m3fn else 2, 1 if fb == torch.float8_e4m3fn else 2))
 
 
+def test_what_the_bits_depend_on():
+    """The sizes and the number of workgroups decide the parts, nothing else; a call with segment bounds has none."""
+    dev = torch.device("cuda:0")
+    a, b = torch.randn(30000, 256, device=dev).bfloat16(), torch.randn(30000, 264, device=dev).bfloat16()
+    s = torch.tensor([17000, 4, 12996], dtype=torch.int32, device=dev)
+    ends = s.cumsum(0).to(torch.int32)
+    runs = {cus: k_grouped_gemm(a, b, s, numSM=cus) for cus in (-1, 64, 100)}
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        again = {cus: k_grouped_gemm(a, b, s.long(), numSM=cus) for cus in runs}
+    torch.cuda.synchronize()
+    assert all(torch.equal(runs[cus], again[cus]) for cus in runs)
+    _native.set_option("kg_split", 0)
+    try:
+        uncut = k_grouped_gemm(a, b, s)
+    finally:
+        _native.set_option("kg_split", 1)
+    assert all(torch.equal(k_grouped_gemm(a, b, s, ends - s, ends, numSM=cus), uncut) for cus in runs)
+    assert all(not torch.equal(r, uncut) for r in runs.values())
+
+
 def _planned_parts(sizes, m, n, unit, tile, part, cost, cus=256):
     """split_plan's choice in Python integers: how many parts each group is cut into."""
     up = lambda a, b: -(-a // b)

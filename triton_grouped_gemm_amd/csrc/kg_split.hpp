@@ -1,7 +1,7 @@
 // K-grouped launches of few tiles and long segments (weight gradients of small outputs over many tokens), cut along K: a segment
 // is computed in parts, each tile of a part by a workgroup of its own, the parts' fp32 sums go to a workspace and a second
 // kernel adds them up in order and rounds once.  How long a part is depends on the sizes, so the device decides (split_plan);
-// the same sizes give the same parts, hence the same bits.
+// the same sizes on as many workgroups give the same parts, hence the same bits.
 #pragma once
 #include "launch.hpp"
 #include "w4_common.hpp"

@@ -49,11 +49,14 @@ def k_grouped_gemm(A: Tensor, B: Tensor, size_per_group: Tensor, group_start: Op
                    group_end: Optional[Tensor] = None, trans_b: bool = False, numSM: int = -1,
                    use_fixed_sm90_config: bool = True, *, queue: Optional[Tensor] = None) -> Tensor:
     """A ``[K_TOTAL, M_DIM]``, B ``[K_TOTAL, N_DIM]`` -> C ``[G, M_DIM, N_DIM]`` (fp32 accumulation over
-    the whole segment, one rounding to the input dtype).
+    the whole segment, one rounding to the input dtype).  With few outputs over many tokens a segment is summed in parts that
+    are added up in fp32 before that rounding; which parts depends on the sizes and on ``numSM``, so the same call gives the
+    same bits and another ``numSM`` may round otherwise.  Calls with ``group_start`` and ``group_end`` sum every segment in one piece.
 
     ``queue`` (not in the reference): the kernel's tile counters, ``_native.QUEUE_WORDS`` zeroed int32 on A's device
-    that the caller owns -- for callers that must not allocate inside the call (graph capture); the kernel hands them
-    back zeroed.  By default the library keeps one such tensor per device and stream."""
+    that the caller owns; the kernel hands them back zeroed.  By default the library keeps one such tensor per device and
+    stream, and a captured call makes one in the graph, with a fill that a caller's own saves.  (The result, and the workspace
+    of a segment summed in parts, are allocated in either case, from the graph's pool under capture.)"""
     if group_start is None and group_end is None and not trans_b and A.is_cuda:
         C = _native.host().k_grouped_gemm(A, B, size_per_group, numSM, _native.work_queue(A.device, queue))
         if C is not None:

@@ -30,8 +30,8 @@ def matmul(x_fp8: Tensor, x_scale: Tensor, y_fp8: Tensor, y_scale: Tensor, token
            M: int, N: int, K: int, num_groups: int, dtype_a: int = 1, dtype_b: int = 1, *,
            queue: Optional[Tensor] = None) -> Tensor:
     """x ``[M, K]``, y ``[N, K]`` fp8 with the token dimension contiguous; dtype codes 1 = e4m3fn,
-    anything else = e5m2 (reference :83-84).  Returns ``[num_groups, M, N]`` bf16.  ``queue`` (not in the
-    reference): caller-owned tile counters, see ``k_grouped_gemm``."""
+    anything else = e5m2 (reference :83-84).  Returns ``[num_groups, M, N]`` bf16; like ``k_grouped_gemm`` it sums
+    a segment in parts where outputs are few.  ``queue`` (not in the reference): caller-owned tile counters, see ``k_grouped_gemm``."""
     assert x_fp8.dim() == 2 and tuple(x_fp8.shape) == (M, K), "x_fp8 must be [M, K]"
     assert y_fp8.dim() == 2 and tuple(y_fp8.shape) == (N, K), "y_fp8 must be [N, K]"
     assert x_fp8.element_size() == 1 and y_fp8.element_size() == 1, "x_fp8 and y_fp8 must hold 8-bit codes"
