@@ -1,82 +1,17 @@
-"""Wait-state hazards around the inline-assembly memory instructions of the HIP kernels.
-
-The compiler inserts the wait states gfx9-family hardware needs between certain instruction pairs, but it does not
-look inside inline assembly.  Three of those pairs involve the hand-written vector-memory instructions of the tuned
-kernels (direct-to-LDS copies, non-temporal stores):
-  * a vector instruction writes a scalar register (v_readlane / v_readfirstlane, e.g. the reload of a spilled scalar)
-    and a vector-memory instruction reads that register fewer than five wait states later: it sees the old value --
-    for a buffer descriptor that means a wild address;
-  * a 12- or 16-byte store is followed within two wait states by a vector instruction that overwrites its data
-    registers: the store writes the new value;
-  * a scalar instruction writes m0 and the very next instruction is a copy to LDS (a buffer load with the lds
-    modifier), which takes its LDS address from m0: one wait state must lie between them.
-The first two were met while developing these kernels (a GPU memory fault, and wrong dwords in the output); the
-third is the rule the compiler applies to its own copies of this kind.  The build keeps
-the device assembly (triton_grouped_gemm_amd/build/*.gfx950.s); this test scans it.  The scanner itself is checked
-on hand-written snippets, so the file tests something even where the library has not been built.
+"""Wait-state hazards around the inline-assembly memory instructions of the HIP kernels, and registers that only their text names
+(triton_grouped_gemm_amd/assembly_checks.py, where the rules are explained).  The build looks its own assembly over and keeps it
+(triton_grouped_gemm_amd/build/*.gfx950.s); these tests scan what was kept, and check the scanners on hand-written
+snippets, so the file tests something even where the library has not been built.
 """
-import re
 from pathlib import Path
 
 import pytest
 
+from triton_grouped_gemm_amd import build
+from triton_grouped_gemm_amd.assembly_checks import (K_GROUPED, accumulator_reads_too_early, compiler_uses_of_named_registers, findings, scan,
+                                                     stray_uses_of_reserved_registers, stray_uses_of_v255, uses_of_reads_in_flight)
+
 BUILD = Path(__file__).resolve().parents[1] / "triton_grouped_gemm_amd" / "build"
-
-
-def _regs(tok: str, kind: str):
-    m = re.match(kind + r"\[(\d+):(\d+)\]$", tok)
-    if m:
-        return set(range(int(m.group(1)), int(m.group(2)) + 1))
-    m = re.match(kind + r"(\d+)$", tok)
-    return {int(m.group(1))} if m else set()
-
-
-def _wait_states(line: str) -> int:
-    m = re.match(r"s_nop (\d+)", line)
-    return int(m.group(1)) + 1 if m else 1
-
-
-def scan(text: str):
-    """Returns a list of (first instruction, second instruction, wait states between them) for every hazard found."""
-    code = []
-    for raw in text.splitlines():
-        line = raw.split(";")[0].strip()
-        if line and not line.startswith(".") and not line.endswith(":"):
-            code.append(line)
-    bad = []
-    for i, line in enumerate(code):
-        op = line.split()[0]
-        toks = [t.strip(",") for t in line.split()[1:]]
-        if not op.startswith(("buffer_", "global_", "flat_", "scratch_")):
-            continue
-        if op.startswith("buffer_load") and toks[-1] == "lds" and i > 0:
-            prev = code[i - 1].split()
-            if prev[0].startswith("s_") and len(prev) > 1 and prev[1].strip(",") == "m0":
-                bad.append((code[i - 1], line, 0))
-        need = set().union(*[_regs(t, "s") for t in toks]) if toks else set()
-        ws = 0
-        for d in range(1, 8):
-            if not need or i - d < 0 or ws >= 5:
-                break
-            prev = code[i - d]
-            ptoks = prev.split()
-            if ptoks[0].startswith("v_") and len(ptoks) > 1 and _regs(ptoks[1].strip(","), "s") & need:
-                bad.append((prev, line, ws))
-                break
-            ws += _wait_states(prev)
-        if re.match(r"(buffer|global|flat|scratch)_store_dwordx[34]", op):
-            data = _regs(toks[0], "v") if op.startswith("buffer") else _regs(toks[1], "v")
-            ws = 0
-            for d in range(1, 4):
-                if i + d >= len(code) or ws >= 2:
-                    break
-                nxt = code[i + d]
-                ntoks = nxt.split()
-                if ntoks[0].startswith("v_") and len(ntoks) > 1 and _regs(ntoks[1].strip(","), "v") & data:
-                    bad.append((line, nxt, ws))
-                    break
-                ws += _wait_states(nxt)
-    return bad
 
 
 def test_scanner_finds_scalar_write_before_vector_memory_read():
@@ -115,33 +50,6 @@ def test_built_kernels_have_no_unspaced_hazard():
         assert not found, f"{f.name}: {len(found)} hazards, first: {found[0]}"
 
 
-# The four-wave kernel keeps operand chunks that are in flight across loop iterations in v[192:255], named in the
-# text of its own load and LDS-write statements; the compiler must never have allocated one of them for itself (it
-# would move or overwrite a value it knows nothing about).
-_RESERVED = set(range(192, 256))
-
-
-def stray_uses_of_reserved_registers(text: str):
-    """Lines of the four-wave kernels that touch v192..v255 other than the staging loads and LDS writes."""
-    stray, inside = [], False
-    for raw in text.splitlines():
-        line = raw.split(";")[0].strip()
-        if line.endswith(":") and not line.startswith("."):
-            inside = "gemm_w4_kernel" in line
-            continue
-        if not inside or not line or line.startswith("."):
-            continue
-        toks = [t.strip(",") for t in line.split()]
-        used = set().union(*[_regs(t, "v") for t in toks[1:]]) & _RESERVED
-        if not used:
-            continue
-        staged_load = toks[0] == "buffer_load_dwordx4" and _regs(toks[1], "v") == used and toks[-1] != "lds"
-        staged_write = toks[0] == "ds_write_b128" and _regs(toks[2], "v") == used
-        if not (staged_load or staged_write):
-            stray.append(line)
-    return stray
-
-
 def test_reserved_register_scanner_on_snippets():
     head = "_ZN3tgg14gemm_w4_kernelILi0ELi0EEEvNS_10GemmParamsE:\n"
     assert stray_uses_of_reserved_registers(head + "buffer_load_dwordx4 v[192:195], v130, s[12:15], s85 offen\n") == []
@@ -160,46 +68,6 @@ def test_four_wave_kernel_keeps_its_reserved_registers_to_itself():
     assert "gemm_w4_kernel" in text
     stray = stray_uses_of_reserved_registers(text)
     assert not stray, f"{len(stray)} compiler-generated uses of v[192:255], first: {stray[0]}"
-
-
-# The four-wave kernel's multiplies are inline assembly, so the compiler does not know when their results land: it
-# places the epilogue's v_accvgpr_read wherever the source order allows.  The source order is written so that a block
-# is read no sooner than three multiplies (48 cycles of issue) after the multiply that wrote it, or behind a
-# statement of idle cycles; this scanner checks the kept assembly for it, in text order (what crosses a loop's back
-# edge is further apart than what it sees).
-_MIN_MULTIPLIES_BETWEEN = 3
-_MIN_IDLE_WAIT_STATES = 12
-
-
-def accumulator_reads_too_early(text: str):
-    """(multiply, read, multiplies in between, idle wait states in between) for every v_accvgpr_read in a four-wave
-    kernel that follows the multiply that wrote its register too closely."""
-    bad, inside = [], False
-    last_write = {}  # accumulator register -> (index of the multiply that wrote it, its text, idle wait states issued so far)
-    n_mul, idle = 0, 0
-    for raw in text.splitlines():
-        line = raw.split(";")[0].strip()
-        if line.endswith(":") and not line.startswith("."):
-            inside = "gemm_w4_kernel" in line
-            last_write, n_mul, idle = {}, 0, 0
-            continue
-        if not inside or not line or line.startswith("."):
-            continue
-        toks = [t.strip(",") for t in line.split()]
-        if toks[0].startswith("v_mfma"):
-            for r in _regs(toks[1], "a"):
-                last_write[r] = (n_mul, line, idle)
-            n_mul += 1
-        elif toks[0] == "s_nop":
-            idle += _wait_states(line)
-        elif toks[0] == "v_accvgpr_read_b32":
-            for r in _regs(toks[2], "a"):
-                if r in last_write:
-                    at, mul, idle_then = last_write[r]
-                    between, waited = n_mul - at - 1, idle - idle_then
-                    if between < _MIN_MULTIPLIES_BETWEEN and waited < _MIN_IDLE_WAIT_STATES:
-                        bad.append((mul, line, between, waited))
-    return bad
 
 
 def test_accumulator_read_scanner_on_snippets():
@@ -221,32 +89,6 @@ def test_four_wave_kernel_reads_no_accumulator_right_behind_its_multiply():
     assert not found, f"{len(found)} reads too close behind the multiply, first: {found[0]}"
 
 
-# The K-grouped four-wave kernels hold a work-queue draw that is in flight across K steps in v255 (KgDraw, w4_common.hpp).
-_K_GROUPED = {"gemm_wgrad": "gemm_wgrad_kernel", "fp8_w4": "fp8_w4_kernel"}  # source file, kernel
-
-
-def _kernel_lines(text: str, kernel: str):
-    inside = False
-    for raw in text.splitlines():
-        line = raw.split(";")[0].strip()
-        if line.endswith(":") and not line.startswith("."):
-            inside = kernel in line
-        elif inside and line and not line.startswith("."):
-            yield line, [t.strip(",") for t in line.split()]
-
-
-def stray_uses_of_v255(text: str, kernel: str):
-    stray = []
-    for line, toks in _kernel_lines(text, kernel):
-        if not any(255 in _regs(t, "v") for t in toks[1:]):
-            continue
-        drawn = toks[0] == "global_atomic_add" and toks[1] == "v255" and toks[-1] == "sc0" and "v255" not in toks[2:]
-        taken = toks[0] == "v_readfirstlane_b32" and toks[2] == "v255"
-        if not (drawn or taken):
-            stray.append(line)
-    return stray
-
-
 def test_v255_scanner_on_snippets():
     head = "_ZN3tgg17gemm_wgrad_kernelILi0EEEvNS_10GemmParamsE:\n"
     found = lambda code, at=head: stray_uses_of_v255(at + code, "gemm_wgrad_kernel")
@@ -255,25 +97,6 @@ def test_v255_scanner_on_snippets():
     assert len(found("ds_read_b128 v[252:255], v3\n")) == 1
     assert len(found("global_atomic_add v255, v255, v2, s[4:5] sc0\n")) == 1
     assert found("v_mov_b32_e32 v255, v3\n", "other_kernel:\n") == []
-
-
-# Their fragment reads are inline assembly as well, and those of fp8_w4.hip are in flight across groups of multiplies and across the
-# slab loop: nothing may touch a register that a read is still to fill.  LDS operations complete in order, so a wait
-# for lgkmcnt(n) leaves the n youngest in flight.
-def uses_of_reads_in_flight(text: str, kernel: str):
-    bad, flight = [], []
-    for line, toks in _kernel_lines(text, kernel):
-        if toks[0] == "s_waitcnt":
-            m = re.search(r"lgkmcnt\((\d+)\)", line)
-            if m:
-                flight = flight[max(0, len(flight) - int(m.group(1))):]
-            continue
-        used = set().union(*[_regs(t, "v") for t in toks[1:]]) if len(toks) > 1 else set()
-        if used & set().union(set(), *flight):
-            bad.append(line)
-        if toks[0].startswith("ds_"):
-            flight.append(_regs(toks[1], "v") if toks[0].startswith("ds_read") else set())
-    return bad
 
 
 def test_reads_in_flight_scanner_on_snippets():
@@ -286,9 +109,9 @@ def test_reads_in_flight_scanner_on_snippets():
     assert found(two + "s_waitcnt vmcnt(3) lgkmcnt(0)\nv_add_u32_e32 v21, v7, v0\n") == []
 
 
-@pytest.mark.parametrize("stem", sorted(_K_GROUPED))
+@pytest.mark.parametrize("stem", sorted(K_GROUPED))
 def test_k_grouped_four_wave_kernels(stem):
-    f, kernel = BUILD / f"{stem}.gfx950.s", _K_GROUPED[stem]
+    f, kernel = BUILD / f"{stem}.gfx950.s", K_GROUPED[stem]
     if not f.exists():
         pytest.skip("no device assembly in the build directory (the library was built elsewhere or not yet)")
     text = f.read_text()
@@ -298,26 +121,6 @@ def test_k_grouped_four_wave_kernels(stem):
                         ("accumulator reads too close behind the multiply", accumulator_reads_too_early(text.replace(kernel, "gemm_w4_kernel")))):
         assert not found, f"{len(found)} {what}, first: {found[0]}"
     assert "scratch_" not in text  # a spilled value would be reloaded behind the copies
-
-
-# The four-wave kernel names its fragments (v[64:191]), staged chunks (v[192:255]) and accumulators (all AGPRs) in the text of its own statements;
-# the compiler, which knows nothing of what they hold, must not use any of them itself.
-def compiler_uses_of_named_registers(text: str):
-    stray, inside, ours = [], False, False
-    for raw in text.splitlines():
-        if "#ASMSTART" in raw or "#ASMEND" in raw:
-            ours = "#ASMSTART" in raw
-            continue
-        line = raw.split(";")[0].strip()
-        if line.endswith(":") and not line.startswith("."):
-            inside = "gemm_w4_kernel" in line
-            continue
-        if not inside or ours or not line or line.startswith("."):
-            continue
-        toks = [t.strip(",") for t in line.split()[1:]]
-        if any(_regs(t, "a") or any(r >= 64 for r in _regs(t, "v")) for t in toks):
-            stray.append(line)
-    return stray
 
 
 def test_named_register_scanner_on_snippets():
@@ -336,3 +139,39 @@ def test_four_wave_kernel_leaves_its_named_registers_alone():
         pytest.skip("no device assembly in the build directory (the library was built elsewhere or not yet)")
     stray = compiler_uses_of_named_registers(f.read_text())
     assert not stray, f"{len(stray)} compiler-generated uses, first: {stray[0]}"
+
+
+def test_the_build_fails_on_what_the_checks_find(monkeypatch, tmp_path):
+    """A library whose assembly breaks a rule is not linked, tests or no tests."""
+    kernel = "_ZN3tgg14gemm_w4_kernelILi0ELi0EEEvNS_10GemmParamsE:\n"
+    csrc, pkg = tmp_path / "csrc", tmp_path / "pkg"
+    csrc.mkdir()
+    pkg.mkdir()
+    (csrc / "gemm_w4.hip").write_text("")
+    monkeypatch.setattr(build, "CSRC", csrc)
+    monkeypatch.setattr(build, "PKG_DIR", pkg)
+    monkeypatch.setattr(build, "LIB_PATH", pkg / "lib.so")
+    monkeypatch.setattr(build, "_compile_host", lambda obj: None)
+    monkeypatch.setattr(build, "_link_host", lambda obj: None)
+    monkeypatch.setattr(build, "_hipcc", lambda: "hipcc")
+    code = {}
+
+    def compiler(cmd):
+        out = Path(cmd[cmd.index("-o") + 1])
+        out.write_text("")
+        if "-c" in cmd:
+            (out.parent / f"gemm_w4-hip-amdgcn-amd-amdhsa-{build.ARCH}.s").write_text(code["text"])
+        return ""
+    monkeypatch.setattr(build, "_run", compiler)
+    code["text"] = kernel + "v_mov_b32_e32 v63, v3\n"
+    assert findings("gemm_w4", code["text"]) == []
+    assert build.build_library() == pkg / "lib.so" and (pkg / "lib.so").exists()
+    (pkg / "lib.so").unlink()
+    for bad in ("v_mov_b32_e32 v64, v3\n", "v_accvgpr_write_b32 a0, v3\n", "s_mov_b32 m0, s2\nbuffer_load_dwordx4 v2, s[44:47], 0 offen lds\n"):
+        code["text"] = kernel + bad
+        with pytest.raises(RuntimeError, match="gemm_w4"):
+            build.build_library()
+        assert not (pkg / "lib.so").exists()
+    code["text"] = "another_kernel:\n"
+    with pytest.raises(RuntimeError, match="no kernel of this name"):
+        build.build_library()

@@ -15,6 +15,8 @@ import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
+from .assembly_checks import findings
+
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "libtgg_amd.so"
@@ -69,8 +71,7 @@ def build_library(verbose: bool = False, jobs: int | None = None) -> Path:
     def compile_one(pair):
         src, obj = pair
         # -save-temps=obj leaves the intermediate files next to the object; only the device assembly is kept
-        # (build/<stem>.gfx950.s): tests/test_isa_hazards.py reads it to check what the compiler cannot check
-        # around the inline-assembly memory instructions.
+        # (build/<stem>.gfx950.s) and looked over for what the compiler cannot check around the inline assembly.
         msg = _run([hipcc, *HIPCC_FLAGS, "-save-temps=obj", "-c", str(src), "-o", str(obj)])
         for tmp in obj_dir.glob(src.stem + "*"):
             if tmp == obj:
@@ -79,6 +80,9 @@ def build_library(verbose: bool = False, jobs: int | None = None) -> Path:
                 os.replace(tmp, obj_dir / f"{src.stem}.{ARCH}.s")
             elif tmp.suffix != ".s" or "-" in tmp.name:
                 tmp.unlink()
+        wrong = findings(src.stem, (obj_dir / f"{src.stem}.{ARCH}.s").read_text())
+        if wrong:
+            raise RuntimeError("the device assembly breaks a rule of assembly_checks.py:\n" + "\n".join(wrong))
         if verbose and msg.strip():
             print(msg, file=sys.stderr)
 

@@ -245,7 +245,7 @@ __global__ __launch_bounds__(Fp8W4Cfg::THREADS) void fp8_w4_kernel(const GemmPar
     i32x4_t v;
     v[0] = (int)x.x; v[1] = (int)x.y; v[2] = (int)y.x; v[3] = (int)y.y;
     const int off = e.off + (16 * i + r) * p.N * 2;
-    // the data registers of a 16-byte store must not be overwritten within two wait states (tests/test_isa_hazards.py)
+    // the data registers of a 16-byte store must not be overwritten within two wait states (assembly_checks.py)
     asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 1" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
   };
   auto epi_flush = [&]() __attribute__((always_inline)) {  // row blocks 4-7 of the workgroup's last tile

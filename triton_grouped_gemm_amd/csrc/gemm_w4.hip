@@ -53,7 +53,7 @@
 //
 // What the compiler does not know about assembly statements, and how it is handled here:
 //   * fragments and accumulators are named in the instruction text and waited for by the K step's wait statement; the compiler's own allocation
-//     is kept below them (amdgpu_num_vgpr; tests/test_isa_hazards.py scans the kept assembly for any other use);
+//     is kept below them (amdgpu_num_vgpr; the build fails where its assembly shows any other use, assembly_checks.py);
 //   * the A chunks are in flight across loop iterations and paths that join: their registers (v[192:255]) are named
 //     in the instruction text too;
 //   * the multiplies write AGPRs: the epilogue's conversions read a block's accumulators no sooner
@@ -297,7 +297,7 @@ __global__ __launch_bounds__(W4Cfg::THREADS) __attribute__((amdgpu_num_vgpr(64))
   // All of them are named in the instruction text: block (i, j)'s accumulators a[32 i + 4 j : + 3], A's fragment i of set s v[64 + 32 s + 4 i : + 3], B's
   // fragment j v[128 + 32 s + 4 j : + 3].  Full and half tiles leave and find different parts of them in use, and where such
   // paths join the compiler moves what it knows of from register to register.  Its own allocation ends below v64 (amdgpu_num_vgpr)
-  // and has no AGPR (they are clobbered at every K step's end; tests/test_isa_hazards.py looks at the kept assembly).
+  // and has no AGPR (they are clobbered at every K step's end; assembly_checks.py looks at the assembly).
   for_each<64>([&](auto Bc) __attribute__((always_inline)) { acc_zero<4 * decltype(Bc)::value>(); });
 
   // read number q (0..15) of the fragments of K step KS of the slab at byte offset `buf_off`, into set SET: B fragments first
@@ -359,7 +359,7 @@ __global__ __launch_bounds__(W4Cfg::THREADS) __attribute__((amdgpu_num_vgpr(64))
     // Two wait states must pass before a 16-byte store's data registers may be overwritten, and the compiler, which
     // considers them free after this statement, reuses them at once: between multiplies the multiply that follows is
     // one wait state (TAIL: a mask may come between them), the flush has none.  No wait states in front: the descriptor sits in scalar registers since the
-    // end of the tile.  Both hazards are checked on the kept assembly (tests/test_isa_hazards.py).
+    // end of the tile.  Both hazards are checked on the kept assembly (assembly_checks.py).
     if (between_multiplies && !TAIL) asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 0" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
     else asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen nt\n\ts_nop 1" : : "v"(v), "v"(off), "s"(pend_rs) : "memory");
   };

@@ -107,7 +107,7 @@ struct KgTiles {
 // Where a four-wave workgroup's tiles of a K-grouped launch come from: the work queue of sched.hpp (largest groups first, one
 // counter per XCD) or, without one, the fixed walk.  Wave 0 draws: request() goes out some K steps before take(), whose
 // caller has waited for it; the answer sits in v255, which is named in the instruction text because a value in
-// flight across K steps must not be known to the compiler (tests/test_isa_hazards.py scans the kept assembly for any other use;
+// flight across K steps must not be known to the compiler (assembly_checks.py scans the assembly for any other use;
 // the kernels' own waits list it as clobbered).  take() leaves the tile id in LDS for the other waves, in front of a
 // barrier.  A counter's value stands for a tile id (sched_queue_id); once it stands for none, the wave looks at all
 // counters at once and goes on with the next one that has tiles left.
