@@ -1,8 +1,11 @@
-"""Shared helpers for the GPU parity tests."""
+"""Shared helpers of the tests."""
+import ctypes
+
 import numpy as np
 import torch
 
 from oracle import gemm_ref
+from triton_grouped_gemm_amd import _native
 
 
 def bf16_ulp_distance(a: torch.Tensor, b: torch.Tensor) -> int:
@@ -54,3 +57,14 @@ def to_np_f32(t: torch.Tensor) -> np.ndarray:
 
 def codes_np(t: torch.Tensor) -> np.ndarray:
     return t.detach().cpu().contiguous().view(torch.uint8).numpy()
+
+
+GENERIC, EIGHT_WAVE, FOUR_WAVE, FOUR_OR_EIGHT, DEEP, WGRAD = range(6)  # tgg_debug_route_16bit
+M_GROUPED, PADDED, MASKED, K_GROUPED = 0, 1, 2, 4
+
+
+def route_16bit(mode, groups, rows, n, k, trans_b=True, aux=0, num_cu=256):
+    """Which kernels a 16-bit launch of these sizes enqueues under the present options (include/tgg_amd.h)."""
+    out = ctypes.c_int32(-1)
+    _native.call("tgg_debug_route_16bit", mode, groups, rows, aux, n, k, int(trans_b), num_cu, ctypes.addressof(out))
+    return out.value

@@ -3,7 +3,7 @@ import pytest
 import torch
 
 from oracle import gemm_ref
-from tests._util import check_16bit_gemm
+from tests._util import FOUR_OR_EIGHT, M_GROUPED, MASKED, check_16bit_gemm, route_16bit
 from triton_grouped_gemm_amd import _native, workloads
 from triton_grouped_gemm_amd.gemm.BF16.k_grouped_gemm_TMA import k_grouped_gemm
 from triton_grouped_gemm_amd.gemm.BF16.m_grouped_gemm_masked_TMA import m_grouped_gemm_masked
@@ -346,7 +346,7 @@ def test_m_grouped_launch_that_both_kernels_look_at(dev, trans_b):
     G, N, K = 96, 1024, 256
     sizes = [(131 * g) % 700 for g in range(G)]
     M = sum(sizes)
-    assert M < 512 * G
+    assert M < 512 * G and route_16bit(M_GROUPED, G, M, N, K, trans_b) == FOUR_OR_EIGHT
     a = _ints((M, K), 51)
     b = _ints((G, N, K) if trans_b else (G, K, N), 52)
     ref = gemm_ref.gmm_fp32(a, b, sizes, trans_b).to(torch.bfloat16)
@@ -374,6 +374,7 @@ def test_masked_launch_that_both_kernels_look_at(dev, counts):
     else:
         masked = [(131 * g) % 513 for g in range(G)]
     masked[5], masked[6] = 0, 512 if counts != "small" else 99
+    assert route_16bit(MASKED, G, G * m_max, N, K, aux=m_max) == FOUR_OR_EIGHT
     lhs = _ints((G * m_max, K), 31)
     rhs = _ints((G, N, K), 32)
     ref = torch.bmm(lhs.float().view(G, m_max, K), rhs.float().transpose(1, 2)).to(torch.bfloat16)

@@ -5,6 +5,7 @@ the plain instantiation, by the default route: alone, and enqueued together with
 import pytest
 import torch
 
+from tests._util import EIGHT_WAVE, FOUR_OR_EIGHT, FOUR_WAVE, M_GROUPED, MASKED, route_16bit
 from triton_grouped_gemm_amd import _native
 from triton_grouped_gemm_amd.gemm.BF16.m_grouped_gemm_masked_TMA import m_grouped_gemm_masked
 from triton_grouped_gemm_amd.gemm.BF16.m_grouped_gemm_TMA import m_grouped_gemm
@@ -73,11 +74,13 @@ def _chosen(sizes, N):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("trans_b, N, K", [(True, 1032, 776), (False, 1032, 768), (False, 1024, 904), (True, 1024, 1024)])
+@pytest.mark.parametrize("trans_b, N, K", [(True, 1032, 776), (False, 1032, 1152), (False, 1024, 904), (True, 1024, 1024)])
 @pytest.mark.parametrize("case, sizes, wide", [
     ("alone", [1500, 2, 1301, 1397], None),                                     # 512 rows a group and more, more than four rounds: the four-wave kernel alone
     ("small groups", [500, 513, 480, 300, 0, 700, 511, 300, 896], True),
     ("small groups", [470] + [40] * 8, False),                                  # groups that fill a fraction of the operand, in 128-row tiles
+    ("small groups", [256] * 16 + [0] * 14, True),                              # 140 rows a group by the operand
+    ("small groups", [100] * 30, False),
     ("few rounds", [330, 255, 180], True),                                      # at most four rounds, of a long K
     ("few rounds", [100, 0, 40], False),                                        # the same operand with few rows: narrow tiles
 ])
@@ -87,6 +90,7 @@ def test_the_default_route(dtype, trans_b, N, K, case, sizes, wide):
     if case == "few rounds":
         rows, K = 768 if N > 1024 else 1024, K + 1024
         assert -(-rows // 256) * -(-N // 128) <= 4 * CUS  # and gemm_w4.hip's likely tiles: 9 / 2 or 11 / 2 rows of them, two rounds of K = 2048
+    assert route_16bit(M_GROUPED, G, rows, N, K, trans_b, num_cu=CUS) == (FOUR_WAVE if wide is None else FOUR_OR_EIGHT)
     if wide is not None:
         assert _chosen(sizes, N) == wide
     gen = torch.Generator(device=dev).manual_seed(K + rows)
@@ -112,6 +116,7 @@ def test_the_default_route_of_masked_launches(dtype, K, masked, wide):
     dev = torch.device("cuda:0")
     N, slots = 1032, 512
     assert _chosen(masked, N) == wide
+    assert route_16bit(MASKED, len(masked), len(masked) * slots, N, K, aux=slots, num_cu=CUS) == (EIGHT_WAVE if K % 128 else FOUR_OR_EIGHT)
     gen = torch.Generator(device=dev).manual_seed(K)
     a = torch.randn(len(masked) * slots, K, device=dev, generator=gen).to(dtype)
     b = (torch.randn(len(masked), N, K, device=dev, generator=gen) * K ** -0.5).to(dtype)
@@ -147,19 +152,21 @@ def test_half_tiles(dtype, num_cu, K, N, trans_b, sizes):
 
 @pytest.mark.parametrize("trans_b", [True, False])
 @pytest.mark.parametrize("N, K, sizes, num_cu", [
-    (512, 768, [1, 1023, 256], 8),        # more than 1.15 rounds of likely tiles, of one group mostly
-    (256, 776, [400, 0, 800], 8),         # a tail, too short for it
-    (264, 1032, [500, 130, 138], 8),      # one that is long enough; N cut as well
+    (512, 768, [1, 1023, 256], 8),        # 1.6 rounds of likely tiles, of one group mostly
+    (256, 776, [400, 0, 800], 8),         # a tail
+    (264, 1032, [500, 130, 138], 8),      # N cut as well
     (256, 768, [400, 3, 797], 8),         # 0.81 of a round
     (256, 896, [256, 767, 1], 8),         # 0.69 of one
-    (256, 768, [512, 0, 1, 511] * 75, -1),  # more groups than threads
+    (256, 768, [512, 0, 1, 511] * 75, -1),  # more groups than the four-wave kernel has threads
 ])
 def test_mid_size_launches(trans_b, N, K, sizes, num_cu):
-    """Launches on both sides of the lines between the four-wave and the eight-wave kernels: the same bits."""
+    """Launches of some size that the four-wave kernel does not get by default, by it and by the eight-wave kernels: the same bits."""
     dev = torch.device("cuda:0")
+    assert route_16bit(M_GROUPED, len(sizes), sum(sizes), N, K, trans_b, num_cu=num_cu) != FOUR_WAVE
     gen = torch.Generator(device=dev).manual_seed(N + K)
     s = torch.tensor(sizes, dtype=torch.int32, device=dev)
     a = torch.randn(sum(sizes), K, device=dev, generator=gen).to(torch.bfloat16)
     b = (torch.randn(len(sizes), *((N, K) if trans_b else (K, N)), device=dev, generator=gen) * K ** -0.5).to(torch.bfloat16)
     run = lambda: _with("deep", 0, 1, lambda: m_grouped_gemm(a, b, s, trans_b, numSM=num_cu))
-    assert torch.equal(run(), _with("force_generic", 1, 0, run))
+    want = _with("force_generic", 1, 0, run)
+    assert torch.equal(run(), want) and torch.equal(_with("four_wave", 2, 1, run), want)

@@ -4,17 +4,8 @@ import ctypes
 
 import pytest
 
+from tests._util import EIGHT_WAVE, FOUR_OR_EIGHT, FOUR_WAVE, M_GROUPED, MASKED, PADDED, route_16bit as route
 from triton_grouped_gemm_amd import _native
-
-GENERIC, EIGHT_WAVE, FOUR_WAVE, FOUR_OR_EIGHT, DEEP, WGRAD = range(6)
-M_GROUPED, PADDED, MASKED, K_GROUPED = 0, 1, 2, 4
-
-
-def route(mode, groups, rows, n, k, trans_b=True, aux=0, num_cu=256):
-    out = ctypes.c_int32(-1)
-    _native.call("tgg_debug_route_16bit", mode, groups, rows, aux, n, k, int(trans_b), num_cu, ctypes.addressof(out))
-    return out.value
-
 
 @pytest.mark.parametrize("trans_b", [True, False])
 @pytest.mark.parametrize("groups", [257, 367, 512])
