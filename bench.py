@@ -63,9 +63,9 @@ MEASURED_TRAFFIC_GB = {
 }
 TRAFFIC_SOURCES = {
     "gemm16": ("common.hpp", "sched.hpp", "fast_common.hpp", "gemm_fast.hip", "gemm_w4.hip", "w4_common.hpp"),
-    "wgrad16": ("common.hpp", "sched.hpp", "fast_common.hpp", "w4_common.hpp", "gemm_wgrad.hip"),
+    "wgrad16": ("common.hpp", "sched.hpp", "fast_common.hpp", "w4_common.hpp", "kg_split.hpp", "gemm_wgrad.hip"),
     "gemm8": ("common.hpp", "sched.hpp", "fast_common.hpp", "gemm_fp8.hip"),
-    "wgrad8": ("common.hpp", "sched.hpp", "fast_common.hpp", "w4_common.hpp", "fp8_w4.hip"),
+    "wgrad8": ("common.hpp", "sched.hpp", "fast_common.hpp", "w4_common.hpp", "kg_split.hpp", "fp8_w4.hip"),
     "quant": ("common.hpp", "sched.hpp", "quant.hip"),
     "permute": ("moe_permute.hip",),
 }

@@ -23,7 +23,7 @@ static std::atomic<int> g_store_nt{1};
 static std::atomic<int> g_n_chunk{0};
 static std::atomic<int> g_kg_second_launch{1};
 static std::atomic<int> g_kg_split{1};
-static std::atomic<int> g_four_wave{1};  // 0 = eight-wave kernels only, 1 = four-wave kernel on large M-grouped NT launches (default), 2 = on every launch it can take
+static std::atomic<int> g_four_wave{1};  // 0 = eight-wave kernels only, 1 = the four-wave kernels where they are the faster ones (default), 2 = on every launch they can take
 
 static std::atomic<int> g_variant{0};  // as given to set_fast_variant and set_fp8_variant
 static std::atomic<int> g_deep{1};  // 0 = never the deep-ring kernel, 1 = on launches of few tiles (default), 2 = on every launch it can take

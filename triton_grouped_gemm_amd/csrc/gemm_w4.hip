@@ -47,9 +47,10 @@
 //
 // Headline shape (G = 128, M = 655360, N = 1536, K = 2048), same box: 3.03 ms against 3.30 ms for the eight-wave
 // kernel; K = 768 shape 1.77 against 1.97 ms; masked decode (G = 128, up to 512 rows per group, N = 4096, K = 1536)
-// 0.51 against 0.56 ms.  Large M-grouped launches take this kernel (w4_supported); masked
-// launches of that size enqueue it together with the eight-wave kernel and the counts decide on the device which of
-// the two runs (GemmParams::wide_gate); everything else goes to the eight-wave kernels.
+// 0.51 against 0.56 ms.  Large M-grouped launches of 512 rows a group and more take this kernel (w4_supported); masked launches of that size, M-grouped
+// ones of smaller groups and those of at most four rounds that are likely to be its enqueue it together with the eight-wave kernel, and the sizes decide on
+// the device which of the two runs (GemmParams::wide_gate).  Launches of few tiles have gone to gemm_deep.hip before this is asked; the rest are
+// the eight-wave kernels'.
 //
 // What the compiler does not know about assembly statements, and how it is handled here:
 //   * fragments and accumulators are named in the instruction text and waited for by the K step's wait statement; the compiler's own allocation
@@ -703,7 +704,7 @@ bool w4_decided_on_device(const GemmParams& p) {
 // The four-wave kernel takes large M-grouped and masked launches, and M-grouped ones of 128 rows and more per group whose likely tiles
 // (every group's last one half full) cost two rounds of K = 2048 or more and would not be chosen for 128-row tiles
 // (sched_wide_tiles_chosen).  Of 574 of those, drawn at random with operands in no cache, 554 were its by their sizes as well and
-// took 0.91 of the eight-wave kernel's time (0.92 with a tail, 0.85-1.01) with the launch that returns in it; 20 were not and lost 4-6 us, 1.03.
+// took 0.91 of the eight-wave kernel's time (0.92 with a tail, 0.85-1.01; before half tiles) with the launch that returns in it; 20 were not and lost 4-6 us, 1.03.
 // Large ones with a tail: 0.93.  32 groups of 1635 rows, N = 1536, K = 3208: 549 -> 487 us; 8 of 1700, N = 3296, K = 1256: 136 -> 123.
 // Smaller launches stay with the eight-wave kernels, which choose narrower tiles on the device.
 bool w4_supported(const GemmParams& p, int dt, int layout, bool any_size) {

@@ -28,7 +28,6 @@ template <int OFF0, int OFF1> TGG_DEV void lds_read_tr(i32x4_t& dst, uint32_t ad
                : "=&v"(lo), "=&v"(hi) : "v"(addr), "n"(OFF0), "n"(OFF1) : "memory");
   dst = __builtin_shufflevector(lo, hi, 0, 1, 2, 3);
 }
-#define TGG_TIE4(f) "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3])
 #define TGG_TIE8(f) "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]), "+v"(f[6]), "+v"(f[7])
 
 // A 16-byte output store of a lane and the wait states behind it (two must pass before the data registers may be overwritten).
