@@ -235,7 +235,7 @@ inline SplitRoom split_room(const GemmParams& p) {
 // last round of tiles lacks; with groups as a Dirichlet(1) draw deals them the largest has about ln G + 0.6 times the average, and
 // the launch takes as long as that one.  The first alone decides where the launch is short, lest equal groups pay for nothing.
 // The host does not know the sizes, so what unequal groups gain equal ones pay for.  Time with a cut offered over without, 800 random launches of 1-256
-// groups: unequal ones 0.31 in the mean (16 bits, up to 1.04) and 0.29 (FP8, up to 1.02).  Equal ones 0.47 and 0.38 with up to 64 groups, 0.84 and 0.81 with 24-256; those in
+// groups: unequal ones 0.35 in the mean (16 bits, up to 1.04) and 0.32 (FP8, up to 1.02).  Equal ones 0.47 and 0.38 with up to 64 groups, 0.84 and 0.81 with 24-256; those in
 // which the device finds nothing to cut pay 7 us, 1.01-1.06 in launches of 160 us and more.  Dearer is that what is not cut runs on the four-wave kernel also where the eight-wave
 // one would be the faster: equal groups, 16 bits, few narrow tiles and a gain of 2000-3000 tokens up to 1.24 (108 groups of 80 x 136, 3738 tokens: 83 -> 102 us; unequal ones
 // of that class 0.38-0.53), FP8, up to 256 columns, 1.02-1.17 (34 of 2080 x 96, 6524 tokens: 199 -> 234; unequal ones 0.48).
